@@ -168,6 +168,13 @@ void build_topology_sah(const float* cen, const float* tbox, int64_t nF, const i
 void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t nQ, float* omega, uint8_t* inside,
                  int32_t* stats, bool device_ptrs);
 void run_bruteforce(Engine& e, const float* Q, int64_t nQ, double* out, bool device_ptrs);
+// The slots-in-lanes traversal (fwn_quad.hip): whether a call goes to it, and its launch over nb
+// batches of kQuadPoints points (metadata as k_traverse's); FP64 near leaves are evaluated in the
+// kernel, flag is set on a stack overflow.
+constexpr int kQuadPoints = 16;
+bool use_quads(const Engine& e, int64_t nQ, int banks);
+void launch_quads(Engine& e, const float* dQ, const uint32_t* perm, const int64_t* q_off, const int64_t* b_off,
+                  const int32_t* order, int M, int64_t nb, float* omega, uint8_t* inside, int32_t* flag, hipStream_t s);
 // Pieces of a query that uses no engine scratch (single-mesh engine, device points): the 32-bit
 // point keys, and the traversal in sorted order `perm` with FP64 near leaves evaluated in place
 // (no work list); meta holds q_off {0, nQ}, b_off {0, batches} and the mesh order {0} (5 int64

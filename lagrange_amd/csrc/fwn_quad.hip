@@ -1,0 +1,307 @@
+// Winding number queries with a node's slots in the lanes of a wave (gfx950): the batched
+// traversal of calls whose points are far apart compared with the mesh's triangles.  Compiled
+// without machine LICM: it would keep the FP64 constants of the near-field evaluation in 40 vector
+// registers through the whole walk (118 registers, 4 waves per SIMD, instead of 68 and 7; 4M
+// uniform points, 199,692 triangles: 1556 -> 1283 us).
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cmath>
+#include <type_traits>
+
+#include "fwn_eval.h"
+#include "fwn_internal.h"
+
+namespace fwn {
+
+namespace {
+
+// Slots-in-lanes traversal of 4-wide trees: 16 points per wave, lane 4 p + s holding point p and
+// taking slot s of every node the wave visits, so that a node's four slots are tested, expanded
+// and (leaves) evaluated in one parallel step.  k_traverse walks 64 points per wave and takes the
+// slots one after the other from scalar registers, which costs less when all 64 lanes have work
+// in the slot; here a wave's points are 4 times closer together, a visit has a quarter of the
+// dependent steps and a call has 4 times the waves.
+//
+// A node is fetched into the LDS buffer of its stack position when it is pushed
+// (global_load_lds), so the wave waits for one fetch on the child popped next and its siblings
+// are there when their turn comes.  The terms of a node reach the point's sum in slot order, as
+// in k_traverse: every lane's pair (a, b), far terms as (t, inv3), near FP32 triangles as
+// (1, value), other slots as (0, 0), goes through om = fmaf(a, b, om) by quad broadcasts (the
+// four lanes of a point hold the same sum).  FP64 near leaves are queued in LDS and evaluated 64
+// at a time, one leaf per lane, their sums added in 2^-40 fixed point (associative) to the
+// point's LDS accumulator.  Results are bit for bit those of k_traverse.
+//
+// Bound: VALU issue (SQ counters, 4M points, F = 199,692: 2,467 VALU instructions per wave of 16
+// uniform points over 38 node visits, 7,733 over 88 visits for points near the surface; 83 and 95 %
+// of the issue slots) once a call has enough waves, the chain of node visits below that.  Whole
+// calls, k_traverse then this kernel: 5,000 uniform points, F = 20,172 443 -> 158 us; 100k points,
+// F = 199,692 673 -> 253 us uniform, 880 -> 330 us near the surface; 4M near 4164 -> 3438 us.
+constexpr int kQuadQueue = 128; // FP64 leaves waiting (at most 63 before a node adds 64)
+constexpr int kQuadNodeBytes = 4 * kSlotWords * 4; // one 4-wide node
+
+template <int S>
+__device__ __forceinline__ float quad_bcast(float v) // lane 4 p + S of each quad
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), S * 0x55, 0xF, 0xF, true));
+}
+// om = fmaf(a_s, b_s, om) for the quad's lanes s = 0..3 in order: the multiplicand of each v_fmac
+// is read through DPP (two instructions a term; the compiler's form takes three)
+__device__ __forceinline__ float quad_terms(float a, float b, float om)
+{
+    float t;
+    asm("s_nop 1\n\t" // a DPP operand is read two wait states after its write at the earliest
+        "v_mov_b32_dpp %1, %3 quad_perm:[0,0,0,0] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %2, %1 quad_perm:[0,0,0,0] row_mask:0xf bank_mask:0xf\n\t"
+        "v_mov_b32_dpp %1, %3 quad_perm:[1,1,1,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %2, %1 quad_perm:[1,1,1,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_mov_b32_dpp %1, %3 quad_perm:[2,2,2,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %2, %1 quad_perm:[2,2,2,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_mov_b32_dpp %1, %3 quad_perm:[3,3,3,3] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %2, %1 quad_perm:[3,3,3,3] row_mask:0xf bank_mask:0xf"
+        : "+v"(om), "=&v"(t)
+        : "v"(a), "v"(b));
+    return om;
+}
+// 64-bit lane masks whose quads are points: s_quadmask_b64 (bit p: any lane of quad p) and its
+// inverse (all four lanes of each point) by two s_bitreplicate_b64_b32; LLVM intrinsics that
+// clang exposes under no builtin name
+extern "C" __device__ uint64_t fwn_llvm_quadmask(uint64_t m) __asm("llvm.amdgcn.s.quadmask.i64");
+extern "C" __device__ uint64_t fwn_llvm_bitreplicate(uint32_t m) __asm("llvm.amdgcn.s.bitreplicate");
+__device__ __forceinline__ uint32_t quad_mask(uint64_t m) { return (uint32_t)fwn_llvm_quadmask(m); }
+__device__ __forceinline__ uint64_t quad_expand(uint32_t m16)
+{
+    return fwn_llvm_bitreplicate((uint32_t)fwn_llvm_bitreplicate(m16));
+}
+
+// LDS: node buffers (lds_nodes of them), the FP64 queue, per point its accumulator and position
+inline size_t quad_lds_bytes(int lds_nodes)
+{
+    return (size_t)lds_nodes * kQuadNodeBytes + kQuadQueue * sizeof(uint2) +
+           kQuadPoints * (sizeof(unsigned long long) + 4 * sizeof(float));
+}
+
+// BUCKET: leaves hold up to 8 triangles (1 otherwise)
+template <bool BUCKET>
+__global__ __launch_bounds__(64) void k_traverse_quad(
+    const uint32_t* __restrict__ slots, const uint32_t* __restrict__ tris, const int32_t* __restrict__ roots,
+    const float* __restrict__ minfo, const float* __restrict__ Q, const uint32_t* __restrict__ perm,
+    const int64_t* __restrict__ q_off, const int64_t* __restrict__ b_off, const int32_t* __restrict__ mesh_order,
+    int M, int64_t n_batches, int lds_nodes, float* __restrict__ omega, uint8_t* __restrict__ inside,
+    int32_t* __restrict__ flag)
+{
+    extern __shared__ uint4 quad_lds[];
+    uint2* queue = reinterpret_cast<uint2*>(reinterpret_cast<char*>(quad_lds) + (size_t)lds_nodes * kQuadNodeBytes);
+    unsigned long long* acc = reinterpret_cast<unsigned long long*>(queue + kQuadQueue);
+    float4* qpos = reinterpret_cast<float4*>(acc + kQuadPoints);
+    constexpr int kNode4 = kQuadNodeBytes / 16; // uint4 per node
+    const int lane = threadIdx.x;
+    const int p = lane >> 2, s = lane & 3;
+    const int64_t batch = xcd_remap(blockIdx.x, gridDim.x);
+    if (batch >= n_batches) return;
+    const int pos = mesh_of64(b_off, M, batch);
+    const int m = mesh_order[pos];
+    const int64_t start = q_off[m] + (batch - b_off[pos]) * kQuadPoints;
+    const int64_t cnt64 = q_off[m + 1] - start;
+    const int cnt = cnt64 < kQuadPoints ? (int)cnt64 : kQuadPoints;
+    const bool valid = p < cnt;
+    const uint32_t jpos = (uint32_t)(start + p);
+    const uint32_t orig = valid ? (perm ? perm[jpos] : jpos) : 0u;
+    const float qx = valid ? Q[3 * (int64_t)orig] : 0.0f;
+    const float qy = valid ? Q[3 * (int64_t)orig + 1] : 0.0f;
+    const float qz = valid ? Q[3 * (int64_t)orig + 2] : 0.0f;
+    const int32_t root = roots[2 * m];
+    const int32_t root_ns = roots[2 * m + 1];
+    const float tau = minfo[8 * m + 6];
+    const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    if (s == 0) {
+        acc[p] = 0ull;
+        qpos[p] = make_float4(qx, qy, qz, 0.0f);
+    }
+
+    float om = 0.0f;
+    int nq = 0; // queued FP64 leaves
+    if (root >= 0) {
+        // stack: entry k in lane k, a node's link and the 16-bit mask of the points that visit it
+        uint32_t st_link = ((uint32_t)root << 4) | (uint32_t)root_ns, st_mask = quad_mask(__ballot(valid));
+        auto fetch = [&](uint32_t lk, int at) __attribute__((always_inline)) {
+            const uint32_t* nb = slots + (size_t)(lk >> 4) * (size_t)(4 * kSlotWords);
+            asm("" : "+s"(nb)); // the node's address stays scalar
+            fetch_node(nb, quad_lds + at * kNode4, 4, lane);
+        };
+        fetch(st_link, 0);
+        int sp = 1;
+        bool overflow = false;
+        for (;;) {
+            if (sp == 0 || nq >= 64) { // 64 queued leaves, or what is left at the end
+                __syncthreads();
+                while (nq >= 64 || (sp == 0 && nq > 0)) {
+                    const int take = min(nq, 64);
+                    nq -= take;
+                    if (lane < take) {
+                        const uint2 it = queue[nq + lane];
+                        const float4 q = qpos[it.y];
+                        const uint32_t first = it.x >> 3, n = (it.x & 7u) + 1u;
+                        double s64 = 0.0;
+                        for (uint32_t t = first; t < first + n; ++t)
+                            s64 += tri_f64(reinterpret_cast<const float*>(tris + (size_t)t * kTriWords), q.x, q.y, q.z);
+                        atomicAdd(&acc[it.y], (unsigned long long)__double2ll_rn(s64 * kFixScale));
+                    }
+                }
+                __syncthreads();
+                if (sp == 0) break;
+            }
+            --sp;
+            const uint32_t e = (uint32_t)__builtin_amdgcn_readlane((int)st_link, sp);
+            const uint32_t m16 = (uint32_t)__builtin_amdgcn_readlane((int)st_mask, sp);
+            uint4 x[kSlotWords / 4];
+            if (sp < lds_nodes) {
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // this node's fetch has landed
+                const uint4* src = quad_lds + sp * kNode4 + s * (kSlotWords / 4);
+#pragma unroll
+                for (int k = 0; k < kSlotWords / 4; ++k) x[k] = src[k];
+            } else { // a stack position without a buffer
+                const uint4* src = reinterpret_cast<const uint4*>(slots + (size_t)(e >> 4) * (size_t)(4 * kSlotWords)) +
+                                   s * (kSlotWords / 4);
+#pragma unroll
+                for (int k = 0; k < kSlotWords / 4; ++k) x[k] = src[k];
+            }
+            // the lanes with a point to test: the points of the mask, the node's occupied slots
+            const uint64_t mk = quad_expand(m16) & __ballot(s < (int)(e & 15u));
+            float w[FWN_W_LINK];
+#pragma unroll
+            for (int k = 0; k < FWN_W_LINK; ++k) w[k] = __uint_as_float(reinterpret_cast<const uint32_t*>(x)[k]);
+            const uint32_t link = x[5].w;
+            const float dx = w[FWN_W_PX] - qx, dy = w[FWN_W_PY] - qy, dz = w[FWN_W_PZ] - qz;
+            const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+            const uint64_t farb = __ballot(d2 > w[FWN_W_THR]);
+            const uint64_t nearm = mk & ~farb;
+            const uint64_t leafm = nearm & __ballot((int32_t)link < 0);
+            // children, in slot order, each fetched as it is pushed: the node's words are in
+            // registers before a fetch overwrites its buffer
+            const uint64_t inner = nearm & ~leafm;
+            if (inner != 0ull) {
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const uint64_t mc = inner & (0x1111111111111111ull << c);
+                    if (mc != 0ull) {
+                        const uint32_t lc = (uint32_t)__builtin_amdgcn_readlane((int)link, c);
+                        st_link = wave_writelane(lc, sp & 63, st_link);
+                        st_mask = wave_writelane(quad_mask(mc), sp & 63, st_mask);
+                        if (sp < lds_nodes) fetch(lc, sp);
+                        ++sp;
+                    }
+                }
+                overflow |= sp > 64; // never with the host's stack bound
+            }
+            float a = 0.0f, b = 0.0f;
+            if (__builtin_amdgcn_inverse_ballot_w64(mk & farb)) far_field_terms(LaneWords{w}, dx, dy, dz, d2, a, b);
+            if (leafm != 0ull) {
+                const bool nl = __builtin_amdgcn_inverse_ballot_w64(leafm);
+                const int32_t first = (int32_t)((link & ~FWN_LINK_LEAF) >> 3);
+                const int32_t tcnt = BUCKET ? (int32_t)(link & 7u) + 1 : 1;
+                bool use64 = false;
+                float v0 = 0.0f;
+                if (nl) { // the whole record in one round trip
+                    const uint4* tp = reinterpret_cast<const uint4*>(tris + (size_t)first * kTriWords);
+                    float tw[kTriWords];
+#pragma unroll
+                    for (int k = 0; k < kTriWords / 4; ++k) {
+                        const uint4 y = tp[k];
+                        tw[4 * k] = __uint_as_float(y.x);
+                        tw[4 * k + 1] = __uint_as_float(y.y);
+                        tw[4 * k + 2] = __uint_as_float(y.z);
+                        tw[4 * k + 3] = __uint_as_float(y.w);
+                    }
+                    const float nd = fmaf(dx, w[FWN_W_NX], fmaf(dy, w[FWN_W_NY], dz * w[FWN_W_NZ]));
+                    use64 = tau > 0.0f && d2 < tw[FWN_T_NEAR2] && (tcnt > 1 || nd * nd < tw[FWN_T_PLANE]);
+                    v0 = tri_f32(tw, qx, qy, qz);
+                    a = use64 ? 0.0f : 1.0f;
+                    b = use64 ? 0.0f : v0;
+                }
+                const uint64_t m64 = __ballot(use64);
+                if (m64 != 0ull) {
+                    if (use64)
+                        queue[nq + (int)__popcll(m64 & lt_mask)] =
+                            make_uint2(((uint32_t)first << 3) | (uint32_t)(tcnt - 1), (uint32_t)p);
+                    nq += (int)__popcll(m64);
+                }
+                if (BUCKET) {
+                    const int n32 = nl && !use64 ? tcnt : 0;
+                    const uint64_t more = __ballot(n32 > 1);
+                    if (more != 0ull) {
+                        // the buckets' other triangles, then every slot's terms in order
+                        float v[8];
+#pragma unroll
+                        for (int k = 1; k < 8; ++k) {
+                            v[k] = 0.0f;
+                            if (k < n32)
+                                v[k] = tri_f32(reinterpret_cast<const float*>(tris + (size_t)(first + k) * kTriWords),
+                                               qx, qy, qz);
+                        }
+                        auto slot_terms = [&](auto c) __attribute__((always_inline)) {
+                            om = fmaf(quad_bcast<c.value>(a), quad_bcast<c.value>(b), om);
+                            if ((more & (0x1111111111111111ull << c.value)) != 0ull) {
+#pragma unroll
+                                for (int k = 1; k < 8; ++k) om += quad_bcast<c.value>(v[k]);
+                            }
+                        };
+                        slot_terms(std::integral_constant<int, 0>{});
+                        slot_terms(std::integral_constant<int, 1>{});
+                        slot_terms(std::integral_constant<int, 2>{});
+                        slot_terms(std::integral_constant<int, 3>{});
+                        continue;
+                    }
+                }
+            }
+            om = quad_terms(a, b, om);
+        }
+        if (overflow && lane == 0) atomicOr(flag, 1);
+    }
+    if (valid && s == 0) {
+        const long long v = (long long)acc[p];
+        if (v != 0) om = (float)((double)om + (double)v * (1.0 / kFixScale));
+        omega[orig] = om;
+        if (inside) inside[orig] = ((double)om / (4.0 * 3.14159265358979323846) > 0.5) ? 1 : 0;
+    }
+}
+
+} // namespace
+
+// Whether a call of nQ points, q_off per mesh, goes to the slots-in-lanes traversal: 4-wide trees
+// of the default launch shape (the other shapes are k_traverse's, chosen by the tuner or the
+// caller), up to kQuadCross * sqrt(F) points for a mesh of F triangles.  The two kernels' costs
+// cross where the 64 points of a k_traverse wave are close together compared with the triangles
+// (uniform points, both kernels in us at 400k / 1.5M / 4M points: F = 972 127 260 557 against 146
+// 428 1032, F = 20,172 279 395 709 against 187 507 1170, F = 199,692 711 698 977 against 260 551
+// 1209, F = 940,800 1016 983 1409 against 288 587 1277), so the line grows with the surface's
+// triangle density along an axis.
+constexpr double kQuadCross = 6300.0;
+bool use_quads(const Engine& e, int64_t nQ, int banks)
+{
+    if (e.width != 4 || banks != 1 || e.opt.launch_mode != FWN_LAUNCH_GRID || e.opt.waves_per_block > 1) return false;
+    double cross = 0.0;
+    for (int m = 0; m < e.n_meshes; ++m) cross += std::sqrt((double)(e.h_f_off[m + 1] - e.h_f_off[m]));
+    return (double)nQ <= kQuadCross * cross;
+}
+
+void launch_quads(Engine& e, const float* dQ, const uint32_t* perm, const int64_t* q_off, const int64_t* b_off,
+                  const int32_t* order, int M, int64_t nb, float* omega, uint8_t* inside, int32_t* flag, hipStream_t s)
+{
+    // node buffers per wave: 20 (9 KB, room for 4 waves per SIMD) while the call has no more waves
+    // than that, else 12 (6 KB: 7 waves per SIMD, the registers' bound too); entries above them are
+    // rare (30k points, F = 199,692: 12 buffers 154 us, 20 147 us; 4M points: 1198 and 1528 us)
+    const int lds_nodes = std::min(nb <= 4096 ? 20 : 12, 1 + 3 * std::max(e.max_depth, 1));
+    const size_t lds = quad_lds_bytes(lds_nodes);
+#define FWN_QUAD(BUCKET)                                                                                            \
+    hipLaunchKernelGGL(k_traverse_quad<BUCKET>, dim3((unsigned)nb), dim3(64), lds, s, e.slots.as<uint32_t>(),      \
+                       e.tris.as<uint32_t>(), e.roots.as<int32_t>(), e.mesh_info.as<float>(), dQ, perm, q_off,     \
+                       b_off, order, M, nb, lds_nodes, omega, inside, flag)
+    if (e.opt.leaf_max > 1) FWN_QUAD(true);
+    else FWN_QUAD(false);
+#undef FWN_QUAD
+    FWN_LAUNCH_CHECK("k_traverse_quad");
+}
+
+} // namespace fwn

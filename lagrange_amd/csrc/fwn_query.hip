@@ -26,6 +26,7 @@
 #include <algorithm>
 #include <cmath>
 
+#include "fwn_eval.h"
 #include "fwn_internal.h"
 
 namespace fwn {
@@ -33,17 +34,6 @@ namespace fwn {
 namespace {
 
 constexpr int QT = 256; // key kernel threads
-
-__device__ __forceinline__ int mesh_of64(const int64_t* off, int M, int64_t t)
-{
-    int lo = 0, hi = M - 1;
-    while (lo < hi) {
-        int mid = (lo + hi + 1) >> 1;
-        if (off[mid] <= t) lo = mid;
-        else hi = mid - 1;
-    }
-    return lo;
-}
 
 // a value equal in every lane of the wave, made visibly uniform (scalar registers)
 __device__ __forceinline__ int64_t wave_uniform64(int64_t v)
@@ -79,52 +69,6 @@ __global__ __launch_bounds__(QT) void k_query_keys(const float* __restrict__ Q, 
     keys[i] = key; // the sort's first pass takes the values to be the positions i
 }
 
-// exact triangle solid angle, FP32, normalised-vector van Oosterom-Strackee form
-__device__ __forceinline__ float tri_f32(const float* __restrict__ t, float qx, float qy, float qz)
-{
-    float ax = t[0] - qx, ay = t[1] - qy, az = t[2] - qz;
-    float bx = t[3] - qx, by = t[4] - qy, bz = t[5] - qz;
-    float cx = t[6] - qx, cy = t[7] - qy, cz = t[8] - qz;
-    float la2 = fmaf(ax, ax, fmaf(ay, ay, az * az));
-    float lb2 = fmaf(bx, bx, fmaf(by, by, bz * bz));
-    float lc2 = fmaf(cx, cx, fmaf(cy, cy, cz * cz));
-    if (la2 == 0.0f || lb2 == 0.0f || lc2 == 0.0f) return 0.0f;
-    float ia = __builtin_amdgcn_rsqf(la2), ib = __builtin_amdgcn_rsqf(lb2), ic = __builtin_amdgcn_rsqf(lc2);
-    ax *= ia; ay *= ia; az *= ia;
-    bx *= ib; by *= ib; bz *= ib;
-    cx *= ic; cy *= ic; cz *= ic;
-    float ux = bx - ax, uy = by - ay, uz = bz - az;
-    float vx = cx - ax, vy = cy - ay, vz = cz - az;
-    float nx = fmaf(uy, vz, -uz * vy);
-    float ny = fmaf(uz, vx, -ux * vz);
-    float nz = fmaf(ux, vy, -uy * vx);
-    float num = fmaf(ax, nx, fmaf(ay, ny, az * nz));
-    if (num == 0.0f) return 0.0f;
-    float ab = fmaf(ax, bx, fmaf(ay, by, az * bz));
-    float ac = fmaf(ax, cx, fmaf(ay, cy, az * cz));
-    float bc = fmaf(bx, cx, fmaf(by, cy, bz * cz));
-    float den = 1.0f + ab + ac + bc;
-    return 2.0f * atan2f(num, den);
-}
-
-// exact triangle solid angle, FP64, 2 atan2(a.(b x c), |a||b||c| + (a.b)|c| + (b.c)|a| + (c.a)|b|)
-__device__ __forceinline__ double tri_f64(const float* __restrict__ t, float qx, float qy, float qz)
-{
-    double q0 = qx, q1 = qy, q2 = qz;
-    double ax = (double)t[0] - q0, ay = (double)t[1] - q1, az = (double)t[2] - q2;
-    double bx = (double)t[3] - q0, by = (double)t[4] - q1, bz = (double)t[5] - q2;
-    double cx = (double)t[6] - q0, cy = (double)t[7] - q1, cz = (double)t[8] - q2;
-    double la = sqrt(ax * ax + ay * ay + az * az);
-    double lb = sqrt(bx * bx + by * by + bz * bz);
-    double lc = sqrt(cx * cx + cy * cy + cz * cz);
-    if (la == 0.0 || lb == 0.0 || lc == 0.0) return 0.0;
-    double num = ax * (by * cz - bz * cy) + ay * (bz * cx - bx * cz) + az * (bx * cy - by * cx);
-    if (num == 0.0) return 0.0;
-    double den = la * lb * lc + (ax * bx + ay * by + az * bz) * lc + (bx * cx + by * cy + bz * cz) * la +
-                 (cx * ax + cy * ay + cz * az) * lb;
-    return 2.0 * atan2(num, den);
-}
-
 // One slot's 24 words held in SGPRs (a 16-dword and an 8-dword scalar load issued together at
 // the top of the slot).  The other waves of the SIMD (8 resident) hide the load latency.
 typedef uint32_t v16u __attribute__((ext_vector_type(16)));
@@ -143,39 +87,6 @@ __device__ __forceinline__ SlotRegs load_slot(const uint32_t* __restrict__ p)
 
 __device__ __forceinline__ uint32_t su(const SlotRegs& r, int k) { return k < 16 ? r.a[k] : r.b[k - 16]; }
 __device__ __forceinline__ float sw(const SlotRegs& r, int k) { return __uint_as_float(su(r, k)); }
-
-// order-2 far field of one slot, split into t and inv3 (the caller adds fmaf(t, inv3, omega)):
-//   omega += inv3 (o0 + inv2 (q1 + inv2 q2)),  inv = 1 / |d|,
-// o0 = d.N, q1 = d^T A d, q2 = B(d, d, d).  The build folds the constant terms (tr M1 of o0 and
-// C.d of q1) into A and B through |d|^2 / |d|^2, so every product has one coefficient operand
-// and no coefficient needs a move into a vector register; q1 and q2 are evaluated in Horner form
-// over the packed coefficients (no monomials needed).  W(k) reads slot word k: scalar registers
-// in the batched traversal, per-lane registers in the single-point kernel (the same operations,
-// so the same bits).
-template <class W>
-__device__ __forceinline__ void far_field_terms(const W& w, float dx, float dy, float dz, float d2, float& t,
-                                                float& inv3)
-{
-    const float inv = __builtin_amdgcn_rsqf(d2);
-    const float inv2 = inv * inv;
-    inv3 = inv2 * inv;
-    const float o0 = fmaf(dx, w(FWN_W_NX), fmaf(dy, w(FWN_W_NY), dz * w(FWN_W_NZ)));
-    const float zz = dz * dz; // shared with the slot test's |d|^2
-    // A: xx yy zz xy yz zx;  q1 = A_zz zz + x (A_xx x + A_xy y + A_zx z) + y (A_yy y + A_yz z)
-    const float a1 = fmaf(w(FWN_W_A), dx, fmaf(w(FWN_W_A + 3), dy, w(FWN_W_A + 5) * dz));
-    const float b1 = fmaf(w(FWN_W_A + 1), dy, w(FWN_W_A + 4) * dz);
-    const float q1 = fmaf(dy, b1, fmaf(dx, a1, w(FWN_W_A + 2) * zz));
-    // B: xxx yyy zzz xxy xxz yyx yyz zzx zzy xyz;
-    // q2 = zz (B_zzx x + B_zzy y + B_zzz z) + x (x (B_xxx x + B_xxy y + B_xxz z) + y (B_yyx y + B_xyz z))
-    //      + y y (B_yyy y + B_yyz z)
-    const float L = fmaf(w(FWN_W_B + 7), dx, fmaf(w(FWN_W_B + 8), dy, w(FWN_W_B + 2) * dz));
-    const float P = fmaf(w(FWN_W_B), dx, fmaf(w(FWN_W_B + 3), dy, w(FWN_W_B + 4) * dz));
-    const float Qv = fmaf(w(FWN_W_B + 5), dy, w(FWN_W_B + 9) * dz);
-    const float X = fmaf(dy, Qv, dx * P);
-    const float R = fmaf(w(FWN_W_B + 1), dy, w(FWN_W_B + 6) * dz);
-    const float q2 = fmaf(dy * dy, R, fmaf(dx, X, zz * L));
-    t = fmaf(inv2, fmaf(inv2, q2, q1), o0);
-}
 
 struct SlotWords {
     const SlotRegs& r;
@@ -467,11 +378,6 @@ __global__ __launch_bounds__(256) void k_bruteforce(const uint32_t* __restrict__
 // fmaf(t, inv3, omega), near FP32 triangles one by one) and the FP64 near leaves in 2^-40 fixed
 // point, so a point gets bit for bit the value a batched call gives it.  Points are read from
 // and results written to pinned host memory.
-struct LaneWords {
-    const float* w;
-    __device__ __forceinline__ float operator()(int k) const { return w[k]; }
-};
-
 __device__ __forceinline__ float readlane_f(float v, int l)
 {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
@@ -483,13 +389,6 @@ constexpr int kPointArgs = 16;
 struct PointArgs {
     float q[kPointArgs][3];
 };
-
-// one node (width x 96 bytes) into LDS: lane l < width * 6 copies 16 bytes
-__device__ __forceinline__ void fetch_node(const uint32_t* __restrict__ nb, uint4* lds, int width, int lane)
-{
-    if (lane < width * (kSlotWords / 4))
-        __builtin_amdgcn_global_load_lds(reinterpret_cast<const uint4*>(nb) + lane, lds, 16, 0, 0);
-}
 
 template <int NB, bool PF>
 __global__ __launch_bounds__(64) void k_point(const uint32_t* __restrict__ slots, int width,
@@ -1349,7 +1248,9 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
     // points per wave: 64, or fewer for small calls so that their waves spread over the device
     // (a point's result does not depend on which points share its wave)
     const bool small = nQ <= kSmallBatch && !stats;
-    const int bpts = small ? (int)std::min<int64_t>(64, std::max<int64_t>(1, (nQ + 1023) / 1024)) : 64;
+    const bool quad = !small && !stats && use_quads(e, nQ, banks);
+    const int bpts = small ? (int)std::min<int64_t>(64, std::max<int64_t>(1, (nQ + 1023) / 1024))
+                           : (quad ? kQuadPoints : 64);
     std::vector<int64_t> boff(M + 1, 0);
     for (int k = 0; k < M; ++k) boff[k + 1] = boff[k] + (qoff[order[k] + 1] - qoff[order[k]] + bpts - 1) / bpts;
     const int64_t nb = boff[M];
@@ -1411,14 +1312,14 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
     if (!e.ev[0])
         for (int k = 0; k < 4; ++k) FWN_HIP(hipEventCreate(&e.ev[k]));
     // per-point FP64 accumulators (sorted positions), kept zero between calls
-    if (e.acc_cap < nQ) {
+    if (!quad && e.acc_cap < nQ) {
         e.q_acc.alloc(sizeof(unsigned long long) * nQ);
         e.acc_cap = nQ;
         hipLaunchKernelGGL(k_fill_u64, dim3(grid_blocks(nQ, 256)), dim3(256), 0, s,
                            e.q_acc.as<unsigned long long>(), nQ);
         FWN_LAUNCH_CHECK("k_fill_u64");
     }
-    if (e.item_cap < std::max<int64_t>(nQ, 1 << 20)) {
+    if (!quad && e.item_cap < std::max<int64_t>(nQ, 1 << 20)) {
         e.item_cap = std::min<int64_t>(std::max<int64_t>(nQ, 1 << 20), (int64_t)UINT32_MAX / 4);
         e.q_items.alloc(sizeof(uint32_t) * 3 * (size_t)e.item_cap);
     }
@@ -1460,19 +1361,24 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
         hipLaunchKernelGGL(k_zero3, dim3(1), dim3(1), 0, s, dflag);
         FWN_HIP(hipEventRecord(e.ev[1], s));
         const uint32_t cap = (uint32_t)e.item_cap;
-        launch_traverse(stats != nullptr, waves, persist, banks, (unsigned)nblk, s, e.slots.as<uint32_t>(), e.width,
-                        e.tris.as<uint32_t>(), e.roots.as<int32_t>(), e.mesh_info.as<float>(), dQ, vp, d_qoff,
-                        d_boff, d_order, M, nb, bpts, beta2, dOm, dIn, dSt, e.q_items.as<uint32_t>(), dnitems, cap,
-                        dflag, dwork);
-        FWN_LAUNCH_CHECK("k_traverse");
-        FWN_HIP(hipEventRecord(e.ev[2], s));
-        const unsigned g64 = small ? 16u : 2048u; // grid-stride loops: any grid size covers every item
-        hipLaunchKernelGGL(k_near64, dim3(g64), dim3(256), 0, s, e.q_items.as<uint32_t>(), dnitems, cap,
-                           e.tris.as<uint32_t>(), dQ, vp, e.q_acc.as<unsigned long long>());
-        FWN_LAUNCH_CHECK("k_near64");
-        hipLaunchKernelGGL(k_near64_combine, dim3(g64), dim3(256), 0, s, e.q_items.as<uint32_t>(), dnitems, cap, vp,
-                           e.q_acc.as<unsigned long long>(), dOm, dIn);
-        FWN_LAUNCH_CHECK("k_near64_combine");
+        if (quad) { // FP64 leaves in the kernel: no work list
+            launch_quads(e, dQ, vp, d_qoff, d_boff, d_order, M, nb, dOm, dIn, dflag, s);
+            FWN_HIP(hipEventRecord(e.ev[2], s));
+        } else {
+            launch_traverse(stats != nullptr, waves, persist, banks, (unsigned)nblk, s, e.slots.as<uint32_t>(),
+                            e.width, e.tris.as<uint32_t>(), e.roots.as<int32_t>(), e.mesh_info.as<float>(), dQ, vp,
+                            d_qoff, d_boff, d_order, M, nb, bpts, beta2, dOm, dIn, dSt, e.q_items.as<uint32_t>(),
+                            dnitems, cap, dflag, dwork);
+            FWN_LAUNCH_CHECK("k_traverse");
+            FWN_HIP(hipEventRecord(e.ev[2], s));
+            const unsigned g64 = small ? 16u : 2048u; // grid-stride loops: any grid size covers every item
+            hipLaunchKernelGGL(k_near64, dim3(g64), dim3(256), 0, s, e.q_items.as<uint32_t>(), dnitems, cap,
+                               e.tris.as<uint32_t>(), dQ, vp, e.q_acc.as<unsigned long long>());
+            FWN_LAUNCH_CHECK("k_near64");
+            hipLaunchKernelGGL(k_near64_combine, dim3(g64), dim3(256), 0, s, e.q_items.as<uint32_t>(), dnitems, cap,
+                               vp, e.q_acc.as<unsigned long long>(), dOm, dIn);
+            FWN_LAUNCH_CHECK("k_near64_combine");
+        }
         FWN_HIP(hipEventRecord(e.ev[3], s));
         int32_t h_fl[2] = {0, 0};
         if (stage_io) { // flags and results in one wait
