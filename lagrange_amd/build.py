@@ -28,6 +28,7 @@ HIP_FLAGS = [
 # VGPRs (the fused MLP's bias/ReLU/BF16 epilogue then reads them without 512 AGPR-to-VGPR moves per
 # tile)
 EXTRA_FLAGS = {
+    "fwn_point.hip": ["-mllvm", "-disable-machine-licm"],
     "fwn_quad.hip": ["-mllvm", "-disable-machine-licm"],
     "fwn_surrogate.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }

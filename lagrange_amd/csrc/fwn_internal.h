@@ -116,6 +116,7 @@ struct Engine {
     // (reused only after the call that filled it has synchronised its stream)
     void* h_stage = nullptr;
     size_t h_stage_bytes = 0;
+    DBuf q_ptflag; // overflow flag of few-point calls
     DBuf q_meta; // device copy of the staged metadata (and small host batches' points)
     std::vector<char> meta_dev; // the metadata bytes q_meta holds (compared before an upload)
     // pipelined host calls: pinned double buffers (points in, results out), a stream per copy
@@ -168,6 +169,16 @@ void build_topology_sah(const float* cen, const float* tbox, int64_t nF, const i
 void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t nQ, float* omega, uint8_t* inside,
                  int32_t* stats, bool device_ptrs);
 void run_bruteforce(Engine& e, const float* Q, int64_t nQ, double* out, bool device_ptrs);
+// pinned staging buffer of at least this many bytes (contents undefined when it grows)
+char* host_stage(Engine& e, size_t bytes);
+// whether the engine has the default launch shape (the others are k_traverse's, chosen by the tuner
+// or the caller)
+inline bool default_shape(const Engine& e)
+{
+    return e.opt.launch_mode == FWN_LAUNCH_GRID && e.opt.waves_per_block <= 1;
+}
+// Calls of few points of a single-mesh engine, one wave per point (fwn_point.hip).
+void run_points(Engine& e, const float* Q, int64_t nQ, float* omega, uint8_t* inside, int banks, bool device_ptrs);
 // The slots-in-lanes traversal (fwn_quad.hip): whether a call goes to it, and its launch over nb
 // batches of kQuadPoints points (metadata as k_traverse's); FP64 near leaves are evaluated in the
 // kernel, flag is set on a stack overflow.

@@ -280,7 +280,7 @@ __global__ __launch_bounds__(64) void k_traverse_quad(
 constexpr double kQuadCross = 6300.0;
 bool use_quads(const Engine& e, int64_t nQ, int banks)
 {
-    if (e.width != 4 || banks != 1 || e.opt.launch_mode != FWN_LAUNCH_GRID || e.opt.waves_per_block > 1) return false;
+    if (e.width != 4 || banks != 1 || !default_shape(e)) return false;
     double cross = 0.0;
     for (int m = 0; m < e.n_meshes; ++m) cross += std::sqrt((double)(e.h_f_off[m + 1] - e.h_f_off[m]));
     return (double)nQ <= kQuadCross * cross;

@@ -27,8 +27,8 @@ def mixed_points(mesh, n, seed):
     return q
 
 
-# 2,049 is the smallest sorted call; 16 k + {0, 1, 15} points end in a full or partial wave
-@pytest.mark.parametrize("n", [2049, 4096, 4111, 30001])
+# 16,385 is the smallest such call of one mesh; 16 k + {0, 1, 15} points end in a full or partial wave
+@pytest.mark.parametrize("n", [16385, 16399, 16400, 30001])
 @pytest.mark.parametrize("leaf", [1, 3, 8])
 @pytest.mark.parametrize("nu,delete", [(1, 0.0), (3, 0.5), (32, 0.0), (64, 0.05)])
 def test_equals_scalar_slot_traversal(n, leaf, nu, delete):
@@ -44,7 +44,7 @@ def test_fp64_queue_wraps():
     # every point has many FP64 leaves (tau of the size of the mesh): the queue fills and drains
     mesh = W.displaced_sphere(12, 3)
     e = FastWindingNumber(mesh, near_fp64_rel=0.3)
-    q = mixed_points(mesh, 3000, 5)
+    q = mixed_points(mesh, 17000, 5)
     a, b = both(e, lambda: e.solid_angle_batch(q))
     assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
