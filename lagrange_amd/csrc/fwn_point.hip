@@ -135,99 +135,87 @@ __device__ __forceinline__ float point_dfs(const uint32_t* __restrict__ slots, i
                 }
             }
         }
-        if (overflow && lane == 0) *flag = 1;
+        if (overflow && lane == 0) { // never with the host's stack bound
+            *flag = 1;
+            __threadfence_system(); // before the mark of a packed result
+        }
     }
     return om;
 }
 
 // Breadth-first single-point walk (calls of a few thousand points; the per-point API).  A depth-first
-// walk is a chain of dependent node loads; here one wave per point takes the tree a level at
-// a time, every slot of up to 64 / width of the level's nodes in its own lane, so the point waits
-// for one load round trip per level step instead of one per node.  Each visited node gets a
-// record in LDS: per slot its kind (far, near internal, near FP32 leaf, near FP64 leaf), the far
-// term's t and inv3, the child's record or the FP32 leaf's triangle values.  FP64 near leaves
-// are evaluated on the way and summed in 2^-40 fixed point (integer addition: any order).
+// walk is a chain of dependent node loads; here one wave per point takes the waiting nodes 64 / W at
+// a time, every slot in its own lane (W = tree width), so the point waits for one load round trip
+// per step (about one per tree level) instead of one per node.  Each visited node gets a record in
+// LDS, in visiting order: its link, its number of FP32 terms and of near children (whose records are
+// consecutive, in slot order), and per slot the pair (a, b) that the term adds as fmaf(a, b, omega)
+// (far terms (t, inv3); a near FP32 triangle (1, value); the values of a larger bucket are kept
+// apart).  FP64 near leaves are evaluated on the way and summed in 2^-40 fixed point (integer
+// addition: any order).
 //
 // The FP32 terms must then be added in the batched traversal's order: a node's own terms in slot
-// order (far terms, then the triangles of near leaves), followed by the subtrees of its near
-// children in reverse slot order (they were pushed in slot order and are popped last first).  So
-// two more level-parallel passes over the records compute, bottom up, every record's number of
-// terms T (kept in its parent's slot entry, beside the other slots' own term counts, so that a
-// pass reads one word per slot) and, top down, where its terms start in that order (a slot's own terms after the
-// node's earlier own terms; a child's subtree after the node's own terms and the subtrees of the
-// children in later slots), writing each term's pair (a, b) to that position of a list.  One
-// chain of fmaf over the list gives the sum: far terms as fmaf(t, inv3, omega) and triangle
-// values as fmaf(1, v, omega) = omega + v (exact product, one rounding), the same operations on
-// the same values as the batched traversal, so a point gets bit for bit the value a batched call
-// gives it.  A walk that needs more than max_rec records, max_tv triangle values or kBfsLevels
+// order, followed by the subtrees of its near children in reverse slot order (they were pushed in
+// slot order and are popped last first).  Two passes over the levels, a lane per record, count each
+// subtree's terms bottom up and hand out the records' places top down; the terms are moved to their
+// places in a list, 64 / W records a step, and one chain of fmaf over the list gives the sum: the
+// same operations on the same values as the batched traversal, so a point gets bit for bit the value
+// a batched call gives it.  A walk that needs more than max_rec records, max_tv bucket values or 63
 // levels is done again by the same wave, depth first (point_dfs, in the same LDS).
 //
-// Points and results: Q and done NULL for points in the kernel arguments; done (host memory): a byte
-// the kernel writes after a point's results, for a few points whose results the host waits for
-// directly; without it the results go to device memory and k_publish follows.
-constexpr uint32_t kRecLeaf64 = 0u, kRecFar = 1u, kRecInner = 2u, kRecLeaf32 = 3u;
-constexpr int kBfsLevels = 63; // level bounds live in the lanes of one register (lane L: first record of level L)
-// slot entry: kind in bits 0-1; a near internal slot: child record << 2; an FP32 leaf:
-// (triangles - 1) << 2 | first value << 5
+// Points: Q, or the kernel arguments (Q NULL).  Results: packed (host memory): one 8-byte store a
+// point with omega, the inside flag and a mark the host waits for; otherwise omega and inside.
+//
+// Bound: latency of one wave's dependent steps for a call of few points (8.8 us of kernel for a random
+// point of 199,692 triangles, 10.3 with slot-wise counting passes and a system fence before a done
+// byte), VALU issue and LDS space for thousands.  Fetching the top three levels into LDS at the start
+// (one round trip instead of three) was measured and not kept: 9.0 us.
 
-// sums over aligned groups of w lanes (w = 2, 4 or 8, all lanes active; ls = lane % w): inclusive
-// prefix and inclusive suffix by DPP row shifts (a group lies inside one 16-lane row, and the
-// lanes a shift brings in from outside the group are masked off)
+// sums over aligned groups of W lanes (2, 4 or 8; all lanes active; ls = lane % W): inclusive prefix
+// by DPP row shifts (a group lies inside one 16-lane row, and the lanes a shift brings in from
+// outside the group are masked off)
 template <int D>
 __device__ __forceinline__ int dpp_shr(int x) { return __builtin_amdgcn_update_dpp(0, x, 0x110 + D, 0xF, 0xF, true); }
-template <int D>
-__device__ __forceinline__ int dpp_shl(int x) { return __builtin_amdgcn_update_dpp(0, x, 0x100 + D, 0xF, 0xF, true); }
-__device__ __forceinline__ int seg_prefix(int x, int ls, int w)
+template <int W>
+__device__ __forceinline__ int seg_prefix(int x, int ls)
 {
     int y = dpp_shr<1>(x);
     x += ls >= 1 ? y : 0;
-    if (w > 2) {
+    if (W > 2) {
         y = dpp_shr<2>(x);
         x += ls >= 2 ? y : 0;
     }
-    if (w > 4) {
+    if (W > 4) {
         y = dpp_shr<4>(x);
         x += ls >= 4 ? y : 0;
     }
     return x;
 }
-__device__ __forceinline__ int seg_suffix(int x, int ls, int w)
-{
-    int y = dpp_shl<1>(x);
-    x += ls + 1 < w ? y : 0;
-    if (w > 2) {
-        y = dpp_shl<2>(x);
-        x += ls + 2 < w ? y : 0;
-    }
-    if (w > 4) {
-        y = dpp_shl<4>(x);
-        x += ls + 4 < w ? y : 0;
-    }
-    return x;
-}
 
-template <int NB>
-__global__ __launch_bounds__(64) void k_point_bfs(const uint32_t* __restrict__ slots, int width,
+// LDS bytes of a record (list places and pairs of its slots, their words, link, info, place, count) and
+// of a bucket value (its place in the list and itself)
+constexpr size_t point_rec_bytes(int W) { return (size_t)W * 20 + 16; }
+constexpr size_t kPointValueBytes = 12;
+
+template <int W, int NB>
+__global__ __launch_bounds__(64) void k_point_bfs(const uint32_t* __restrict__ slots,
                                                   const uint32_t* __restrict__ tris, int32_t root, int32_t root_ns,
                                                   float tau, const float* __restrict__ Q, PointArgs pa, int max_rec,
                                                   int max_tv, int lds_nodes, float* __restrict__ omega,
                                                   uint8_t* __restrict__ inside, int32_t* __restrict__ flag,
-                                                  uint8_t* __restrict__ done)
+                                                  uint64_t* __restrict__ packed)
 {
-    // LDS: the list of term pairs (at most one per slot entry and FP32 value); per record its
-    // node link, its parent's slot entry and its start; per slot entry its kind word (kind 0 for
-    // a node's unused slots), t, inv3 and its term count (own terms; T of the child for a near
-    // internal slot); the FP32 triangle values
-    extern __shared__ float2 terms[];
-    const int nsl = max_rec * width; // slot entries
-    uint32_t* rec_node = reinterpret_cast<uint32_t*>(terms + nsl + max_tv);
-    int* rec_par = reinterpret_cast<int*>(rec_node + max_rec);
-    int* rec_S = rec_par + max_rec;
-    uint32_t* rec_k = reinterpret_cast<uint32_t*>(rec_S + max_rec);
-    float* rec_a = reinterpret_cast<float*>(rec_k + nsl);
-    float* rec_b = rec_a + nsl;
-    int* slot_n = reinterpret_cast<int*>(rec_b + nsl);
-    float* trival = reinterpret_cast<float*>(slot_n + nsl);
+    constexpr int kPer = 64 / W;                     // nodes per step
+    constexpr uint32_t kGroup = (1u << W) - 1u;
+    extern __shared__ uint4 lds[];
+    const int nsl = max_rec * W; // slot entries
+    float2* terms = reinterpret_cast<float2*>(lds);                // the list
+    float2* slot_ab = terms + nsl + max_tv;                        // per slot its pair
+    uint32_t* slot_w = reinterpret_cast<uint32_t*>(slot_ab + nsl); // terms | offset in the record << 4 | value << 12
+    uint32_t* rec_node = slot_w + nsl;
+    uint32_t* rec_info = rec_node + max_rec; // own terms | near children << 8 | first child's record << 16
+    int* rec_S = reinterpret_cast<int*>(rec_info + max_rec);
+    int* rec_T = rec_S + max_rec;
+    float* trival = reinterpret_cast<float*>(rec_T + max_rec);
     const int i = blockIdx.x;
     const int lane = threadIdx.x;
     float qx, qy, qz;
@@ -242,69 +230,57 @@ __global__ __launch_bounds__(64) void k_point_bfs(const uint32_t* __restrict__ s
         qz = pa.q[i][2];
     }
     const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    const int per = 64 / width;       // nodes per step
-    const int ln = lane / width;      // this lane's node within the step
-    const int ls = lane - ln * width; // and slot
+    const int ln = lane / W;      // this lane's node within the step
+    const int ls = lane - ln * W; // and slot
     float om = 0.0f;
     unsigned long long acc_lane = 0ull; // this lane's FP64 near leaves, 2^-40 fixed point
     bool redo = false;
-    int lvl = 0; // lane L: the first record of level L (level L holds records [lvl_L, lvl_L+1))
+    uint32_t lvl = 0u; // lane L: the first record of level L
+    const uint64_t before = (1ull << (ln * W)) - 1ull; // lanes of the step's earlier nodes
     if (root >= 0) {
-        if (lane == 0) {
-            rec_node[0] = ((uint32_t)root << 4) | (uint32_t)root_ns;
-            rec_S[0] = 0;
-            rec_par[0] = -1;
-        }
+        if (lane == 0) rec_node[0] = ((uint32_t)root << 4) | (uint32_t)root_ns;
         __syncthreads();
-        // pass 1: the walk, a level at a time
-        int b = 0, e = 1, nfree = 1, tvfree = 0, nlev = 0;
-        while (b < e) {
-            if (nlev == kBfsLevels) {
-                redo = true;
-                break;
+        int nrec = 1, ntv = 0; // records and bucket values so far
+        int nlev = 0, next = 1; // levels finished, first record of the level after this one
+        for (int c = 0; c < nrec;) {
+            const int took = min(kPer, next - c); // of the level's nodes
+            const int r = c + ln;
+            const bool in_r = ln < took;
+            const uint32_t ne = in_r ? rec_node[r] : 0u;
+            const bool act = in_r && ls < (int)(ne & 15u);
+            uint4 x[kSlotWords / 4];
+            if (act) {
+                const uint4* src =
+                    reinterpret_cast<const uint4*>(slots + ((size_t)(ne >> 4) * (size_t)W + ls) * kSlotWords);
+#pragma unroll
+                for (int k = 0; k < kSlotWords / 4; ++k) x[k] = src[k];
             }
-            for (int c = b; c < e; c += per) {
-                const int r = c + ln;
-                const bool in_r = ln < per && r < e;
-                const uint32_t ne = in_r ? rec_node[r] : 0u;
-                const bool act = in_r && ls < (int)(ne & 15u);
-                float w[FWN_W_LINK];
-                uint32_t link = FWN_LINK_EMPTY;
-                float dx = 0.0f, dy = 0.0f, dz = 0.0f, d2 = 0.0f, t = 0.0f, inv3 = 0.0f;
-                bool far = false;
-                if (act) {
-                    const uint4* src =
-                        reinterpret_cast<const uint4*>(slots + ((size_t)(ne >> 4) * (size_t)width + ls) * kSlotWords);
-                    uint32_t u[kSlotWords];
+            float w[FWN_W_LINK];
 #pragma unroll
-                    for (int k = 0; k < kSlotWords / 4; ++k) {
-                        const uint4 v = src[k];
-                        u[4 * k] = v.x;
-                        u[4 * k + 1] = v.y;
-                        u[4 * k + 2] = v.z;
-                        u[4 * k + 3] = v.w;
-                    }
-#pragma unroll
-                    for (int k = 0; k < FWN_W_LINK; ++k) w[k] = __uint_as_float(u[k]);
-                    link = u[FWN_W_LINK];
-                    dx = w[FWN_W_PX] - qx;
-                    dy = w[FWN_W_PY] - qy;
-                    dz = w[FWN_W_PZ] - qz;
-                    d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-                    far = d2 > w[FWN_W_THR];
-                    far_field_terms(LaneWords{w}, dx, dy, dz, d2, t, inv3);
-                }
-                const bool inner = act && !far && (int32_t)link >= 0;
-                const bool nleaf = act && !far && (int32_t)link < 0;
-                // a near leaf: its first triangle's record (vertices and the FP64 rule's
-                // thresholds) in one round trip
-                int32_t first = 0, tcnt = 0;
-                float tw[kTriWords];
-                bool use64 = false;
+            for (int k = 0; k < FWN_W_LINK; ++k) w[k] = __uint_as_float(reinterpret_cast<const uint32_t*>(x)[k]);
+            const uint32_t link = x[5].w;
+            const float dx = w[FWN_W_PX] - qx, dy = w[FWN_W_PY] - qy, dz = w[FWN_W_PZ] - qz;
+            const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+            const bool far = act && d2 > w[FWN_W_THR];
+            const bool inner = act && !far && (int32_t)link >= 0;
+            const bool nleaf = act && !far && (int32_t)link < 0;
+            float ta = 0.0f, tb = 0.0f;
+            if (far) far_field_terms(LaneWords{w}, dx, dy, dz, d2, ta, tb);
+            // records of the near children, in lane order
+            const uint64_t im = __ballot(inner);
+            const int cnt = __popcll(im);
+            int n = far ? 1 : 0; // FP32 terms of the slot
+            int32_t first = 0;
+            bool use64 = false;
+            float v0 = 0.0f;
+            const uint64_t leafm = __ballot(nleaf);
+            if (leafm != 0ull) {
                 if (nleaf) {
+                    // the first triangle's record (vertices, the FP64 rule's thresholds) in one round trip
                     first = (int32_t)((link & ~FWN_LINK_LEAF) >> 3);
-                    tcnt = (int32_t)(link & 7u) + 1;
+                    const int32_t tcnt = (int32_t)(link & 7u) + 1;
                     const uint4* tp = reinterpret_cast<const uint4*>(tris + (size_t)first * kTriWords);
+                    float tw[kTriWords];
 #pragma unroll
                     for (int k = 0; k < kTriWords / 4; ++k) {
                         const uint4 v = tp[k];
@@ -315,128 +291,133 @@ __global__ __launch_bounds__(64) void k_point_bfs(const uint32_t* __restrict__ s
                     }
                     const float nd = fmaf(dx, w[FWN_W_NX], fmaf(dy, w[FWN_W_NY], dz * w[FWN_W_NZ]));
                     use64 = tau > 0.0f && d2 < tw[FWN_T_NEAR2] && (tcnt > 1 || nd * nd < tw[FWN_T_PLANE]);
+                    if (use64) {
+                        double s64 = tri_f64(tw, qx, qy, qz);
+                        for (int32_t k = 1; k < tcnt; ++k)
+                            s64 += tri_f64(reinterpret_cast<const float*>(tris + (size_t)(first + k) * kTriWords), qx,
+                                           qy, qz);
+                        acc_lane += (unsigned long long)__double2ll_rn(s64 * kFixScale);
+                    } else {
+                        n = tcnt;
+                        v0 = tri_f32(tw, qx, qy, qz);
+                        ta = 1.0f;
+                        tb = v0;
+                    }
                 }
-                const bool use32 = nleaf && !use64;
-                // records of the near children and places for the FP32 values, in lane order
-                const uint64_t im = __ballot(inner);
-                const int cnt = __popcll(im);
-                const int c32 = use32 ? tcnt : 0; // 1..8: four bits
-                int pre = 0, tot = 0;
+            }
+            // the slot's terms within its record
+            const uint64_t big = __ballot(n > 1);
+            int off, own, tv = 0, tot = 0;
+            if (big == 0ull) {
+                const uint32_t g = (uint32_t)(__ballot(n == 1) >> (ln * W)) & kGroup;
+                off = __popc(g & ((1u << ls) - 1u));
+                own = __popc(g);
+            } else { // buckets: their values get places in the value array, in lane order
+                const int incl = seg_prefix<W>(n, ls);
+                off = incl - n;
+                own = __shfl(incl, ln * W + W - 1);
+                const int nb = n > 1 ? n : 0; // 2..8: four bits
 #pragma unroll
                 for (int bit = 0; bit < 4; ++bit) {
-                    const uint64_t bm = __ballot((c32 >> bit) & 1);
-                    pre += __popcll(bm & lt_mask) << bit;
+                    const uint64_t bm = __ballot((nb >> bit) & 1);
+                    tv += __popcll(bm & lt_mask) << bit;
                     tot += __popcll(bm) << bit;
                 }
-                if (nfree + cnt > max_rec || tvfree + tot > max_tv) {
+                tv += ntv;
+            }
+            if (nrec + cnt > max_rec || ntv + tot > max_tv) {
+                redo = true;
+                break;
+            }
+            if (n > 1) {
+                trival[tv] = v0;
+                for (int32_t k = 1; k < n; ++k)
+                    trival[tv + k] = tri_f32(reinterpret_cast<const float*>(tris + (size_t)(first + k) * kTriWords), qx,
+                                             qy, qz);
+            }
+            if (inner) rec_node[nrec + __popcll(im & lt_mask)] = link;
+            if (in_r) {
+                slot_ab[r * W + ls] = make_float2(ta, tb);
+                slot_w[r * W + ls] = (uint32_t)n | ((uint32_t)off << 4) | ((uint32_t)tv << 12);
+                if (ls == 0)
+                    rec_info[r] = (uint32_t)own | ((uint32_t)__popc((uint32_t)(im >> (ln * W)) & kGroup) << 8) |
+                                  ((uint32_t)(nrec + __popcll(im & before)) << 16);
+            }
+            __syncthreads(); // the step's records before the next step reads them
+            nrec += cnt;
+            ntv += tot;
+            c += took;
+            if (c == next) { // the level is done
+                ++nlev;
+                lvl = wave_writelane((uint32_t)c, nlev, lvl);
+                next = nrec;
+                if (nlev == 63 && c < nrec) {
                     redo = true;
                     break;
                 }
-                const int child = nfree + __popcll(im & lt_mask);
-                if (inner) {
-                    rec_node[child] = link;
-                    rec_par[child] = r * width + ls;
-                }
-                if (use32) {
-                    float* tv = trival + tvfree + pre;
-                    tv[0] = tri_f32(tw, qx, qy, qz);
-                    for (int32_t k = 1; k < tcnt; ++k)
-                        tv[k] = tri_f32(reinterpret_cast<const float*>(tris + (size_t)(first + k) * kTriWords), qx, qy, qz);
-                }
-                if (use64) {
-                    double s64 = tri_f64(tw, qx, qy, qz);
-                    for (int32_t k = 1; k < tcnt; ++k)
-                        s64 += tri_f64(reinterpret_cast<const float*>(tris + (size_t)(first + k) * kTriWords), qx, qy, qz);
-                    acc_lane += (unsigned long long)__double2ll_rn(s64 * kFixScale);
-                }
-                if (in_r) {
-                    const int k = r * width + ls;
-                    rec_k[k] = !act ? kRecLeaf64 : far ? kRecFar
-                                   : (inner ? (kRecInner | ((uint32_t)child << 2))
-                                            : (use32 ? (kRecLeaf32 | ((uint32_t)(tcnt - 1) << 2) |
-                                                        ((uint32_t)(tvfree + pre) << 5))
-                                                     : kRecLeaf64));
-                    rec_a[k] = t;
-                    rec_b[k] = inv3;
-                    slot_n[k] = (act && far) ? 1 : (use32 ? (int)tcnt : 0); // internal: set by pass 2
-                }
-                nfree += cnt;
-                tvfree += tot;
             }
-            if (redo) break;
-            ++nlev;
-            if (lane == nlev) lvl = e; // the level just walked is [b, e); the next, [e, nfree)
-            __syncthreads(); // the level's records before the next level reads them
-            b = e;
-            e = nfree;
         }
         if (!redo) {
-            // pass 2, bottom up: T, the terms of a record's subtree, into its parent's slot entry
-            int t_root = 0;
+            // bottom up, a lane per record: the terms T of a record's subtree
             for (int L = nlev - 1; L >= 0; --L) {
                 const int lb = __builtin_amdgcn_readlane(lvl, L), le = __builtin_amdgcn_readlane(lvl, L + 1);
-                for (int c = lb; c < le; c += per) {
-                    const int r = c + ln;
-                    const bool in_r = ln < per && r < le;
-                    int n = 0, par = -1;
-                    if (in_r) {
-                        n = slot_n[r * width + ls];
-                        par = rec_par[r];
-                    }
-                    n = seg_prefix(n, ls, width) + seg_suffix(n, ls, width) - n; // the group's total
-                    if (in_r && ls == 0) {
-                        if (par >= 0) slot_n[par] = n;
-                        else t_root = n;
-                    }
+                for (int r = lb + lane; r < le; r += 64) {
+                    const uint32_t in = rec_info[r];
+                    const int kids = (int)(in >> 8) & 15, f = (int)(in >> 16);
+                    int T = (int)(in & 255u);
+#pragma unroll
+                    for (int k = 0; k < W; ++k) T += k < kids ? rec_T[f + k] : 0;
+                    rec_T[r] = T;
                 }
                 __syncthreads();
             }
-            t_root = __builtin_amdgcn_readfirstlane(t_root); // lane 0 holds the root's record
-            // pass 3, top down: where each record's terms start; each term's location in the list
+            const int nt = rec_T[0]; // at most one term per slot entry and bucket value
+            // top down: where a record's terms start; its children's follow its own, last child first
+            if (lane == 0) rec_S[0] = 0;
             for (int L = 0; L < nlev; ++L) {
                 const int lb = __builtin_amdgcn_readlane(lvl, L), le = __builtin_amdgcn_readlane(lvl, L + 1);
-                for (int c = lb; c < le; c += per) {
-                    const int r = c + ln;
-                    const bool in_r = ln < per && r < le;
-                    const int k = r * width + ls;
-                    uint32_t kk = 0u;
-                    int sr = 0, nk = 0;
-                    float ta = 0.0f, tb = 0.0f;
-                    if (in_r) { // one round trip: every word of the slot and the record's start
-                        kk = rec_k[k];
-                        sr = rec_S[r];
-                        ta = rec_a[k];
-                        tb = rec_b[k];
-                        nk = slot_n[k];
-                    }
-                    const uint32_t kind = kk & 3u;
-                    const int own = kind == kRecInner ? 0 : nk;
-                    const int sub = kind == kRecInner ? nk : 0;
-                    const int own_incl = seg_prefix(own, ls, width);
-                    const int own_all = own_incl + seg_suffix(own, ls, width) - own; // the node's own terms
-                    const int sub_incl = seg_suffix(sub, ls, width);
-                    if (kind == kRecFar) {
-                        terms[sr + own_incl - 1] = make_float2(ta, tb);
-                    } else if (kind == kRecLeaf32) {
-                        const int p0 = sr + own_incl - own;
-                        const float* tv = trival + (kk >> 5);
-                        for (int j = 0; j < own; ++j) terms[p0 + j] = make_float2(1.0f, tv[j]);
-                    } else if (kind == kRecInner) {
-                        rec_S[kk >> 2] = sr + own_all + sub_incl - sub;
-                    }
+                for (int r = lb + lane; r < le; r += 64) {
+                    const uint32_t in = rec_info[r];
+                    const int kids = (int)(in >> 8) & 15, f = (int)(in >> 16);
+                    int S = rec_S[r] + (int)(in & 255u);
+#pragma unroll
+                    for (int k = W - 1; k >= 0; --k)
+                        if (k < kids) {
+                            rec_S[f + k] = S;
+                            S += rec_T[f + k];
+                        }
                 }
                 __syncthreads();
             }
+            // the terms to their places
+            for (int c = 0; c < nrec; c += kPer) {
+                const int r = c + ln;
+                if (r < nrec) {
+                    const uint32_t sw = slot_w[r * W + ls];
+                    const float2 ab = slot_ab[r * W + ls];
+                    const int n = (int)(sw & 15u), p0 = rec_S[r] + (int)((sw >> 4) & 255u);
+                    if (n == 1) {
+                        terms[p0] = ab;
+                    } else if (n > 1) {
+                        const float* tv = trival + (sw >> 12);
+                        for (int j = 0; j < n; ++j) terms[p0 + j] = make_float2(1.0f, tv[j]);
+                    }
+                }
+            }
+            __syncthreads();
             // the sum, in list order: one fmaf per term (every lane runs the chain on broadcast
-            // reads, 16 reads in flight ahead of their fmaf)
-            const int nt = min(t_root, nsl + max_tv); // at most one term per slot entry and value
+            // reads, 16 terms in flight ahead of their fmaf)
+            const float4* two = reinterpret_cast<const float4*>(terms);
             int j = 0;
             for (; j + 16 <= nt; j += 16) {
-                float2 v[16];
+                float4 v[8];
 #pragma unroll
-                for (int u = 0; u < 16; ++u) v[u] = terms[j + u];
+                for (int u = 0; u < 8; ++u) v[u] = two[j / 2 + u];
 #pragma unroll
-                for (int u = 0; u < 16; ++u) om = fmaf(v[u].x, v[u].y, om);
+                for (int u = 0; u < 8; ++u) {
+                    om = fmaf(v[u].x, v[u].y, om);
+                    om = fmaf(v[u].z, v[u].w, om);
+                }
             }
             for (; j < nt; ++j) {
                 const float2 v = terms[j];
@@ -447,8 +428,7 @@ __global__ __launch_bounds__(64) void k_point_bfs(const uint32_t* __restrict__ s
     unsigned long long acc = 0ull;
     if (redo) { // more records than the LDS holds: the same point depth first
         __syncthreads();
-        om = point_dfs<NB>(slots, width, tris, root, root_ns, tau, qx, qy, qz, reinterpret_cast<uint4*>(terms),
-                           lds_nodes, lane, flag, acc);
+        om = point_dfs<NB>(slots, W, tris, root, root_ns, tau, qx, qy, qz, lds, lds_nodes, lane, flag, acc);
     } else { // the wave's FP64 sum
         for (uint64_t m = __ballot(acc_lane != 0ull); m != 0ull; m &= m - 1ull) {
             const int l = (int)__builtin_ctzll(m);
@@ -459,12 +439,14 @@ __global__ __launch_bounds__(64) void k_point_bfs(const uint32_t* __restrict__ s
     }
     const long long v = (long long)acc;
     if (v != 0) om = (float)((double)om + (double)v * (1.0 / kFixScale));
+    const uint32_t in = ((double)om / (4.0 * 3.14159265358979323846) > 0.5) ? 1u : 0u;
     if (lane == 0) {
-        omega[i] = om;
-        if (inside) inside[i] = ((double)om / (4.0 * 3.14159265358979323846) > 0.5) ? 1 : 0;
-        if (done) { // the host waits on this byte: the results and the overflow flag go first
-            __threadfence_system();
-            *(volatile uint8_t*)(done + i) = 1;
+        if (packed) { // omega, the flag and the mark in one store: they arrive together
+            __hip_atomic_store(packed + i, (uint64_t)__float_as_uint(om) | ((uint64_t)(2u | in) << 32),
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        } else {
+            omega[i] = om;
+            if (inside) inside[i] = (uint8_t)in;
         }
     }
 }
@@ -491,12 +473,30 @@ __global__ __launch_bounds__(1024) void k_publish(const uint4* __restrict__ om, 
 
 __global__ void k_clear(int32_t* p) { *p = 0; }
 
-// results of up to this many points go straight to host memory, each wave writing its own and a
-// done byte (three bus writes a point); more are collected in device memory first
+// results of up to this many points go straight to host memory, one 8-byte store each; more are
+// collected in device memory first
 constexpr int64_t kPointDirect = 128;
 // LDS of a k_point_bfs wave: as much as lets all waves of the call be resident, within these bounds
-// (a point's walk takes 108 bytes a visited 4-wide node and 12 an FP32 triangle)
 constexpr size_t kPointLdsMax = 65536, kPointLdsMin = 20480;
+
+template <int W>
+void launch_points(Engine& e, int banks, int64_t nQ, const float* dq, const PointArgs& pa, float* omega,
+                   uint8_t* inside, int32_t* flag, uint64_t* packed, hipStream_t s)
+{
+    const size_t per_cu = (size_t)((nQ + 255) / 256);
+    const size_t lds = std::min(kPointLdsMax, std::max(kPointLdsMin, (size_t)163840 / per_cu & ~(size_t)1023));
+    const int lds_nodes = (int)(lds / ((size_t)W * kSlotWords * 4));
+    const int max_tv = e.opt.leaf_max > 1 ? (int)(lds / 64) : 0;
+    const int max_rec = (int)((lds - max_tv * kPointValueBytes) / point_rec_bytes(W));
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)nQ), dim3(64), lds, s, e.slots.as<uint32_t>(), e.tris.as<uint32_t>(),
+                           e.h_roots[0], e.h_roots[1], e.h_tau[0], dq, pa, max_rec, max_tv, lds_nodes, omega,
+                           inside, flag, packed);
+        FWN_LAUNCH_CHECK("k_point_bfs");
+    };
+    if (banks == 1) go(k_point_bfs<W, 1>);
+    else go(k_point_bfs<W, 3>);
+}
 
 } // namespace
 
@@ -507,25 +507,25 @@ void run_points(Engine& e, const float* Q, int64_t nQ, float* omega, uint8_t* in
     const bool direct = !dev && nQ <= kPointDirect;
     const bool timed = dev || nQ > 2048;
     auto up16 = [](size_t b) { return (b + 15) & ~(size_t)15; };
-    const size_t done_b = up16(direct ? (size_t)nQ : 4);
     const size_t pts_b = dev ? 0 : up16(sizeof(float) * 3 * (size_t)nQ);
-    const size_t om_b = dev ? 0 : up16(sizeof(float) * (size_t)nQ), in_b = dev ? 0 : up16((size_t)nQ);
-    // stage: overflow flag (16 B), done bytes or word, points, omega, inside
+    const size_t om_b = dev || direct ? 0 : up16(sizeof(float) * (size_t)nQ), in_b = dev || direct ? 0 : up16((size_t)nQ);
+    const size_t done_b = direct ? sizeof(uint64_t) * (size_t)kPointDirect : 16;
+    // stage: overflow flag (16 B), packed results or the done word, points, omega, inside
     char* hs = host_stage(e, 16 + done_b + pts_b + om_b + in_b);
     int32_t* hflag = reinterpret_cast<int32_t*>(hs);
-    uint8_t* hdone = reinterpret_cast<uint8_t*>(hs + 16);
+    uint64_t* hdone = reinterpret_cast<uint64_t*>(hs + 16);
     float* hq = reinterpret_cast<float*>(hs + 16 + done_b);
     float* hom = reinterpret_cast<float*>(hs + 16 + done_b + pts_b);
     uint8_t* hin = reinterpret_cast<uint8_t*>(hs + 16 + done_b + pts_b + om_b);
     *hflag = 0;
-    std::memset(hdone, 0, done_b);
+    std::memset(hdone, 0, direct ? sizeof(uint64_t) * (size_t)nQ : 8);
     PointArgs pa;
-    std::memset(&pa, 0, sizeof(pa));
     const float* dq = Q; // device points, points in the pinned stage, or in the arguments (nullptr)
     if (!dev) {
-        dq = nullptr;
         if (nQ <= kPointArgs) {
+            std::memset(&pa, 0, sizeof(pa));
             std::memcpy(pa.q, Q, sizeof(float) * 3 * (size_t)nQ);
+            dq = nullptr;
         } else {
             std::memcpy(hq, Q, sizeof(float) * 3 * (size_t)nQ);
             dq = hq;
@@ -534,10 +534,7 @@ void run_points(Engine& e, const float* Q, int64_t nQ, float* omega, uint8_t* in
     float* dom = omega;
     uint8_t* din = inside;
     int32_t* dflag = hflag;
-    if (direct) {
-        dom = hom;
-        din = hin;
-    } else if (!dev) {
+    if (!dev && !direct) {
         if (!e.q_ptflag.p) { // kept zero between calls
             e.q_ptflag.alloc(sizeof(int32_t));
             hipLaunchKernelGGL(k_clear, dim3(1), dim3(1), 0, s, e.q_ptflag.as<int32_t>());
@@ -554,21 +551,10 @@ void run_points(Engine& e, const float* Q, int64_t nQ, float* omega, uint8_t* in
             for (int k = 0; k < 4; ++k) FWN_HIP(hipEventCreate(&e.ev[k]));
         FWN_HIP(hipEventRecord(e.ev[0], s));
     }
-    const int32_t root = e.h_roots[0], root_ns = e.h_roots[1];
-    const float tau = e.h_tau[0];
-    const size_t per_cu = (size_t)((nQ + 255) / 256);
-    const size_t lds = std::min(kPointLdsMax, std::max(kPointLdsMin, (size_t)163840 / per_cu & ~(size_t)1023));
-    const int max_tv = (int)(lds / 64);
-    const int max_rec = (int)((lds / sizeof(uint32_t) - 3 * (size_t)max_tv) / (size_t)(3 + 6 * e.width));
-    const int lds_nodes = (int)(lds / ((size_t)e.width * kSlotWords * sizeof(uint32_t)));
-#define FWN_POINT(NB)                                                                                               \
-    hipLaunchKernelGGL(k_point_bfs<NB>, dim3((unsigned)nQ), dim3(64), lds, s, e.slots.as<uint32_t>(), e.width,     \
-                       e.tris.as<uint32_t>(), root, root_ns, tau, dq, pa, max_rec, max_tv, lds_nodes, dom, din,    \
-                       dflag, direct ? hdone : nullptr)
-    if (banks == 1) FWN_POINT(1);
-    else FWN_POINT(3);
-#undef FWN_POINT
-    FWN_LAUNCH_CHECK("k_point_bfs");
+    uint64_t* packed = direct ? hdone : nullptr;
+    if (e.width == 4) launch_points<4>(e, banks, nQ, dq, pa, dom, din, dflag, packed, s);
+    else if (e.width == 2) launch_points<2>(e, banks, nQ, dq, pa, dom, din, dflag, packed, s);
+    else launch_points<8>(e, banks, nQ, dq, pa, dom, din, dflag, packed, s);
     if (timed) FWN_HIP(hipEventRecord(e.ev[3], s));
     if (!dev && !direct) {
         hipLaunchKernelGGL(k_publish, dim3(1), dim3(1024), 0, s, e.q_om.as<uint4>(), (int64_t)(om_b / 16),
@@ -576,13 +562,13 @@ void run_points(Engine& e, const float* Q, int64_t nQ, float* omega, uint8_t* in
                            reinterpret_cast<uint4*>(hin), dflag, hflag, reinterpret_cast<uint32_t*>(hdone), 1u);
         FWN_LAUNCH_CHECK("k_publish");
     }
-    // host results are waited for by polling the bytes (or word) written after them: no stream
+    // host results are waited for by polling the marks (or the word) that arrive with them: no stream
     // synchronisation in the round trip.  Every 256 polls the stream is asked whether it has
     // finished, so a failed launch ends the wait.
     if (dev) {
         FWN_HIP(hipStreamSynchronize(s));
     } else {
-        const volatile uint8_t* vd = hdone;
+        const volatile uint64_t* vd = hdone;
         const int64_t n = direct ? nQ : 1;
         bool polled = false;
         int64_t k = 0;
@@ -598,7 +584,13 @@ void run_points(Engine& e, const float* Q, int64_t nQ, float* omega, uint8_t* in
         if (!polled) FWN_HIP(hipStreamSynchronize(s));
     }
     if (*hflag) fail(FWN_LIMIT_EXCEEDED, "traversal stack overflow");
-    if (!dev) {
+    if (direct) {
+        for (int64_t k = 0; k < nQ; ++k) {
+            const uint32_t w = (uint32_t)hdone[k];
+            std::memcpy(omega + k, &w, sizeof(w));
+            if (inside) inside[k] = (uint8_t)((hdone[k] >> 32) & 1u);
+        }
+    } else if (!dev) {
         std::memcpy(omega, hom, sizeof(float) * (size_t)nQ);
         if (inside) std::memcpy(inside, hin, (size_t)nQ);
     }
