@@ -12,14 +12,18 @@
 //   k_karras        binary radix tree over the sorted keys (Karras 2012), ties broken by index
 //   k_find_roots    the node covering exactly one mesh's triangles is that mesh's root
 //   k_leaf_records  sorted triangle records + FP32 per-triangle moments
+//   k_merge_mid, k_merge_top
+//                   SAH trees: moments of subtrees of up to 1,024 triangles, a workgroup each, then
+//                   of the nodes above them; each node merges its two children, FP32 for small
+//                   nodes and FP64 for nodes with >= fp64_moment_min triangles
 //   k_node_depth, k_depth_bucket, k_merge_level
-//                   moments level by level from the deepest internal nodes up: each node merges
-//                   its two children, FP32 for small nodes and FP64 for nodes with
-//                   >= fp64_moment_min triangles (kernel boundaries order the levels)
+//                   Morton trees: the same merges level by level from the deepest internal nodes up
+//                   (kernel boundaries order the levels)
 //   k_bottom_up     the same merges by an arrival-counter walk to the roots, for trees deeper
 //                   than kMaxLevels
 //   k_collapse_*    level by level, each wide node takes the binary node's children and
-//                   repeatedly opens the largest non-leaf slot until it has tree_width slots
+//                   repeatedly opens the largest non-leaf slot until it has tree_width slots (Morton
+//                   trees), or whole binary levels (SAH trees)
 //   k_write_slots   FP64 records -> the 32-word FP32 slot format of fwn.h, plus each slot's box
 //                   (6 floats, rounded outward) for distance queries
 //
@@ -270,6 +274,13 @@ __global__ void k_fill_i32(int32_t* __restrict__ p, int64_t n, int32_t v)
     if (i < n) p[i] = v;
 }
 
+__global__ void k_gather_i32(const int32_t* __restrict__ from, const int32_t* __restrict__ at, int32_t n,
+                             int32_t* __restrict__ to)
+{
+    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) to[i] = from[at[i]];
+}
+
 __global__ __launch_bounds__(BT) void k_find_roots(const int32_t* __restrict__ first, const int32_t* __restrict__ last,
                                                    int64_t n, const uint64_t* __restrict__ keys,
                                                    const int64_t* __restrict__ f_off, int M,
@@ -495,24 +506,92 @@ __global__ __launch_bounds__(BT) void k_merge_level(const int32_t* __restrict__ 
     else merge2<float>(a, b, rec + (int64_t)p * kRecWords);
 }
 
+// ---- moments of an SAH tree ----------------------------------------------------------------------
+// The same merges, a workgroup per mid segment (a subtree of at most kSahMid triangles over
+// neighbouring positions, its nodes' ids in [lo, hi - 2]), then one workgroup for the nodes above
+// them: threads climb from the leaves (the subtrees' roots) and the second child to arrive at a node
+// merges it.  Arrivals and records stay within a workgroup, so block-scope fences order them: two
+// launches where the levels took one each and a host round trip for their sizes.  Bound: the 768
+// bytes of records a merge reads and writes (101,568 triangles: 0.12 + 0.04 ms; 22 launches and the
+// wait before 0.25 ms; 256 threads a workgroup instead of 512: 0.17 ms for the first).
+constexpr int kMergeThreads = 512;
+__global__ __launch_bounds__(kMergeThreads) void k_merge_mid(const int32_t* __restrict__ seg, const int32_t* __restrict__ left,
+                                                  const int32_t* __restrict__ right, const int32_t* __restrict__ parent,
+                                                  const int32_t* __restrict__ first, const int32_t* __restrict__ last,
+                                                  int64_t n, int32_t fp64_min, double* rec,
+                                                  int32_t* __restrict__ seg_root, int32_t* __restrict__ visits)
+{
+    __shared__ int32_t cnt[kSahMid];
+    const int32_t lo = seg[4 * (int64_t)blockIdx.x], hi = seg[4 * (int64_t)blockIdx.x + 1];
+    for (int k = threadIdx.x; k < hi - lo; k += kMergeThreads) cnt[k] = 0;
+    if (threadIdx.x == 0) { // the nodes above the subtrees are the splits between them
+        if (lo > 0) visits[lo - 1] = 0;
+        visits[hi - 1] = 0;
+    }
+    __syncthreads();
+    for (int32_t j = lo + (int32_t)threadIdx.x; j < hi; j += kMergeThreads) {
+        int32_t u = (int32_t)(n - 1) + j;
+        for (;;) {
+            const int32_t p = parent[u];
+            if (p < lo || p > hi - 2) { // the subtree's root
+                seg_root[blockIdx.x] = u;
+                break;
+            }
+            __threadfence_block();
+            if (atomicAdd(&cnt[p - lo], 1) == 0) break; // the sibling's thread finishes this node
+            __threadfence_block();
+            const double* a = rec + (int64_t)left[p] * kRecWords;
+            const double* b = rec + (int64_t)right[p] * kRecWords;
+            if (last[p] - first[p] + 1 >= fp64_min) merge2<double>(a, b, rec + (int64_t)p * kRecWords);
+            else merge2<float>(a, b, rec + (int64_t)p * kRecWords);
+            u = p;
+        }
+    }
+}
+
+constexpr int kTopThreads = 1024;
+__global__ __launch_bounds__(kTopThreads) void k_merge_top(const int32_t* __restrict__ seg_root, int64_t n_seg,
+                                                           const int32_t* __restrict__ left,
+                                                           const int32_t* __restrict__ right,
+                                                           const int32_t* __restrict__ parent,
+                                                           const int32_t* __restrict__ first,
+                                                           const int32_t* __restrict__ last, int32_t fp64_min,
+                                                           double* rec, int32_t* visits)
+{
+    for (int64_t k = threadIdx.x; k < n_seg; k += kTopThreads) {
+        int32_t u = seg_root[k];
+        for (;;) {
+            const int32_t p = parent[u];
+            if (p < 0) break;
+            __threadfence_block();
+            if (atomicAdd(&visits[p], 1) == 0) break;
+            __threadfence_block();
+            const double* a = rec + (int64_t)left[p] * kRecWords;
+            const double* b = rec + (int64_t)right[p] * kRecWords;
+            if (last[p] - first[p] + 1 >= fp64_min) merge2<double>(a, b, rec + (int64_t)p * kRecWords);
+            else merge2<float>(a, b, rec + (int64_t)p * kRecWords);
+            u = p;
+        }
+    }
+}
+
 // ---- collapse into wide nodes -----------------------------------------------------------------
 __device__ __forceinline__ int32_t node_count(int32_t u, int64_t n, const int32_t* first, const int32_t* last)
 {
     return (u >= n - 1) ? 1 : last[u] - first[u] + 1;
 }
 
-__global__ __launch_bounds__(BT) void k_collapse_level(const int32_t* __restrict__ level_bin, int32_t cnt,
-                                                       int32_t gbase, const int32_t* __restrict__ left,
-                                                       const int32_t* __restrict__ right,
-                                                       const int32_t* __restrict__ first,
-                                                       const int32_t* __restrict__ last, int64_t n, int leaf_max,
-                                                       int width, int rounds, int32_t* __restrict__ wide_slot_bin,
-                                                       int32_t* __restrict__ wide_ns, int32_t* __restrict__ newcount)
+struct BinTree {
+    const int32_t *left, *right, *first, *last;
+    int64_t n;
+};
+
+// the slots of binary node b's wide node: binary nodes sl[], their triangle counts sc[]; returns how many
+__device__ __forceinline__ int wide_slots(int32_t b, const BinTree& t, int leaf_max, int width, int rounds,
+                                          int32_t (&sl)[kWidth], int32_t (&sc)[kWidth])
 {
-    int i = blockIdx.x * BT + threadIdx.x;
-    if (i >= cnt) return;
-    int32_t b = level_bin[i];
-    int32_t sl[kWidth], sc[kWidth];
+    const int32_t *left = t.left, *right = t.right, *first = t.first, *last = t.last;
+    const int64_t n = t.n;
     int ns;
     if (b >= n - 1 || node_count(b, n, first, last) <= leaf_max) {
         sl[0] = b;
@@ -570,38 +649,130 @@ __global__ __launch_bounds__(BT) void k_collapse_level(const int32_t* __restrict
             ++ns;
         }
     }
-    int g = gbase + i;
-    int nc = 0;
-    for (int s = 0; s < kWidth; ++s) {
-        wide_slot_bin[(int64_t)g * kWidth + s] = (s < ns) ? sl[s] : -1;
-        if (s < ns && sc[s] > leaf_max) ++nc;
-    }
-    wide_ns[g] = ns;
-    newcount[i] = nc;
+    return ns;
 }
 
-__global__ __launch_bounds__(BT) void k_collapse_assign(int32_t cnt, int32_t gbase, int32_t next_base,
-                                                        const int32_t* __restrict__ wide_slot_bin,
-                                                        const int32_t* __restrict__ first,
-                                                        const int32_t* __restrict__ last, int64_t n, int leaf_max,
-                                                        const int32_t* __restrict__ offs,
-                                                        int32_t* __restrict__ child_wide,
-                                                        int32_t* __restrict__ level_next)
+// Wide nodes are numbered level by level, each level in slot order.  The level in work is a list of
+// binary nodes; its state (nodes, number of the first one, levels done, list array) stays on the
+// device, one entry per level, so that the host enqueues as many levels as it expects and reads the
+// state once.  k_collapse_top takes the levels of up to 1,024 nodes in one workgroup; a larger level
+// takes two launches: slots and block sums of new nodes, then the numbers of the children (every
+// block adds up the sums of the blocks before it).
+struct LevelState {
+    int32_t cnt, base, depth, cur;
+};
+struct Wide {
+    int32_t *slot_bin, *child; // width entries per wide node
+    int32_t* ns;
+    int32_t* lvl[2];
+};
+
+// exclusive scan over a workgroup of T threads (T / 64 waves); total of all
+template <int T>
+__device__ __forceinline__ int block_scan(int v, int32_t* part, int& total)
 {
-    int i = blockIdx.x * BT + threadIdx.x;
-    if (i >= cnt) return;
-    int g = gbase + i;
-    int k = offs[i];
-    for (int s = 0; s < kWidth; ++s) {
-        int32_t u = wide_slot_bin[(int64_t)g * kWidth + s];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int x = v;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(x, o);
+        if (lane >= o) x += y;
+    }
+    if (lane == 63) part[w] = x;
+    __syncthreads();
+    int before = 0;
+    total = 0;
+    for (int k = 0; k < T / 64; ++k) {
+        if (k < w) before += part[k];
+        total += part[k];
+    }
+    __syncthreads();
+    return before + x - v;
+}
+
+// writes wide node g's children numbers (from `next` on) and the next level's list
+__device__ __forceinline__ void link_children(const Wide& w, int64_t g, int width, int leaf_max, const BinTree& t,
+                                              int32_t next_base, int k, int32_t* __restrict__ level_next)
+{
+    for (int s = 0; s < width; ++s) {
+        const int32_t u = w.slot_bin[g * width + s];
         int32_t cw = -1;
-        if (u >= 0 && node_count(u, n, first, last) > leaf_max) {
+        if (u >= 0 && node_count(u, t.n, t.first, t.last) > leaf_max) {
             cw = next_base + k;
             level_next[k] = u;
             ++k;
         }
-        child_wide[(int64_t)g * kWidth + s] = cw;
+        w.child[g * width + s] = cw;
     }
+}
+
+// writes wide node g's slots; returns its number of children
+__device__ __forceinline__ int put_slots(const Wide& w, int64_t g, int32_t b, const BinTree& t, int leaf_max, int width,
+                                         int rounds)
+{
+    int32_t sl[kWidth], sc[kWidth];
+    const int ns = b < 0 ? 0 : wide_slots(b, t, leaf_max, width, rounds, sl, sc); // b < 0: no root was found
+    int nc = 0;
+    for (int s = 0; s < width; ++s) {
+        w.slot_bin[g * width + s] = (s < ns) ? sl[s] : -1;
+        if (s < ns && sc[s] > leaf_max) ++nc;
+    }
+    w.ns[g] = ns;
+    return nc;
+}
+
+constexpr int kTopNodes = 1024;
+__global__ __launch_bounds__(kTopNodes) void k_collapse_top(Wide w, BinTree t, int32_t cnt, int leaf_max, int width,
+                                                            int rounds, LevelState* __restrict__ state)
+{
+    __shared__ int32_t part[kTopNodes / 64];
+    LevelState st{cnt, 0, 0, 0};
+    while (st.cnt > 0 && st.cnt <= kTopNodes) { // uniform
+        const int i = threadIdx.x;
+        const bool live = i < st.cnt;
+        const int nc = live ? put_slots(w, st.base + i, w.lvl[st.cur][i], t, leaf_max, width, rounds) : 0;
+        int total;
+        const int k = block_scan<kTopNodes>(nc, part, total);
+        if (live) link_children(w, st.base + i, width, leaf_max, t, st.base + st.cnt, k, w.lvl[st.cur ^ 1]);
+        __syncthreads(); // the next level's list
+        st = LevelState{total, st.base + st.cnt, st.depth + 1, st.cur ^ 1};
+    }
+    if (threadIdx.x == 0) state[0] = st;
+}
+
+__global__ __launch_bounds__(BT) void k_collapse_slots(Wide w, BinTree t, int leaf_max, int width, int rounds,
+                                                       const LevelState* __restrict__ state,
+                                                       int32_t* __restrict__ newcount, int32_t* __restrict__ sums)
+{
+    __shared__ int32_t part[BT / 64];
+    const LevelState st = *state;
+    if ((int64_t)blockIdx.x * BT >= st.cnt) return;
+    const int i = blockIdx.x * BT + threadIdx.x;
+    const int nc = i < st.cnt ? put_slots(w, st.base + i, w.lvl[st.cur][i], t, leaf_max, width, rounds) : 0;
+    if (i < st.cnt) newcount[i] = nc;
+    int total;
+    block_scan<BT>(nc, part, total);
+    if (threadIdx.x == 0) sums[blockIdx.x] = total;
+}
+
+__global__ __launch_bounds__(BT) void k_collapse_link(Wide w, BinTree t, int leaf_max, int width,
+                                                      LevelState* __restrict__ state,
+                                                      const int32_t* __restrict__ newcount,
+                                                      const int32_t* __restrict__ sums)
+{
+    __shared__ int32_t part[BT / 64];
+    const LevelState st = state[0];
+    if ((int64_t)blockIdx.x * BT >= st.cnt) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) state[1] = st; // no level left
+        return;
+    }
+    int before = 0, own;
+    for (int k = threadIdx.x; k < blockIdx.x; k += BT) before += sums[k];
+    (void)block_scan<BT>(before, part, before);
+    const int i = blockIdx.x * BT + threadIdx.x;
+    const int k = before + block_scan<BT>(i < st.cnt ? newcount[i] : 0, part, own);
+    if (i < st.cnt) link_children(w, st.base + i, width, leaf_max, t, st.base + st.cnt, k, w.lvl[st.cur ^ 1]);
+    if ((int64_t)(blockIdx.x + 1) * BT >= st.cnt && threadIdx.x == 0)
+        state[1] = LevelState{before + own, st.base + st.cnt, st.depth + 1, st.cur ^ 1};
 }
 
 __global__ __launch_bounds__(BT) void k_write_slots(int64_t W, int width, const int32_t* __restrict__ wide_slot_bin,
@@ -620,7 +791,7 @@ __global__ __launch_bounds__(BT) void k_write_slots(int64_t W, int width, const 
     int s = (int)(idx % width);
     uint32_t* w = slots + idx * kSlotWords;
     float* bx = boxes + idx * 6;
-    int64_t src = g * kWidth + s; // collapse scratch keeps kWidth entries per node
+    const int64_t src = idx; // the collapse's tables have width entries per node
     int32_t u = wide_slot_bin[src];
     if (s >= wide_ns[g] || u < 0) {
         for (int k = 0; k < FWN_W_LINK; ++k) w[k] = 0u;
@@ -720,140 +891,155 @@ void build_engine(Engine& e, int32_t M, const float* V_host, const int64_t* v_of
     hipEvent_t b0, b1;
     FWN_HIP(hipEventCreate(&b0));
     FWN_HIP(hipEventCreate(&b1));
+    struct Events {
+        hipEvent_t a, b;
+        ~Events()
+        {
+            (void)hipEventDestroy(a);
+            (void)hipEventDestroy(b);
+        }
+    } events{b0, b1};
     FWN_HIP(hipEventRecord(b0, s));
 
-    DBuf dV, dF, dvo, dfo, boxes, err, cinfo, cen, keys, vals, keys2, vals2, hist, rowsum;
-    dV.alloc(sizeof(float) * 3 * (size_t)std::max<int64_t>(nV, 1));
-    dF.alloc(sizeof(int32_t) * 3 * (size_t)std::max<int64_t>(nF, 1));
-    dvo.alloc(sizeof(int64_t) * (M + 1));
-    dfo.alloc(sizeof(int64_t) * (M + 1));
-    if (nV) FWN_HIP(hipMemcpyAsync(dV.p, V_host, sizeof(float) * 3 * nV, hipMemcpyHostToDevice, s));
-    if (nF) FWN_HIP(hipMemcpyAsync(dF.p, F_host, sizeof(int32_t) * 3 * nF, hipMemcpyHostToDevice, s));
-    FWN_HIP(hipMemcpyAsync(dvo.p, v_off, sizeof(int64_t) * (M + 1), hipMemcpyHostToDevice, s));
-    FWN_HIP(hipMemcpyAsync(dfo.p, f_off, sizeof(int64_t) * (M + 1), hipMemcpyHostToDevice, s));
-
-    boxes.alloc(sizeof(int32_t) * 12 * M);
-    err.alloc(sizeof(int32_t));
-    cinfo.alloc(sizeof(float) * 6 * M);
-    e.mesh_info.alloc(sizeof(float) * 8 * M);
-    hipLaunchKernelGGL(k_init, dim3(grid_blocks(12 * M, 256)), dim3(256), 0, s, boxes.as<int32_t>(), M,
-                       err.as<int32_t>());
-    FWN_LAUNCH_CHECK("k_init");
-
     const bool sah = e.opt.tree_builder == FWN_TREE_SAH;
-    DBuf tbox;
-    cen.alloc(sizeof(float) * 3 * (size_t)std::max<int64_t>(nF, 1));
-    if (sah) tbox.alloc(sizeof(float) * 6 * (size_t)std::max<int64_t>(nF, 1));
+    const int64_t n = nF;
+    // scratch bytes per triangle: mesh 24, centroid and box 36, orders 8, binary tree 32, the SAH lists
+    // 24, moment records 512, collapse 8 width + 16
+    Arena ar((size_t)(12 * nV + (660 + 8 * width) * nF + 256 * (int64_t)M + (1 << 16)));
+    float* dV = ar.take<float>(3 * nV);
+    int32_t* dF = ar.take<int32_t>(3 * nF);
+    int64_t* dvo = ar.take<int64_t>(M + 1);
+    int64_t* dfo = ar.take<int64_t>(M + 1);
+    if (nV) FWN_HIP(hipMemcpyAsync(dV, V_host, sizeof(float) * 3 * nV, hipMemcpyHostToDevice, s));
+    if (nF) FWN_HIP(hipMemcpyAsync(dF, F_host, sizeof(int32_t) * 3 * nF, hipMemcpyHostToDevice, s));
+    FWN_HIP(hipMemcpyAsync(dvo, v_off, sizeof(int64_t) * (M + 1), hipMemcpyHostToDevice, s));
+    FWN_HIP(hipMemcpyAsync(dfo, f_off, sizeof(int64_t) * (M + 1), hipMemcpyHostToDevice, s));
+
+    int32_t* boxes = ar.take<int32_t>(12 * (int64_t)M);
+    int32_t* err = ar.take<int32_t>(1);
+    float* cinfo = ar.take<float>(6 * (int64_t)M);
+    e.mesh_info.alloc(sizeof(float) * 8 * M);
+    hipLaunchKernelGGL(k_init, dim3(grid_blocks(12 * M, 256)), dim3(256), 0, s, boxes, M, err);
+    FWN_LAUNCH_CHECK("k_init");
+    float* cen = ar.take<float>(3 * nF);
+    float* tbox = sah ? ar.take<float>(6 * nF) : nullptr;
     if (nF) {
-        hipLaunchKernelGGL(k_tri_setup, dim3(grid_blocks(nF, TS)), dim3(TS), 0, s, dV.as<float>(), dF.as<int32_t>(),
-                           nF, dfo.as<int64_t>(), dvo.as<int64_t>(), M, cen.as<float>(), boxes.as<int32_t>(),
-                           sah ? tbox.as<float>() : nullptr, err.as<int32_t>());
+        hipLaunchKernelGGL(k_tri_setup, dim3(grid_blocks(nF, TS)), dim3(TS), 0, s, dV, dF, nF, dfo, dvo, M, cen, boxes,
+                           tbox, err);
         FWN_LAUNCH_CHECK("k_tri_setup");
     }
-    hipLaunchKernelGGL(k_box_final, dim3(grid_blocks(M, 64)), dim3(64), 0, s, boxes.as<int32_t>(), M,
-                       e.opt.near_fp64_rel, cinfo.as<float>(), e.mesh_info.as<float>());
+    hipLaunchKernelGGL(k_box_final, dim3(grid_blocks(M, 64)), dim3(64), 0, s, boxes, M, e.opt.near_fp64_rel, cinfo,
+                       e.mesh_info.as<float>());
     FWN_LAUNCH_CHECK("k_box_final");
-    int32_t h_err = 0;
-    FWN_HIP(hipMemcpyAsync(&h_err, err.p, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    FWN_HIP(hipStreamSynchronize(s));
-    if (h_err & 1) fail(FWN_INVALID_ARGUMENT, "facet index out of range of its mesh's vertices");
-    if (h_err & 2) fail(FWN_INVALID_ARGUMENT, "non-finite vertex position");
-
-    e.h_tau.assign(M, 0.0f);
-    {
-        std::vector<float> mi(8 * (size_t)M);
-        FWN_HIP(hipMemcpyAsync(mi.data(), e.mesh_info.p, sizeof(float) * 8 * M, hipMemcpyDeviceToHost, s));
-        FWN_HIP(hipStreamSynchronize(s));
-        for (int m = 0; m < M; ++m) e.h_tau[m] = mi[8 * m + 6];
-    }
 
     e.tris.alloc(sizeof(uint32_t) * kTriWords * (size_t)std::max<int64_t>(nF, 1));
     e.roots.alloc(sizeof(int32_t) * 2 * M);
     e.h_roots.assign(2 * (size_t)M, -1);
     for (int m = 0; m < M; ++m) e.h_roots[2 * m + 1] = 0;
+    e.h_tau.assign(M, 0.0f);
+    // what the host reads at the end: input errors and each mesh's tau (the tree of a mesh with
+    // input errors is built from clamped indices and thrown away)
+    auto read_setup = [&](char* to) {
+        FWN_HIP(hipMemcpyAsync(to, err, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+        FWN_HIP(hipMemcpyAsync(to + 16, e.mesh_info.p, sizeof(float) * 8 * M, hipMemcpyDeviceToHost, s));
+    };
+    auto check_setup = [&](const char* from) {
+        const int32_t h_err = *reinterpret_cast<const int32_t*>(from);
+        if (h_err & 1) fail(FWN_INVALID_ARGUMENT, "facet index out of range of its mesh's vertices");
+        if (h_err & 2) fail(FWN_INVALID_ARGUMENT, "non-finite vertex position");
+        const float* mi = reinterpret_cast<const float*>(from + 16);
+        for (int m = 0; m < M; ++m) e.h_tau[m] = mi[8 * m + 6];
+    };
+    const size_t setup_b = 16 + sizeof(float) * 8 * (size_t)M;
 
     if (nF == 0) {
+        char* hs = host_stage(e, setup_b);
+        read_setup(hs);
         e.slots.alloc(sizeof(uint32_t) * width * kSlotWords);
         e.boxes.alloc(sizeof(float) * width * 6);
         e.n_nodes = 0;
         e.max_depth = 0;
         FWN_HIP(hipMemcpyAsync(e.roots.p, e.h_roots.data(), sizeof(int32_t) * 2 * M, hipMemcpyHostToDevice, s));
         FWN_HIP(hipStreamSynchronize(s));
-        FWN_HIP(hipEventDestroy(b0));
-        FWN_HIP(hipEventDestroy(b1));
+        check_setup(hs);
         return;
     }
 
     // ---- binary tree topology: Morton-order radix tree, or top-down SAH splits ----
-    const int64_t n = nF;
     const int64_t nnodes = 2 * n - 1;
-    DBuf left, right, parent, first, last, isroot, rootbin, rec, visits;
-    left.alloc(sizeof(int32_t) * std::max<int64_t>(n - 1, 1));
-    right.alloc(sizeof(int32_t) * std::max<int64_t>(n - 1, 1));
-    first.alloc(sizeof(int32_t) * std::max<int64_t>(n - 1, 1));
-    last.alloc(sizeof(int32_t) * std::max<int64_t>(n - 1, 1));
-    parent.alloc(sizeof(int32_t) * nnodes);
-    isroot.alloc(nnodes);
-    rootbin.alloc(sizeof(int32_t) * M);
-    FWN_HIP(hipMemsetAsync(isroot.p, 0, nnodes, s));
-    hipLaunchKernelGGL(k_fill_i32, dim3(grid_blocks(nnodes, 256)), dim3(256), 0, s, parent.as<int32_t>(), nnodes, -1);
-    hipLaunchKernelGGL(k_fill_i32, dim3(grid_blocks(M, 256)), dim3(256), 0, s, rootbin.as<int32_t>(), (int64_t)M, -1);
+    int32_t* left = ar.take<int32_t>(n - 1);
+    int32_t* right = ar.take<int32_t>(n - 1);
+    int32_t* first = ar.take<int32_t>(n - 1);
+    int32_t* last = ar.take<int32_t>(n - 1);
+    int32_t* parent = ar.take<int32_t>(nnodes);
+    uint8_t* isroot = ar.take<uint8_t>((nnodes + 3) & ~(int64_t)3);
+    int32_t* rootbin = ar.take<int32_t>(M);
+    hipLaunchKernelGGL(k_fill_i32, dim3(grid_blocks((nnodes + 3) / 4, 256)), dim3(256), 0, s,
+                       reinterpret_cast<int32_t*>(isroot), (nnodes + 3) / 4, 0);
+    hipLaunchKernelGGL(k_fill_i32, dim3(grid_blocks(M, 256)), dim3(256), 0, s, rootbin, (int64_t)M, -1);
     FWN_LAUNCH_CHECK("k_fill_i32");
-    vals.alloc(sizeof(uint32_t) * nF);
-    uint32_t* vp = vals.as<uint32_t>();
+    uint32_t* vp = ar.take<uint32_t>(nF);
+    SahMids mids{nullptr, 0};
     if (sah) {
-        build_topology_sah(cen.as<float>(), tbox.as<float>(), nF, f_off, M, reinterpret_cast<int32_t*>(vp),
-                           left.as<int32_t>(), right.as<int32_t>(), parent.as<int32_t>(), first.as<int32_t>(),
-                           last.as<int32_t>(), isroot.as<uint8_t>(), rootbin.as<int32_t>(), s);
-        tbox.release();
+        mids = build_topology_sah(e, ar, cen, tbox, boxes, nF, f_off, M, reinterpret_cast<int32_t*>(vp), left, right,
+                                  parent, first, last, isroot, rootbin);
     } else {
-        keys.alloc(sizeof(uint64_t) * nF);
-        keys2.alloc(sizeof(uint64_t) * nF);
-        vals2.alloc(sizeof(uint32_t) * nF);
-        hipLaunchKernelGGL(k_tri_keys, dim3(grid_blocks(nF, BT)), dim3(BT), 0, s, cen.as<float>(), nF,
-                           dfo.as<int64_t>(), M, cinfo.as<float>(), keys.as<uint64_t>(), vp);
+        hipLaunchKernelGGL(k_fill_i32, dim3(grid_blocks(nnodes, 256)), dim3(256), 0, s, parent, nnodes, -1);
+        FWN_LAUNCH_CHECK("k_fill_i32");
+        DBuf hist, rowsum;
+        uint64_t* kp = ar.take<uint64_t>(nF);
+        uint64_t* kp2 = ar.take<uint64_t>(nF);
+        uint32_t* vp2 = ar.take<uint32_t>(nF);
+        hipLaunchKernelGGL(k_tri_keys, dim3(grid_blocks(nF, BT)), dim3(BT), 0, s, cen, nF, dfo, M, cinfo, kp, vp);
         FWN_LAUNCH_CHECK("k_tri_keys");
         int mesh_bits = 0;
         while ((1 << mesh_bits) < M) ++mesh_bits;
         int nbits = (M > 1) ? 32 + mesh_bits : 30;
-        uint64_t* kp = keys.as<uint64_t>();
-        uint64_t* kp2 = keys2.as<uint64_t>();
-        uint32_t* vp2 = vals2.as<uint32_t>();
         radix_sort_pairs(kp, vp, kp2, vp2, nF, nbits, hist, rowsum, s);
         if (n > 1) {
-            hipLaunchKernelGGL(k_karras, dim3(grid_blocks(n - 1, BT)), dim3(BT), 0, s, kp, n, left.as<int32_t>(),
-                               right.as<int32_t>(), parent.as<int32_t>(), first.as<int32_t>(), last.as<int32_t>());
+            hipLaunchKernelGGL(k_karras, dim3(grid_blocks(n - 1, BT)), dim3(BT), 0, s, kp, n, left, right, parent,
+                               first, last);
             FWN_LAUNCH_CHECK("k_karras");
         }
-        hipLaunchKernelGGL(k_find_roots, dim3(grid_blocks(std::max<int64_t>(n - 1, M), BT)), dim3(BT), 0, s,
-                           first.as<int32_t>(), last.as<int32_t>(), n, kp, dfo.as<int64_t>(), M,
-                           rootbin.as<int32_t>(), isroot.as<uint8_t>());
+        hipLaunchKernelGGL(k_find_roots, dim3(grid_blocks(std::max<int64_t>(n - 1, M), BT)), dim3(BT), 0, s, first,
+                           last, n, kp, dfo, M, rootbin, isroot);
         FWN_LAUNCH_CHECK("k_find_roots");
+        FWN_HIP(hipStreamSynchronize(s)); // the sort's own scratch is freed here
     }
 
     // ---- moments ----
-    rec.alloc(sizeof(double) * kRecWords * nnodes);
-    hipLaunchKernelGGL(k_leaf_records, dim3(grid_blocks(n, BT)), dim3(BT), 0, s, vp, n, dV.as<float>(),
-                       dF.as<int32_t>(), dfo.as<int64_t>(), dvo.as<int64_t>(), M, e.tris.as<uint32_t>(),
-                       rec.as<double>());
+    double* rec = ar.take<double>(kRecWords * nnodes);
+    hipLaunchKernelGGL(k_leaf_records, dim3(grid_blocks(n, BT)), dim3(BT), 0, s, vp, n, dV, dF, dfo, dvo, M,
+                       e.tris.as<uint32_t>(), rec);
     FWN_LAUNCH_CHECK("k_leaf_records");
-    if (n > 1) {
+    if (n > 1 && sah && e.opt.moment_pass == FWN_MOMENTS_LEVELS) {
+        int32_t* seg_root = ar.take<int32_t>(mids.count);
+        int32_t* visits = ar.take<int32_t>(n);
+        hipLaunchKernelGGL(k_merge_mid, dim3((unsigned)mids.count), dim3(kMergeThreads), 0, s, mids.seg, left, right, parent, first,
+                           last, n, e.opt.fp64_moment_min, rec, seg_root, visits);
+        FWN_LAUNCH_CHECK("k_merge_mid");
+        if (mids.count > 1) {
+            hipLaunchKernelGGL(k_merge_top, dim3(1), dim3(kTopThreads), 0, s, seg_root, mids.count, left, right, parent,
+                               first, last, e.opt.fp64_moment_min, rec, visits);
+            FWN_LAUNCH_CHECK("k_merge_top");
+        }
+    } else if (n > 1) {
         const int64_t n_int = n - 1;
-        DBuf depth, lvl_hist, lvl_off, order;
-        depth.alloc(sizeof(int32_t) * n_int);
-        lvl_hist.alloc(sizeof(int32_t) * (2 * kMaxLevels + 1)); // hist[kMaxLevels], cursor[kMaxLevels], deep
-        lvl_off.alloc(sizeof(int32_t) * kMaxLevels);
-        order.alloc(sizeof(int32_t) * n_int);
-        int32_t* hist_d = lvl_hist.as<int32_t>();
-        hipLaunchKernelGGL(k_fill_i32, dim3(grid_blocks(2 * kMaxLevels + 1, 256)), dim3(256), 0, s, hist_d,
-                           (int64_t)(2 * kMaxLevels + 1), 0);
-        hipLaunchKernelGGL(k_node_depth, dim3(grid_blocks(n_int, BT)), dim3(BT), 0, s, parent.as<int32_t>(),
-                           isroot.as<uint8_t>(), n_int, depth.as<int32_t>(), hist_d, hist_d + 2 * kMaxLevels);
-        FWN_LAUNCH_CHECK("k_node_depth");
-        std::vector<int32_t> hh(kMaxLevels + 1);
-        FWN_HIP(hipMemcpyAsync(hh.data(), hist_d, sizeof(int32_t) * kMaxLevels, hipMemcpyDeviceToHost, s));
-        FWN_HIP(hipMemcpyAsync(&hh[kMaxLevels], hist_d + 2 * kMaxLevels, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-        FWN_HIP(hipStreamSynchronize(s));
+        int32_t* depth = ar.take<int32_t>(n_int);
+        int32_t* hist_d = ar.take<int32_t>(2 * kMaxLevels + 1); // hist[kMaxLevels], cursor[kMaxLevels], deep
+        int32_t* lvl_off = ar.take<int32_t>(kMaxLevels);
+        int32_t* order = ar.take<int32_t>(n_int);
+        std::vector<int32_t> hh(kMaxLevels + 1, 0);
+        if (e.opt.moment_pass == FWN_MOMENTS_LEVELS) {
+            hipLaunchKernelGGL(k_fill_i32, dim3(grid_blocks(2 * kMaxLevels + 1, 256)), dim3(256), 0, s, hist_d,
+                               (int64_t)(2 * kMaxLevels + 1), 0);
+            hipLaunchKernelGGL(k_node_depth, dim3(grid_blocks(n_int, BT)), dim3(BT), 0, s, parent, isroot, n_int, depth,
+                               hist_d, hist_d + 2 * kMaxLevels);
+            FWN_LAUNCH_CHECK("k_node_depth");
+            FWN_HIP(hipMemcpyAsync(hh.data(), hist_d, sizeof(int32_t) * kMaxLevels, hipMemcpyDeviceToHost, s));
+            FWN_HIP(hipMemcpyAsync(&hh[kMaxLevels], hist_d + 2 * kMaxLevels, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+            FWN_HIP(hipStreamSynchronize(s));
+        }
         if (hh[kMaxLevels] == 0 && e.opt.moment_pass == FWN_MOMENTS_LEVELS) {
             std::vector<int32_t> off(kMaxLevels, 0);
             int levels = 0;
@@ -862,109 +1048,116 @@ void build_engine(Engine& e, int32_t M, const float* V_host, const int64_t* v_of
                 acc += hh[d];
                 if (hh[d] > 0) levels = d + 1;
             }
-            FWN_HIP(hipMemcpyAsync(lvl_off.p, off.data(), sizeof(int32_t) * kMaxLevels, hipMemcpyHostToDevice, s));
-            hipLaunchKernelGGL(k_depth_bucket, dim3(grid_blocks(n_int, BT)), dim3(BT), 0, s, depth.as<int32_t>(),
-                               n_int, lvl_off.as<int32_t>(), hist_d + kMaxLevels, order.as<int32_t>());
+            FWN_HIP(hipMemcpyAsync(lvl_off, off.data(), sizeof(int32_t) * kMaxLevels, hipMemcpyHostToDevice, s));
+            hipLaunchKernelGGL(k_depth_bucket, dim3(grid_blocks(n_int, BT)), dim3(BT), 0, s, depth, n_int, lvl_off,
+                               hist_d + kMaxLevels, order);
             FWN_LAUNCH_CHECK("k_depth_bucket");
             for (int d = levels - 1; d >= 0; --d) {
                 if (hh[d] == 0) continue;
-                hipLaunchKernelGGL(k_merge_level, dim3(grid_blocks(hh[d], BT)), dim3(BT), 0, s,
-                                   order.as<int32_t>() + off[d], hh[d], left.as<int32_t>(), right.as<int32_t>(),
-                                   first.as<int32_t>(), last.as<int32_t>(), e.opt.fp64_moment_min, rec.as<double>());
+                hipLaunchKernelGGL(k_merge_level, dim3(grid_blocks(hh[d], BT)), dim3(BT), 0, s, order + off[d], hh[d],
+                                   left, right, first, last, e.opt.fp64_moment_min, rec);
                 FWN_LAUNCH_CHECK("k_merge_level");
             }
-            // the host vectors above are read by copies already waited for; off by the bucket kernel
+            // off is read by the bucket kernel's upload
             FWN_HIP(hipStreamSynchronize(s));
         } else {
-            visits.alloc(sizeof(int32_t) * n_int);
-            hipLaunchKernelGGL(k_fill_i32, dim3(grid_blocks(n_int, 256)), dim3(256), 0, s, visits.as<int32_t>(),
-                               n_int, 0);
-            hipLaunchKernelGGL(k_bottom_up, dim3(grid_blocks(n, BT)), dim3(BT), 0, s, parent.as<int32_t>(),
-                               left.as<int32_t>(), right.as<int32_t>(), first.as<int32_t>(), last.as<int32_t>(),
-                               isroot.as<uint8_t>(), n, e.opt.fp64_moment_min, rec.as<double>(),
-                               visits.as<int32_t>());
+            int32_t* visits = ar.take<int32_t>(n_int);
+            hipLaunchKernelGGL(k_fill_i32, dim3(grid_blocks(n_int, 256)), dim3(256), 0, s, visits, n_int, 0);
+            hipLaunchKernelGGL(k_bottom_up, dim3(grid_blocks(n, BT)), dim3(BT), 0, s, parent, left, right, first, last,
+                               isroot, n, e.opt.fp64_moment_min, rec, visits);
             FWN_LAUNCH_CHECK("k_bottom_up");
         }
     }
 
     // ---- collapse ----
-    std::vector<int32_t> rb(M);
-    FWN_HIP(hipMemcpyAsync(rb.data(), rootbin.p, sizeof(int32_t) * M, hipMemcpyDeviceToHost, s));
-    FWN_HIP(hipStreamSynchronize(s));
-    std::vector<int32_t> level0;
-    std::vector<int32_t> mesh_wide(M, -1);
-    for (int m = 0; m < M; ++m) {
+    // the first level: the roots of the meshes that have facets, in mesh order (gathered on the device)
+    std::vector<int32_t> mesh_wide(M, -1), level0_mesh;
+    for (int m = 0; m < M; ++m)
         if (f_off[m + 1] > f_off[m]) {
-            if (rb[m] < 0) fail(FWN_HIP_ERROR, "tree build: mesh root not found");
-            mesh_wide[m] = (int32_t)level0.size();
-            level0.push_back(rb[m]);
+            mesh_wide[m] = (int32_t)level0_mesh.size();
+            level0_mesh.push_back(m);
         }
-    }
-    DBuf wsb, wns, cw, lvl[2], newc, offs, scan_tmp;
+    const int32_t cnt0 = (int32_t)level0_mesh.size();
     // every wide node is a distinct binary node with more than leaf_max triangles, or a mesh root
-    int64_t wcap = n + M;
-    wsb.alloc(sizeof(int32_t) * kWidth * wcap);
-    cw.alloc(sizeof(int32_t) * kWidth * wcap);
-    wns.alloc(sizeof(int32_t) * wcap);
-    lvl[0].alloc(sizeof(int32_t) * wcap);
-    lvl[1].alloc(sizeof(int32_t) * wcap);
-    newc.alloc(sizeof(int32_t) * wcap);
-    offs.alloc(sizeof(int32_t) * (wcap + 1));
-    FWN_HIP(hipMemcpyAsync(lvl[0].p, level0.data(), sizeof(int32_t) * level0.size(), hipMemcpyHostToDevice, s));
+    const int64_t wcap = n + M;
+    Wide w;
+    w.slot_bin = ar.take<int32_t>(width * wcap);
+    w.child = ar.take<int32_t>(width * wcap);
+    w.ns = ar.take<int32_t>(wcap);
+    w.lvl[0] = ar.take<int32_t>(wcap);
+    w.lvl[1] = ar.take<int32_t>(wcap);
+    int32_t* newc = ar.take<int32_t>(wcap);
+    int32_t* sums = ar.take<int32_t>((wcap + BT - 1) / BT);
+    const BinTree bt{left, right, first, last, n};
     int rounds = 0; // binary levels per wide node for the SAH layout: log2(width)
     while ((1 << rounds) < width) ++rounds;
-    int32_t cnt = (int32_t)level0.size(), gbase = 0, depth = 0;
-    int cur = 0;
-    while (cnt > 0) {
-        hipLaunchKernelGGL(k_collapse_level, dim3(grid_blocks(cnt, BT)), dim3(BT), 0, s, lvl[cur].as<int32_t>(), cnt,
-                           gbase, left.as<int32_t>(), right.as<int32_t>(), first.as<int32_t>(), last.as<int32_t>(),
-                           n, leaf_max, width, sah ? rounds : 0, wsb.as<int32_t>(), wns.as<int32_t>(),
-                           newc.as<int32_t>());
-        FWN_LAUNCH_CHECK("k_collapse_level");
-        exclusive_scan_i32(newc.as<int32_t>(), offs.as<int32_t>(), cnt, scan_tmp, s);
-        int32_t next_base = gbase + cnt;
-        hipLaunchKernelGGL(k_collapse_assign, dim3(grid_blocks(cnt, BT)), dim3(BT), 0, s, cnt, gbase, next_base,
-                           wsb.as<int32_t>(), first.as<int32_t>(), last.as<int32_t>(), n, leaf_max,
-                           offs.as<int32_t>(), cw.as<int32_t>(), lvl[cur ^ 1].as<int32_t>());
-        FWN_LAUNCH_CHECK("k_collapse_assign");
-        int32_t total = 0;
-        FWN_HIP(hipMemcpyAsync(&total, offs.as<int32_t>() + cnt, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-        FWN_HIP(hipStreamSynchronize(s));
-        ++depth;
-        gbase = next_base;
-        cnt = total;
-        cur ^= 1;
-        if (gbase + (int64_t)cnt > wcap) fail(FWN_HIP_ERROR, "tree build: wide node bound exceeded");
+    if (!sah) rounds = 0;
+    // levels a balanced tree needs after the first workgroup's, and a few for uneven ones; more are
+    // enqueued while there are nodes
+    int group = 3;
+    for (int64_t c = n / leaf_max / kTopNodes; c > 0; c /= width) ++group;
+    LevelState* state = ar.take<LevelState>(group + 1);
+    char* hs = host_stage(e, setup_b + sizeof(LevelState) + sizeof(int32_t) * 2 * (size_t)M);
+    LevelState* h_state = reinterpret_cast<LevelState*>(hs + setup_b);
+    int32_t* h_small = reinterpret_cast<int32_t*>(hs + setup_b + sizeof(LevelState)); // M ints, twice
+    if (cnt0 == M) { // the list is the roots array itself
+        FWN_HIP(hipMemcpyAsync(w.lvl[0], rootbin, sizeof(int32_t) * M, hipMemcpyDeviceToDevice, s));
+    } else {
+        std::copy(level0_mesh.begin(), level0_mesh.end(), h_small);
+        FWN_HIP(hipMemcpyAsync(w.lvl[1], h_small, sizeof(int32_t) * cnt0, hipMemcpyHostToDevice, s));
+        hipLaunchKernelGGL(k_gather_i32, dim3(grid_blocks(cnt0, 256)), dim3(256), 0, s, rootbin, w.lvl[1], cnt0,
+                           w.lvl[0]);
+        FWN_LAUNCH_CHECK("k_gather_i32");
     }
-    const int64_t W = gbase;
-    e.n_nodes = W;
-    e.max_depth = depth;
-    e.slots.alloc(sizeof(uint32_t) * width * kSlotWords * (size_t)std::max<int64_t>(W, 1));
-    e.boxes.alloc(sizeof(float) * width * 6 * (size_t)std::max<int64_t>(W, 1));
+    hipLaunchKernelGGL(k_collapse_top, dim3(1), dim3(kTopNodes), 0, s, w, bt, cnt0, leaf_max, width, rounds, state);
+    FWN_LAUNCH_CHECK("k_collapse_top");
+    int64_t bound = std::max<int64_t>((int64_t)kTopNodes * width, cnt0); // nodes of the level in work
+    for (;;) {
+        for (int k = 0; k < group; ++k) {
+            const int blocks = grid_blocks(std::min(bound, wcap), BT);
+            hipLaunchKernelGGL(k_collapse_slots, dim3(blocks), dim3(BT), 0, s, w, bt, leaf_max, width, rounds, state + k,
+                               newc, sums);
+            FWN_LAUNCH_CHECK("k_collapse_slots");
+            hipLaunchKernelGGL(k_collapse_link, dim3(blocks), dim3(BT), 0, s, w, bt, leaf_max, width, state + k, newc,
+                               sums);
+            FWN_LAUNCH_CHECK("k_collapse_link");
+            bound = std::min(bound * width, wcap);
+        }
+        FWN_HIP(hipMemcpyAsync(h_state, state + group, sizeof(LevelState), hipMemcpyDeviceToHost, s));
+        read_setup(hs);
+        FWN_HIP(hipMemcpyAsync(h_small, rootbin, sizeof(int32_t) * M, hipMemcpyDeviceToHost, s));
+        FWN_HIP(hipMemcpyAsync(h_small + M, w.ns, sizeof(int32_t) * cnt0, hipMemcpyDeviceToHost, s));
+        FWN_HIP(hipStreamSynchronize(s));
+        if (h_state->cnt == 0) break;
+        FWN_HIP(hipMemcpyAsync(state, state + group, sizeof(LevelState), hipMemcpyDeviceToDevice, s));
+    }
+    check_setup(hs);
+    for (int m = 0; m < M; ++m)
+        if (mesh_wide[m] >= 0 && h_small[m] < 0) fail(FWN_HIP_ERROR, "tree build: mesh root not found");
+    const int64_t W = h_state->base;
+    if (W < 1 || W > wcap) fail(FWN_HIP_ERROR, "tree build: wide node bound exceeded");
     if (W >= ((int64_t)1 << 27)) fail(FWN_LIMIT_EXCEEDED, "more than 2^27 tree nodes");
-    hipLaunchKernelGGL(k_write_slots, dim3(grid_blocks(W * width, BT)), dim3(BT), 0, s, W, width, wsb.as<int32_t>(),
-                       wns.as<int32_t>(), cw.as<int32_t>(), rec.as<double>(), first.as<int32_t>(), last.as<int32_t>(),
-                       n, e.opt.accuracy_scale * e.opt.accuracy_scale, dfo.as<int64_t>(), M,
-                       e.mesh_info.as<float>(), e.slots.as<uint32_t>(), e.boxes.as<float>(), e.tris.as<uint32_t>());
-    FWN_LAUNCH_CHECK("k_write_slots");
-    std::vector<int32_t> ns_root(level0.size());
-    if (!level0.empty())
-        FWN_HIP(hipMemcpyAsync(ns_root.data(), wns.p, sizeof(int32_t) * level0.size(), hipMemcpyDeviceToHost, s));
-    FWN_HIP(hipStreamSynchronize(s));
+    e.n_nodes = W;
+    e.max_depth = h_state->depth;
     for (int m = 0; m < M; ++m) {
         if (mesh_wide[m] >= 0) {
             e.h_roots[2 * m] = mesh_wide[m];
-            e.h_roots[2 * m + 1] = ns_root[mesh_wide[m]];
+            e.h_roots[2 * m + 1] = h_small[M + mesh_wide[m]];
         }
     }
-    FWN_HIP(hipMemcpyAsync(e.roots.p, e.h_roots.data(), sizeof(int32_t) * 2 * M, hipMemcpyHostToDevice, s));
+    e.slots.alloc(sizeof(uint32_t) * width * kSlotWords * (size_t)W);
+    e.boxes.alloc(sizeof(float) * width * 6 * (size_t)W);
+    hipLaunchKernelGGL(k_write_slots, dim3(grid_blocks(W * width, BT)), dim3(BT), 0, s, W, width, w.slot_bin, w.ns,
+                       w.child, rec, first, last, n, e.opt.accuracy_scale * e.opt.accuracy_scale, dfo, M,
+                       e.mesh_info.as<float>(), e.slots.as<uint32_t>(), e.boxes.as<float>(), e.tris.as<uint32_t>());
+    FWN_LAUNCH_CHECK("k_write_slots");
+    std::copy(e.h_roots.begin(), e.h_roots.end(), h_small);
+    FWN_HIP(hipMemcpyAsync(e.roots.p, h_small, sizeof(int32_t) * 2 * M, hipMemcpyHostToDevice, s));
     FWN_HIP(hipEventRecord(b1, s));
     FWN_HIP(hipStreamSynchronize(s));
     float ms = 0.0f;
     FWN_HIP(hipEventElapsedTime(&ms, b0, b1));
     e.build_ms = ms;
-    FWN_HIP(hipEventDestroy(b0));
-    FWN_HIP(hipEventDestroy(b1));
 }
 
 } // namespace fwn

@@ -5,7 +5,9 @@
 
 #include <condition_variable>
 #include <cstdint>
+#include <algorithm>
 #include <atomic>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <string>
@@ -156,14 +158,49 @@ void exclusive_scan_i32(const int32_t* in, int32_t* out, int64_t n, DBuf& tmp, h
 void build_engine(Engine& e, int32_t n_meshes, const float* V_host, const int64_t* v_off, const int32_t* F_host,
                   const int64_t* f_off);
 
+// Scratch of one build: pieces taken from a few device allocations, all freed at the end.  The
+// allocations stay below 64 MB where a single piece does not need more (hipFree takes 12-25 us up to
+// 64 MB and 300 us above, per allocation).
+struct Arena {
+    static constexpr size_t kBlock = (size_t)60 << 20;
+    std::vector<std::unique_ptr<DBuf>> blocks;
+    size_t used = 0, expect = 0; // of the last block; bytes still expected to be taken
+    explicit Arena(size_t expected) : expect(expected) {}
+    void* take_bytes(size_t n)
+    {
+        n = (std::max<size_t>(n, 1) + 255) & ~(size_t)255;
+        if (blocks.empty() || used + n > blocks.back()->bytes) {
+            blocks.emplace_back(new DBuf());
+            blocks.back()->alloc(std::max(n, std::min(kBlock, std::max<size_t>(expect, (size_t)1 << 20))));
+            used = 0;
+        }
+        void* p = static_cast<char*>(blocks.back()->p) + used;
+        used += n;
+        expect -= std::min(expect, n);
+        return p;
+    }
+    template <class T>
+    T* take(int64_t count)
+    {
+        return static_cast<T*>(take_bytes(sizeof(T) * (size_t)std::max<int64_t>(count, 0)));
+    }
+};
+
 // SAH topology (fwn_sah.hip): top-down binned box-area splits of each mesh's triangles down to
 // single triangles, in the binary tree layout of the LBVH path: internal nodes [0, n-1), leaf j
 // -> n-1+j for the triangle at sorted position j, `items` = sorted position -> triangle,
-// left/right/first/last per internal node, parent per node (the caller fills -1 first),
-// is_root (the caller fills 0) and root_bin per mesh.
-void build_topology_sah(const float* cen, const float* tbox, int64_t nF, const int64_t* f_off, int M,
-                        int32_t* items, int32_t* left, int32_t* right, int32_t* parent, int32_t* first,
-                        int32_t* last, uint8_t* is_root, int32_t* root_bin, hipStream_t s);
+// left/right/first/last per internal node, parent per node of a mesh's tree, is_root (the caller
+// fills 0) and root_bin per mesh.  boxes: the triangle setup's 12 ints per mesh.  A mid segment (at
+// most kSahMid triangles, 4 ints in the returned list: lo, hi, parent, side) is a subtree over the
+// sorted positions [lo, hi) whose internal nodes have the ids [lo, hi - 2].
+constexpr int kSahMid = 1024;
+struct SahMids {
+    const int32_t* seg; // device
+    int64_t count;
+};
+SahMids build_topology_sah(Engine& e, Arena& ar, const float* cen, const float* tbox, const int32_t* boxes, int64_t nF,
+                           const int64_t* f_off, int M, int32_t* items, int32_t* left, int32_t* right, int32_t* parent,
+                           int32_t* first, int32_t* last, uint8_t* is_root, int32_t* root_bin);
 
 // queries (fwn_query.hip)
 void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t nQ, float* omega, uint8_t* inside,
