@@ -13,6 +13,8 @@ from __future__ import annotations
 
 import numpy as np
 
+from .bounds import column_bounds
+
 DEFAULT_VOXEL_SIZE = -0.01  # MeshToVolumeOptions::voxel_size (mesh_to_volume.h:40)
 NARROW_BAND = 3             # exterior / interior bandwidth in voxels (mesh_to_volume.cpp:164-165)
 
@@ -24,7 +26,8 @@ def bbox_diagonal(vertices) -> float:
     if V.ndim != 2 or V.shape[1] != 3 or V.shape[0] == 0:
         raise ValueError("vertices must be a non-empty (N, 3) array")
     t = V.dtype.type if V.dtype in (np.float32, np.float64) else np.float64
-    d = (V.max(axis=0) - V.min(axis=0)).astype(t)
+    lo, hi = column_bounds(V)
+    d = (hi - lo).astype(t)
     return float(np.sqrt(t(d[0] * d[0] + d[1] * d[1]) + t(d[2] * d[2])))
 
 
@@ -51,8 +54,9 @@ def index_box(vertices, voxel_size: float, band: int = NARROW_BAND):
     by ``band`` voxels on every side (a dense superset of OpenVDB's narrow band)."""
     V = np.asarray(vertices, dtype=np.float64)
     vs = float(voxel_size)
-    lo = np.floor((V.min(axis=0) - vs * 0.5) / vs).astype(np.int64) - band
-    hi = np.ceil((V.max(axis=0) - vs * 0.5) / vs).astype(np.int64) + band
+    vlo, vhi = column_bounds(V)
+    lo = np.floor((vlo - vs * 0.5) / vs).astype(np.int64) - band
+    hi = np.ceil((vhi - vs * 0.5) / vs).astype(np.int64) + band
     if (lo < np.iinfo(np.int32).min).any() or (hi > np.iinfo(np.int32).max).any():
         raise ValueError("voxel indices beyond int32: voxel size too small")
     return lo.astype(np.int32), (hi - lo + 1).astype(np.int32)

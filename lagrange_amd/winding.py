@@ -19,6 +19,7 @@ import weakref
 import numpy as np
 
 from . import _lib as L
+from .bounds import column_bounds
 
 
 class LagrangeError(RuntimeError):
@@ -48,8 +49,10 @@ def _mesh_arrays(mesh):
     if F.ndim != 2 or F.shape[1] != 3:
         raise LagrangeError("Fast winding number engine only supports triangle meshes")
     # the reference's internal copy: float positions, int indices (FastWindingNumber.cpp:39-52)
-    return (np.ascontiguousarray(V, dtype=np.float32),
-            np.ascontiguousarray(F.astype(np.int64, copy=False).astype(np.int32), dtype=np.int32))
+    # (float or unsigned indices go through int64, as before their narrowing to int)
+    if F.dtype != np.int32:
+        F = F.astype(np.int64, copy=False).astype(np.int32)
+    return np.ascontiguousarray(V, dtype=np.float32), np.ascontiguousarray(F)
 
 
 def _ptr(a) -> int:
@@ -195,8 +198,7 @@ class FastWindingNumber(_EngineBase):
         self.num_vertices = V.shape[0]
         self.num_facets = F.shape[0]
         # float bounding box of the mesh (mesh_bbox<3> of a float mesh), for sampling
-        self.bbox = ((V.min(axis=0), V.max(axis=0)) if V.shape[0] else
-                     (np.zeros(3, np.float32), np.zeros(3, np.float32)))
+        self.bbox = column_bounds(V) if V.shape[0] else (np.zeros(3, np.float32), np.zeros(3, np.float32))
 
     @classmethod
     def tuned(cls, mesh, points, leaf_sizes=(1, 2, 4, 8), *, options: L.Options | None = None, **opts):
@@ -210,8 +212,7 @@ class FastWindingNumber(_EngineBase):
         self._handle = h
         self.num_vertices = V.shape[0]
         self.num_facets = F.shape[0]
-        self.bbox = ((V.min(axis=0), V.max(axis=0)) if V.shape[0] else
-                     (np.zeros(3, np.float32), np.zeros(3, np.float32)))
+        self.bbox = column_bounds(V) if V.shape[0] else (np.zeros(3, np.float32), np.zeros(3, np.float32))
         self.tuning = {"leaf_max": leaf, "query_ms": ms}
         return self
 
