@@ -25,7 +25,8 @@
 //                   repeatedly opens the largest non-leaf slot until it has tree_width slots (Morton
 //                   trees), or whole binary levels (SAH trees)
 //   k_write_slots   FP64 records -> the 32-word FP32 slot format of fwn.h, plus each slot's box
-//                   (6 floats, rounded outward) for distance queries
+//                   (6 floats, rounded outward) and link for distance queries
+//   k_slot_disks    each slot's disk (a slab around its triangles) for distance queries
 //
 // Several meshes are built together: their keys carry the mesh id above the Morton bits, so
 // each mesh is one subtree of a single radix tree and every kernel runs once for all meshes.
@@ -790,13 +791,14 @@ __global__ __launch_bounds__(BT) void k_write_slots(int64_t W, int width, const 
     int64_t g = idx / width;
     int s = (int)(idx % width);
     uint32_t* w = slots + idx * kSlotWords;
-    float* bx = boxes + idx * 6;
+    float* bx = boxes + idx * kBoxWords;
     const int64_t src = idx; // the collapse's tables have width entries per node
     int32_t u = wide_slot_bin[src];
     if (s >= wide_ns[g] || u < 0) {
         for (int k = 0; k < FWN_W_LINK; ++k) w[k] = 0u;
         w[FWN_W_LINK] = FWN_LINK_EMPTY;
-        for (int k = 0; k < 6; ++k) bx[k] = 0.0f;
+        for (int k = 0; k < kBoxWords; ++k) bx[k] = 0.0f;
+        bx[6] = __uint_as_float(FWN_LINK_EMPTY);
         return;
     }
     const double* r = rec + (int64_t)u * kRecWords;
@@ -846,12 +848,14 @@ __global__ __launch_bounds__(BT) void k_write_slots(int64_t W, int width, const 
     const int32_t cw = child_wide[src];
     if (cw >= 0) {
         w[FWN_W_LINK] = ((uint32_t)cw << 4) | (uint32_t)wide_ns[cw];
+        bx[6] = __uint_as_float(w[FWN_W_LINK]);
         return;
     }
     const bool bin_leaf = u >= n - 1;
     const int64_t tf = bin_leaf ? (u - (n - 1)) : first[u];
     const int32_t tc = bin_leaf ? 1 : last[u] - first[u] + 1;
     w[FWN_W_LINK] = FWN_LINK_LEAF | ((uint32_t)tf << 3) | (uint32_t)(tc - 1);
+    bx[6] = __uint_as_float(w[FWN_W_LINK]);
     // the leaf's FP64 near-field rule, in its first triangle: q is within tau of the leaf's
     // bounding sphere when |d|^2 < (sqrt(r2) + tau)^2 and, for a single triangle, within tau of
     // its plane when (d.N)^2 < tau^2 |N|^2
@@ -861,6 +865,79 @@ __global__ __launch_bounds__(BT) void k_write_slots(int64_t W, int width, const 
     uint32_t* tw = tris + tf * kTriWords;
     tw[FWN_T_NEAR2] = __float_as_uint(rr * rr);
     tw[FWN_T_PLANE] = __float_as_uint((tau * tau) * nn);
+}
+
+// Each slot's disk, from its triangles' vertices in double; a row of 16 lanes per slot.  A slot of more
+// than kDiskTris triangles (nearly always entered, and a serial loop here) or with a sliver (sine below 1e-4: its evaluated
+// distance may be off by more than the bound allows for) gets no bound.
+constexpr int64_t kDiskTris = 1024;
+__global__ __launch_bounds__(BT) void k_slot_disks(int64_t nslots, const int32_t* __restrict__ slot_bin,
+                                                   const double* __restrict__ rec, const int32_t* __restrict__ first,
+                                                   const int32_t* __restrict__ last, int64_t n,
+                                                   const uint32_t* __restrict__ tris, float* __restrict__ boxes)
+{
+    const int64_t idx = ((int64_t)blockIdx.x * BT + threadIdx.x) >> 4;
+    const int lane = threadIdx.x & 15;
+    if (idx >= nslots) return;
+    float* o = boxes + idx * kBoxWords;
+    if (__float_as_uint(o[6]) == FWN_LINK_EMPTY) return;
+    const int32_t u = slot_bin[idx];
+    const int64_t t0 = u >= n - 1 ? u - (n - 1) : first[u], t1 = u >= n - 1 ? t0 : last[u];
+    const double* r = rec + (int64_t)u * kRecWords;
+    const double c0[3] = {r[R_P], r[R_P + 1], r[R_P + 2]};
+    double nn[3] = {r[R_N], r[R_N + 1], r[R_N + 2]};
+    const double A = sqrt(nn[0] * nn[0] + nn[1] * nn[1] + nn[2] * nn[2]);
+    for (int d = 0; d < 3; ++d) nn[d] /= A;
+    bool none = t1 - t0 >= kDiskTris || !(A > 0.0);
+    float lo = INFINITY, hi = -INFINITY, rr = 0.0f; // rounded outward
+    if (!none) {
+        for (int64_t t = t0 + lane; t <= t1; t += 16) {
+            const float* tw = reinterpret_cast<const float*>(tris + t * kTriWords);
+            double w[3][3];
+            for (int k = 0; k < 3; ++k)
+                for (int d = 0; d < 3; ++d) w[k][d] = (double)tw[3 * k + d] - c0[d];
+            double e1[3], e2[3];
+            for (int d = 0; d < 3; ++d) {
+                e1[d] = w[1][d] - w[0][d];
+                e2[d] = w[2][d] - w[0][d];
+            }
+            const double N[3] = {e1[1] * e2[2] - e1[2] * e2[1], e1[2] * e2[0] - e1[0] * e2[2],
+                                 e1[0] * e2[1] - e1[1] * e2[0]};
+            none |= !(N[0] * N[0] + N[1] * N[1] + N[2] * N[2] >
+                      1e-8 * (e1[0] * e1[0] + e1[1] * e1[1] + e1[2] * e1[2]) *
+                          (e2[0] * e2[0] + e2[1] * e2[1] + e2[2] * e2[2]));
+            for (int k = 0; k < 3; ++k) {
+                const double h = w[k][0] * nn[0] + w[k][1] * nn[1] + w[k][2] * nn[2];
+                double q = 0.0;
+                for (int d = 0; d < 3; ++d) q += (w[k][d] - h * nn[d]) * (w[k][d] - h * nn[d]);
+                lo = fminf(lo, __double2float_rd(h));
+                hi = fmaxf(hi, __double2float_ru(h));
+                rr = fmaxf(rr, __double2float_ru(q));
+            }
+        }
+    }
+    for (int m = 8; m > 0; m >>= 1) {
+        lo = fminf(lo, __shfl_xor(lo, m, 16));
+        hi = fmaxf(hi, __shfl_xor(hi, m, 16));
+        rr = fmaxf(rr, __shfl_xor(rr, m, 16));
+        none |= __shfl_xor((int)none, m, 16) != 0;
+    }
+    if (lane != 0) return;
+    float c[3] = {0, 0, 0};
+    double margin = 0.0; // the rounding of c and n
+    for (int d = 0; d < 3; ++d) {
+        c[d] = (float)(c0[d] + nn[d] * 0.5 * ((double)lo + (double)hi));
+        margin += 1e-7 * fabs((double)c[d]);
+    }
+    const double t = 0.5 * ((double)hi - (double)lo), R = sqrt((double)rr);
+    margin += 3e-7 * (t + R);
+    o[7] = none ? INFINITY : __double2float_ru(t + margin);
+    o[11] = none ? INFINITY : __double2float_ru(R + margin);
+    for (int d = 0; d < 3; ++d) {
+        o[8 + d] = none ? 0.0f : c[d];
+        o[12 + d] = none ? 0.0f : (float)nn[d];
+    }
+    o[15] = 0.0f;
 }
 
 } // namespace
@@ -956,7 +1033,7 @@ void build_engine(Engine& e, int32_t M, const float* V_host, const int64_t* v_of
         char* hs = host_stage(e, setup_b);
         read_setup(hs);
         e.slots.alloc(sizeof(uint32_t) * width * kSlotWords);
-        e.boxes.alloc(sizeof(float) * width * 6);
+        e.boxes.alloc(sizeof(float) * width * kBoxWords);
         e.n_nodes = 0;
         e.max_depth = 0;
         FWN_HIP(hipMemcpyAsync(e.roots.p, e.h_roots.data(), sizeof(int32_t) * 2 * M, hipMemcpyHostToDevice, s));
@@ -1146,11 +1223,14 @@ void build_engine(Engine& e, int32_t M, const float* V_host, const int64_t* v_of
         }
     }
     e.slots.alloc(sizeof(uint32_t) * width * kSlotWords * (size_t)W);
-    e.boxes.alloc(sizeof(float) * width * 6 * (size_t)W);
+    e.boxes.alloc(sizeof(float) * width * kBoxWords * (size_t)W);
     hipLaunchKernelGGL(k_write_slots, dim3(grid_blocks(W * width, BT)), dim3(BT), 0, s, W, width, w.slot_bin, w.ns,
                        w.child, rec, first, last, n, e.opt.accuracy_scale * e.opt.accuracy_scale, dfo, M,
                        e.mesh_info.as<float>(), e.slots.as<uint32_t>(), e.boxes.as<float>(), e.tris.as<uint32_t>());
     FWN_LAUNCH_CHECK("k_write_slots");
+    hipLaunchKernelGGL(k_slot_disks, dim3(grid_blocks(W * width * 16, BT)), dim3(BT), 0, s, W * width, w.slot_bin, rec,
+                       first, last, n, e.tris.as<uint32_t>(), e.boxes.as<float>());
+    FWN_LAUNCH_CHECK("k_slot_disks");
     std::copy(e.h_roots.begin(), e.h_roots.end(), h_small);
     FWN_HIP(hipMemcpyAsync(e.roots.p, h_small, sizeof(int32_t) * 2 * M, hipMemcpyHostToDevice, s));
     FWN_HIP(hipEventRecord(b1, s));

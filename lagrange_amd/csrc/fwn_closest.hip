@@ -10,9 +10,19 @@
 // entries as in the winding-number traversal; a lane takes part in a slot while the slot's box is
 // nearer than the lane's best distance so far.  Leaf slots are evaluated before a node's children
 // are pushed (to tighten the bounds early) and children are pushed farthest first, ordered by the
-// box distance of each slot's first participating lane, so the nearest is walked next.  Inside a
-// leaf, a triangle is evaluated only for lanes whose best distance its vertex box does not
-// exceed.  Slot boxes come from the build (each slot's vertex box, rounded outward to float).
+// box distance of each slot's first participating lane, so the nearest is walked next.  A slot that
+// no participating lane's best reaches by its disk (a slab around the triangles: a box is fat where
+// the surface runs askew, and deep inside a mesh the box walk opened nearly every leaf) is left out
+// as a whole, which changes neither a mask nor a best distance anywhere else: the facet of an exact
+// tie is the first in the walk's order, with or without the disks.  Inside a leaf bucket, a triangle
+// is evaluated only for lanes whose best distance its vertex box does not exceed.
+//
+// Bound: issue and latency of the longest waves (points deep inside, whose 64 lanes' nearest
+// triangles lie on all sides): 400,000 points over 200k triangles keep 3.3 waves of a compute unit in
+// flight on average, and an average wave issues 87k vector and 52k scalar instructions.  Against the
+// walk with double box distances from vector loads and no disks (333k and 330k), that call takes
+// 4.28 ms instead of 43.2: 16.1 ms with the float box distances and record loads below, 12.7 with
+// disks of single triangles, and the rest from the disks of the inner slots.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -247,12 +257,51 @@ __device__ __forceinline__ double tri_box_dist2(const float* __restrict__ tw, do
     return box_dist2(b, qx, qy, qz);
 }
 
-template <int NB>
-__global__ __launch_bounds__(64) void k_closest(const uint32_t* __restrict__ slots, const float* __restrict__ boxes,
-                                                int width, const uint32_t* __restrict__ tris, int32_t root,
-                                                int32_t root_ns, const float* __restrict__ Q,
-                                                const uint32_t* __restrict__ perm, int64_t nQ,
-                                                double* __restrict__ d2_out, int32_t* __restrict__ tri_out,
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef v16f v16f_a4 __attribute__((aligned(4)));
+
+// A lane's FP64 best distance as float bounds: a float box distance below `lo` is certainly below
+// the best, one above `hi` certainly not (the float distance is within 3e-7 of the double one, the
+// bounds leave 1e-6); between them, and where the best is too small or too large for that, the
+// double distance decides.
+struct BestBounds {
+    float lo = INFINITY, hi = INFINITY;
+    __device__ __forceinline__ void set(double best)
+    {
+        const float b = (float)best;
+        lo = b > 1e-30f && b < 1e38f ? b * (1.0f - 1e-6f) : 0.0f;
+        hi = b < 1e38f ? (b > 1e-30f ? b * (1.0f + 1e-6f) : 1e-29f) : INFINITY;
+    }
+};
+
+// Lower bound on the squared distance from q to what a slot's disk holds (its triangles: within t of
+// the plane through c normal to n, and within R of the axis), less the float arithmetic's error.  With
+// r = c - q, h its part along n and rho the one along the plane, the distance is at least |h| - t along
+// n and rho - R along the plane.  The float results are within 2.4e-6 |r|^2 (six roundings of relative
+// 2^-24 in h, three in |r|^2, and (rho - R) / rho <= 1 for the square root); 4e-6 |r|^2 is taken off,
+// and 1e-13 R^2 for the rounding of the exact evaluation this stands for.  t = R = infinity bounds
+// nothing, and NaN (overflow) compares as no bound.
+__device__ __forceinline__ float disk_bound(float t, float cx, float cy, float cz, float R, float nx, float ny,
+                                            float nz, float fx, float fy, float fz)
+{
+    const float rx = cx - fx, ry = cy - fy, rz = cz - fz;
+    const float r2 = fmaf(rx, rx, fmaf(ry, ry, rz * rz));
+    const float hc = fmaf(rx, nx, fmaf(ry, ny, rz * nz));
+    const float h = fmaxf(fabsf(hc) - t, 0.0f);
+    const float out = fmaxf(__builtin_amdgcn_sqrtf(fmaxf(fmaf(-hc, hc, r2), 0.0f)) - R, 0.0f);
+    return fmaf(-4e-6f, r2, fmaf(-1e-13f * R, R, fmaf(out, out, h * h)));
+}
+
+// One wave per 64 sorted points; W = tree width.  Decisions (which lanes take part in a slot, the
+// order of the children, which triangle wins) are those of the double arithmetic throughout; float
+// distances settle all but the closest calls: 14 instructions a box instead of 40, its operands
+// straight from scalar registers.  A slot's box, link and disk are one 64-byte scalar load.
+// (Measured and not taken: the disks of a node's leaves all tested before any is evaluated, 13.1 ms
+// for 12.7; one selected division and evaluation in place of the region branches, 4.80 for 4.28.)
+template <int NB, int W>
+__global__ __launch_bounds__(64) void k_closest(const float* __restrict__ boxes, const uint32_t* __restrict__ tris,
+                                                int32_t root, int32_t root_ns, const float* __restrict__ Q,
+                                                const uint32_t* __restrict__ perm, int64_t nQ, double* __restrict__ d2_out, int32_t* __restrict__ tri_out,
                                                 double* __restrict__ cp_out, int32_t* __restrict__ flag)
 {
     const int lane = threadIdx.x;
@@ -260,10 +309,12 @@ __global__ __launch_bounds__(64) void k_closest(const uint32_t* __restrict__ slo
     const int64_t jpos = batch * 64 + lane;
     const bool valid = jpos < nQ;
     const uint32_t orig = valid ? perm[jpos] : 0u;
-    const double qx = valid ? (double)Q[3 * (int64_t)orig] : 0.0;
-    const double qy = valid ? (double)Q[3 * (int64_t)orig + 1] : 0.0;
-    const double qz = valid ? (double)Q[3 * (int64_t)orig + 2] : 0.0;
+    const float fx = valid ? Q[3 * (int64_t)orig] : 0.0f;
+    const float fy = valid ? Q[3 * (int64_t)orig + 1] : 0.0f;
+    const float fz = valid ? Q[3 * (int64_t)orig + 2] : 0.0f;
+    const double qx = fx, qy = fy, qz = fz;
     double best = INFINITY, bs = 0.0, bt = 0.0;
+    BestBounds bb;
     int32_t btri = -1;
     if (root >= 0) {
         WaveStack<NB> S;
@@ -275,85 +326,107 @@ __global__ __launch_bounds__(64) void k_closest(const uint32_t* __restrict__ slo
             uint32_t e;
             uint64_t mk;
             S.pop(sp, e, mk);
-            const bool act = __builtin_amdgcn_inverse_ballot_w64(mk); // this lane's bit of mk, as a mask
-            const int64_t node = e >> 4;
-            const int ns = (int)(e & 15u);
-            const uint32_t* nb = slots + (size_t)node * (size_t)width * kSlotWords;
-            const float* nbx = boxes + (size_t)node * (size_t)width * 6;
-            double db[kWidth];
-            uint32_t link[kWidth]; // leaf slots have the top bit set
+            const float* nbx = boxes + (size_t)(e >> 4) * (size_t)(W * kBoxWords);
+            float db[W];     // squared box distances
+            int32_t link[W]; // negative: a leaf, -1: unoccupied (its box is zeros)
+            v16f rec[W];
 #pragma unroll
-            for (int s = 0; s < kWidth; ++s) {
-                db[s] = INFINITY;
-                link[s] = 0u;
-                if (s < ns) {
-                    db[s] = box_dist2(nbx + 6 * s, qx, qy, qz);
-                    link[s] = nb[s * kSlotWords + FWN_W_LINK];
-                }
+            for (int s = 0; s < W; ++s) {
+                const v16f b = *reinterpret_cast<const v16f_a4*>(nbx + kBoxWords * s); // one scalar load
+                const float x = fmaxf(fmaxf(b[0] - fx, fx - b[3]), 0.0f);
+                const float y = fmaxf(fmaxf(b[1] - fy, fy - b[4]), 0.0f);
+                const float z = fmaxf(fmaxf(b[2] - fz, fz - b[5]), 0.0f);
+                db[s] = fmaf(z, z, fmaf(y, y, x * x));
+                link[s] = __float_as_int(b[6]);
+                rec[s] = b;
             }
+            // lanes of the node whose double box distance to slot s is below their best
+            auto nearer = [&](int s, float d) __attribute__((always_inline)) -> uint64_t {
+                const uint64_t yes = __ballot(d < bb.lo);
+                const uint64_t open = mk & ~yes & ~__ballot(d > bb.hi);
+                if (open == 0ull) return mk & yes;
+                return mk & __ballot(box_dist2(nbx + kBoxWords * s, qx, qy, qz) < best);
+            };
+            // of lanes m, those whose best the slot's disk may reach
+            auto reached = [&](int s, uint64_t m) __attribute__((always_inline)) -> uint64_t {
+                const v16f b = rec[s];
+                return m & ~__ballot(disk_bound(b[7], b[8], b[9], b[10], b[11], b[12], b[13], b[14], fx, fy, fz) > bb.hi);
+            };
             // leaf slots first
 #pragma unroll
-            for (int s = 0; s < kWidth; ++s) {
-                if (s < ns && (link[s] & FWN_LINK_LEAF) != 0u) {
-                    const bool go = act && db[s] < best;
-                    if (__ballot(go) != 0ull) {
-                        const int32_t first = (int32_t)((link[s] & ~FWN_LINK_LEAF) >> 3);
-                        const int32_t cnt = (int32_t)(link[s] & 7u) + 1;
-                        for (int32_t t = first; t < first + cnt; ++t) {
-                            const float* tw = reinterpret_cast<const float*>(tris + (size_t)t * kTriWords);
-                            // a triangle whose box is farther than the lane's best cannot improve it;
-                            // the 1e-12 margin is far above the rounding of the bound and of the
-                            // exact evaluation, so the nearest triangle (and the first of equally
-                            // near ones) is always evaluated and results do not change
-                            if (go && tri_box_dist2(tw, qx, qy, qz) <= best * (1.0 + 1e-12)) {
-                                double ss, tt;
-                                const double d = tri_closest_f64(tw, qx, qy, qz, ss, tt);
-                                if (d < best) {
-                                    best = d;
-                                    btri = t;
-                                    bs = ss;
-                                    bt = tt;
-                                }
-                            }
+            for (int s = 0; s < W; ++s) {
+                if (link[s] >= -1) continue;
+                uint64_t lanes = nearer(s, db[s]);
+                if (lanes == 0ull) continue;
+                lanes = reached(s, lanes);
+                if (lanes == 0ull) continue;
+                const bool go = __builtin_amdgcn_inverse_ballot_w64(lanes);
+                const int32_t first = (int32_t)(((uint32_t)link[s] & ~FWN_LINK_LEAF) >> 3);
+                const int32_t cnt = (link[s] & 7) + 1;
+                for (int32_t t = first; t < first + cnt; ++t) {
+                    const float* tw = reinterpret_cast<const float*>(tris + (size_t)t * kTriWords);
+                    // a triangle whose box is farther than the lane's best cannot improve it; the 1e-12
+                    // margin is far above the rounding of the bound and of the exact evaluation, so the
+                    // nearest triangle (and the first of equally near ones) is always evaluated and results
+                    // do not change.  A single triangle's box is the slot's, already compared
+                    if (go && (cnt == 1 || tri_box_dist2(tw, qx, qy, qz) <= best * (1.0 + 1e-12))) {
+                        double ss, tt;
+                        const double d = tri_closest_f64(tw, qx, qy, qz, ss, tt);
+                        if (d < best) {
+                            best = d;
+                            btri = t;
+                            bs = ss;
+                            bt = tt;
+                            bb.set(best);
                         }
                     }
                 }
             }
-            // inner slots: push farthest first so the nearest is walked next
-            uint64_t pm[kWidth];
-            float key[kWidth];
+            // inner slots: pushed farthest first so the nearest is walked next, ordered by the box
+            // distance (rounded to float, the later slot first among equals) that the slot's first
+            // participating lane sees (the wave's points are close together; the order only steers
+            // the walk).  A slot goes to the stack position its rank gives
+            uint64_t pm[W];
+            int32_t key[W]; // bits of a non-negative float; -1: not pushed
+            int n = 0;
 #pragma unroll
-            for (int s = 0; s < kWidth; ++s) {
-                const bool go = s < ns && (link[s] & FWN_LINK_LEAF) == 0u && act && db[s] < best;
-                pm[s] = __ballot(go);
-                // ordering key: the box distance seen by the slot's first participating lane (the
-                // wave's points are close together; the order only steers the walk)
-                key[s] = pm[s] ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int((float)db[s]),
-                                                                          (int)__builtin_ctzll(pm[s])))
-                               : -1.0f;
+            for (int s = 0; s < W; ++s) {
+                pm[s] = link[s] >= 0 ? nearer(s, db[s]) : 0ull;
+                if (pm[s] != 0ull && reached(s, pm[s]) == 0ull) pm[s] = 0ull;
+                key[s] = pm[s] ? __builtin_amdgcn_readlane(__float_as_int(db[s]), (int)__builtin_ctzll(pm[s])) : -1;
+                n += pm[s] ? 1 : 0;
             }
-            for (int k = 0; k < kWidth; ++k) {
-                int sel = -1;
-                float kmax = -1.0f;
+            if (n == 0) continue;
+            if (n > 1) {
+                // float distances a few units apart may be in the other order in double (a zero is exact)
+                bool close = false;
 #pragma unroll
-                for (int s = 0; s < kWidth; ++s)
-                    if (pm[s] != 0ull && key[s] >= kmax) {
-                        kmax = key[s];
-                        sel = s;
-                    }
-                if (sel < 0) break;
+                for (int s = 0; s < W; ++s)
 #pragma unroll
-                for (int s = 0; s < kWidth; ++s) {
-                    if (s == sel) {
-                        if (sp < WaveStack<NB>::kCap) {
-                            S.push(sp, lane, link[s], pm[s]); // (child << 4) | its slot count
-                            ++sp;
-                        } else {
-                            overflow = true;
-                        }
-                        pm[s] = 0ull;
-                    }
+                    for (int t = s + 1; t < W; ++t)
+                        close |= key[s] >= 0 && key[t] >= 0 && (key[s] | key[t]) != 0 &&
+                                 (uint32_t)(key[t] - key[s] + 32) <= 64u;
+                if (close) {
+#pragma unroll
+                    for (int s = 0; s < W; ++s)
+                        if (pm[s] != 0ull)
+                            key[s] = __builtin_amdgcn_readlane(
+                                __float_as_int((float)box_dist2(nbx + kBoxWords * s, qx, qy, qz)),
+                                (int)__builtin_ctzll(pm[s]));
                 }
+            }
+            if (sp + n <= WaveStack<NB>::kCap) {
+#pragma unroll
+                for (int s = 0; s < W; ++s) {
+                    int rank = 0;
+#pragma unroll
+                    for (int t = 0; t < W; ++t)
+                        if (t != s) rank += (t > s ? key[t] >= key[s] : key[t] > key[s]) ? 1 : 0;
+                    if (pm[s] != 0ull) S.push(sp + rank, lane, (uint32_t)link[s], pm[s]); // (child << 4) | its slots
+                }
+                sp += n;
+            } else {
+                overflow = true;
             }
         }
         if (overflow && lane == 0) atomicOr(flag, 1);
@@ -409,15 +482,14 @@ void run_closest(Engine& e, const float* Q, int64_t nQ, double* d2, int32_t* tri
     FWN_HIP(hipMemsetAsync(dflag, 0, sizeof(int32_t), s));
     const int64_t nb = (nQ + 63) / 64;
     if (nb > INT32_MAX) fail(FWN_LIMIT_EXCEEDED, "too many point batches");
-    if (banks == 1)
-        hipLaunchKernelGGL(k_closest<1>, dim3((unsigned)nb), dim3(64), 0, s, e.slots.as<uint32_t>(),
-                           e.boxes.as<float>(), e.width, e.tris.as<uint32_t>(), e.h_roots[0], e.h_roots[1], dQ, perm,
-                           nQ, dD, dT, dC, dflag);
-    else
-        hipLaunchKernelGGL(k_closest<3>, dim3((unsigned)nb), dim3(64), 0, s, e.slots.as<uint32_t>(),
-                           e.boxes.as<float>(), e.width, e.tris.as<uint32_t>(), e.h_roots[0], e.h_roots[1], dQ, perm,
-                           nQ, dD, dT, dC, dflag);
-    FWN_LAUNCH_CHECK("k_closest");
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)nb), dim3(64), 0, s, e.boxes.as<float>(), e.tris.as<uint32_t>(),
+                           e.h_roots[0], e.h_roots[1], dQ, perm, nQ, dD, dT, dC, dflag);
+        FWN_LAUNCH_CHECK("k_closest");
+    };
+    if (e.width == 4) go(banks == 1 ? k_closest<1, 4> : k_closest<3, 4>);
+    else if (e.width == 2) go(banks == 1 ? k_closest<1, 2> : k_closest<3, 2>);
+    else go(banks == 1 ? k_closest<1, 8> : k_closest<3, 8>);
     int32_t h_flag = 0;
     FWN_HIP(hipMemcpyAsync(&h_flag, dflag, sizeof(int32_t), hipMemcpyDeviceToHost, s));
     if (!dev) {

@@ -39,6 +39,7 @@ void hip_check(hipError_t e, const char* what, const char* file, int line);
 constexpr int kWidth = FWN_WIDTH;          // maximum slots per node
 constexpr int kSlotWords = FWN_SLOT_WORDS; // 32-bit words per slot
 constexpr int kTriWords = FWN_TRI_WORDS;   // 32-bit words per stored triangle
+constexpr int kBoxWords = 16;              // 32-bit words per slot box record
 constexpr int kRecWords = 32;              // doubles per binary-node moment record
 constexpr int kStack = 192;                // per-wave traversal stack entries
 constexpr double kFixScale = 1099511627776.0; // 2^40: fixed-point scale of FP64 near-field sums
@@ -93,7 +94,9 @@ struct Engine {
 
     // tree (resident)
     DBuf slots;      // n_nodes * width * kSlotWords u32
-    DBuf boxes;      // n_nodes * width * 6 floats: each slot's box (lo, hi), for distance queries
+    DBuf boxes;      // n_nodes * width * kBoxWords, for distance queries: each slot's box (lo, hi), its link and its
+                     // disk (t, c, R, n): the triangles are within t of the plane through c normal to n and within
+                     // R of the axis; infinity where that bounds nothing
     DBuf tris;       // n_tris * kTriWords u32
     DBuf roots;      // 2 int32 per mesh: wide root, occupied slots
     DBuf mesh_info;  // per mesh: 8 floats: qbox lo[3], qbox inv[3], tau, pad
