@@ -23,12 +23,13 @@ HIP_FLAGS = [
 ]
 
 
-# per-source additions: the slots-in-lanes traversal's FP64 constants must not be hoisted out of its
-# walk (68 vector registers instead of 118); the surrogate's MFMA kernels keep their accumulators in
-# VGPRs (the fused MLP's bias/ReLU/BF16 epilogue then reads them without 512 AGPR-to-VGPR moves per
-# tile)
+# per-source additions: the traversals' FP64 constants must not be hoisted out of their walks (61
+# vector registers instead of 112, slots in lanes 68 instead of 118); the surrogate's MFMA kernels
+# keep their accumulators in VGPRs (the fused MLP's bias/ReLU/BF16 epilogue then reads them without
+# 512 AGPR-to-VGPR moves per tile)
 EXTRA_FLAGS = {
     "fwn_point.hip": ["-mllvm", "-disable-machine-licm"],
+    "fwn_query.hip": ["-mllvm", "-disable-machine-licm"],
     "fwn_quad.hip": ["-mllvm", "-disable-machine-licm"],
     "fwn_surrogate.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }

@@ -868,8 +868,8 @@ __global__ __launch_bounds__(BT) void k_write_slots(int64_t W, int width, const 
 }
 
 // Each slot's disk, from its triangles' vertices in double; a row of 16 lanes per slot.  A slot of more
-// than kDiskTris triangles (nearly always entered, and a serial loop here) or with a sliver (sine below 1e-4: its evaluated
-// distance may be off by more than the bound allows for) gets no bound.
+// than kDiskTris triangles (nearly always entered, and a serial loop here) or with a sliver (sine below
+// 1e-4: its evaluated distance may be off by more than the bound allows for) gets no bound.
 constexpr int64_t kDiskTris = 1024;
 __global__ __launch_bounds__(BT) void k_slot_disks(int64_t nslots, const int32_t* __restrict__ slot_bin,
                                                    const double* __restrict__ rec, const int32_t* __restrict__ first,

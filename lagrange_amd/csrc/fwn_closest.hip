@@ -301,7 +301,8 @@ __device__ __forceinline__ float disk_bound(float t, float cx, float cy, float c
 template <int NB, int W>
 __global__ __launch_bounds__(64) void k_closest(const float* __restrict__ boxes, const uint32_t* __restrict__ tris,
                                                 int32_t root, int32_t root_ns, const float* __restrict__ Q,
-                                                const uint32_t* __restrict__ perm, int64_t nQ, double* __restrict__ d2_out, int32_t* __restrict__ tri_out,
+                                                const uint32_t* __restrict__ perm, int64_t nQ,
+                                                double* __restrict__ d2_out, int32_t* __restrict__ tri_out,
                                                 double* __restrict__ cp_out, int32_t* __restrict__ flag)
 {
     const int lane = threadIdx.x;
@@ -350,7 +351,8 @@ __global__ __launch_bounds__(64) void k_closest(const float* __restrict__ boxes,
             // of lanes m, those whose best the slot's disk may reach
             auto reached = [&](int s, uint64_t m) __attribute__((always_inline)) -> uint64_t {
                 const v16f b = rec[s];
-                return m & ~__ballot(disk_bound(b[7], b[8], b[9], b[10], b[11], b[12], b[13], b[14], fx, fy, fz) > bb.hi);
+                const float d = disk_bound(b[7], b[8], b[9], b[10], b[11], b[12], b[13], b[14], fx, fy, fz);
+                return m & ~__ballot(d > bb.hi);
             };
             // leaf slots first
 #pragma unroll

@@ -111,11 +111,6 @@ struct Engine {
     DBuf c_V, c_F, c_err, c_out, c_pos, c_scan, c_outp; // orientation / sampling scratch
     DBuf d_d2, d_tri, d_cp;                               // closest-point outputs for host callers
     int n_cu = 0;
-    // deferred FP64 near-field work: (sorted point, first triangle, count) items and per-point
-    // fixed-point accumulators (zero between calls)
-    DBuf q_items, q_acc;
-    int64_t item_cap = 0;
-    int64_t acc_cap = 0;
 
     // pinned host staging for small calls: metadata, points and results in one copy each way
     // (reused only after the call that filled it has synchronised its stream)
@@ -227,8 +222,7 @@ bool use_quads(const Engine& e, int64_t nQ, int banks);
 void launch_quads(Engine& e, const float* dQ, const uint32_t* perm, const int64_t* q_off, const int64_t* b_off,
                   const int32_t* order, int M, int64_t nb, float* omega, uint8_t* inside, int32_t* flag, hipStream_t s);
 // Pieces of a query that uses no engine scratch (single-mesh engine, device points): the 32-bit
-// point keys, and the traversal in sorted order `perm` with FP64 near leaves evaluated in place
-// (no work list); meta holds q_off {0, nQ}, b_off {0, batches} and the mesh order {0} (5 int64
+// point keys, and the traversal in sorted order `perm`; meta holds q_off {0, nQ}, b_off {0, batches} and the mesh order {0} (5 int64
 // words), flag one int32 (set on stack overflow).  Results equal run_queries' bit for bit.
 void launch_point_keys(Engine& e, const float* dQ, int64_t nQ, uint32_t* keys, hipStream_t s);
 void launch_traverse_inplace(Engine& e, int banks, const float* dQ, const uint32_t* perm, const int64_t* meta,

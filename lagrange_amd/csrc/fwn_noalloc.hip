@@ -5,8 +5,7 @@
 // Its scratch lives in one file-scope device array of fixed size; the host reaches each device's
 // copy through hipGetSymbolAddress, taken once per device with that device current.  The same
 // kernels as the allocating path run: point keys, the 24-bit radix sort (histograms in the
-// array), and the traversal with the FP64 near leaves evaluated in place (no work list), which
-// gives the deferred pass's value exactly.
+// array) and the traversal.
 #include <hip/hip_runtime.h>
 
 #include <mutex>

@@ -35,8 +35,8 @@ namespace {
 // Bound: VALU issue (SQ counters, 4M points, F = 199,692: 2,467 VALU instructions per wave of 16
 // uniform points over 38 node visits, 7,733 over 88 visits for points near the surface; 83 and 95 %
 // of the issue slots) once a call has enough waves, the chain of node visits below that.  Whole
-// calls, k_traverse then this kernel: 5,000 uniform points, F = 20,172 443 -> 158 us; 100k points,
-// F = 199,692 673 -> 253 us uniform, 880 -> 330 us near the surface; 4M near 4164 -> 3438 us.
+// calls, k_traverse then this kernel: 20,000 uniform points, F = 20,172 427 -> 176 us; 100k points,
+// F = 199,692 734 -> 244 us uniform, 820 -> 320 us near the surface.
 constexpr int kQuadQueue = 128; // FP64 leaves waiting (at most 63 before a node adds 64)
 constexpr int kQuadNodeBytes = 4 * kSlotWords * 4; // one 4-wide node
 
@@ -271,18 +271,22 @@ __global__ __launch_bounds__(64) void k_traverse_quad(
 
 // Whether a call of nQ points, q_off per mesh, goes to the slots-in-lanes traversal: 4-wide trees
 // of the default launch shape (the other shapes are k_traverse's, chosen by the tuner or the
-// caller), up to kQuadCross * sqrt(F) points for a mesh of F triangles.  The two kernels' costs
-// cross where the 64 points of a k_traverse wave are close together compared with the triangles
-// (uniform points, both kernels in us at 400k / 1.5M / 4M points: F = 972 127 260 557 against 146
-// 428 1032, F = 20,172 279 395 709 against 187 507 1170, F = 199,692 711 698 977 against 260 551
-// 1209, F = 940,800 1016 983 1409 against 288 587 1277), so the line grows with the surface's
-// triangle density along an axis.
-constexpr double kQuadCross = 6300.0;
+// caller), up to kQuadCross * cbrt(F) points for a mesh of F triangles.  The two kernels' costs
+// cross where the 64 points of a k_traverse wave are close together compared with the nodes they
+// visit, for points near the surface (both kernels walk to the triangles) at fewer points than for
+// uniform ones; the line lies between the two crossings.  k_traverse / this kernel in us,
+//   uniform: F = 972 171 / 156 (200k points) and 191 / 212 (400k); F = 20,172 341 / 257 (400k),
+//     366 / 368 (800k), 467 / 578 (1.5M); F = 199,692 713 / 431 (800k), 800 / 627 (1.5M), 1095 /
+//     1333 (4M); F = 940,800 1182 / 681 (1.5M), 1576 / 1408 (4M);
+//   near the surface: F = 972 179 / 179 (200k); F = 20,172 431 / 396 (400k), 507 / 619 (800k);
+//     F = 199,692 724 / 586 (400k), 886 / 913 (800k), 1156 / 1465 (1.5M); F = 940,800 1472 / 1343
+//     (800k), 1834 / 2128 (1.5M).
+constexpr double kQuadCross = 24000.0;
 bool use_quads(const Engine& e, int64_t nQ, int banks)
 {
     if (e.width != 4 || banks != 1 || !default_shape(e)) return false;
     double cross = 0.0;
-    for (int m = 0; m < e.n_meshes; ++m) cross += std::sqrt((double)(e.h_f_off[m + 1] - e.h_f_off[m]));
+    for (int m = 0; m < e.n_meshes; ++m) cross += std::cbrt((double)(e.h_f_off[m + 1] - e.h_f_off[m]));
     return (double)nQ <= kQuadCross * cross;
 }
 

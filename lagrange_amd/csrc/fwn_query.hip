@@ -16,7 +16,14 @@
 //    traversal (children pushed in slot order, popped last-in-first-out), so each point gets
 //    the same result the per-point reference loop would give on this tree.
 // Triangles closer than tau (near_fp64_rel x bbox diagonal) to the leaf's bounding sphere
-// use the FP64 van Oosterom-Strackee formula.
+// use the FP64 van Oosterom-Strackee formula, 64 leaves at a time from a queue in LDS.
+//
+// Bound: VALU issue for points close together (16.7M grid points, F = 940,800: 98 % of the issue
+// slots).  Compiled without machine LICM, which would hold the FP64 constants in 45 vector registers
+// through the walk (112 registers, 4 waves per SIMD, instead of 61 and 8).  Before the queue, FP64
+// leaves went to a work list in memory for two more kernels, its slots claimed 64 at a time from one
+// counter, which points near the surface saturated: 4M of them, F = 199,692, 4.30 -> 2.29 ms (the
+// three kernels 3.44 + 0.30 + 0.27 -> 2.05 ms), the grid 3.54 -> 3.52 ms.
 #include <hip/hip_runtime.h>
 
 #include <cstring>
@@ -99,42 +106,27 @@ __device__ __forceinline__ float far_field_acc(const SlotRegs& r, float dx, floa
     return fmaf(t, inv3, om);
 }
 
-// Deferred FP64 items are written in chunks of kItemChunk slots: a wave claims a chunk with one
-// atomic on the chunk counter and fills it over several leaves, so the shared counter sees one
-// atomic per 64 items instead of one per leaf event.  Unfilled slots of a chunk are written as
-// empty items (count 0), which the FP64 kernels skip.
-constexpr uint32_t kItemChunk = 64;
-struct ItemChunk {
-    uint32_t base = 0u;         // first item slot of the wave's open chunk
-    uint32_t fill = kItemChunk; // slots used in it (kItemChunk: no chunk open)
-};
-
-__device__ __forceinline__ void pad_chunk(const ItemChunk& ch, int lane, uint32_t* __restrict__ items,
-                                          uint32_t item_cap)
+// LDS of a traversal wave: the queue of FP64 near leaves (link without its leaf bit, lane), at most 63
+// left over and a node's 64 per slot, and the lanes' FP64 sums in 2^-40 fixed point
+__host__ __device__ __forceinline__ constexpr int queue_entries(int width) { return 64 + 64 * width; }
+__host__ __device__ __forceinline__ constexpr size_t traverse_lds_bytes(int width)
 {
-    if ((uint32_t)lane >= ch.fill) {
-        const uint32_t k = ch.base + (uint32_t)lane;
-        if (k < item_cap) {
-            items[3 * (size_t)k] = 0u;
-            items[3 * (size_t)k + 1] = 0u;
-            items[3 * (size_t)k + 2] = 0u;
-        }
-    }
+    return sizeof(uint2) * (size_t)queue_entries(width) + sizeof(unsigned long long) * 64;
 }
 
 // One batch of up to bpts <= 64 points (one per lane) of one mesh, walked through that mesh's
-// tree (bpts is 64 except in small calls, which spread their points over more waves).  INL:
-// FP64 near leaves are evaluated in place (each leaf's FP64 sum in 2^-40 fixed point, the
-// point's total added once at the end: the value the deferred pass gives) instead of being
-// deferred to the work list; for calls that use no work list.
-template <bool STATS, int NB, bool INL = false>
+// tree (bpts is 64 except in small calls, which spread their points over more waves).  FP64 near
+// leaves are queued in LDS and evaluated 64 at a time, one leaf per lane whichever point it
+// belongs to; a leaf's sum goes to its point's accumulator in 2^-40 fixed point (integer addition
+// is associative: the total does not depend on the order) and the total is added once at the end.
+template <bool STATS, int NB>
 __device__ __forceinline__ void traverse_batch(
     int64_t batch, const uint32_t* __restrict__ slots, int width, const uint32_t* __restrict__ tris,
     const int32_t* __restrict__ roots, const float* __restrict__ minfo, const float* __restrict__ Q,
     const uint32_t* __restrict__ perm, const int64_t* __restrict__ q_off, const int64_t* __restrict__ b_off,
     const int32_t* __restrict__ mesh_order, int M, int bpts, float beta2, float* __restrict__ omega,
-    uint8_t* __restrict__ inside, int32_t* __restrict__ stats, uint32_t* __restrict__ items,
-    uint32_t* __restrict__ n_chunks, uint32_t item_cap, int32_t* __restrict__ flag, ItemChunk& ch)
+    uint8_t* __restrict__ inside, int32_t* __restrict__ stats, int32_t* __restrict__ flag, uint2* queue,
+    unsigned long long* acc)
 {
     const int lane = threadIdx.x & 63;
     // batches are numbered over the meshes in mesh_order; b_off is the prefix over that order
@@ -144,120 +136,127 @@ __device__ __forceinline__ void traverse_batch(
     const int64_t cnt64 = q_off[m + 1] - start;
     const int cnt = cnt64 < bpts ? (int)cnt64 : bpts;
     const bool valid = lane < cnt;
-    const uint32_t jpos = (uint32_t)(start + lane); // sorted position of this lane's point
-    const uint32_t orig = valid ? (perm ? perm[jpos] : jpos) : 0u;
+    const uint32_t orig = valid ? (perm ? perm[start + lane] : (uint32_t)(start + lane)) : 0u;
     const float qx = valid ? Q[3 * (int64_t)orig] : 0.0f;
     const float qy = valid ? Q[3 * (int64_t)orig + 1] : 0.0f;
     const float qz = valid ? Q[3 * (int64_t)orig + 2] : 0.0f;
     const int32_t root = roots[2 * m];
     const int32_t root_ns = roots[2 * m + 1];
     const float tau = minfo[8 * m + 6];
-    const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
 
+    const uint32_t node_words = (uint32_t)width * kSlotWords;
     float om = 0.0f;
-    unsigned long long acc64 = 0ull; // INL: FP64 near leaves in 2^-40 fixed point
+    int nq = 0;  // queued FP64 leaves
+    int n64 = 0; // all that were queued
     int32_t n_test = 0, n_far = 0, n_t32 = 0, n_t64 = 0;
-    if (root >= 0) {
+    if (root >= 0 && root_ns > 0) { // an inner node has a slot at least
         WaveStack<NB> S;
         S.push(0, lane, ((uint32_t)root << 4) | (uint32_t)root_ns, __ballot(valid));
         int sp = 1;
-        bool overflow = false;
-        while (sp > 0) {
-            --sp;
-            uint32_t e;
-            uint64_t mk;
-            S.pop(sp, e, mk);
-            const bool act = __builtin_amdgcn_inverse_ballot_w64(mk); // this lane's bit of mk, as a mask
-            const uint32_t* nb = slots + (size_t)(e >> 4) * (size_t)width * kSlotWords;
-            const int ns = (int)(e & 15u);
-            if (ns == 0) continue;
-            // one slot: test, far term, leaf triangles or push of the child
-            auto slot = [&](const SlotRegs& cur) __attribute__((always_inline)) {
-                const float dx = sw(cur, FWN_W_PX) - qx, dy = sw(cur, FWN_W_PY) - qy, dz = sw(cur, FWN_W_PZ) - qz;
-                const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-                const bool far = d2 > sw(cur, FWN_W_THR); // beta^2 r^2, written by the build
-                // near lanes: active and not far (scalar mask arithmetic on the compare's ballot,
-                // taken before the divergent far-field branch)
-                const uint64_t nearm = mk & ~__ballot(far);
-                if (STATS) n_test += act ? 1 : 0;
-                if (act && far) {
-                    om = far_field_acc(cur, dx, dy, dz, d2, om);
-                    if (STATS) ++n_far;
-                }
-                const uint32_t link = su(cur, FWN_W_LINK);
-                if (nearm == 0ull) return;
-                // written above the stack top for every slot with near lanes, kept (sp advanced)
-                // only for an internal slot: the writelanes then sit in a branch-free block and
-                // the stack registers need no copies.  The position written is below the
-                // capacity (the host keeps a one-entry margin for it), so the entries below stay
-                // intact; an overflow is checked once per node.  The link of an internal slot is
-                // the stack entry: (child << 4) | its slot count
-                S.push(sp, lane, link, nearm);
-                const bool leaf = (int32_t)link < 0; // FWN_LINK_LEAF is the sign bit
-                sp += leaf ? 0 : 1;
-                if (leaf) {
-                    const int32_t first = (int32_t)((link & ~FWN_LINK_LEAF) >> 3);
-                    const int32_t tcnt = (int32_t)(link & 7u) + 1;
-                    const bool nl = __builtin_amdgcn_inverse_ballot_w64(nearm);
-                    // FP64 for points within tau of the leaf's bounding sphere and, for a single
-                    // triangle, within tau of its plane (p lies on that plane); both thresholds are
-                    // stored in the leaf's first triangle
-                    const float* t0 = reinterpret_cast<const float*>(tris + (size_t)first * kTriWords);
-                    const float near2 = t0[FWN_T_NEAR2], plane = t0[FWN_T_PLANE];
-                    const float nd = fmaf(dx, sw(cur, FWN_W_NX), fmaf(dy, sw(cur, FWN_W_NY), dz * sw(cur, FWN_W_NZ)));
-                    const bool use64 = nl && tau > 0.0f && d2 < near2 && (tcnt > 1 || nd * nd < plane);
-                    const bool use32 = nl && !use64;
-                    if (__ballot(use32) != 0ull) {
-                        for (int32_t t = first; t < first + tcnt; ++t) {
-                            const float* tw = reinterpret_cast<const float*>(tris + (size_t)t * kTriWords);
-                            if (use32) {
-                                om += tri_f32(tw, qx, qy, qz);
-                                if (STATS) ++n_t32;
+        int sp_max = 1;
+        do {
+            while (((sp - 1) | (63 - nq)) >= 0) { // sp > 0 and nq < 64
+                --sp;
+                uint32_t e;
+                uint64_t mk;
+                S.pop(sp, e, mk);
+                const bool act = __builtin_amdgcn_inverse_ballot_w64(mk); // this lane's bit of mk, as a mask
+                const uint32_t* nb = slots + (size_t)(e >> 4) * node_words;
+                const int ns = (int)(e & 15u);
+                // one slot: test, far term, leaf triangles or push of the child
+                auto slot = [&](const SlotRegs& cur) __attribute__((always_inline)) {
+                    const float dx = sw(cur, FWN_W_PX) - qx, dy = sw(cur, FWN_W_PY) - qy, dz = sw(cur, FWN_W_PZ) - qz;
+                    const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                    const bool far = d2 > sw(cur, FWN_W_THR); // beta^2 r^2, written by the build
+                    // near lanes: active and not far (scalar mask arithmetic on the compare's ballot,
+                    // taken before the divergent far-field branch)
+                    const uint64_t nearm = mk & ~__ballot(far);
+                    if (STATS) n_test += act ? 1 : 0;
+                    if (act && far) {
+                        om = far_field_acc(cur, dx, dy, dz, d2, om);
+                        if (STATS) ++n_far;
+                    }
+                    const uint32_t link = su(cur, FWN_W_LINK);
+                    if (nearm == 0ull) return;
+                    // written above the stack top for every slot with near lanes, kept (sp advanced)
+                    // only for an internal slot: the writelanes then sit in a branch-free block and
+                    // the stack registers need no copies.  The position written is below the
+                    // capacity (the host keeps a one-entry margin for it), so the entries below stay
+                    // intact; an overflow is checked once per node.  The link of an internal slot is
+                    // the stack entry: (child << 4) | its slot count
+                    S.push(sp, lane, link, nearm);
+                    const bool leaf = (int32_t)link < 0; // FWN_LINK_LEAF is the sign bit
+                    sp += leaf ? 0 : 1;
+                    if (leaf) {
+                        const int32_t first = (int32_t)((link & ~FWN_LINK_LEAF) >> 3);
+                        const int32_t tcnt = (int32_t)(link & 7u) + 1;
+                        const bool nl = __builtin_amdgcn_inverse_ballot_w64(nearm);
+                        // FP64 for points within tau of the leaf's bounding sphere and, for a single
+                        // triangle, within tau of its plane (p lies on that plane); both thresholds are
+                        // stored in the leaf's first triangle
+                        const float* t0 = reinterpret_cast<const float*>(tris + (size_t)first * kTriWords);
+                        const float near2 = t0[FWN_T_NEAR2], plane = t0[FWN_T_PLANE];
+                        const float nd =
+                            fmaf(dx, sw(cur, FWN_W_NX), fmaf(dy, sw(cur, FWN_W_NY), dz * sw(cur, FWN_W_NZ)));
+                        const bool use64 = nl && tau > 0.0f && d2 < near2 && (tcnt > 1 || nd * nd < plane);
+                        const bool use32 = nl && !use64;
+                        if (__ballot(use32) != 0ull) {
+                            for (int32_t t = first; t < first + tcnt; ++t) {
+                                const float* tw = reinterpret_cast<const float*>(tris + (size_t)t * kTriWords);
+                                if (use32) {
+                                    om += tri_f32(tw, qx, qy, qz);
+                                    if (STATS) ++n_t32;
+                                }
                             }
                         }
-                    }
-                    const uint64_t m64 = __ballot(use64);
-                    if (INL && m64 != 0ull) {
-                        if (use64) {
-                            double s64 = 0.0;
-                            for (int32_t t = first; t < first + tcnt; ++t)
-                                s64 += tri_f64(reinterpret_cast<const float*>(tris + (size_t)t * kTriWords), qx, qy, qz);
-                            acc64 += (unsigned long long)__double2ll_rn(s64 * kFixScale);
-                            if (STATS) n_t64 += tcnt;
-                        }
-                    } else if (m64 != 0ull) {
-                        // deferred: (point, leaf) items, evaluated in FP64 by k_near64
-                        const uint32_t c = (uint32_t)__popcll(m64);
-                        if (ch.fill + c > kItemChunk) {
-                            pad_chunk(ch, lane, items, item_cap);
-                            uint32_t nc = 0u;
-                            if (lane == 0) nc = atomicAdd(n_chunks, 1u);
-                            nc = __builtin_amdgcn_readfirstlane(nc);
-                            ch.base = min(nc, 0xFFFFFFFFu / kItemChunk) * kItemChunk;
-                            ch.fill = 0u;
-                        }
-                        if (use64) {
-                            const uint32_t k = ch.base + ch.fill + (uint32_t)__popcll(m64 & lt_mask);
-                            if (k < item_cap) {
-                                items[3 * (size_t)k] = jpos;
-                                items[3 * (size_t)k + 1] = (uint32_t)first;
-                                items[3 * (size_t)k + 2] = (uint32_t)tcnt;
+                        const uint64_t m64 = __ballot(use64);
+                        if (m64 != 0ull) {
+                            if (n64 == 0) acc[lane] = 0ull;
+                            if (use64) {
+                                const uint32_t below = __builtin_amdgcn_mbcnt_hi(
+                                    (uint32_t)(m64 >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m64, 0u));
+                                queue[nq + (int)below] = make_uint2(link & ~FWN_LINK_LEAF, (uint32_t)lane);
+                                if (STATS) n_t64 += tcnt;
                             }
-                            if (STATS) n_t64 += tcnt;
+                            nq += (int)__popcll(m64);
+                            n64 += (int)__popcll(m64);
                         }
-                        ch.fill += c;
                     }
+                };
+                const uint32_t* sl = nb;
+                int s = 0;
+                do {
+                    slot(load_slot(sl));
+                    sl += kSlotWords;
+                } while (++s < ns);
+                // the host only launches trees whose stack bound 1 + (width - 1) depth fits; a push
+                // past the capacity is reported
+                sp_max = max(sp_max, sp);
+            }
+            // 64 queued leaves, or what is left at the end
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            while (nq >= 64 || (sp == 0 && nq > 0)) {
+                const int take = min(nq, 64);
+                nq -= take;
+                const uint2 it = queue[nq + (lane < take ? lane : 0)];
+                // the leaf's point, from its own lane's registers
+                const float x = __shfl(qx, (int)it.y), y = __shfl(qy, (int)it.y), z = __shfl(qz, (int)it.y);
+                if (lane < take) {
+                    const uint32_t first = it.x >> 3, n = (it.x & 7u) + 1u;
+                    double s64 = 0.0;
+                    for (uint32_t t = first; t < first + n; ++t)
+                        s64 += tri_f64(reinterpret_cast<const float*>(tris + (size_t)t * kTriWords), x, y, z);
+                    atomicAdd(&acc[it.y], (unsigned long long)__double2ll_rn(s64 * kFixScale));
                 }
-            };
-            const uint32_t* sl = nb;
-            for (int s = 0; s < ns; ++s, sl += kSlotWords) slot(load_slot(sl));
-            // the host only launches trees whose stack bound 1 + (width - 1) depth fits; a push
-            // past the capacity is reported
-            overflow |= sp > WaveStack<NB>::kCap;
-        }
-        if (overflow && lane == 0) atomicOr(flag, 1);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        } while (sp > 0);
+        if (sp_max > WaveStack<NB>::kCap && lane == 0) atomicOr(flag, 1);
     }
-    if (INL && acc64 != 0ull) om = (float)((double)om + (double)(long long)acc64 * (1.0 / kFixScale));
+    if (n64 > 0) {
+        const long long v = (long long)acc[lane];
+        if (v != 0) om = (float)((double)om + (double)v * (1.0 / kFixScale));
+    }
     if (valid) {
         omega[orig] = om;
         if (inside) inside[orig] = ((double)om / (4.0 * 3.14159265358979323846) > 0.5) ? 1 : 0;
@@ -273,81 +272,33 @@ __device__ __forceinline__ void traverse_batch(
 // Grid launch: one wave per batch, XCD-aware block order.  Persistent launch: a grid sized to
 // the device's resident waves; each wave takes batches from a work counter until none is left
 // (the batch numbering puts the meshes with the most triangles first).
-template <bool STATS, int WAVES, bool PERSIST, int NB, bool INL = false>
+template <bool STATS, int WAVES, bool PERSIST, int NB>
 __global__ __launch_bounds__(WAVES * 64) void k_traverse(
     const uint32_t* __restrict__ slots, int width, const uint32_t* __restrict__ tris,
     const int32_t* __restrict__ roots, const float* __restrict__ minfo, const float* __restrict__ Q,
     const uint32_t* __restrict__ perm, const int64_t* __restrict__ q_off, const int64_t* __restrict__ b_off,
     const int32_t* __restrict__ mesh_order, int M, int64_t n_batches, int bpts, float beta2, float* __restrict__ omega,
-    uint8_t* __restrict__ inside, int32_t* __restrict__ stats, uint32_t* __restrict__ items,
-    uint32_t* __restrict__ n_chunks, uint32_t item_cap, int32_t* __restrict__ flag, uint32_t* __restrict__ work)
+    uint8_t* __restrict__ inside, int32_t* __restrict__ stats, int32_t* __restrict__ flag, uint32_t* __restrict__ work)
 {
-    ItemChunk ch;
+    extern __shared__ uint4 traverse_lds[];
+    char* lds = reinterpret_cast<char*>(traverse_lds) + (size_t)(threadIdx.x >> 6) * traverse_lds_bytes(width);
+    unsigned long long* acc = reinterpret_cast<unsigned long long*>(lds);
+    uint2* queue = reinterpret_cast<uint2*>(acc + 64);
     if (!PERSIST) {
         const int64_t batch = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * WAVES + (threadIdx.x >> 6);
         if (batch >= n_batches) return; // whole wave
-        traverse_batch<STATS, NB, INL>(batch, slots, width, tris, roots, minfo, Q, perm, q_off, b_off, mesh_order, M, bpts,
-                                  beta2, omega, inside, stats, items, n_chunks, item_cap, flag, ch);
+        traverse_batch<STATS, NB>(batch, slots, width, tris, roots, minfo, Q, perm, q_off, b_off, mesh_order, M, bpts,
+                                  beta2, omega, inside, stats, flag, queue, acc);
     } else {
         for (;;) {
             uint32_t b = 0u;
             if ((threadIdx.x & 63) == 0) b = atomicAdd(work, 1u);
             b = __builtin_amdgcn_readfirstlane(b);
             if ((int64_t)b >= n_batches) break; // every wave leaves once the counter passes the end
-            traverse_batch<STATS, NB, INL>((int64_t)b, slots, width, tris, roots, minfo, Q, perm, q_off, b_off, mesh_order, M,
-                                      bpts, beta2, omega, inside, stats, items, n_chunks, item_cap, flag, ch);
+            traverse_batch<STATS, NB>((int64_t)b, slots, width, tris, roots, minfo, Q, perm, q_off, b_off, mesh_order, M,
+                                      bpts, beta2, omega, inside, stats, flag, queue, acc);
         }
     }
-    if (!INL) pad_chunk(ch, threadIdx.x & 63, items, item_cap); // close the wave's open chunk
-}
-
-// FP64 solid angles of the deferred (point, leaf) items, summed per point in 2^-40 fixed
-// point: integer addition is associative, so the per-point sum does not depend on the order
-// in which items are processed.
-__global__ __launch_bounds__(256) void k_near64(const uint32_t* __restrict__ items,
-                                                const uint32_t* __restrict__ n_chunks, uint32_t item_cap,
-                                                const uint32_t* __restrict__ tris, const float* __restrict__ Q,
-                                                const uint32_t* __restrict__ perm,
-                                                unsigned long long* __restrict__ acc)
-{
-    const uint32_t n = (uint32_t)min((uint64_t)*n_chunks * kItemChunk, (uint64_t)item_cap);
-    for (uint32_t k = blockIdx.x * 256u + threadIdx.x; k < n; k += gridDim.x * 256u) {
-        const uint32_t j = items[3 * (size_t)k], first = items[3 * (size_t)k + 1], cnt = items[3 * (size_t)k + 2];
-        if (cnt == 0u) continue; // unfilled slot of a chunk
-        const uint32_t orig = perm ? perm[j] : j;
-        const float qx = Q[3 * (size_t)orig], qy = Q[3 * (size_t)orig + 1], qz = Q[3 * (size_t)orig + 2];
-        double s = 0.0;
-        for (uint32_t t = first; t < first + cnt; ++t)
-            s += tri_f64(reinterpret_cast<const float*>(tris + (size_t)t * kTriWords), qx, qy, qz);
-        atomicAdd(&acc[j], (unsigned long long)__double2ll_rn(s * kFixScale));
-    }
-}
-
-// omega = fp32 sum + FP64 near-field sum, once per point: the item that takes the accumulator
-// (atomic exchange with 0) does the update, which also leaves the accumulator zeroed.
-__global__ __launch_bounds__(256) void k_near64_combine(const uint32_t* __restrict__ items,
-                                                        const uint32_t* __restrict__ n_chunks, uint32_t item_cap,
-                                                        const uint32_t* __restrict__ perm,
-                                                        unsigned long long* __restrict__ acc,
-                                                        float* __restrict__ omega, uint8_t* __restrict__ inside)
-{
-    const uint32_t n = (uint32_t)min((uint64_t)*n_chunks * kItemChunk, (uint64_t)item_cap);
-    for (uint32_t k = blockIdx.x * 256u + threadIdx.x; k < n; k += gridDim.x * 256u) {
-        if (items[3 * (size_t)k + 2] == 0u) continue; // unfilled slot of a chunk
-        const uint32_t j = items[3 * (size_t)k];
-        const long long v = (long long)atomicExch(&acc[j], 0ull);
-        if (v == 0) continue;
-        const uint32_t orig = perm ? perm[j] : j;
-        const float om = (float)((double)omega[orig] + (double)v * (1.0 / kFixScale));
-        omega[orig] = om;
-        if (inside) inside[orig] = ((double)om / (4.0 * 3.14159265358979323846) > 0.5) ? 1 : 0;
-    }
-}
-
-__global__ void k_fill_u64(unsigned long long* __restrict__ p, int64_t n)
-{
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0ull;
 }
 
 __global__ __launch_bounds__(256) void k_bruteforce(const uint32_t* __restrict__ tris, int64_t first, int64_t cnt,
@@ -363,11 +314,10 @@ __global__ __launch_bounds__(256) void k_bruteforce(const uint32_t* __restrict__
     if (valid) out[i] = s;
 }
 
-__global__ void k_zero3(int32_t* a)
+__global__ void k_zero2(int32_t* a) // overflow flag, work counter
 {
     a[0] = 0;
     a[1] = 0;
-    a[2] = 0;
 }
 
 template <bool ST, int WV, bool PE, int NB>
@@ -378,12 +328,16 @@ void* traverse_fn()
 
 // banks: traversal stack banks the tree needs (1: 64 entries, 3: kStack entries)
 template <typename... Args>
-void launch_traverse(bool stats, int waves, bool persist, int banks, unsigned nblk, hipStream_t s, Args... args)
+void launch_traverse(bool stats, int waves, bool persist, int banks, int width, unsigned nblk, hipStream_t s,
+                     Args... args)
 {
-#define FWN_TRAV(ST, WV, PE)                                                                                  \
-    do {                                                                                                      \
-        if (banks == 1) hipLaunchKernelGGL((k_traverse<ST, WV, PE, 1>), dim3(nblk), dim3(WV * 64), 0, s, args...); \
-        else hipLaunchKernelGGL((k_traverse<ST, WV, PE, 3>), dim3(nblk), dim3(WV * 64), 0, s, args...);        \
+#define FWN_TRAV(ST, WV, PE)                                                                               \
+    do {                                                                                                   \
+        const size_t lds = (WV) * traverse_lds_bytes(width);                                               \
+        if (banks == 1)                                                                                    \
+            hipLaunchKernelGGL((k_traverse<ST, WV, PE, 1>), dim3(nblk), dim3(WV * 64), lds, s, args...);   \
+        else                                                                                               \
+            hipLaunchKernelGGL((k_traverse<ST, WV, PE, 3>), dim3(nblk), dim3(WV * 64), lds, s, args...);   \
     } while (0)
     if (stats) {
         FWN_TRAV(true, 1, false);
@@ -404,7 +358,7 @@ void launch_traverse(bool stats, int waves, bool persist, int banks, unsigned nb
 }
 
 // resident workgroups per CU of a traversal variant (persistent grid size)
-int resident_blocks(bool persist, int waves, int banks)
+int resident_blocks(bool persist, int waves, int banks, int width)
 {
     const void* f = nullptr;
     const bool one = banks == 1;
@@ -416,7 +370,7 @@ int resident_blocks(bool persist, int waves, int banks)
     default: fail(FWN_INVALID_ARGUMENT, "unknown persistent launch shape (waves per block 1, 2, 4 or 8)");
     }
     int nb = 0;
-    FWN_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, waves * 64, 0));
+    FWN_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, waves * 64, waves * traverse_lds_bytes(width)));
     return nb > 0 ? nb : 1;
 }
 
@@ -516,17 +470,6 @@ void run_queries_pipelined(Engine& e, const float* Q, int64_t nQ, float* omega, 
         e.q_keys[k].reserve(sizeof(uint32_t) * C);
         e.q_vals[k].reserve(sizeof(uint32_t) * C);
     }
-    if (e.acc_cap < C) {
-        e.q_acc.alloc(sizeof(unsigned long long) * C);
-        e.acc_cap = C;
-        hipLaunchKernelGGL(k_fill_u64, dim3(grid_blocks(C, 256)), dim3(256), 0, s, e.q_acc.as<unsigned long long>(),
-                           C);
-        FWN_LAUNCH_CHECK("k_fill_u64");
-    }
-    if (e.item_cap < std::max<int64_t>(C, 1 << 20)) {
-        e.item_cap = std::max<int64_t>(C, 1 << 20);
-        e.q_items.alloc(sizeof(uint32_t) * 3 * (size_t)e.item_cap);
-    }
     // per chunk: q_off {0, n}, b_off {0, batches}, mesh order {0} (5 int64 words)
     std::vector<int64_t> meta(5 * nch, 0);
     for (int64_t k = 0; k < nch; ++k) {
@@ -536,7 +479,7 @@ void run_queries_pipelined(Engine& e, const float* Q, int64_t nQ, float* omega, 
     }
     e.q_pmeta.reserve(sizeof(int64_t) * meta.size());
     FWN_HIP(hipMemcpyAsync(e.q_pmeta.p, meta.data(), sizeof(int64_t) * meta.size(), hipMemcpyHostToDevice, s));
-    e.q_pflags.reserve(sizeof(int32_t) * 4 * nch);
+    e.q_pflags.reserve(sizeof(int32_t) * 2 * nch);
     const int waves = e.opt.waves_per_block > 0 ? e.opt.waves_per_block : 1;
     const bool persist = e.opt.launch_mode == FWN_LAUNCH_PERSISTENT;
     if (persist && e.n_cu == 0) {
@@ -545,7 +488,6 @@ void run_queries_pipelined(Engine& e, const float* Q, int64_t nQ, float* omega, 
         e.n_cu = prop.multiProcessorCount;
     }
     const float beta2 = e.opt.accuracy_scale * e.opt.accuracy_scale;
-    const uint32_t cap = (uint32_t)e.item_cap;
 
     for (int64_t k = 0; k <= nch; ++k) {
         if (k < nch) {
@@ -558,7 +500,7 @@ void run_queries_pipelined(Engine& e, const float* Q, int64_t nQ, float* omega, 
                                    e.cs_in));
             FWN_HIP(hipEventRecord(e.pev[sl], e.cs_in));
             FWN_HIP(hipStreamWaitEvent(s, e.pev[sl], 0));
-            // chunk k on the engine's stream: sort, traversal, FP64 pass (no host wait)
+            // chunk k on the engine's stream: sort and traversal (no host wait)
             const float* dQ = dIn3 + 3 * off;
             const int64_t* d_qoff = e.q_pmeta.as<int64_t>() + 5 * k;
             const int64_t* d_boff = d_qoff + 2;
@@ -573,24 +515,17 @@ void run_queries_pipelined(Engine& e, const float* Q, int64_t nQ, float* omega, 
             radix_sort_pairs32(kp, vp, kp2, vp2, ck, 8, 32, true, e.q_hist, e.q_rowsum, s);
             const int64_t nb = (ck + 63) / 64;
             int64_t nblk = (nb + waves - 1) / waves;
-            if (persist) nblk = std::min<int64_t>(nblk, (int64_t)e.n_cu * resident_blocks(true, waves, banks));
-            int32_t* dflag = e.q_pflags.as<int32_t>() + 4 * k;
-            uint32_t* dnitems = reinterpret_cast<uint32_t*>(dflag + 1);
-            uint32_t* dwork = reinterpret_cast<uint32_t*>(dflag + 2);
-            hipLaunchKernelGGL(k_zero3, dim3(1), dim3(1), 0, s, dflag);
+            if (persist) nblk = std::min<int64_t>(nblk, (int64_t)e.n_cu * resident_blocks(true, waves, banks, e.width));
+            int32_t* dflag = e.q_pflags.as<int32_t>() + 2 * k;
+            uint32_t* dwork = reinterpret_cast<uint32_t*>(dflag + 1);
+            hipLaunchKernelGGL(k_zero2, dim3(1), dim3(1), 0, s, dflag);
             FWN_HIP(hipEventRecord(e.tev[2 * k], s));
-            launch_traverse(false, waves, persist, banks, (unsigned)nblk, s, e.slots.as<uint32_t>(), e.width,
+            launch_traverse(false, waves, persist, banks, e.width, (unsigned)nblk, s, e.slots.as<uint32_t>(), e.width,
                             e.tris.as<uint32_t>(), e.roots.as<int32_t>(), e.mesh_info.as<float>(), dQ, vp, d_qoff,
                             d_boff, d_order, 1, nb, 64, beta2, dOm + off, dIn ? dIn + off : nullptr, (int32_t*)nullptr,
-                            e.q_items.as<uint32_t>(), dnitems, cap, dflag, dwork);
+                            dflag, dwork);
             FWN_LAUNCH_CHECK("k_traverse");
             FWN_HIP(hipEventRecord(e.tev[2 * k + 1], s));
-            hipLaunchKernelGGL(k_near64, dim3(2048), dim3(256), 0, s, e.q_items.as<uint32_t>(), dnitems, cap,
-                               e.tris.as<uint32_t>(), dQ, vp, e.q_acc.as<unsigned long long>());
-            FWN_LAUNCH_CHECK("k_near64");
-            hipLaunchKernelGGL(k_near64_combine, dim3(2048), dim3(256), 0, s, e.q_items.as<uint32_t>(), dnitems,
-                               cap, vp, e.q_acc.as<unsigned long long>(), dOm + off, dIn ? dIn + off : nullptr);
-            FWN_LAUNCH_CHECK("k_near64_combine");
             FWN_HIP(hipEventRecord(e.pev[2 + sl], s));
             // chunk k's results back to the pinned buffer on the other copy stream; chunk k-2's
             // results were copied out of that buffer in the previous iteration
@@ -610,8 +545,8 @@ void run_queries_pipelined(Engine& e, const float* Q, int64_t nQ, float* omega, 
             if (inside) parallel_copy(inside + off, pin_i8(sl), (size_t)cj);
         }
     }
-    std::vector<int32_t> fl(4 * nch);
-    FWN_HIP(hipMemcpyAsync(fl.data(), e.q_pflags.p, sizeof(int32_t) * 4 * nch, hipMemcpyDeviceToHost, s));
+    std::vector<int32_t> fl(2 * nch);
+    FWN_HIP(hipMemcpyAsync(fl.data(), e.q_pflags.p, sizeof(int32_t) * 2 * nch, hipMemcpyDeviceToHost, s));
     FWN_HIP(hipStreamSynchronize(s));
     FWN_HIP(hipStreamSynchronize(e.cs_in));
     FWN_HIP(hipStreamSynchronize(e.cs_out));
@@ -625,18 +560,8 @@ void run_queries_pipelined(Engine& e, const float* Q, int64_t nQ, float* omega, 
     }
     e.last_traverse_ms = t_tr / (double)nch; // average over the chunks' launches
     e.last_total_ms = t_all;
-    for (int64_t k = 0; k < nch; ++k) {
-        if (fl[4 * k]) fail(FWN_LIMIT_EXCEEDED, "traversal stack overflow");
-        const int64_t need = (int64_t)(uint32_t)fl[4 * k + 1] * kItemChunk;
-        if (need > (int64_t)cap) { // the chunk's FP64 work list overflowed its capacity in the
-                                   // pipeline (a redo may have grown it since): answer it again
-            const int64_t off = k * C, ck = std::min(C, nQ - off);
-            const double tr = e.last_traverse_ms, tot = e.last_total_ms;
-            run_queries(e, Q + 3 * off, nullptr, ck, omega + off, inside ? inside + off : nullptr, nullptr, false);
-            e.last_traverse_ms = tr;
-            e.last_total_ms = tot + e.last_total_ms; // the redo is part of this call's device time
-        }
-    }
+    for (int64_t k = 0; k < nch; ++k)
+        if (fl[2 * k]) fail(FWN_LIMIT_EXCEEDED, "traversal stack overflow");
 }
 
 } // namespace
@@ -657,14 +582,9 @@ void launch_traverse_inplace(Engine& e, int banks, const float* dQ, const uint32
     const int64_t* q_off = meta;
     const int64_t* b_off = meta + 2;
     const int32_t* order = reinterpret_cast<const int32_t*>(meta + 4);
-#define FWN_TRAV_INL(NB)                                                                                            \
-    hipLaunchKernelGGL((k_traverse<false, 1, false, NB, true>), dim3((unsigned)nb), dim3(64), 0, s,                \
-                       e.slots.as<uint32_t>(), e.width, e.tris.as<uint32_t>(), e.roots.as<int32_t>(),              \
-                       e.mesh_info.as<float>(), dQ, perm, q_off, b_off, order, 1, nb, 64, beta2, omega, inside,    \
-                       (int32_t*)nullptr, (uint32_t*)nullptr, (uint32_t*)nullptr, 0u, flag, (uint32_t*)nullptr)
-    if (banks == 1) FWN_TRAV_INL(1);
-    else FWN_TRAV_INL(3);
-#undef FWN_TRAV_INL
+    launch_traverse(false, 1, false, banks, e.width, (unsigned)nb, s, e.slots.as<uint32_t>(), e.width,
+                    e.tris.as<uint32_t>(), e.roots.as<int32_t>(), e.mesh_info.as<float>(), dQ, perm, q_off, b_off,
+                    order, 1, nb, 64, beta2, omega, inside, (int32_t*)nullptr, flag, (uint32_t*)nullptr);
     FWN_LAUNCH_CHECK("k_traverse");
 }
 
@@ -765,7 +685,7 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
             dSt = e.q_stats.as<int32_t>();
         }
     }
-    e.q_flag.reserve(3 * sizeof(int32_t));
+    e.q_flag.reserve(2 * sizeof(int32_t));
 
     for (int k = 0; k < 2; ++k) {
         e.q_keys[k].reserve(sizeof(uint32_t) * nQ);
@@ -773,18 +693,6 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
     }
     if (!e.ev[0])
         for (int k = 0; k < 4; ++k) FWN_HIP(hipEventCreate(&e.ev[k]));
-    // per-point FP64 accumulators (sorted positions), kept zero between calls
-    if (!quad && e.acc_cap < nQ) {
-        e.q_acc.alloc(sizeof(unsigned long long) * nQ);
-        e.acc_cap = nQ;
-        hipLaunchKernelGGL(k_fill_u64, dim3(grid_blocks(nQ, 256)), dim3(256), 0, s,
-                           e.q_acc.as<unsigned long long>(), nQ);
-        FWN_LAUNCH_CHECK("k_fill_u64");
-    }
-    if (!quad && e.item_cap < std::max<int64_t>(nQ, 1 << 20)) {
-        e.item_cap = std::min<int64_t>(std::max<int64_t>(nQ, 1 << 20), (int64_t)UINT32_MAX / 4);
-        e.q_items.alloc(sizeof(uint32_t) * 3 * (size_t)e.item_cap);
-    }
 
     FWN_HIP(hipEventRecord(e.ev[0], s));
     // sorted position -> input index (nullptr: small calls keep the input order)
@@ -812,56 +720,35 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
             FWN_HIP(hipGetDeviceProperties(&prop, e.device));
             e.n_cu = prop.multiProcessorCount;
         }
-        nblk = std::min<int64_t>(nblk, (int64_t)e.n_cu * resident_blocks(true, waves, banks));
+        nblk = std::min<int64_t>(nblk, (int64_t)e.n_cu * resident_blocks(true, waves, banks, e.width));
     }
     if (nblk > INT32_MAX) fail(FWN_LIMIT_EXCEEDED, "too many point batches");
     const float beta2 = e.opt.accuracy_scale * e.opt.accuracy_scale;
     int32_t* dflag = e.q_flag.as<int32_t>();
-    uint32_t* dnitems = reinterpret_cast<uint32_t*>(dflag + 1); // chunks of FP64 items claimed
-    uint32_t* dwork = reinterpret_cast<uint32_t*>(dflag + 2);
-    for (int attempt = 0;; ++attempt) {
-        hipLaunchKernelGGL(k_zero3, dim3(1), dim3(1), 0, s, dflag);
-        FWN_HIP(hipEventRecord(e.ev[1], s));
-        const uint32_t cap = (uint32_t)e.item_cap;
-        if (quad) { // FP64 leaves in the kernel: no work list
-            launch_quads(e, dQ, vp, d_qoff, d_boff, d_order, M, nb, dOm, dIn, dflag, s);
-            FWN_HIP(hipEventRecord(e.ev[2], s));
-        } else {
-            launch_traverse(stats != nullptr, waves, persist, banks, (unsigned)nblk, s, e.slots.as<uint32_t>(),
-                            e.width, e.tris.as<uint32_t>(), e.roots.as<int32_t>(), e.mesh_info.as<float>(), dQ, vp,
-                            d_qoff, d_boff, d_order, M, nb, bpts, beta2, dOm, dIn, dSt, e.q_items.as<uint32_t>(),
-                            dnitems, cap, dflag, dwork);
-            FWN_LAUNCH_CHECK("k_traverse");
-            FWN_HIP(hipEventRecord(e.ev[2], s));
-            const unsigned g64 = small ? 16u : 2048u; // grid-stride loops: any grid size covers every item
-            hipLaunchKernelGGL(k_near64, dim3(g64), dim3(256), 0, s, e.q_items.as<uint32_t>(), dnitems, cap,
-                               e.tris.as<uint32_t>(), dQ, vp, e.q_acc.as<unsigned long long>());
-            FWN_LAUNCH_CHECK("k_near64");
-            hipLaunchKernelGGL(k_near64_combine, dim3(g64), dim3(256), 0, s, e.q_items.as<uint32_t>(), dnitems, cap,
-                               vp, e.q_acc.as<unsigned long long>(), dOm, dIn);
-            FWN_LAUNCH_CHECK("k_near64_combine");
-        }
-        FWN_HIP(hipEventRecord(e.ev[3], s));
-        int32_t h_fl[2] = {0, 0};
-        if (stage_io) { // flags and results in one wait
-            FWN_HIP(hipMemcpyAsync(hs, dflag, sizeof(h_fl), hipMemcpyDeviceToHost, s));
-            FWN_HIP(hipMemcpyAsync(hs + 16, dOm, sizeof(float) * nQ, hipMemcpyDeviceToHost, s));
-            if (inside) FWN_HIP(hipMemcpyAsync(hs + 16 + sizeof(float) * nQ, dIn, nQ, hipMemcpyDeviceToHost, s));
-            FWN_HIP(hipStreamSynchronize(s));
-            std::memcpy(h_fl, hs, sizeof(h_fl));
-        } else { // through the pinned stage too (its metadata bytes were uploaded before, in order)
-            FWN_HIP(hipMemcpyAsync(hs, dflag, sizeof(h_fl), hipMemcpyDeviceToHost, s));
-            FWN_HIP(hipStreamSynchronize(s));
-            std::memcpy(h_fl, hs, sizeof(h_fl));
-        }
-        if (h_fl[0]) fail(FWN_LIMIT_EXCEEDED, "traversal stack overflow");
-        const int64_t need = (int64_t)(uint32_t)h_fl[1] * kItemChunk; // claimed chunks x slots
-        if (need <= e.item_cap) break;
-        if (attempt > 0 || need > (int64_t)UINT32_MAX / 4)
-            fail(FWN_LIMIT_EXCEEDED, "FP64 near-field work list too large");
-        e.item_cap = need + need / 4;
-        e.q_items.alloc(sizeof(uint32_t) * 3 * (size_t)e.item_cap);
+    uint32_t* dwork = reinterpret_cast<uint32_t*>(dflag + 1);
+    hipLaunchKernelGGL(k_zero2, dim3(1), dim3(1), 0, s, dflag);
+    FWN_HIP(hipEventRecord(e.ev[1], s));
+    if (quad) {
+        launch_quads(e, dQ, vp, d_qoff, d_boff, d_order, M, nb, dOm, dIn, dflag, s);
+    } else {
+        launch_traverse(stats != nullptr, waves, persist, banks, e.width, (unsigned)nblk, s, e.slots.as<uint32_t>(),
+                        e.width, e.tris.as<uint32_t>(), e.roots.as<int32_t>(), e.mesh_info.as<float>(), dQ, vp, d_qoff,
+                        d_boff, d_order, M, nb, bpts, beta2, dOm, dIn, dSt, dflag, dwork);
+        FWN_LAUNCH_CHECK("k_traverse");
     }
+    FWN_HIP(hipEventRecord(e.ev[2], s));
+    FWN_HIP(hipEventRecord(e.ev[3], s));
+    // the flag (and a small host call's results in the same wait) through the pinned stage, whose
+    // metadata bytes were uploaded before, in order
+    int32_t h_fl = 0;
+    FWN_HIP(hipMemcpyAsync(hs, dflag, sizeof(h_fl), hipMemcpyDeviceToHost, s));
+    if (stage_io) {
+        FWN_HIP(hipMemcpyAsync(hs + 16, dOm, sizeof(float) * nQ, hipMemcpyDeviceToHost, s));
+        if (inside) FWN_HIP(hipMemcpyAsync(hs + 16 + sizeof(float) * nQ, dIn, nQ, hipMemcpyDeviceToHost, s));
+    }
+    FWN_HIP(hipStreamSynchronize(s));
+    std::memcpy(&h_fl, hs, sizeof(h_fl));
+    if (h_fl) fail(FWN_LIMIT_EXCEEDED, "traversal stack overflow");
     if (stage_io) {
         std::memcpy(omega, hs + 16, sizeof(float) * nQ);
         if (inside) std::memcpy(inside, hs + 16 + sizeof(float) * nQ, nQ);
@@ -869,8 +756,8 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
         FWN_HIP(hipMemcpyAsync(omega, dOm, sizeof(float) * nQ, hipMemcpyDeviceToHost, s));
         if (inside) FWN_HIP(hipMemcpyAsync(inside, dIn, nQ, hipMemcpyDeviceToHost, s));
         if (stats) FWN_HIP(hipMemcpyAsync(stats, dSt, sizeof(int32_t) * 4 * nQ, hipMemcpyDeviceToHost, s));
+        FWN_HIP(hipStreamSynchronize(s));
     }
-    FWN_HIP(hipStreamSynchronize(s));
     float t_tr = 0.0f, t_all = 0.0f;
     FWN_HIP(hipEventElapsedTime(&t_tr, e.ev[1], e.ev[2]));
     FWN_HIP(hipEventElapsedTime(&t_all, e.ev[0], e.ev[3]));
