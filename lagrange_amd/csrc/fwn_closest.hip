@@ -21,8 +21,8 @@
 // triangles lie on all sides): 400,000 points over 200k triangles keep 3.3 waves of a compute unit in
 // flight on average, and an average wave issues 87k vector and 52k scalar instructions.  Against the
 // walk with double box distances from vector loads and no disks (333k and 330k), that call takes
-// 4.28 ms instead of 43.2: 16.1 ms with the float box distances and record loads below, 12.7 with
-// disks of single triangles, and the rest from the disks of the inner slots.
+// 4.1 ms instead of 43.2: 16.1 ms with the float box distances and record loads below, 12.7 with
+// disks of single triangles, 4.3 with the disks of the inner slots, the rest by the blocks' order.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -306,7 +306,9 @@ __global__ __launch_bounds__(64) void k_closest(const float* __restrict__ boxes,
                                                 double* __restrict__ cp_out, int32_t* __restrict__ flag)
 {
     const int lane = threadIdx.x;
-    const int64_t batch = xcd_remap(blockIdx.x, gridDim.x);
+    // runs of 256 waves: the expensive waves lie together (400k points: 4.20 ms in one run per XCD,
+    // 3.96 in runs of 64, 3.88 of 256, 4.25 of 1,024)
+    const int64_t batch = xcd_remap_runs(blockIdx.x, gridDim.x, 256u);
     const int64_t jpos = batch * 64 + lane;
     const bool valid = jpos < nQ;
     const uint32_t orig = valid ? perm[jpos] : 0u;

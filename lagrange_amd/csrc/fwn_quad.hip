@@ -97,7 +97,7 @@ __global__ __launch_bounds__(64) void k_traverse_quad(
     constexpr int kNode4 = kQuadNodeBytes / 16; // uint4 per node
     const int lane = threadIdx.x;
     const int p = lane >> 2, s = lane & 3;
-    const int64_t batch = xcd_remap(blockIdx.x, gridDim.x);
+    const int64_t batch = xcd_batch(blockIdx.x, gridDim.x, M);
     if (batch >= n_batches) return;
     const int pos = mesh_of64(b_off, M, batch);
     const int m = mesh_order[pos];
@@ -271,7 +271,9 @@ __global__ __launch_bounds__(64) void k_traverse_quad(
 
 // Whether a call of nQ points, q_off per mesh, goes to the slots-in-lanes traversal: 4-wide trees
 // of the default launch shape (the other shapes are k_traverse's, chosen by the tuner or the
-// caller), up to kQuadCross * cbrt(F) points for a mesh of F triangles.  The two kernels' costs
+// caller), up to kQuadCross * cbrt(F) points for a mesh of F triangles (several: of the mean F)
+// and, for several meshes, kQuadSparse points a triangle more, as each mesh's share of the points
+// is sparse on it however many the call has.  The two kernels' costs
 // cross where the 64 points of a k_traverse wave are close together compared with the nodes they
 // visit, for points near the surface (both kernels walk to the triangles) at fewer points than for
 // uniform ones; the line lies between the two crossings.  k_traverse / this kernel in us,
@@ -280,14 +282,17 @@ __global__ __launch_bounds__(64) void k_traverse_quad(
 //     1333 (4M); F = 940,800 1182 / 681 (1.5M), 1576 / 1408 (4M);
 //   near the surface: F = 972 179 / 179 (200k); F = 20,172 431 / 396 (400k), 507 / 619 (800k);
 //     F = 199,692 724 / 586 (400k), 886 / 913 (800k), 1156 / 1465 (1.5M); F = 940,800 1472 / 1343
-//     (800k), 1834 / 2128 (1.5M).
-constexpr double kQuadCross = 24000.0;
+//     (800k), 1834 / 2128 (1.5M);
+//   several meshes, uniform / near the surface (the kernels alone): 64 x 20k points, F = 199,692
+//     1872 / 873 and 5661 / 3039, F = 19,200 1113 / 738 and 1649 / 1328, F = 1,728 553 / 587 and 623 /
+//     778; 32 x 100k points, F = 19,200 1350 / 1274 and 1974 / 2362; 8 meshes of 14k to 48k, 1M
+//     points, 720 / 462; 32 of 1.7k to 181k, 3.7M points, 1208 / 1297.
+constexpr double kQuadCross = 24000.0, kQuadSparse = 2.0;
 bool use_quads(const Engine& e, int64_t nQ, int banks)
 {
     if (e.width != 4 || banks != 1 || !default_shape(e)) return false;
-    double cross = 0.0;
-    for (int m = 0; m < e.n_meshes; ++m) cross += std::cbrt((double)(e.h_f_off[m + 1] - e.h_f_off[m]));
-    return (double)nQ <= kQuadCross * cross;
+    const double F = (double)e.h_f_off[e.n_meshes];
+    return (double)nQ <= kQuadCross * std::cbrt(F / e.n_meshes) + (e.n_meshes > 1 ? kQuadSparse * F : 0.0);
 }
 
 void launch_quads(Engine& e, const float* dQ, const uint32_t* perm, const int64_t* q_off, const int64_t* b_off,

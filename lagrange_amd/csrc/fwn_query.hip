@@ -285,7 +285,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_traverse(
     unsigned long long* acc = reinterpret_cast<unsigned long long*>(lds);
     uint2* queue = reinterpret_cast<uint2*>(acc + 64);
     if (!PERSIST) {
-        const int64_t batch = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * WAVES + (threadIdx.x >> 6);
+        const int64_t batch = (int64_t)xcd_batch(blockIdx.x, gridDim.x, M) * WAVES + (threadIdx.x >> 6);
         if (batch >= n_batches) return; // whole wave
         traverse_batch<STATS, NB>(batch, slots, width, tris, roots, minfo, Q, perm, q_off, b_off, mesh_order, M, bpts,
                                   beta2, omega, inside, stats, flag, queue, acc);

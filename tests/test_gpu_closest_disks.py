@@ -78,3 +78,13 @@ def test_closest_scales(oracle, scale, offset):
     V, F = _mesh("open")
     V = (V.astype(np.float64) * scale + offset).astype(np.float32)
     _compare(V, F, _points(V, F, np.random.default_rng(6)), oracle)
+
+
+def test_closest_of_many_waves():
+    """Above 2,048 waves the blocks are dealt to the XCDs in runs: with runs and a remainder, the
+    distances are those of calls too small for runs."""
+    V, F = _mesh("open")
+    Q = np.random.default_rng(9).uniform(-1.3, 1.3, (2 * 131072 + 64 * 300 + 5, 3)).astype(np.float32)
+    e = FastWindingNumber((V, F))
+    want = np.concatenate([e.closest_point(Q[k:k + 50000])[0] for k in range(0, Q.shape[0], 50000)])
+    np.testing.assert_array_equal(e.closest_point(Q)[0], want)
