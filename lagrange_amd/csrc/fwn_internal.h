@@ -200,9 +200,12 @@ SahMids build_topology_sah(Engine& e, Arena& ar, const float* cen, const float* 
                            const int64_t* f_off, int M, int32_t* items, int32_t* left, int32_t* right, int32_t* parent,
                            int32_t* first, int32_t* last, uint8_t* is_root, int32_t* root_bin);
 
-// queries (fwn_query.hip)
+// queries (fwn_query.hip).  order: device positions -> points of one mesh that are already in an order
+// of waves (nullptr: the call sorts its points); not read by calls that need no order (few_points).
 void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t nQ, float* omega, uint8_t* inside,
-                 int32_t* stats, bool device_ptrs);
+                 int32_t* stats, bool device_ptrs, const uint32_t* order = nullptr);
+// whether a device call of nQ points of one mesh runs one wave per point
+bool few_points(const Engine& e, int64_t nQ);
 void run_bruteforce(Engine& e, const float* Q, int64_t nQ, double* out, bool device_ptrs);
 // pinned staging buffer of at least this many bytes (contents undefined when it grows)
 char* host_stage(Engine& e, size_t bytes);

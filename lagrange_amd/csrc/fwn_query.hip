@@ -588,8 +588,13 @@ void launch_traverse_inplace(Engine& e, int banks, const float* dQ, const uint32
     FWN_LAUNCH_CHECK("k_traverse");
 }
 
+bool few_points(const Engine& e, int64_t nQ)
+{
+    return nQ <= kPointCalls && default_shape(e);
+}
+
 void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t nQ, float* omega, uint8_t* inside,
-                 int32_t* stats, bool dev)
+                 int32_t* stats, bool dev, const uint32_t* point_order)
 {
     hipStream_t s = e.stream;
     const int M = e.n_meshes;
@@ -615,7 +620,7 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
         return;
     }
     if (!stats && M == 1 &&
-        ((!dev && nQ <= kSmallBatch) || (nQ <= kPointCalls && default_shape(e)))) {
+        ((!dev && nQ <= kSmallBatch) || few_points(e, nQ))) {
         run_points(e, Q, nQ, omega, inside, banks, dev);
         return;
     }
@@ -687,28 +692,31 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
     }
     e.q_flag.reserve(2 * sizeof(int32_t));
 
-    for (int k = 0; k < 2; ++k) {
-        e.q_keys[k].reserve(sizeof(uint32_t) * nQ);
-        e.q_vals[k].reserve(sizeof(uint32_t) * nQ);
+    if (!small && !point_order) {
+        for (int k = 0; k < 2; ++k) {
+            e.q_keys[k].reserve(sizeof(uint32_t) * nQ);
+            e.q_vals[k].reserve(sizeof(uint32_t) * nQ);
+        }
     }
     if (!e.ev[0])
         for (int k = 0; k < 4; ++k) FWN_HIP(hipEventCreate(&e.ev[k]));
 
     FWN_HIP(hipEventRecord(e.ev[0], s));
     // sorted position -> input index (nullptr: small calls keep the input order)
-    uint32_t* vp = nullptr;
-    if (!small) {
+    const uint32_t* vp = small ? nullptr : point_order;
+    if (!small && !point_order) {
         uint32_t* kp = e.q_keys[0].as<uint32_t>();
         uint32_t* kp2 = e.q_keys[1].as<uint32_t>();
         uint32_t* vp2 = e.q_vals[1].as<uint32_t>();
-        vp = e.q_vals[0].as<uint32_t>();
+        uint32_t* vals = e.q_vals[0].as<uint32_t>();
         int mesh_bits = 0;
         while ((1 << mesh_bits) < M) ++mesh_bits;
         if (mesh_bits > 24) fail(FWN_LIMIT_EXCEEDED, "more than 2^24 meshes in one engine");
         hipLaunchKernelGGL(k_query_keys, dim3(grid_blocks(nQ, QT)), dim3(QT), 0, s, dQ, nQ, d_qoff, M, mesh_bits,
                            e.mesh_info.as<float>(), kp);
         FWN_LAUNCH_CHECK("k_query_keys");
-        radix_sort_pairs32(kp, vp, kp2, vp2, nQ, 8, 32, true, e.q_hist, e.q_rowsum, s);
+        radix_sort_pairs32(kp, vals, kp2, vp2, nQ, 8, 32, true, e.q_hist, e.q_rowsum, s);
+        vp = vals;
     }
 
     const int waves = e.opt.waves_per_block > 0 ? e.opt.waves_per_block : 1;

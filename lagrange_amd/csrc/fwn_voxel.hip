@@ -23,17 +23,57 @@ __device__ __forceinline__ float voxel_coord(int64_t idx, double vs, double half
     return (float)(w + half);
 }
 
-// dense box: voxel t = x + dx (y + dy z) has index lo + (x, y, z)
-__global__ __launch_bounds__(256) void k_voxel_box(int32_t lx, int32_t ly, int32_t lz, int64_t dx, int64_t dy,
-                                                   int64_t n, double vs, float* __restrict__ P)
+// a / b for b that may be beyond 32 bits (then 0: a is not)
+__device__ __forceinline__ uint32_t quotient(uint32_t a, uint64_t b)
 {
-    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (t >= n) return;
-    const int64_t x = t % dx, r = t / dx, y = r % dy, z = r / dy;
+    return b > a ? 0u : a / (uint32_t)b;
+}
+
+// Dense box: voxel t = x + dx (y + dy z) has index lo + (x, y, z); n < 2^31 voxels.  With `order`, also
+// the voxels in the order the batched traversals want them, close together in space: blocks of 4 x 4
+// x 4 (those at the far faces cut short), x fastest, a whole block's voxels in Morton order so that
+// every 8 and 16 of them are compact too.  A wave of 64 points is a block, or parts of two neighbours
+// after a cut one.  One 4-byte write per voxel in place of point keys and three sort passes (3.5M
+// voxels: 21 us, the centres and the sort before 17 + 100; the traversal 791 -> 779 us in this order).
+__global__ __launch_bounds__(256) void k_voxel_box(int32_t lx, int32_t ly, int32_t lz, uint32_t dx, uint32_t dy,
+                                                   uint32_t dz, uint32_t n, double vs, float* __restrict__ P,
+                                                   uint32_t* __restrict__ order)
+{
+    const uint32_t j = blockIdx.x * 256u + threadIdx.x;
+    if (j >= n) return;
+    const uint64_t layer = (uint64_t)dx * dy;
+    uint32_t x, y, z;
+    if (!order) {
+        z = quotient(j, layer);
+        const uint32_t r = j - z * (uint32_t)layer;
+        y = r / dx;
+        x = r - y * dx;
+    } else {
+        const uint32_t z0 = quotient(j, 4 * layer) * 4, hz = min(dz - z0, 4u);
+        const uint32_t in_layer = j - z0 * (uint32_t)layer;
+        const uint32_t y0 = quotient(in_layer, (uint64_t)dx * 4 * hz) * 4, hy = min(dy - y0, 4u);
+        const uint32_t in_row = in_layer - y0 * dx * hz;
+        const uint32_t x0 = in_row / (4 * hy * hz) * 4, hx = min(dx - x0, 4u);
+        const uint32_t k = in_row - x0 * hy * hz;
+        if (hx == 4 && hy == 4 && hz == 4) {
+            x = (k & 1) | ((k >> 2) & 2);
+            y = ((k >> 1) & 1) | ((k >> 3) & 2);
+            z = ((k >> 2) & 1) | ((k >> 4) & 2);
+        } else {
+            x = k % hx;
+            y = k / hx % hy;
+            z = k / (hx * hy);
+        }
+        x += x0;
+        y += y0;
+        z += z0;
+    }
+    const uint32_t t = x + dx * (y + dy * z);
+    if (order) order[j] = t;
     const double half = vs * 0.5;
-    P[3 * t + 0] = voxel_coord(lx + x, vs, half);
-    P[3 * t + 1] = voxel_coord(ly + y, vs, half);
-    P[3 * t + 2] = voxel_coord(lz + z, vs, half);
+    P[3 * (size_t)t + 0] = voxel_coord((int64_t)lx + x, vs, half);
+    P[3 * (size_t)t + 1] = voxel_coord((int64_t)ly + y, vs, half);
+    P[3 * (size_t)t + 2] = voxel_coord((int64_t)lz + z, vs, half);
 }
 
 // explicit list of (i, j, k) int32 triples
@@ -47,13 +87,14 @@ __global__ __launch_bounds__(256) void k_voxel_list(const int32_t* __restrict__ 
 
 } // namespace
 
-// Generate the centres into the engine's scratch and answer them; outputs host or device.
+// Generate the centres (and, for a box, their order) into the engine's scratch and answer them;
+// outputs host or device.
 static void sign_centres(Engine& e, int64_t n, uint8_t* inside, float* omega, bool dev,
-                         void (*gen)(Engine&, float*, const void*), const void* arg)
+                         const uint32_t* (*gen)(Engine&, float*, const void*), const void* arg)
 {
     hipStream_t s = e.stream;
     e.v_pts.reserve(sizeof(float) * 3 * n);
-    gen(e, e.v_pts.as<float>(), arg);
+    const uint32_t* order = gen(e, e.v_pts.as<float>(), arg);
     float* dOm = omega;
     uint8_t* dIn = inside;
     if (!dev || !omega) {
@@ -64,7 +105,7 @@ static void sign_centres(Engine& e, int64_t n, uint8_t* inside, float* omega, bo
         e.v_in.reserve(n);
         dIn = e.v_in.as<uint8_t>();
     }
-    run_queries(e, e.v_pts.as<float>(), nullptr, n, dOm, dIn, nullptr, true);
+    run_queries(e, e.v_pts.as<float>(), nullptr, n, dOm, dIn, nullptr, true, order);
     if (!dev) {
         FWN_HIP(hipMemcpyAsync(inside, dIn, n, hipMemcpyDeviceToHost, s));
         if (omega) FWN_HIP(hipMemcpyAsync(omega, dOm, sizeof(float) * n, hipMemcpyDeviceToHost, s));
@@ -85,15 +126,21 @@ struct ListArg {
     bool dev;
 };
 
-static void gen_box(Engine& e, float* P, const void* a)
+static const uint32_t* gen_box(Engine& e, float* P, const void* a)
 {
     const BoxArg& b = *static_cast<const BoxArg*>(a);
+    uint32_t* order = nullptr;
+    if (!few_points(e, b.n)) { // those are answered in any order
+        e.q_vals[0].reserve(sizeof(uint32_t) * b.n);
+        order = e.q_vals[0].as<uint32_t>();
+    }
     hipLaunchKernelGGL(k_voxel_box, dim3(grid_blocks(b.n, 256)), dim3(256), 0, e.stream, b.lo[0], b.lo[1], b.lo[2],
-                       b.dims[0], b.dims[1], b.n, b.vs, P);
+                       (uint32_t)b.dims[0], (uint32_t)b.dims[1], (uint32_t)b.dims[2], (uint32_t)b.n, b.vs, P, order);
     FWN_LAUNCH_CHECK("k_voxel_box");
+    return order;
 }
 
-static void gen_list(Engine& e, float* P, const void* a)
+static const uint32_t* gen_list(Engine& e, float* P, const void* a)
 {
     const ListArg& l = *static_cast<const ListArg*>(a);
     const int32_t* dijk = l.ijk;
@@ -104,6 +151,7 @@ static void gen_list(Engine& e, float* P, const void* a)
     }
     hipLaunchKernelGGL(k_voxel_list, dim3(grid_blocks(3 * l.n, 256)), dim3(256), 0, e.stream, dijk, l.n, l.vs, P);
     FWN_LAUNCH_CHECK("k_voxel_list");
+    return nullptr;
 }
 
 static void check_voxel_size(double vs)
