@@ -146,6 +146,13 @@ void radix_sort_pairs32(uint32_t*& keys, uint32_t*& vals, uint32_t*& keys_alt, u
 // The same over caller-provided histogram scratch (no allocation): hist holds
 // radix_sort_hist_words(n) int32, rowsum 256 int32.
 int64_t radix_sort_hist_words(int64_t n);
+// The top 20 bits of at most kFewTiles tiles of keys, whose first 10-bit digit (bits 12 to 21) the kernel
+// that made them has counted into hist (kFewTile keys a tile, 1,024 int32 each): vals receives the input
+// positions in stable order of those bits.
+constexpr int kFewTile = 4096, kFewTiles = 128;
+inline int few_tiles(int64_t n) { return (int)((n + kFewTile - 1) / kFewTile); }
+void sort_few_tiles(const uint32_t* keys, uint32_t* keys_alt, uint32_t* vals_alt, uint32_t* vals, int64_t n,
+                    int32_t* hist, hipStream_t s);
 void radix_sort_pairs32_scratch(uint32_t*& keys, uint32_t*& vals, uint32_t*& keys_alt, uint32_t*& vals_alt, int64_t n,
                                 int begin_bit, int end_bit, bool vals_are_index, int32_t* hist, int32_t* rowsum,
                                 hipStream_t s);
@@ -322,6 +329,19 @@ __device__ __forceinline__ uint32_t morton30(float x, float y, float z, const fl
 {
     return (expand10(quant10(x, lo[0], inv[0])) << 2) | (expand10(quant10(y, lo[1], inv[1])) << 1) |
            expand10(quant10(z, lo[2], inv[2]));
+}
+
+// one key's digit into the block's counters; called with whole waves (a wave whose keys share one
+// digit adds its count with one atomic: LDS atomics on one address serialise)
+__device__ __forceinline__ void count_digit(int32_t* cnt, uint32_t d, bool valid)
+{
+    const uint64_t live = __ballot(valid);
+    const uint32_t d0 = __builtin_amdgcn_readfirstlane(d);
+    if ((__ballot(d != d0) & live) == 0ull) {
+        if ((threadIdx.x & 63) == 0 && live != 0ull) atomicAdd(&cnt[d0], (int32_t)__popcll(live));
+    } else if (valid) {
+        atomicAdd(&cnt[d], 1);
+    }
 }
 
 // order-preserving float <-> int maps for atomic min/max

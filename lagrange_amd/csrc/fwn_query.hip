@@ -53,12 +53,10 @@ __device__ __forceinline__ int64_t wave_uniform64(int64_t v)
 // 30-bit Morton code in its mesh's box.  Only the 24 top bits are sorted: a wave needs its 64
 // points close together, not in exact curve order, and every point's result is independent of
 // which points share its wave.
-__global__ __launch_bounds__(QT) void k_query_keys(const float* __restrict__ Q, int64_t nQ,
-                                                   const int64_t* __restrict__ q_off, int M, int mesh_bits,
-                                                   const float* __restrict__ minfo, uint32_t* __restrict__ keys)
+__device__ __forceinline__ uint32_t point_key(const float* __restrict__ Q, int64_t nQ, int64_t i,
+                                              const int64_t* __restrict__ q_off, int M, int mesh_bits,
+                                              const float* __restrict__ minfo)
 {
-    int64_t i = (int64_t)blockIdx.x * QT + threadIdx.x;
-    if (i >= nQ) return;
     int m = 0;
     if (M > 1) {
         // the wave's first and last points (wave-uniform: scalar loads); only a wave that spans a
@@ -72,7 +70,40 @@ __global__ __launch_bounds__(QT) void k_query_keys(const float* __restrict__ Q, 
     const int mbits = 32 - mesh_bits; // bits left for the Morton code
     uint32_t key = (mbits >= 30) ? mc : (mc >> (30 - mbits));
     if (mesh_bits > 0) key |= (uint32_t)m << mbits;
-    keys[i] = key; // the sort's first pass takes the values to be the positions i
+    return key; // the sort's first pass takes the values to be the positions i
+}
+
+// flags (nullptr: none): the traversal's overflow flag and work counter, cleared on the way
+__global__ __launch_bounds__(QT) void k_query_keys(const float* __restrict__ Q, int64_t nQ,
+                                                   const int64_t* __restrict__ q_off, int M, int mesh_bits,
+                                                   const float* __restrict__ minfo, uint32_t* __restrict__ keys,
+                                                   int32_t* __restrict__ flags)
+{
+    const int64_t i = (int64_t)blockIdx.x * QT + threadIdx.x;
+    if (i < 2 && flags) flags[i] = 0;
+    if (i < nQ) keys[i] = point_key(Q, nQ, i, q_off, M, mesh_bits, minfo);
+}
+
+// the same in tiles of kFewTile points, with the tile's counts of the sort's first digit
+__global__ __launch_bounds__(1024) void k_query_keys_few(const float* __restrict__ Q, int64_t nQ,
+                                                         const int64_t* __restrict__ q_off, int M, int mesh_bits,
+                                                         const float* __restrict__ minfo, uint32_t* __restrict__ keys,
+                                                         int32_t* __restrict__ hist, int32_t* __restrict__ flags)
+{
+    __shared__ int32_t cnt[1024];
+    if (blockIdx.x == 0 && threadIdx.x < 2) flags[threadIdx.x] = 0;
+    cnt[threadIdx.x] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kFewTile / 1024; ++r) {
+        const int64_t i = (int64_t)blockIdx.x * kFewTile + r * 1024 + threadIdx.x;
+        const bool valid = i < nQ;
+        const uint32_t key = valid ? point_key(Q, nQ, i, q_off, M, mesh_bits, minfo) : 0u;
+        if (valid) keys[i] = key;
+        count_digit(cnt, key >> 12 & 1023u, valid);
+    }
+    __syncthreads();
+    hist[(int64_t)blockIdx.x * 1024 + threadIdx.x] = cnt[threadIdx.x];
 }
 
 // One slot's 24 words held in SGPRs (a 16-dword and an 8-dword scalar load issued together at
@@ -510,7 +541,7 @@ void run_queries_pipelined(Engine& e, const float* Q, int64_t nQ, float* omega, 
             uint32_t* kp2 = e.q_keys[1].as<uint32_t>();
             uint32_t* vp2 = e.q_vals[1].as<uint32_t>();
             hipLaunchKernelGGL(k_query_keys, dim3(grid_blocks(ck, QT)), dim3(QT), 0, s, dQ, ck, d_qoff, 1, 0,
-                               e.mesh_info.as<float>(), kp);
+                               e.mesh_info.as<float>(), kp, (int32_t*)nullptr);
             FWN_LAUNCH_CHECK("k_query_keys");
             radix_sort_pairs32(kp, vp, kp2, vp2, ck, 8, 32, true, e.q_hist, e.q_rowsum, s);
             const int64_t nb = (ck + 63) / 64;
@@ -569,7 +600,7 @@ void run_queries_pipelined(Engine& e, const float* Q, int64_t nQ, float* omega, 
 void launch_point_keys(Engine& e, const float* dQ, int64_t nQ, uint32_t* keys, hipStream_t s)
 {
     hipLaunchKernelGGL(k_query_keys, dim3(grid_blocks(nQ, QT)), dim3(QT), 0, s, dQ, nQ, (const int64_t*)nullptr, 1, 0,
-                       e.mesh_info.as<float>(), keys);
+                       e.mesh_info.as<float>(), keys, (int32_t*)nullptr);
     FWN_LAUNCH_CHECK("k_query_keys");
 }
 
@@ -702,20 +733,34 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
         for (int k = 0; k < 4; ++k) FWN_HIP(hipEventCreate(&e.ev[k]));
 
     FWN_HIP(hipEventRecord(e.ev[0], s));
+    int32_t* dflag = e.q_flag.as<int32_t>();
+    uint32_t* dwork = reinterpret_cast<uint32_t*>(dflag + 1);
     // sorted position -> input index (nullptr: small calls keep the input order)
     const uint32_t* vp = small ? nullptr : point_order;
-    if (!small && !point_order) {
+    if (small || point_order) {
+        hipLaunchKernelGGL(k_zero2, dim3(1), dim3(1), 0, s, dflag);
+    } else {
         uint32_t* kp = e.q_keys[0].as<uint32_t>();
         uint32_t* kp2 = e.q_keys[1].as<uint32_t>();
-        uint32_t* vp2 = e.q_vals[1].as<uint32_t>();
         uint32_t* vals = e.q_vals[0].as<uint32_t>();
+        uint32_t* vp2 = e.q_vals[1].as<uint32_t>();
         int mesh_bits = 0;
         while ((1 << mesh_bits) < M) ++mesh_bits;
         if (mesh_bits > 24) fail(FWN_LIMIT_EXCEEDED, "more than 2^24 meshes in one engine");
-        hipLaunchKernelGGL(k_query_keys, dim3(grid_blocks(nQ, QT)), dim3(QT), 0, s, dQ, nQ, d_qoff, M, mesh_bits,
-                           e.mesh_info.as<float>(), kp);
-        FWN_LAUNCH_CHECK("k_query_keys");
-        radix_sort_pairs32(kp, vals, kp2, vp2, nQ, 8, 32, true, e.q_hist, e.q_rowsum, s);
+        // few tiles: 20 bits (the mesh among them) separate 2^20 cells, or about 60,000 along a
+        // surface, where at most 524,288 points leave nothing for more bits to order
+        if (few_tiles(nQ) <= kFewTiles && mesh_bits <= 8) {
+            e.q_hist.reserve(sizeof(int32_t) * 1024 * (size_t)few_tiles(nQ));
+            hipLaunchKernelGGL(k_query_keys_few, dim3(few_tiles(nQ)), dim3(1024), 0, s, dQ, nQ, d_qoff, M, mesh_bits,
+                               e.mesh_info.as<float>(), kp, e.q_hist.as<int32_t>(), dflag);
+            FWN_LAUNCH_CHECK("k_query_keys_few");
+            sort_few_tiles(kp, kp2, vp2, vals, nQ, e.q_hist.as<int32_t>(), s);
+        } else {
+            hipLaunchKernelGGL(k_query_keys, dim3(grid_blocks(nQ, QT)), dim3(QT), 0, s, dQ, nQ, d_qoff, M, mesh_bits,
+                               e.mesh_info.as<float>(), kp, dflag);
+            FWN_LAUNCH_CHECK("k_query_keys");
+            radix_sort_pairs32(kp, vals, kp2, vp2, nQ, 8, 32, true, e.q_hist, e.q_rowsum, s);
+        }
         vp = vals;
     }
 
@@ -732,9 +777,6 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
     }
     if (nblk > INT32_MAX) fail(FWN_LIMIT_EXCEEDED, "too many point batches");
     const float beta2 = e.opt.accuracy_scale * e.opt.accuracy_scale;
-    int32_t* dflag = e.q_flag.as<int32_t>();
-    uint32_t* dwork = reinterpret_cast<uint32_t*>(dflag + 1);
-    hipLaunchKernelGGL(k_zero2, dim3(1), dim3(1), 0, s, dflag);
     FWN_HIP(hipEventRecord(e.ev[1], s));
     if (quad) {
         launch_quads(e, dQ, vp, d_qoff, d_boff, d_order, M, nb, dOm, dIn, dflag, s);
@@ -745,7 +787,6 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
         FWN_LAUNCH_CHECK("k_traverse");
     }
     FWN_HIP(hipEventRecord(e.ev[2], s));
-    FWN_HIP(hipEventRecord(e.ev[3], s));
     // the flag (and a small host call's results in the same wait) through the pinned stage, whose
     // metadata bytes were uploaded before, in order
     int32_t h_fl = 0;
@@ -768,7 +809,7 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
     }
     float t_tr = 0.0f, t_all = 0.0f;
     FWN_HIP(hipEventElapsedTime(&t_tr, e.ev[1], e.ev[2]));
-    FWN_HIP(hipEventElapsedTime(&t_all, e.ev[0], e.ev[3]));
+    FWN_HIP(hipEventElapsedTime(&t_all, e.ev[0], e.ev[2]));
     e.last_traverse_ms = t_tr;
     e.last_total_ms = t_all;
 }
@@ -787,7 +828,7 @@ const uint32_t* sort_points_single(Engine& e, const float* dQ, int64_t nQ)
     uint32_t* kp2 = e.q_keys[1].as<uint32_t>();
     uint32_t* vp2 = e.q_vals[1].as<uint32_t>();
     hipLaunchKernelGGL(k_query_keys, dim3(grid_blocks(nQ, QT)), dim3(QT), 0, s, dQ, nQ, (const int64_t*)nullptr, 1, 0,
-                       e.mesh_info.as<float>(), kp);
+                       e.mesh_info.as<float>(), kp, (int32_t*)nullptr);
     FWN_LAUNCH_CHECK("k_query_keys");
     radix_sort_pairs32(kp, vp, kp2, vp2, nQ, 8, 32, true, e.q_hist, e.q_rowsum, s);
     return vp;

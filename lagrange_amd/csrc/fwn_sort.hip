@@ -26,18 +26,20 @@ constexpr int RS_ROUNDS = 16;
 constexpr int RS_TILE = RS_THREADS * RS_ROUNDS;
 constexpr int RS_WAVES = RS_THREADS / kWave;
 typedef __attribute__((address_space(3))) volatile int32_t lds_vint;
+typedef __attribute__((address_space(3))) volatile uint16_t lds_vshort;
 
-// lanes of the wave holding the same 8-bit digit d as this lane (among the lanes in `live`, a
+// lanes of the wave holding the same digit d (BITS wide) as this lane (among the lanes in `live`, a
 // prefix of the wave).  Morton keys of nearby points often share a digit across the whole wave:
 // one compare settles that case; otherwise 8 bit ballots separate the digits.  Called with every
 // lane of the wave active.
+template <int BITS = 8>
 __device__ __forceinline__ uint64_t digit_peers(uint32_t d, uint64_t live)
 {
     const uint32_t d0 = __builtin_amdgcn_readfirstlane(d);
     if ((__ballot(d != d0) & live) == 0ull) return live;
     uint64_t peers = live;
 #pragma unroll
-    for (int b = 0; b < 8; ++b) {
+    for (int b = 0; b < BITS; ++b) {
         const bool bit = (d >> b) & 1u;
         const uint64_t m = __ballot(bit);
         peers &= bit ? m : ~m;
@@ -247,7 +249,131 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const KeyT* __restric
         const KeyT key = lk[t];
         const uint32_t d = (uint32_t)(key >> shift) & 255u;
         const int32_t pos = gbase[d] + (t - toff[d]);
-        kout[pos] = key;
+        if (kout) kout[pos] = key;
+        vout[pos] = lv[t];
+    }
+}
+
+// ---- point keys of few tiles ----------------------------------------------------------------
+// Sorts of at most kFewTiles tiles of 4,096 keys take two passes of 10 bits, each a histogram (the
+// first counted by the kernel that makes the keys) and a scatter that sums the tiles' histograms
+// itself, instead of three of 8 bits with a scan kernel between: 4 launches for 10.  Such sorts are
+// bound by launches and by the latency inside each: 1,024 threads rank a tile in 4 rounds, and a tile's
+// 1,024 threads read the up to 128 rows of counts in 16 rounds of loads.  100k and 400k points: the
+// kernels of keys and sort 60 and 63 us before, 34 and 44 now, and six gaps between launches fewer.
+// With more tiles the rows cost more than a scan kernel, and runs of 4 keys a digit scatter worse than
+// runs of 16.
+constexpr int FS_ROUNDS = kFewTile / 1024;
+
+__global__ __launch_bounds__(1024) void k_fs_hist(const uint32_t* __restrict__ keys, int n, int shift,
+                                                  int32_t* __restrict__ hist)
+{
+    __shared__ int32_t cnt[1024];
+    const int tid = threadIdx.x, base = blockIdx.x * kFewTile;
+    uint32_t kr[FS_ROUNDS];
+#pragma unroll
+    for (int r = 0; r < FS_ROUNDS; ++r) {
+        const int i = base + r * 1024 + tid;
+        kr[r] = i < n ? keys[i] : 0u;
+    }
+    cnt[tid] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < FS_ROUNDS; ++r) count_digit(cnt, kr[r] >> shift & 1023u, base + r * 1024 + tid < n);
+    __syncthreads();
+    hist[blockIdx.x * 1024 + tid] = cnt[tid];
+}
+
+__global__ __launch_bounds__(1024) void k_fs_scatter(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
+                                                     uint32_t* __restrict__ kout, uint32_t* __restrict__ vout, int n,
+                                                     int shift, const int32_t* __restrict__ hist, int ntiles)
+{
+    constexpr int kWaves = 16, kWaveKeys = kFewTile / kWaves;
+    __shared__ int32_t gbase[1024];         // global position of the tile's place 0, were it of this digit
+    __shared__ uint16_t wrun[kWaves][1024]; // per wave: keys of each digit (run length, then place in the tile)
+    __shared__ uint32_t lk[kFewTile], lv[kFewTile];
+    __shared__ int32_t sums[2][kWaves];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int base = blockIdx.x * kFewTile, tile_n = min(n - base, kFewTile);
+    uint32_t kr[FS_ROUNDS], vr[FS_ROUNDS];
+#pragma unroll
+    for (int r = 0; r < FS_ROUNDS; ++r) {
+        const int li = wave * kWaveKeys + r * 64 + lane;
+        kr[r] = li < tile_n ? kin[base + li] : 0u;
+        vr[r] = vin ? (li < tile_n ? vin[base + li] : 0u) : (uint32_t)(base + li);
+    }
+    // keys of digit tid: in all tiles, in earlier ones and in this one
+    int32_t total = 0, before = 0, mine = 0;
+    for (int t = 0; t < ntiles; t += 8) {
+        int32_t c[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) c[k] = t + k < ntiles ? hist[(t + k) * 1024 + tid] : 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            total += c[k];
+            before += t + k < (int)blockIdx.x ? c[k] : 0;
+            mine = t + k == (int)blockIdx.x ? c[k] : mine;
+        }
+    }
+    for (int k = 0; k < kWaves / 2; ++k) reinterpret_cast<uint32_t*>(wrun)[k * 1024 + tid] = 0u;
+    // exclusive scans over the digits of the totals and of the tile's counts
+    int32_t st = total, sm = mine;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int32_t a = __shfl_up(st, off), b = __shfl_up(sm, off);
+        if (lane >= off) {
+            st += a;
+            sm += b;
+        }
+    }
+    if (lane == 63) {
+        sums[0][wave] = st;
+        sums[1][wave] = sm;
+    }
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) {
+        st += sums[0][w];
+        sm += sums[1][w];
+    }
+    const int32_t place = sm - mine; // the tile's first place of digit tid
+    gbase[tid] = st - total + before - place;
+    // each wave: the place of every key in the wave's run of its digit
+    const uint64_t lt = lane == 0 ? 0ull : ~0ull >> (64 - lane);
+    lds_vshort* run_of = (lds_vshort*)wrun[wave];
+    int lp[FS_ROUNDS];
+#pragma unroll
+    for (int r = 0; r < FS_ROUNDS; ++r) {
+        const bool valid = wave * kWaveKeys + r * 64 + lane < tile_n;
+        const uint32_t d = kr[r] >> shift & 1023u;
+        const uint64_t peers = digit_peers<10>(d, __ballot(valid));
+        const int rank = __popcll(peers & lt);
+        const int run = valid ? run_of[d] : 0;
+        lp[r] = run + rank;
+        // in order, as in k_rs_scatter
+        if (valid && rank == 0) run_of[d] = (uint16_t)(run + (int)__popcll(peers));
+    }
+    __syncthreads();
+    int at = place;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+        const int len = wrun[w][tid];
+        wrun[w][tid] = (uint16_t)at;
+        at += len;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < FS_ROUNDS; ++r) {
+        if (wave * kWaveKeys + r * 64 + lane < tile_n) {
+            const int pos = wrun[wave][kr[r] >> shift & 1023u] + lp[r];
+            lk[pos] = kr[r];
+            lv[pos] = vr[r];
+        }
+    }
+    __syncthreads();
+    for (int t = tid; t < tile_n; t += 1024) {
+        const uint32_t key = lk[t];
+        const int pos = gbase[key >> shift & 1023u] + t;
+        if (kout) kout[pos] = key;
         vout[pos] = lv[t];
     }
 }
@@ -324,10 +450,10 @@ __global__ __launch_bounds__(256) void k_iota(uint32_t* __restrict__ v, int64_t 
 }
 
 // the passes over caller-provided histogram scratch: hist holds 256 x ceil(n / RS_TILE) and
-// rowsum 256 int32
+// rowsum 256 int32.  keys_out: the caller reads the sorted keys (else the last pass writes none)
 template <typename KeyT>
 void radix_sort_core(KeyT*& keys, uint32_t*& vals, KeyT*& keys_alt, uint32_t*& vals_alt, int64_t n, int begin_bit,
-                     int end_bit, bool vals_are_index, int32_t* hist, int32_t* rowsum, hipStream_t s)
+                     int end_bit, bool vals_are_index, bool keys_out, int32_t* hist, int32_t* rowsum, hipStream_t s)
 {
     if (n <= 1 || begin_bit >= end_bit) {
         if (n >= 1 && vals_are_index) {
@@ -344,8 +470,9 @@ void radix_sort_core(KeyT*& keys, uint32_t*& vals, KeyT*& keys_alt, uint32_t*& v
         hipLaunchKernelGGL(k_rs_rows, dim3(256), dim3(256), 0, s, hist, nblocks, rowsum);
         FWN_LAUNCH_CHECK("k_rs_rows");
         const uint32_t* vin = (vals_are_index && shift == begin_bit) ? nullptr : vals;
-        hipLaunchKernelGGL(k_rs_scatter<KeyT>, dim3(nblocks), dim3(RS_THREADS), 0, s, keys, vin, keys_alt,
-                           vals_alt, n, shift, hist, rowsum, nblocks);
+        KeyT* kout = keys_out || shift + 8 < end_bit ? keys_alt : nullptr;
+        hipLaunchKernelGGL(k_rs_scatter<KeyT>, dim3(nblocks), dim3(RS_THREADS), 0, s, keys, vin, kout, vals_alt, n,
+                           shift, hist, rowsum, nblocks);
         FWN_LAUNCH_CHECK("k_rs_scatter");
         std::swap(keys, keys_alt);
         std::swap(vals, vals_alt);
@@ -354,15 +481,15 @@ void radix_sort_core(KeyT*& keys, uint32_t*& vals, KeyT*& keys_alt, uint32_t*& v
 
 template <typename KeyT>
 void radix_sort_impl(KeyT*& keys, uint32_t*& vals, KeyT*& keys_alt, uint32_t*& vals_alt, int64_t n, int begin_bit,
-                     int end_bit, bool vals_are_index, DBuf& hist, DBuf& rowsum, hipStream_t s)
+                     int end_bit, bool vals_are_index, bool keys_out, DBuf& hist, DBuf& rowsum, hipStream_t s)
 {
     if (n > 1 && begin_bit < end_bit) {
         const int64_t nblocks = (n + RS_TILE - 1) / RS_TILE;
         hist.reserve(sizeof(int32_t) * 256 * (size_t)nblocks);
         rowsum.reserve(sizeof(int32_t) * 256);
     }
-    radix_sort_core<KeyT>(keys, vals, keys_alt, vals_alt, n, begin_bit, end_bit, vals_are_index, hist.as<int32_t>(),
-                          rowsum.as<int32_t>(), s);
+    radix_sort_core<KeyT>(keys, vals, keys_alt, vals_alt, n, begin_bit, end_bit, vals_are_index, keys_out,
+                          hist.as<int32_t>(), rowsum.as<int32_t>(), s);
 }
 
 } // namespace
@@ -370,13 +497,14 @@ void radix_sort_impl(KeyT*& keys, uint32_t*& vals, KeyT*& keys_alt, uint32_t*& v
 void radix_sort_pairs(uint64_t*& keys, uint32_t*& vals, uint64_t*& keys_alt, uint32_t*& vals_alt, int64_t n,
                       int nbits, DBuf& hist, DBuf& rowsum, hipStream_t s)
 {
-    radix_sort_impl<uint64_t>(keys, vals, keys_alt, vals_alt, n, 0, nbits, false, hist, rowsum, s);
+    radix_sort_impl<uint64_t>(keys, vals, keys_alt, vals_alt, n, 0, nbits, false, true, hist, rowsum, s);
 }
 
 void radix_sort_pairs32(uint32_t*& keys, uint32_t*& vals, uint32_t*& keys_alt, uint32_t*& vals_alt, int64_t n,
                         int begin_bit, int end_bit, bool vals_are_index, DBuf& hist, DBuf& rowsum, hipStream_t s)
 {
-    radix_sort_impl<uint32_t>(keys, vals, keys_alt, vals_alt, n, begin_bit, end_bit, vals_are_index, hist, rowsum, s);
+    radix_sort_impl<uint32_t>(keys, vals, keys_alt, vals_alt, n, begin_bit, end_bit, vals_are_index, false, hist, rowsum,
+                              s);
 }
 
 int64_t radix_sort_hist_words(int64_t n)
@@ -388,7 +516,22 @@ void radix_sort_pairs32_scratch(uint32_t*& keys, uint32_t*& vals, uint32_t*& key
                                 int begin_bit, int end_bit, bool vals_are_index, int32_t* hist, int32_t* rowsum,
                                 hipStream_t s)
 {
-    radix_sort_core<uint32_t>(keys, vals, keys_alt, vals_alt, n, begin_bit, end_bit, vals_are_index, hist, rowsum, s);
+    radix_sort_core<uint32_t>(keys, vals, keys_alt, vals_alt, n, begin_bit, end_bit, vals_are_index, false, hist, rowsum,
+                              s);
+}
+
+void sort_few_tiles(const uint32_t* keys, uint32_t* keys_alt, uint32_t* vals_alt, uint32_t* vals, int64_t n,
+                    int32_t* hist, hipStream_t s)
+{
+    const int tiles = few_tiles(n);
+    hipLaunchKernelGGL(k_fs_scatter, dim3(tiles), dim3(1024), 0, s, keys, (const uint32_t*)nullptr, keys_alt, vals_alt,
+                       (int)n, 12, hist, tiles);
+    FWN_LAUNCH_CHECK("k_fs_scatter");
+    hipLaunchKernelGGL(k_fs_hist, dim3(tiles), dim3(1024), 0, s, keys_alt, (int)n, 22, hist);
+    FWN_LAUNCH_CHECK("k_fs_hist");
+    hipLaunchKernelGGL(k_fs_scatter, dim3(tiles), dim3(1024), 0, s, keys_alt, vals_alt, (uint32_t*)nullptr, vals, (int)n,
+                       22, hist, tiles);
+    FWN_LAUNCH_CHECK("k_fs_scatter");
 }
 
 // out must hold n+1 entries; out[n] receives the total.
