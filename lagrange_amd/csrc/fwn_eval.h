@@ -28,7 +28,9 @@ __device__ __forceinline__ float tri_f32(const float* __restrict__ t, float qx, 
     float la2 = fmaf(ax, ax, fmaf(ay, ay, az * az));
     float lb2 = fmaf(bx, bx, fmaf(by, by, bz * bz));
     float lc2 = fmaf(cx, cx, fmaf(cy, cy, cz * cz));
-    if (la2 == 0.0f || lb2 == 0.0f || lc2 == 0.0f) return 0.0f;
+    // a zero where a corner or the plane is hit, selected at the end: two branches around the rest cost
+    // more than they save
+    const bool corner = la2 == 0.0f || lb2 == 0.0f || lc2 == 0.0f;
     float ia = __builtin_amdgcn_rsqf(la2), ib = __builtin_amdgcn_rsqf(lb2), ic = __builtin_amdgcn_rsqf(lc2);
     ax *= ia; ay *= ia; az *= ia;
     bx *= ib; by *= ib; bz *= ib;
@@ -39,12 +41,11 @@ __device__ __forceinline__ float tri_f32(const float* __restrict__ t, float qx, 
     float ny = fmaf(uz, vx, -ux * vz);
     float nz = fmaf(ux, vy, -uy * vx);
     float num = fmaf(ax, nx, fmaf(ay, ny, az * nz));
-    if (num == 0.0f) return 0.0f;
     float ab = fmaf(ax, bx, fmaf(ay, by, az * bz));
     float ac = fmaf(ax, cx, fmaf(ay, cy, az * cz));
     float bc = fmaf(bx, cx, fmaf(by, cy, bz * cz));
     float den = 1.0f + ab + ac + bc;
-    return 2.0f * atan2f(num, den);
+    return corner || num == 0.0f ? 0.0f : 2.0f * atan2f(num, den);
 }
 
 // exact triangle solid angle, FP64, 2 atan2(a.(b x c), |a||b||c| + (a.b)|c| + (b.c)|a| + (c.a)|b|)

@@ -125,6 +125,17 @@ __device__ __forceinline__ SlotRegs load_slot(const uint32_t* __restrict__ p)
 __device__ __forceinline__ uint32_t su(const SlotRegs& r, int k) { return k < 16 ? r.a[k] : r.b[k - 16]; }
 __device__ __forceinline__ float sw(const SlotRegs& r, int k) { return __uint_as_float(su(r, k)); }
 
+// a triangle's record in SGPRs: two scalar loads issued together
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+typedef v4u v4u_a4 __attribute__((aligned(4)));
+__device__ __forceinline__ void load_tri(const uint32_t* __restrict__ p, float (&t)[kTriWords])
+{
+    const v8u a = *reinterpret_cast<const v8u_a4*>(p);
+    const v4u b = *reinterpret_cast<const v4u_a4*>(p + 8);
+#pragma unroll
+    for (int k = 0; k < kTriWords; ++k) t[k] = __uint_as_float(k < 8 ? a[k] : b[k - 8]);
+}
+
 struct SlotWords {
     const SlotRegs& r;
     __device__ __forceinline__ float operator()(int k) const { return sw(r, k); }
@@ -173,7 +184,7 @@ __device__ __forceinline__ void traverse_batch(
     const float qz = valid ? Q[3 * (int64_t)orig + 2] : 0.0f;
     const int32_t root = roots[2 * m];
     const int32_t root_ns = roots[2 * m + 1];
-    const float tau = minfo[8 * m + 6];
+    const uint64_t tau_mask = __ballot(minfo[8 * m + 6] > 0.0f); // all lanes or none
 
     const uint32_t node_words = (uint32_t)width * kSlotWords;
     float om = 0.0f;
@@ -221,29 +232,30 @@ __device__ __forceinline__ void traverse_batch(
                     if (leaf) {
                         const int32_t first = (int32_t)((link & ~FWN_LINK_LEAF) >> 3);
                         const int32_t tcnt = (int32_t)(link & 7u) + 1;
-                        const bool nl = __builtin_amdgcn_inverse_ballot_w64(nearm);
                         // FP64 for points within tau of the leaf's bounding sphere and, for a single
                         // triangle, within tau of its plane (p lies on that plane); both thresholds are
                         // stored in the leaf's first triangle
-                        const float* t0 = reinterpret_cast<const float*>(tris + (size_t)first * kTriWords);
-                        const float near2 = t0[FWN_T_NEAR2], plane = t0[FWN_T_PLANE];
+                        float t0[kTriWords]; // the whole first triangle at once
+                        load_tri(tris + (size_t)first * kTriWords, t0);
                         const float nd =
                             fmaf(dx, sw(cur, FWN_W_NX), fmaf(dy, sw(cur, FWN_W_NY), dz * sw(cur, FWN_W_NZ)));
-                        const bool use64 = nl && tau > 0.0f && d2 < near2 && (tcnt > 1 || nd * nd < plane);
-                        const bool use32 = nl && !use64;
-                        if (__ballot(use32) != 0ull) {
-                            for (int32_t t = first; t < first + tcnt; ++t) {
-                                const float* tw = reinterpret_cast<const float*>(tris + (size_t)t * kTriWords);
+                        uint64_t m64 = nearm & tau_mask & __ballot(d2 < t0[FWN_T_NEAR2]);
+                        if (tcnt == 1) m64 &= __ballot(nd * nd < t0[FWN_T_PLANE]);
+                        const uint64_t m32 = nearm & ~m64;
+                        if (m32 != 0ull) {
+                            const bool use32 = __builtin_amdgcn_inverse_ballot_w64(m32);
+                            for (int32_t t = first;;) {
                                 if (use32) {
-                                    om += tri_f32(tw, qx, qy, qz);
+                                    om += tri_f32(t0, qx, qy, qz);
                                     if (STATS) ++n_t32;
                                 }
+                                if (++t == first + tcnt) break;
+                                load_tri(tris + (size_t)t * kTriWords, t0);
                             }
                         }
-                        const uint64_t m64 = __ballot(use64);
                         if (m64 != 0ull) {
                             if (n64 == 0) acc[lane] = 0ull;
-                            if (use64) {
+                            if (__builtin_amdgcn_inverse_ballot_w64(m64)) {
                                 const uint32_t below = __builtin_amdgcn_mbcnt_hi(
                                     (uint32_t)(m64 >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m64, 0u));
                                 queue[nq + (int)below] = make_uint2(link & ~FWN_LINK_LEAF, (uint32_t)lane);
