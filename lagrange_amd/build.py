@@ -24,7 +24,7 @@ HIP_FLAGS = [
 
 
 # per-source additions: the traversals' FP64 constants must not be hoisted out of their walks (61
-# vector registers instead of 112, slots in lanes 68 instead of 118); the surrogate's MFMA kernels
+# vector registers instead of 112, slots in lanes 64 instead of 118); the surrogate's MFMA kernels
 # keep their accumulators in VGPRs (the fused MLP's bias/ReLU/BF16 epilogue then reads them without
 # 512 AGPR-to-VGPR moves per tile)
 EXTRA_FLAGS = {

@@ -1,8 +1,8 @@
 // Winding number queries with a node's slots in the lanes of a wave (gfx950): the batched
 // traversal of calls whose points are far apart compared with the mesh's triangles.  Compiled
 // without machine LICM: it would keep the FP64 constants of the near-field evaluation in 40 vector
-// registers through the whole walk (118 registers, 4 waves per SIMD, instead of 68 and 7; 4M
-// uniform points, 199,692 triangles: 1556 -> 1283 us).
+// registers through the whole walk (118 registers, 4 waves per SIMD, instead of 64 and the 6 and a
+// half that the LDS allows).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -32,11 +32,13 @@ namespace {
 // at a time, one leaf per lane, their sums added in 2^-40 fixed point (associative) to the
 // point's LDS accumulator.  Results are bit for bit those of k_traverse.
 //
-// Bound: VALU issue (SQ counters, 4M points, F = 199,692: 2,467 VALU instructions per wave of 16
-// uniform points over 38 node visits, 7,733 over 88 visits for points near the surface; 83 and 95 %
-// of the issue slots) once a call has enough waves, the chain of node visits below that.  Whole
-// calls, k_traverse then this kernel: 20,000 uniform points, F = 20,172 427 -> 176 us; 100k points,
-// F = 199,692 734 -> 244 us uniform, 820 -> 320 us near the surface.
+// Bound: VALU issue (400k points near the surface, F = 190k: 9,700 VALU and 6,100 SALU instructions per
+// wave over 100 node visits, three quarters of the issue slots) once a call has enough waves, the chain
+// of node visits below that.  Leaf triangles are loaded before the far terms they arrive behind, FP64
+// leaves flushed outside the node loop and their lanes not evaluated in FP32 too: 400k points, F =
+// 199,692, 254 -> 221 us uniform and 564 -> 497 near the surface.  Kernels alone, k_traverse then this
+// one: 20,000 uniform points, F = 20,172 353 and 97 us; 100k points, F = 199,692 667 and 146 us uniform,
+// 754 and 216 near the surface.
 constexpr int kQuadQueue = 128; // FP64 leaves waiting (at most 63 before a node adds 64)
 constexpr int kQuadNodeBytes = 4 * kSlotWords * 4; // one 4-wide node
 
@@ -112,8 +114,7 @@ __global__ __launch_bounds__(64) void k_traverse_quad(
     const float qz = valid ? Q[3 * (int64_t)orig + 2] : 0.0f;
     const int32_t root = roots[2 * m];
     const int32_t root_ns = roots[2 * m + 1];
-    const float tau = minfo[8 * m + 6];
-    const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    const uint64_t tau_mask = __ballot(minfo[8 * m + 6] > 0.0f); // all lanes or none
     if (s == 0) {
         acc[p] = 0ull;
         qpos[p] = make_float4(qx, qy, qz, 0.0f);
@@ -130,134 +131,140 @@ __global__ __launch_bounds__(64) void k_traverse_quad(
             fetch_node(nb, quad_lds + at * kNode4, 4, lane);
         };
         fetch(st_link, 0);
-        int sp = 1;
-        bool overflow = false;
-        for (;;) {
-            if (sp == 0 || nq >= 64) { // 64 queued leaves, or what is left at the end
-                __syncthreads();
-                while (nq >= 64 || (sp == 0 && nq > 0)) {
-                    const int take = min(nq, 64);
-                    nq -= take;
-                    if (lane < take) {
-                        const uint2 it = queue[nq + lane];
-                        const float4 q = qpos[it.y];
-                        const uint32_t first = it.x >> 3, n = (it.x & 7u) + 1u;
-                        double s64 = 0.0;
-                        for (uint32_t t = first; t < first + n; ++t)
-                            s64 += tri_f64(reinterpret_cast<const float*>(tris + (size_t)t * kTriWords), q.x, q.y, q.z);
-                        atomicAdd(&acc[it.y], (unsigned long long)__double2ll_rn(s64 * kFixScale));
-                    }
+        int sp = 1, sp_max = 1;
+        do {
+            while (((sp - 1) | (63 - nq)) >= 0) { // sp > 0 and nq < 64
+                --sp;
+                const uint32_t e = (uint32_t)__builtin_amdgcn_readlane((int)st_link, sp);
+                const uint32_t m16 = (uint32_t)__builtin_amdgcn_readlane((int)st_mask, sp);
+                uint4 x[kSlotWords / 4];
+                if (sp < lds_nodes) {
+                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // this node's fetch has landed
+                    const uint4* src = quad_lds + sp * kNode4 + s * (kSlotWords / 4);
+#pragma unroll
+                    for (int k = 0; k < kSlotWords / 4; ++k) x[k] = src[k];
+                } else { // a stack position without a buffer
+                    const char* nb = reinterpret_cast<const char*>(slots + (size_t)(e >> 4) * (size_t)(4 * kSlotWords));
+                    const uint4* src = reinterpret_cast<const uint4*>(nb + (uint32_t)s * (kSlotWords * 4));
+#pragma unroll
+                    for (int k = 0; k < kSlotWords / 4; ++k) x[k] = src[k];
                 }
-                __syncthreads();
-                if (sp == 0) break;
-            }
-            --sp;
-            const uint32_t e = (uint32_t)__builtin_amdgcn_readlane((int)st_link, sp);
-            const uint32_t m16 = (uint32_t)__builtin_amdgcn_readlane((int)st_mask, sp);
-            uint4 x[kSlotWords / 4];
-            if (sp < lds_nodes) {
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // this node's fetch has landed
-                const uint4* src = quad_lds + sp * kNode4 + s * (kSlotWords / 4);
+                // the lanes with a point to test: the points of the mask, the node's occupied slots
+                const uint64_t mk = quad_expand(m16) & __ballot(s < (int)(e & 15u));
+                float w[FWN_W_LINK];
 #pragma unroll
-                for (int k = 0; k < kSlotWords / 4; ++k) x[k] = src[k];
-            } else { // a stack position without a buffer
-                const uint4* src = reinterpret_cast<const uint4*>(slots + (size_t)(e >> 4) * (size_t)(4 * kSlotWords)) +
-                                   s * (kSlotWords / 4);
+                for (int k = 0; k < FWN_W_LINK; ++k) w[k] = __uint_as_float(reinterpret_cast<const uint32_t*>(x)[k]);
+                const uint32_t link = x[5].w;
+                const float dx = w[FWN_W_PX] - qx, dy = w[FWN_W_PY] - qy, dz = w[FWN_W_PZ] - qz;
+                const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                const uint64_t farb = __ballot(d2 > w[FWN_W_THR]);
+                const uint64_t nearm = mk & ~farb;
+                const uint64_t leafm = nearm & __ballot((int32_t)link < 0);
+                // children, in slot order, each fetched as it is pushed: the node's words are in
+                // registers before a fetch overwrites its buffer
+                const uint64_t inner = nearm & ~leafm;
+                if (inner != 0ull) {
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
-                for (int k = 0; k < kSlotWords / 4; ++k) x[k] = src[k];
-            }
-            // the lanes with a point to test: the points of the mask, the node's occupied slots
-            const uint64_t mk = quad_expand(m16) & __ballot(s < (int)(e & 15u));
-            float w[FWN_W_LINK];
-#pragma unroll
-            for (int k = 0; k < FWN_W_LINK; ++k) w[k] = __uint_as_float(reinterpret_cast<const uint32_t*>(x)[k]);
-            const uint32_t link = x[5].w;
-            const float dx = w[FWN_W_PX] - qx, dy = w[FWN_W_PY] - qy, dz = w[FWN_W_PZ] - qz;
-            const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-            const uint64_t farb = __ballot(d2 > w[FWN_W_THR]);
-            const uint64_t nearm = mk & ~farb;
-            const uint64_t leafm = nearm & __ballot((int32_t)link < 0);
-            // children, in slot order, each fetched as it is pushed: the node's words are in
-            // registers before a fetch overwrites its buffer
-            const uint64_t inner = nearm & ~leafm;
-            if (inner != 0ull) {
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const uint64_t mc = inner & (0x1111111111111111ull << c);
-                    if (mc != 0ull) {
-                        const uint32_t lc = (uint32_t)__builtin_amdgcn_readlane((int)link, c);
-                        st_link = wave_writelane(lc, sp & 63, st_link);
-                        st_mask = wave_writelane(quad_mask(mc), sp & 63, st_mask);
-                        if (sp < lds_nodes) fetch(lc, sp);
-                        ++sp;
+                    for (int c = 0; c < 4; ++c) {
+                        const uint64_t mc = inner & (0x1111111111111111ull << c);
+                        if (mc != 0ull) {
+                            const uint32_t lc = (uint32_t)__builtin_amdgcn_readlane((int)link, c);
+                            st_link = wave_writelane(lc, sp & 63, st_link);
+                            st_mask = wave_writelane(quad_mask(mc), sp & 63, st_mask);
+                            if (sp < lds_nodes) fetch(lc, sp);
+                            ++sp;
+                        }
                     }
+                    sp_max = max(sp_max, sp);
                 }
-                overflow |= sp > 64; // never with the host's stack bound
-            }
-            float a = 0.0f, b = 0.0f;
-            if (__builtin_amdgcn_inverse_ballot_w64(mk & farb)) far_field_terms(LaneWords{w}, dx, dy, dz, d2, a, b);
-            if (leafm != 0ull) {
-                const bool nl = __builtin_amdgcn_inverse_ballot_w64(leafm);
+                // the leaves' triangles are on their way while the far terms are evaluated
                 const int32_t first = (int32_t)((link & ~FWN_LINK_LEAF) >> 3);
                 const int32_t tcnt = BUCKET ? (int32_t)(link & 7u) + 1 : 1;
-                bool use64 = false;
-                float v0 = 0.0f;
-                if (nl) { // the whole record in one round trip
-                    const uint4* tp = reinterpret_cast<const uint4*>(tris + (size_t)first * kTriWords);
+                uint4 y[kTriWords / 4];
+                if (leafm != 0ull) { // lanes without a leaf: the first triangle, in one line for all of them
+                    const uint32_t at = __builtin_amdgcn_inverse_ballot_w64(leafm) ? (uint32_t)first : 0u;
+                    const uint4* tp = reinterpret_cast<const uint4*>(tris + (size_t)at * kTriWords);
+#pragma unroll
+                    for (int k = 0; k < kTriWords / 4; ++k) y[k] = tp[k];
+                }
+                float a = 0.0f, b = 0.0f;
+                if (__builtin_amdgcn_inverse_ballot_w64(mk & farb))
+                    far_field_terms(LaneWords{w}, dx, dy, dz, d2, a, b);
+                if (leafm != 0ull) {
                     float tw[kTriWords];
 #pragma unroll
                     for (int k = 0; k < kTriWords / 4; ++k) {
-                        const uint4 y = tp[k];
-                        tw[4 * k] = __uint_as_float(y.x);
-                        tw[4 * k + 1] = __uint_as_float(y.y);
-                        tw[4 * k + 2] = __uint_as_float(y.z);
-                        tw[4 * k + 3] = __uint_as_float(y.w);
+                        tw[4 * k] = __uint_as_float(y[k].x);
+                        tw[4 * k + 1] = __uint_as_float(y[k].y);
+                        tw[4 * k + 2] = __uint_as_float(y[k].z);
+                        tw[4 * k + 3] = __uint_as_float(y[k].w);
                     }
                     const float nd = fmaf(dx, w[FWN_W_NX], fmaf(dy, w[FWN_W_NY], dz * w[FWN_W_NZ]));
-                    use64 = tau > 0.0f && d2 < tw[FWN_T_NEAR2] && (tcnt > 1 || nd * nd < tw[FWN_T_PLANE]);
-                    v0 = tri_f32(tw, qx, qy, qz);
-                    a = use64 ? 0.0f : 1.0f;
-                    b = use64 ? 0.0f : v0;
-                }
-                const uint64_t m64 = __ballot(use64);
-                if (m64 != 0ull) {
-                    if (use64)
-                        queue[nq + (int)__popcll(m64 & lt_mask)] =
-                            make_uint2(((uint32_t)first << 3) | (uint32_t)(tcnt - 1), (uint32_t)p);
-                    nq += (int)__popcll(m64);
-                }
-                if (BUCKET) {
-                    const int n32 = nl && !use64 ? tcnt : 0;
-                    const uint64_t more = __ballot(n32 > 1);
-                    if (more != 0ull) {
-                        // the buckets' other triangles, then every slot's terms in order
-                        float v[8];
-#pragma unroll
-                        for (int k = 1; k < 8; ++k) {
-                            v[k] = 0.0f;
-                            if (k < n32)
-                                v[k] = tri_f32(reinterpret_cast<const float*>(tris + (size_t)(first + k) * kTriWords),
-                                               qx, qy, qz);
+                    uint64_t plane = __ballot(nd * nd < tw[FWN_T_PLANE]);
+                    if (BUCKET) plane |= __ballot(tcnt > 1);
+                    const uint64_t m64 = leafm & tau_mask & plane & __ballot(d2 < tw[FWN_T_NEAR2]);
+                    const bool use64 = __builtin_amdgcn_inverse_ballot_w64(m64);
+                    const bool use32 = __builtin_amdgcn_inverse_ballot_w64(leafm & ~m64);
+                    if (use32) {
+                        a = 1.0f;
+                        b = tri_f32(tw, qx, qy, qz);
+                    }
+                    if (m64 != 0ull) {
+                        if (use64) {
+                            const uint32_t below = __builtin_amdgcn_mbcnt_hi(
+                                (uint32_t)(m64 >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m64, 0u));
+                            queue[nq + (int)below] = make_uint2(link & ~FWN_LINK_LEAF, (uint32_t)p);
                         }
-                        auto slot_terms = [&](auto c) __attribute__((always_inline)) {
-                            om = fmaf(quad_bcast<c.value>(a), quad_bcast<c.value>(b), om);
-                            if ((more & (0x1111111111111111ull << c.value)) != 0ull) {
+                        nq += (int)__popcll(m64);
+                    }
+                    if (BUCKET) {
+                        const int n32 = use32 ? tcnt : 0;
+                        const uint64_t more = __ballot(n32 > 1);
+                        if (more != 0ull) {
+                            // the buckets' other triangles, then every slot's terms in order
+                            float v[8];
 #pragma unroll
-                                for (int k = 1; k < 8; ++k) om += quad_bcast<c.value>(v[k]);
+                            for (int k = 1; k < 8; ++k) {
+                                v[k] = 0.0f;
+                                const uint32_t* tk = tris + (size_t)(first + k) * kTriWords;
+                                if (k < n32) v[k] = tri_f32(reinterpret_cast<const float*>(tk), qx, qy, qz);
                             }
-                        };
-                        slot_terms(std::integral_constant<int, 0>{});
-                        slot_terms(std::integral_constant<int, 1>{});
-                        slot_terms(std::integral_constant<int, 2>{});
-                        slot_terms(std::integral_constant<int, 3>{});
-                        continue;
+                            auto slot_terms = [&](auto c) __attribute__((always_inline)) {
+                                om = fmaf(quad_bcast<c.value>(a), quad_bcast<c.value>(b), om);
+                                if ((more & (0x1111111111111111ull << c.value)) != 0ull) {
+#pragma unroll
+                                    for (int k = 1; k < 8; ++k) om += quad_bcast<c.value>(v[k]);
+                                }
+                            };
+                            slot_terms(std::integral_constant<int, 0>{});
+                            slot_terms(std::integral_constant<int, 1>{});
+                            slot_terms(std::integral_constant<int, 2>{});
+                            slot_terms(std::integral_constant<int, 3>{});
+                            continue;
+                        }
                     }
                 }
+                om = quad_terms(a, b, om);
             }
-            om = quad_terms(a, b, om);
-        }
-        if (overflow && lane == 0) atomicOr(flag, 1);
+            // 64 queued leaves, or what is left at the end
+            __syncthreads();
+            while (nq >= 64 || (sp == 0 && nq > 0)) {
+                const int take = min(nq, 64);
+                nq -= take;
+                if (lane < take) {
+                    const uint2 it = queue[nq + lane];
+                    const float4 q = qpos[it.y];
+                    const uint32_t first = it.x >> 3, n = BUCKET ? (it.x & 7u) + 1u : 1u;
+                    double s64 = 0.0;
+                    for (uint32_t t = first; t < first + n; ++t)
+                        s64 += tri_f64(reinterpret_cast<const float*>(tris + (size_t)t * kTriWords), q.x, q.y, q.z);
+                    atomicAdd(&acc[it.y], (unsigned long long)__double2ll_rn(s64 * kFixScale));
+                }
+            }
+            __syncthreads();
+        } while (sp > 0);
+        if (sp_max > 64 && lane == 0) atomicOr(flag, 1); // never with the host's stack bound
     }
     if (valid && s == 0) {
         const long long v = (long long)acc[p];
@@ -273,20 +280,20 @@ __global__ __launch_bounds__(64) void k_traverse_quad(
 // of the default launch shape (the other shapes are k_traverse's, chosen by the tuner or the
 // caller), up to kQuadCross * cbrt(F) points for a mesh of F triangles (several: of the mean F)
 // and, for several meshes, kQuadSparse points a triangle more, as each mesh's share of the points
-// is sparse on it however many the call has.  The two kernels' costs
-// cross where the 64 points of a k_traverse wave are close together compared with the nodes they
+// is sparse on it however many the call has.  The two kernels' costs cross where the 64 points of a k_traverse wave are close together compared with the nodes they
 // visit, for points near the surface (both kernels walk to the triangles) at fewer points than for
-// uniform ones; the line lies between the two crossings.  k_traverse / this kernel in us,
-//   uniform: F = 972 171 / 156 (200k points) and 191 / 212 (400k); F = 20,172 341 / 257 (400k),
-//     366 / 368 (800k), 467 / 578 (1.5M); F = 199,692 713 / 431 (800k), 800 / 627 (1.5M), 1095 /
-//     1333 (4M); F = 940,800 1182 / 681 (1.5M), 1576 / 1408 (4M);
-//   near the surface: F = 972 179 / 179 (200k); F = 20,172 431 / 396 (400k), 507 / 619 (800k);
-//     F = 199,692 724 / 586 (400k), 886 / 913 (800k), 1156 / 1465 (1.5M); F = 940,800 1472 / 1343
-//     (800k), 1834 / 2128 (1.5M);
+// uniform ones; the line lies between the two crossings.  k_traverse / this kernel in us, with the
+// sort,
+//   uniform: F = 972 138 / 120 (200k points) and 170 / 182 (400k); F = 20,172 349 / 336 (800k), 455 /
+//     516 (1.5M); F = 199,692 731 / 567 (1.5M), 858 / 814 (2.5M), 1038 / 1215 (4M); F = 940,800
+//     1278 / 883 (2.5M), 1456 / 1269 (4M);
+//   near the surface: F = 972 150 / 143 (200k), 187 / 225 (400k); F = 20,172 348 / 350 (400k), 495 /
+//     567 (800k); F = 199,692 861 / 844 (800k), 1119 / 1355 (1.5M); F = 940,800 1380 / 1287 (800k), 1800 /
+//     2021 (1.5M);
 //   several meshes, uniform / near the surface (the kernels alone): 64 x 20k points, F = 199,692
-//     1872 / 873 and 5661 / 3039, F = 19,200 1113 / 738 and 1649 / 1328, F = 1,728 553 / 587 and 623 /
-//     778; 32 x 100k points, F = 19,200 1350 / 1274 and 1974 / 2362; 8 meshes of 14k to 48k, 1M
-//     points, 720 / 462; 32 of 1.7k to 181k, 3.7M points, 1208 / 1297.
+//     1800 / 808 and 5516 / 2818, F = 19,200 1058 / 669 and 1589 / 1241, F = 1,728 535 / 528 and 608 /
+//     713; 32 x 100k points, F = 19,200 1322 / 1169 and 1920 / 2164; 8 meshes of 14k to 48k, 1M
+//     points, 703 / 409; 32 of 1.7k to 181k, 3.7M points, 1199 / 1214.
 constexpr double kQuadCross = 24000.0, kQuadSparse = 2.0;
 bool use_quads(const Engine& e, int64_t nQ, int banks)
 {
@@ -299,8 +306,9 @@ void launch_quads(Engine& e, const float* dQ, const uint32_t* perm, const int64_
                   const int32_t* order, int M, int64_t nb, float* omega, uint8_t* inside, int32_t* flag, hipStream_t s)
 {
     // node buffers per wave: 20 (9 KB, room for 4 waves per SIMD) while the call has no more waves
-    // than that, else 12 (6 KB: 7 waves per SIMD, the registers' bound too); entries above them are
-    // rare (30k points, F = 199,692: 12 buffers 154 us, 20 147 us; 4M points: 1198 and 1528 us)
+    // than that, else 12 (6 KB: 6 and a half); entries above them are rare.  F = 199,692, uniform and
+    // near the surface, 9 / 12 / 20 buffers: 20k points 135 / 132 / 118 and 215 / 200 / 178 us, 400k
+    // points 224 / 221 / 246 and 573 / 497 / 565 us
     const int lds_nodes = std::min(nb <= 4096 ? 20 : 12, 1 + 3 * std::max(e.max_depth, 1));
     const size_t lds = quad_lds_bytes(lds_nodes);
 #define FWN_QUAD(BUCKET)                                                                                            \
