@@ -867,77 +867,124 @@ __global__ __launch_bounds__(BT) void k_write_slots(int64_t W, int width, const 
     tw[FWN_T_PLANE] = __float_as_uint((tau * tau) * nn);
 }
 
-// Each slot's disk, from its triangles' vertices in double; a row of 16 lanes per slot.  A slot of more
-// than kDiskTris triangles (nearly always entered, and a serial loop here) or with a sliver (sine below
-// 1e-4: its evaluated distance may be off by more than the bound allows for) gets no bound.
-constexpr int64_t kDiskTris = 1024;
+// Each slot's disk, from its triangles' vertices in double.  A thread takes a slot of one triangle by
+// itself (three in four); the block's other slots are listed and taken by rows of 16 lanes, those above
+// kDiskRow triangles by waves.  A block's slots are spread over the array, as the large ones come first.  101,568 triangles: 48 us with a row
+// for every slot, 41 so, and 940,800 395 us and 182.  A slot of more than kDiskTris triangles (nearly always entered, and a serial
+// loop here) or with a sliver (sine below 1e-4: its evaluated distance may be off by more than the bound
+// allows for) gets no bound (400k closest points, F = 199,692: limit 128 4.33 ms, 512 4.07, 1,024 3.98).
+constexpr int64_t kDiskTris = 1024, kDiskRow = 64;
+
+struct DiskSpan { // of a slot's triangles about a point and a normal; rounded outward
+    float lo = INFINITY, hi = -INFINITY, rr = 0.0f;
+    bool none = false;
+};
+
+__device__ __forceinline__ void disk_triangle(const float* __restrict__ tw, const double (&c0)[3],
+                                              const double (&nn)[3], DiskSpan& S)
+{
+    double w[3][3];
+    for (int k = 0; k < 3; ++k)
+        for (int d = 0; d < 3; ++d) w[k][d] = (double)tw[3 * k + d] - c0[d];
+    double e1[3], e2[3];
+    for (int d = 0; d < 3; ++d) {
+        e1[d] = w[1][d] - w[0][d];
+        e2[d] = w[2][d] - w[0][d];
+    }
+    const double N[3] = {e1[1] * e2[2] - e1[2] * e2[1], e1[2] * e2[0] - e1[0] * e2[2],
+                         e1[0] * e2[1] - e1[1] * e2[0]};
+    S.none |= !(N[0] * N[0] + N[1] * N[1] + N[2] * N[2] >
+                1e-8 * (e1[0] * e1[0] + e1[1] * e1[1] + e1[2] * e1[2]) *
+                    (e2[0] * e2[0] + e2[1] * e2[1] + e2[2] * e2[2]));
+    for (int k = 0; k < 3; ++k) {
+        const double h = w[k][0] * nn[0] + w[k][1] * nn[1] + w[k][2] * nn[2];
+        double q = 0.0;
+        for (int d = 0; d < 3; ++d) q += (w[k][d] - h * nn[d]) * (w[k][d] - h * nn[d]);
+        S.lo = fminf(S.lo, __double2float_rd(h));
+        S.hi = fmaxf(S.hi, __double2float_ru(h));
+        S.rr = fmaxf(S.rr, __double2float_ru(q));
+    }
+}
+
+__device__ __forceinline__ void write_disk(float* __restrict__ o, const double (&c0)[3], const double (&nn)[3],
+                                           const DiskSpan& S)
+{
+    float c[3];
+    double margin = 0.0; // the rounding of c and n
+    for (int d = 0; d < 3; ++d) {
+        c[d] = (float)(c0[d] + nn[d] * 0.5 * ((double)S.lo + (double)S.hi));
+        margin += 1e-7 * fabs((double)c[d]);
+    }
+    const double t = 0.5 * ((double)S.hi - (double)S.lo), R = sqrt((double)S.rr);
+    margin += 3e-7 * (t + R);
+    o[7] = S.none ? INFINITY : __double2float_ru(t + margin);
+    o[11] = S.none ? INFINITY : __double2float_ru(R + margin);
+    for (int d = 0; d < 3; ++d) {
+        o[8 + d] = S.none ? 0.0f : c[d];
+        o[12 + d] = S.none ? 0.0f : (float)nn[d];
+    }
+    o[15] = 0.0f;
+}
+
+// the point and unit normal that a slot's disk is about; false: no normal
+__device__ __forceinline__ bool disk_frame(const double* __restrict__ r, double (&c0)[3], double (&nn)[3])
+{
+    for (int d = 0; d < 3; ++d) {
+        c0[d] = r[R_P + d];
+        nn[d] = r[R_N + d];
+    }
+    const double A = sqrt(nn[0] * nn[0] + nn[1] * nn[1] + nn[2] * nn[2]);
+    for (int d = 0; d < 3; ++d) nn[d] /= A;
+    return A > 0.0;
+}
+
 __global__ __launch_bounds__(BT) void k_slot_disks(int64_t nslots, const int32_t* __restrict__ slot_bin,
                                                    const double* __restrict__ rec, const int32_t* __restrict__ first,
                                                    const int32_t* __restrict__ last, int64_t n,
                                                    const uint32_t* __restrict__ tris, float* __restrict__ boxes)
 {
-    const int64_t idx = ((int64_t)blockIdx.x * BT + threadIdx.x) >> 4;
-    const int lane = threadIdx.x & 15;
-    if (idx >= nslots) return;
-    float* o = boxes + idx * kBoxWords;
-    if (__float_as_uint(o[6]) == FWN_LINK_EMPTY) return;
-    const int32_t u = slot_bin[idx];
-    const int64_t t0 = u >= n - 1 ? u - (n - 1) : first[u], t1 = u >= n - 1 ? t0 : last[u];
-    const double* r = rec + (int64_t)u * kRecWords;
-    const double c0[3] = {r[R_P], r[R_P + 1], r[R_P + 2]};
-    double nn[3] = {r[R_N], r[R_N + 1], r[R_N + 2]};
-    const double A = sqrt(nn[0] * nn[0] + nn[1] * nn[1] + nn[2] * nn[2]);
-    for (int d = 0; d < 3; ++d) nn[d] /= A;
-    bool none = t1 - t0 >= kDiskTris || !(A > 0.0);
-    float lo = INFINITY, hi = -INFINITY, rr = 0.0f; // rounded outward
-    if (!none) {
-        for (int64_t t = t0 + lane; t <= t1; t += 16) {
-            const float* tw = reinterpret_cast<const float*>(tris + t * kTriWords);
-            double w[3][3];
-            for (int k = 0; k < 3; ++k)
-                for (int d = 0; d < 3; ++d) w[k][d] = (double)tw[3 * k + d] - c0[d];
-            double e1[3], e2[3];
-            for (int d = 0; d < 3; ++d) {
-                e1[d] = w[1][d] - w[0][d];
-                e2[d] = w[2][d] - w[0][d];
-            }
-            const double N[3] = {e1[1] * e2[2] - e1[2] * e2[1], e1[2] * e2[0] - e1[0] * e2[2],
-                                 e1[0] * e2[1] - e1[1] * e2[0]};
-            none |= !(N[0] * N[0] + N[1] * N[1] + N[2] * N[2] >
-                      1e-8 * (e1[0] * e1[0] + e1[1] * e1[1] + e1[2] * e1[2]) *
-                          (e2[0] * e2[0] + e2[1] * e2[1] + e2[2] * e2[2]));
-            for (int k = 0; k < 3; ++k) {
-                const double h = w[k][0] * nn[0] + w[k][1] * nn[1] + w[k][2] * nn[2];
-                double q = 0.0;
-                for (int d = 0; d < 3; ++d) q += (w[k][d] - h * nn[d]) * (w[k][d] - h * nn[d]);
-                lo = fminf(lo, __double2float_rd(h));
-                hi = fmaxf(hi, __double2float_ru(h));
-                rr = fmaxf(rr, __double2float_ru(q));
-            }
+    __shared__ int32_t list[BT], large[BT];
+    __shared__ int32_t count[2];
+    if (threadIdx.x < 2) count[threadIdx.x] = 0;
+    __syncthreads();
+    // slot of the block's thread t: runs of 16
+    auto slot_of = [&](int t) { return ((int64_t)(t >> 4) * gridDim.x + blockIdx.x) * 16 + (t & 15); };
+    const int64_t idx = slot_of(threadIdx.x);
+    if (idx < nslots && __float_as_uint(boxes[idx * kBoxWords + 6]) != FWN_LINK_EMPTY) {
+        const int64_t u = slot_bin[idx];
+        if (u >= n - 1) {
+            double c0[3], nn[3];
+            DiskSpan S;
+            S.none = !disk_frame(rec + u * kRecWords, c0, nn);
+            disk_triangle(reinterpret_cast<const float*>(tris + (u - (n - 1)) * kTriWords), c0, nn, S);
+            write_disk(boxes + idx * kBoxWords, c0, nn, S);
+        } else if (last[u] - first[u] < kDiskRow) {
+            list[atomicAdd(&count[0], 1)] = threadIdx.x;
+        } else {
+            large[atomicAdd(&count[1], 1)] = threadIdx.x;
         }
     }
-    for (int m = 8; m > 0; m >>= 1) {
-        lo = fminf(lo, __shfl_xor(lo, m, 16));
-        hi = fmaxf(hi, __shfl_xor(hi, m, 16));
-        rr = fmaxf(rr, __shfl_xor(rr, m, 16));
-        none |= __shfl_xor((int)none, m, 16) != 0;
-    }
-    if (lane != 0) return;
-    float c[3] = {0, 0, 0};
-    double margin = 0.0; // the rounding of c and n
-    for (int d = 0; d < 3; ++d) {
-        c[d] = (float)(c0[d] + nn[d] * 0.5 * ((double)lo + (double)hi));
-        margin += 1e-7 * fabs((double)c[d]);
-    }
-    const double t = 0.5 * ((double)hi - (double)lo), R = sqrt((double)rr);
-    margin += 3e-7 * (t + R);
-    o[7] = none ? INFINITY : __double2float_ru(t + margin);
-    o[11] = none ? INFINITY : __double2float_ru(R + margin);
-    for (int d = 0; d < 3; ++d) {
-        o[8 + d] = none ? 0.0f : c[d];
-        o[12 + d] = none ? 0.0f : (float)nn[d];
-    }
-    o[15] = 0.0f;
+    __syncthreads();
+    // a group of g lanes takes a slot
+    auto take = [&](int t, int g) {
+        const int64_t at = slot_of(t);
+        const int64_t u = slot_bin[at], t0 = first[u], t1 = last[u];
+        double c0[3], nn[3];
+        DiskSpan S;
+        S.none = !disk_frame(rec + u * kRecWords, c0, nn) || t1 - t0 >= kDiskTris;
+        if (!S.none)
+            for (int64_t k = t0 + (threadIdx.x & (g - 1)); k <= t1; k += g)
+                disk_triangle(reinterpret_cast<const float*>(tris + k * kTriWords), c0, nn, S);
+        for (int m = g / 2; m > 0; m >>= 1) {
+            S.lo = fminf(S.lo, __shfl_xor(S.lo, m));
+            S.hi = fmaxf(S.hi, __shfl_xor(S.hi, m));
+            S.rr = fmaxf(S.rr, __shfl_xor(S.rr, m));
+            S.none |= __shfl_xor((int)S.none, m) != 0;
+        }
+        if ((threadIdx.x & (g - 1)) == 0) write_disk(boxes + at * kBoxWords, c0, nn, S);
+    };
+    for (int k = threadIdx.x >> 6; k < count[1]; k += BT / 64) take(large[k], 64);
+    for (int k = threadIdx.x >> 4; k < count[0]; k += BT / 16) take(list[k], 16);
 }
 
 } // namespace
@@ -1228,7 +1275,7 @@ void build_engine(Engine& e, int32_t M, const float* V_host, const int64_t* v_of
                        w.child, rec, first, last, n, e.opt.accuracy_scale * e.opt.accuracy_scale, dfo, M,
                        e.mesh_info.as<float>(), e.slots.as<uint32_t>(), e.boxes.as<float>(), e.tris.as<uint32_t>());
     FWN_LAUNCH_CHECK("k_write_slots");
-    hipLaunchKernelGGL(k_slot_disks, dim3(grid_blocks(W * width * 16, BT)), dim3(BT), 0, s, W * width, w.slot_bin, rec,
+    hipLaunchKernelGGL(k_slot_disks, dim3(grid_blocks(W * width, BT)), dim3(BT), 0, s, W * width, w.slot_bin, rec,
                        first, last, n, e.tris.as<uint32_t>(), e.boxes.as<float>());
     FWN_LAUNCH_CHECK("k_slot_disks");
     std::copy(e.h_roots.begin(), e.h_roots.end(), h_small);

@@ -54,7 +54,7 @@ namespace fwn {
 namespace {
 
 constexpr int kSahBins = 16;
-constexpr int kChunk = 2048;   // triangles per workgroup in the level-synchronous stage
+constexpr int kChunk = 1024;   // triangles per workgroup in the level-synchronous stage
 constexpr int kThreads = 256;  // its threads
 constexpr int kMidThreads = 512;
 constexpr int kMidWaves = kMidThreads / 64;
