@@ -379,15 +379,20 @@ __device__ void merge2(const double* __restrict__ a, const double* __restrict__ 
     for (int s = 0; s < 10; ++s) o[R_S + s] = S[s];
 }
 
-__global__ __launch_bounds__(BT) void k_leaf_records(const uint32_t* __restrict__ vals, int64_t n,
+// Records and slots go through LDS on their way out where a thread makes one by itself: 64 lanes writing
+// 256 bytes each touch a cache line per lane and store.  101,568 and 940,800 triangles: k_leaf_records 15
+// and 99 us, 10 and 64 so; k_write_slots 25 and 216 us, 19 and 166 so (its reads through LDS too: 28 and 252).
+constexpr int RT = 128;                  // threads (and records) of such a block
+constexpr int kRecPad = kRecWords + 1;   // doubles per record in LDS: the rows start on different banks
+__global__ __launch_bounds__(RT) void k_leaf_records(const uint32_t* __restrict__ vals, int64_t n,
                                                      const float* __restrict__ V, const int32_t* __restrict__ F,
                                                      const int64_t* __restrict__ f_off,
                                                      const int64_t* __restrict__ v_off, int M,
                                                      uint32_t* __restrict__ tris, double* __restrict__ rec)
 {
-    int64_t j = (int64_t)blockIdx.x * BT + threadIdx.x;
-    if (j >= n) return;
-    int64_t t = vals[j];
+    __shared__ double lds[RT * kRecPad];
+    const int64_t j0 = (int64_t)blockIdx.x * RT, j = j0 + threadIdx.x;
+    int64_t t = vals[min(j, n - 1)];
     int m = mesh_of(f_off, M, t);
     int64_t nv = v_off[m + 1] - v_off[m];
     float v[3][3];
@@ -397,13 +402,18 @@ __global__ __launch_bounds__(BT) void k_leaf_records(const uint32_t* __restrict_
         int64_t g = v_off[m] + idx;
         for (int d = 0; d < 3; ++d) v[k][d] = (nv > 0) ? V[3 * g + d] : 0.0f;
     }
-    uint32_t* tw = tris + j * kTriWords;
-    for (int k = 0; k < 3; ++k)
-        for (int d = 0; d < 3; ++d) tw[3 * k + d] = __float_as_uint(v[k][d]);
-    tw[FWN_T_FACET] = (uint32_t)(t - f_off[m]);
-    tw[FWN_T_NEAR2] = 0u; // the leaf data of a leaf's first triangle is written with the slots
-    tw[FWN_T_PLANE] = 0u;
-    tri_record<float>(v, rec + (n - 1 + j) * kRecWords);
+    if (j < n) {
+        float tw[kTriWords] = {}; // a leaf's near-field thresholds are written with the slots
+        for (int k = 0; k < 3; ++k)
+            for (int d = 0; d < 3; ++d) tw[3 * k + d] = v[k][d];
+        tw[FWN_T_FACET] = __uint_as_float((uint32_t)(t - f_off[m]));
+        float4* o = reinterpret_cast<float4*>(tris + j * kTriWords);
+        for (int k = 0; k < kTriWords; k += 4) o[k / 4] = make_float4(tw[k], tw[k + 1], tw[k + 2], tw[k + 3]);
+    }
+    tri_record<float>(v, lds + threadIdx.x * kRecPad);
+    __syncthreads();
+    const int words = (int)min((int64_t)RT, n - j0) * kRecWords;
+    for (int k = threadIdx.x; k < words; k += RT) rec[(n - 1 + j0) * kRecWords + k] = lds[k + k / kRecWords];
 }
 
 __global__ __launch_bounds__(BT) void k_bottom_up(const int32_t* __restrict__ parent,
@@ -516,11 +526,10 @@ __global__ __launch_bounds__(BT) void k_merge_level(const int32_t* __restrict__ 
 // bytes of records a merge reads and writes (101,568 triangles: 0.12 + 0.04 ms; 22 launches and the
 // wait before 0.25 ms; 256 threads a workgroup instead of 512: 0.17 ms for the first).
 constexpr int kMergeThreads = 512;
-__global__ __launch_bounds__(kMergeThreads) void k_merge_mid(const int32_t* __restrict__ seg, const int32_t* __restrict__ left,
-                                                  const int32_t* __restrict__ right, const int32_t* __restrict__ parent,
-                                                  const int32_t* __restrict__ first, const int32_t* __restrict__ last,
-                                                  int64_t n, int32_t fp64_min, double* rec,
-                                                  int32_t* __restrict__ seg_root, int32_t* __restrict__ visits)
+__global__ __launch_bounds__(kMergeThreads) void k_merge_mid(
+    const int32_t* __restrict__ seg, const int32_t* __restrict__ left, const int32_t* __restrict__ right,
+    const int32_t* __restrict__ parent, const int32_t* __restrict__ first, const int32_t* __restrict__ last, int64_t n,
+    int32_t fp64_min, double* rec, int32_t* __restrict__ seg_root, int32_t* __restrict__ visits)
 {
     __shared__ int32_t cnt[kSahMid];
     const int32_t lo = seg[4 * (int64_t)blockIdx.x], hi = seg[4 * (int64_t)blockIdx.x + 1];
@@ -776,25 +785,17 @@ __global__ __launch_bounds__(BT) void k_collapse_link(Wide w, BinTree t, int lea
         state[1] = LevelState{before + own, st.base + st.cnt, st.depth + 1, st.cur ^ 1};
 }
 
-__global__ __launch_bounds__(BT) void k_write_slots(int64_t W, int width, const int32_t* __restrict__ wide_slot_bin,
-                                                    const int32_t* __restrict__ wide_ns,
-                                                    const int32_t* __restrict__ child_wide,
-                                                    const double* __restrict__ rec,
-                                                    const int32_t* __restrict__ first,
-                                                    const int32_t* __restrict__ last, int64_t n, float beta2,
-                                                    const int64_t* __restrict__ f_off, int M,
-                                                    const float* __restrict__ minfo, uint32_t* __restrict__ slots,
-                                                    float* __restrict__ boxes, uint32_t* __restrict__ tris)
+// one slot: its words into w, its box and link into bx, a leaf's near-field rule into its first triangle
+__device__ __forceinline__ void write_slot(int64_t idx, int width, const int32_t* __restrict__ wide_slot_bin,
+                                           const int32_t* __restrict__ wide_ns, const int32_t* __restrict__ child_wide,
+                                           const double* __restrict__ rec, const int32_t* __restrict__ first,
+                                           const int32_t* __restrict__ last, int64_t n, float beta2,
+                                           const int64_t* __restrict__ f_off, int M, const float* __restrict__ minfo,
+                                           uint32_t* w, float* __restrict__ bx, uint32_t* __restrict__ tris)
 {
-    int64_t idx = (int64_t)blockIdx.x * BT + threadIdx.x;
-    if (idx >= W * width) return;
-    int64_t g = idx / width;
-    int s = (int)(idx % width);
-    uint32_t* w = slots + idx * kSlotWords;
-    float* bx = boxes + idx * kBoxWords;
     const int64_t src = idx; // the collapse's tables have width entries per node
     int32_t u = wide_slot_bin[src];
-    if (s >= wide_ns[g] || u < 0) {
+    if ((int)(idx % width) >= wide_ns[idx / width] || u < 0) {
         for (int k = 0; k < FWN_W_LINK; ++k) w[k] = 0u;
         w[FWN_W_LINK] = FWN_LINK_EMPTY;
         for (int k = 0; k < kBoxWords; ++k) bx[k] = 0.0f;
@@ -803,10 +804,13 @@ __global__ __launch_bounds__(BT) void k_write_slots(int64_t W, int width, const 
     }
     const double* r = rec + (int64_t)u * kRecWords;
     // the slot's box for distance queries, rounded outward so it still contains the triangles
+    float box[8];
     for (int d = 0; d < 3; ++d) {
-        bx[d] = __double2float_rd(r[R_LO + d]);
-        bx[3 + d] = __double2float_ru(r[R_HI + d]);
+        box[d] = __double2float_rd(r[R_LO + d]);
+        box[3 + d] = __double2float_ru(r[R_HI + d]);
     }
+    float4* b4 = reinterpret_cast<float4*>(bx); // the link here, the disk by k_slot_disks
+    b4[0] = make_float4(box[0], box[1], box[2], box[3]);
     double r2 = 0.0;
     for (int d = 0; d < 3; ++d) {
         double a = fabs(r[R_P + d] - r[R_LO + d]), b = fabs(r[R_HI + d] - r[R_P + d]);
@@ -848,14 +852,14 @@ __global__ __launch_bounds__(BT) void k_write_slots(int64_t W, int width, const 
     const int32_t cw = child_wide[src];
     if (cw >= 0) {
         w[FWN_W_LINK] = ((uint32_t)cw << 4) | (uint32_t)wide_ns[cw];
-        bx[6] = __uint_as_float(w[FWN_W_LINK]);
+        b4[1] = make_float4(box[4], box[5], __uint_as_float(w[FWN_W_LINK]), 0.0f);
         return;
     }
     const bool bin_leaf = u >= n - 1;
     const int64_t tf = bin_leaf ? (u - (n - 1)) : first[u];
     const int32_t tc = bin_leaf ? 1 : last[u] - first[u] + 1;
     w[FWN_W_LINK] = FWN_LINK_LEAF | ((uint32_t)tf << 3) | (uint32_t)(tc - 1);
-    bx[6] = __uint_as_float(w[FWN_W_LINK]);
+    b4[1] = make_float4(box[4], box[5], __uint_as_float(w[FWN_W_LINK]), 0.0f);
     // the leaf's FP64 near-field rule, in its first triangle: q is within tau of the leaf's
     // bounding sphere when |d|^2 < (sqrt(r2) + tau)^2 and, for a single triangle, within tau of
     // its plane when (d.N)^2 < tau^2 |N|^2
@@ -867,12 +871,35 @@ __global__ __launch_bounds__(BT) void k_write_slots(int64_t W, int width, const 
     tw[FWN_T_PLANE] = __float_as_uint((tau * tau) * nn);
 }
 
+__global__ __launch_bounds__(RT) void k_write_slots(int64_t W, int width, const int32_t* __restrict__ wide_slot_bin,
+                                                    const int32_t* __restrict__ wide_ns,
+                                                    const int32_t* __restrict__ child_wide,
+                                                    const double* __restrict__ rec,
+                                                    const int32_t* __restrict__ first,
+                                                    const int32_t* __restrict__ last, int64_t n, float beta2,
+                                                    const int64_t* __restrict__ f_off, int M,
+                                                    const float* __restrict__ minfo, uint32_t* __restrict__ slots,
+                                                    float* __restrict__ boxes, uint32_t* __restrict__ tris)
+{
+    // the block's slots, written together below
+    __shared__ uint32_t lds[RT * (kSlotWords + 1)];
+    const int64_t idx0 = (int64_t)blockIdx.x * RT, idx = idx0 + threadIdx.x;
+    if (idx < W * width)
+        write_slot(idx, width, wide_slot_bin, wide_ns, child_wide, rec, first, last, n, beta2, f_off, M, minfo,
+                   lds + threadIdx.x * (kSlotWords + 1), boxes + idx * kBoxWords, tris);
+    __syncthreads();
+    const int words = (int)min((int64_t)RT, W * width - idx0) * kSlotWords;
+    for (int k = threadIdx.x; k < words; k += RT) slots[idx0 * kSlotWords + k] = lds[k + k / kSlotWords];
+}
+
 // Each slot's disk, from its triangles' vertices in double.  A thread takes a slot of one triangle by
 // itself (three in four); the block's other slots are listed and taken by rows of 16 lanes, those above
-// kDiskRow triangles by waves.  A block's slots are spread over the array, as the large ones come first.  101,568 triangles: 48 us with a row
-// for every slot, 41 so, and 940,800 395 us and 182.  A slot of more than kDiskTris triangles (nearly always entered, and a serial
-// loop here) or with a sliver (sine below 1e-4: its evaluated distance may be off by more than the bound
-// allows for) gets no bound (400k closest points, F = 199,692: limit 128 4.33 ms, 512 4.07, 1,024 3.98).
+// kDiskRow triangles by waves.  A block's slots are spread over the array, as the large ones come first.
+// Bound: the chain of loads of a slot's triangles; 101,568 and 940,800 triangles 48 and 395 us with a row
+// for every slot, 41 and 182 so.  A slot of more than kDiskTris triangles (nearly always entered, and a
+// serial loop here) or with a sliver (sine below 1e-4: its evaluated distance may be off by more than
+// the bound allows for) gets no bound (400k closest points, F = 199,692: limit 128 4.33 ms, 512 4.07,
+// 1,024 3.98).
 constexpr int64_t kDiskTris = 1024, kDiskRow = 64;
 
 struct DiskSpan { // of a slot's triangles about a point and a normal; rounded outward
@@ -1133,7 +1160,7 @@ void build_engine(Engine& e, int32_t M, const float* V_host, const int64_t* v_of
 
     // ---- moments ----
     double* rec = ar.take<double>(kRecWords * nnodes);
-    hipLaunchKernelGGL(k_leaf_records, dim3(grid_blocks(n, BT)), dim3(BT), 0, s, vp, n, dV, dF, dfo, dvo, M,
+    hipLaunchKernelGGL(k_leaf_records, dim3(grid_blocks(n, RT)), dim3(RT), 0, s, vp, n, dV, dF, dfo, dvo, M,
                        e.tris.as<uint32_t>(), rec);
     FWN_LAUNCH_CHECK("k_leaf_records");
     if (n > 1 && sah && e.opt.moment_pass == FWN_MOMENTS_LEVELS) {
@@ -1271,7 +1298,7 @@ void build_engine(Engine& e, int32_t M, const float* V_host, const int64_t* v_of
     }
     e.slots.alloc(sizeof(uint32_t) * width * kSlotWords * (size_t)W);
     e.boxes.alloc(sizeof(float) * width * kBoxWords * (size_t)W);
-    hipLaunchKernelGGL(k_write_slots, dim3(grid_blocks(W * width, BT)), dim3(BT), 0, s, W, width, w.slot_bin, w.ns,
+    hipLaunchKernelGGL(k_write_slots, dim3(grid_blocks(W * width, RT)), dim3(RT), 0, s, W, width, w.slot_bin, w.ns,
                        w.child, rec, first, last, n, e.opt.accuracy_scale * e.opt.accuracy_scale, dfo, M,
                        e.mesh_info.as<float>(), e.slots.as<uint32_t>(), e.boxes.as<float>(), e.tris.as<uint32_t>());
     FWN_LAUNCH_CHECK("k_write_slots");
