@@ -224,11 +224,12 @@ inline bool default_shape(const Engine& e)
 }
 // Calls of few points of a single-mesh engine, one wave per point (fwn_point.hip).
 void run_points(Engine& e, const float* Q, int64_t nQ, float* omega, uint8_t* inside, int banks, bool device_ptrs);
-// The slots-in-lanes traversal (fwn_quad.hip): whether a call goes to it, and its launch over nb
-// batches of kQuadPoints points (metadata as k_traverse's); FP64 near leaves are evaluated in the
+// The slots-in-lanes traversal (fwn_quad.hip): whether a call goes to it (Spread: if its points spread
+// over the mesh's box), and its launch over nb batches of kQuadPoints points (metadata as k_traverse's); FP64 near leaves are evaluated in the
 // kernel, flag is set on a stack overflow.
 constexpr int kQuadPoints = 16;
-bool use_quads(const Engine& e, int64_t nQ, int banks);
+enum class Quads { No, Yes, Spread };
+Quads use_quads(const Engine& e, int64_t nQ, int banks);
 void launch_quads(Engine& e, const float* dQ, const uint32_t* perm, const int64_t* q_off, const int64_t* b_off,
                   const int32_t* order, int M, int64_t nb, float* omega, uint8_t* inside, int32_t* flag, hipStream_t s);
 // Pieces of a query that uses no engine scratch (single-mesh engine, device points): the 32-bit

@@ -294,12 +294,19 @@ __global__ __launch_bounds__(64) void k_traverse_quad(
 //     1800 / 808 and 5516 / 2818, F = 19,200 1058 / 669 and 1589 / 1241, F = 1,728 535 / 528 and 608 /
 //     713; 32 x 100k points, F = 19,200 1322 / 1169 and 1920 / 2164; 8 meshes of 14k to 48k, 1M
 //     points, 703 / 409; 32 of 1.7k to 181k, 3.7M points, 1199 / 1214.
-constexpr double kQuadCross = 24000.0, kQuadSparse = 2.0;
-bool use_quads(const Engine& e, int64_t nQ, int banks)
+//
+// Points in a thin layer (at a distance from the surface above all, where few walks go deep) are close
+// together at far fewer points than these lines say: a layer 5 % of the diagonal off F = 940,800 takes
+// 300 / 333 us at 588k points and 660 / 990 at 2.3M, one 1 % off 858 / 744 and 1521 / 1955; F =
+// 199,692 333 / 384 at 701k and 781 / 743.  Above kQuadAny points of one mesh the slots-in-lanes
+// traversal is therefore taken only for points that spread over the mesh's box (Quads::Spread).
+constexpr double kQuadCross = 24000.0, kQuadSparse = 2.0, kQuadAny = 500000.0;
+Quads use_quads(const Engine& e, int64_t nQ, int banks)
 {
-    if (e.width != 4 || banks != 1 || !default_shape(e)) return false;
+    if (e.width != 4 || banks != 1 || !default_shape(e)) return Quads::No;
     const double F = (double)e.h_f_off[e.n_meshes];
-    return (double)nQ <= kQuadCross * std::cbrt(F / e.n_meshes) + (e.n_meshes > 1 ? kQuadSparse * F : 0.0);
+    if ((double)nQ > kQuadCross * std::cbrt(F / e.n_meshes) + (e.n_meshes > 1 ? kQuadSparse * F : 0.0)) return Quads::No;
+    return e.n_meshes == 1 && (double)nQ > kQuadAny ? Quads::Spread : Quads::Yes;
 }
 
 void launch_quads(Engine& e, const float* dQ, const uint32_t* perm, const int64_t* q_off, const int64_t* b_off,

@@ -106,6 +106,36 @@ __global__ __launch_bounds__(1024) void k_query_keys_few(const float* __restrict
     hist[(int64_t)blockIdx.x * 1024 + threadIdx.x] = cnt[threadIdx.x];
 }
 
+// How many of the 32^3 cells of the mesh's box (points outside it count at its faces) hold one of 32,768
+// points taken evenly from the call: uniform points and grids in the box or 20 % beyond it fill 0.52 to
+// 0.63 of them, layers up to 10 % of the diagonal off the surface 0.12 to 0.22.  One block; about 6 us,
+// of which the host sees nothing: it reads the count while the sort runs.
+constexpr int kSpreadPoints = 32768, kSpreadCells = 32768, kSpreadLeast = (int)(0.3 * kSpreadCells);
+__global__ __launch_bounds__(1024) void k_point_spread(const float* __restrict__ Q, int64_t nQ,
+                                                       const float* __restrict__ minfo, int32_t* __restrict__ cells)
+{
+    __shared__ uint32_t bits[kSpreadCells / 32];
+    __shared__ int32_t part[16];
+    bits[threadIdx.x] = 0u;
+    __syncthreads();
+#pragma unroll 8
+    for (int r = 0; r < kSpreadPoints / 1024; ++r) {
+        const int64_t i = (int64_t)(r * 1024 + threadIdx.x) * nQ / kSpreadPoints;
+        const uint32_t c = morton30(Q[3 * i], Q[3 * i + 1], Q[3 * i + 2], minfo, minfo + 3) >> 15;
+        atomicOr(&bits[c >> 5], 1u << (c & 31u));
+    }
+    __syncthreads();
+    int32_t n = __popc(bits[threadIdx.x]);
+    for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = n;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        n = 0;
+        for (int w = 0; w < 16; ++w) n += part[w];
+        *cells = n;
+    }
+}
+
 // One slot's 24 words held in SGPRs (a 16-dword and an 8-dword scalar load issued together at
 // the top of the slot).  The other waves of the SIMD (8 resident) hide the load latency.
 typedef uint32_t v16u __attribute__((ext_vector_type(16)));
@@ -678,12 +708,13 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
     // points per wave: 64, or fewer for small calls so that their waves spread over the device
     // (a point's result does not depend on which points share its wave)
     const bool small = nQ <= kSmallBatch && !stats;
-    const bool quad = !small && !stats && use_quads(e, nQ, banks);
+    const Quads choice = small || stats ? Quads::No : use_quads(e, nQ, banks);
+    bool quad = choice == Quads::Yes; // Quads::Spread: known once the points are looked at
     const int bpts = small ? (int)std::min<int64_t>(64, std::max<int64_t>(1, (nQ + 1023) / 1024))
                            : (quad ? kQuadPoints : 64);
     std::vector<int64_t> boff(M + 1, 0);
     for (int k = 0; k < M; ++k) boff[k + 1] = boff[k] + (qoff[order[k] + 1] - qoff[order[k]] + bpts - 1) / bpts;
-    const int64_t nb = boff[M];
+    int64_t nb = boff[M];
 
     const bool stage_io = small && !dev; // points in and results out through the pinned stage
     // metadata (and the points of a small host batch) in one staged copy:
@@ -691,7 +722,8 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
     const size_t meta_b = (sizeof(int64_t) * 2 * (M + 1) + sizeof(int32_t) * M + 15) & ~(size_t)15;
     const size_t in_b = meta_b + (stage_io ? sizeof(float) * 3 * (size_t)nQ : 0);
     const size_t out_b = stage_io ? 16 + (sizeof(float) + 1) * (size_t)nQ : 0; // flags, omega, inside
-    char* hs = host_stage(e, std::max(in_b, out_b));
+    const size_t spread_at = (std::max(in_b, out_b) + 15) & ~(size_t)15; // the spread comes back behind it all
+    char* hs = host_stage(e, spread_at + 16);
     std::memcpy(hs, qoff.data(), sizeof(int64_t) * (M + 1));
     std::memcpy(hs + sizeof(int64_t) * (M + 1), boff.data(), sizeof(int64_t) * (M + 1));
     std::memcpy(hs + sizeof(int64_t) * 2 * (M + 1), order.data(), sizeof(int32_t) * M);
@@ -733,7 +765,7 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
             dSt = e.q_stats.as<int32_t>();
         }
     }
-    e.q_flag.reserve(2 * sizeof(int32_t));
+    e.q_flag.reserve(3 * sizeof(int32_t));
 
     if (!small && !point_order) {
         for (int k = 0; k < 2; ++k) {
@@ -747,6 +779,12 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
     FWN_HIP(hipEventRecord(e.ev[0], s));
     int32_t* dflag = e.q_flag.as<int32_t>();
     uint32_t* dwork = reinterpret_cast<uint32_t*>(dflag + 1);
+    if (choice == Quads::Spread) {
+        hipLaunchKernelGGL(k_point_spread, dim3(1), dim3(1024), 0, s, dQ, nQ, e.mesh_info.as<float>(), dflag + 2);
+        FWN_LAUNCH_CHECK("k_point_spread");
+        FWN_HIP(hipMemcpyAsync(hs + spread_at, dflag + 2, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+        FWN_HIP(hipEventRecord(e.ev[3], s));
+    }
     // sorted position -> input index (nullptr: small calls keep the input order)
     const uint32_t* vp = small ? nullptr : point_order;
     if (small || point_order) {
@@ -774,6 +812,13 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
             radix_sort_pairs32(kp, vals, kp2, vp2, nQ, 8, 32, true, e.q_hist, e.q_rowsum, s);
         }
         vp = vals;
+    }
+    if (choice == Quads::Spread) {
+        FWN_HIP(hipEventSynchronize(e.ev[3])); // the sort is under way
+        int32_t cells = 0;
+        std::memcpy(&cells, hs + spread_at, sizeof(cells));
+        quad = cells >= kSpreadLeast;
+        if (quad) nb = (nQ + kQuadPoints - 1) / kQuadPoints; // of one mesh: its b_off is not read
     }
 
     const int waves = e.opt.waves_per_block > 0 ? e.opt.waves_per_block : 1;

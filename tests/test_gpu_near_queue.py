@@ -66,3 +66,21 @@ def test_queue_with_several_meshes():
     for k, m in enumerate(meshes):
         np.testing.assert_array_equal(om[off[k]:off[k + 1]],
                                       FastWindingNumber(m, near_fp64_rel=0.05).solid_angle_batch(q[k]))
+
+
+@pytest.mark.parametrize("n", [499999, 500000, 500001, 640001])
+@pytest.mark.parametrize("where", ["box", "layer", "one"])
+def test_calls_that_look_at_their_spread(where, n):
+    """Above 500,000 points of one mesh the kernel is chosen by how the points spread over the mesh's box:
+    the same results on both sides of the line and of the choice (24,000 cbrt(F) = 643,000 here)."""
+    V, F = W.icosphere(31).f32()
+    e = FastWindingNumber((V, F))
+    rng = np.random.default_rng(n)
+    q = rng.uniform(-1.1, 1.1, (n, 3))
+    if where == "layer":
+        q *= 1.05 / np.linalg.norm(q, axis=1, keepdims=True)
+    elif where == "one":
+        q[:] = (0.4, 0.1, -0.2)
+    q = q.astype(np.float32)
+    take = rng.integers(0, n, 8192)
+    np.testing.assert_array_equal(e.solid_angle_batch(q)[take], e.solid_angle_batch(q[take]))
