@@ -225,13 +225,15 @@ inline bool default_shape(const Engine& e)
 // Calls of few points of a single-mesh engine, one wave per point (fwn_point.hip).
 void run_points(Engine& e, const float* Q, int64_t nQ, float* omega, uint8_t* inside, int banks, bool device_ptrs);
 // The slots-in-lanes traversal (fwn_quad.hip): whether a call goes to it (Spread: if its points spread
-// over the mesh's box), and its launch over nb batches of kQuadPoints points (metadata as k_traverse's); FP64 near leaves are evaluated in the
-// kernel, flag is set on a stack overflow.
+// over the mesh's box), and its launch over nb batches of bpts points (metadata as k_traverse's); FP64
+// near leaves are evaluated in the kernel, flag is set on a stack overflow.
 constexpr int kQuadPoints = 16;
 enum class Quads { No, Yes, Spread };
 Quads use_quads(const Engine& e, int64_t nQ, int banks);
 void launch_quads(Engine& e, const float* dQ, const uint32_t* perm, const int64_t* q_off, const int64_t* b_off,
-                  const int32_t* order, int M, int64_t nb, float* omega, uint8_t* inside, int32_t* flag, hipStream_t s);
+                  const int32_t* order, int M, int64_t nb, int bpts, float* omega, uint8_t* inside, int32_t* flag,
+                  hipStream_t s);
+int quad_points(const Engine& e, int64_t nQ); // points per wave, kQuadPoints at most
 // Pieces of a query that uses no engine scratch (single-mesh engine, device points): the 32-bit
 // point keys, and the traversal in sorted order `perm`; meta holds q_off {0, nQ}, b_off {0, batches} and the mesh order {0} (5 int64
 // words), flag one int32 (set on stack overflow).  Results equal run_queries' bit for bit.

@@ -89,7 +89,7 @@ __global__ __launch_bounds__(64) void k_traverse_quad(
     const uint32_t* __restrict__ slots, const uint32_t* __restrict__ tris, const int32_t* __restrict__ roots,
     const float* __restrict__ minfo, const float* __restrict__ Q, const uint32_t* __restrict__ perm,
     const int64_t* __restrict__ q_off, const int64_t* __restrict__ b_off, const int32_t* __restrict__ mesh_order,
-    int M, int64_t n_batches, int lds_nodes, float* __restrict__ omega, uint8_t* __restrict__ inside,
+    int M, int64_t n_batches, int bpts, int lds_nodes, float* __restrict__ omega, uint8_t* __restrict__ inside,
     int32_t* __restrict__ flag)
 {
     extern __shared__ uint4 quad_lds[];
@@ -103,9 +103,9 @@ __global__ __launch_bounds__(64) void k_traverse_quad(
     if (batch >= n_batches) return;
     const int pos = mesh_of64(b_off, M, batch);
     const int m = mesh_order[pos];
-    const int64_t start = q_off[m] + (batch - b_off[pos]) * kQuadPoints;
+    const int64_t start = q_off[m] + (batch - b_off[pos]) * bpts;
     const int64_t cnt64 = q_off[m + 1] - start;
-    const int cnt = cnt64 < kQuadPoints ? (int)cnt64 : kQuadPoints;
+    const int cnt = cnt64 < bpts ? (int)cnt64 : bpts;
     const bool valid = p < cnt;
     const uint32_t jpos = (uint32_t)(start + p);
     const uint32_t orig = valid ? (perm ? perm[jpos] : jpos) : 0u;
@@ -309,8 +309,18 @@ Quads use_quads(const Engine& e, int64_t nQ, int banks)
     return e.n_meshes == 1 && (double)nQ > kQuadAny ? Quads::Spread : Quads::Yes;
 }
 
+// Points per wave: 16, the wave's lanes, or 8 where so few waves run that the longest decides (up to 500
+// cbrt(F) points of one mesh, at most 32,000).  8 / 16 in us: 20k points, F = 199,692 97 / 115 uniform,
+// 142 / 184 near the surface, F = 940,800 106 / 128 and 197 / 278; 30k points 103 / 127 and 159 / 178,
+// 109 / 135 and 202 / 270; against it 50k points near the surface, 199 / 172 and 314 / 279, and F = 20,172,
+// 30k points near the surface 94 / 86.
+int quad_points(const Engine& e, int64_t nQ)
+{
+    return e.n_meshes == 1 && (double)nQ <= std::min(500.0 * std::cbrt((double)e.h_f_off[1]), 32000.0) ? 8 : kQuadPoints;
+}
+
 void launch_quads(Engine& e, const float* dQ, const uint32_t* perm, const int64_t* q_off, const int64_t* b_off,
-                  const int32_t* order, int M, int64_t nb, float* omega, uint8_t* inside, int32_t* flag, hipStream_t s)
+                  const int32_t* order, int M, int64_t nb, int bpts, float* omega, uint8_t* inside, int32_t* flag, hipStream_t s)
 {
     // node buffers per wave: 20 (9 KB, room for 4 waves per SIMD) while the call has no more waves
     // than that, else 12 (6 KB: 6 and a half); entries above them are rare.  F = 199,692, uniform and
@@ -321,7 +331,7 @@ void launch_quads(Engine& e, const float* dQ, const uint32_t* perm, const int64_
 #define FWN_QUAD(BUCKET)                                                                                            \
     hipLaunchKernelGGL(k_traverse_quad<BUCKET>, dim3((unsigned)nb), dim3(64), lds, s, e.slots.as<uint32_t>(),      \
                        e.tris.as<uint32_t>(), e.roots.as<int32_t>(), e.mesh_info.as<float>(), dQ, perm, q_off,     \
-                       b_off, order, M, nb, lds_nodes, omega, inside, flag)
+                       b_off, order, M, nb, bpts, lds_nodes, omega, inside, flag)
     if (e.opt.leaf_max > 1) FWN_QUAD(true);
     else FWN_QUAD(false);
 #undef FWN_QUAD

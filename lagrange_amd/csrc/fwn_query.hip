@@ -711,7 +711,7 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
     const Quads choice = small || stats ? Quads::No : use_quads(e, nQ, banks);
     bool quad = choice == Quads::Yes; // Quads::Spread: known once the points are looked at
     const int bpts = small ? (int)std::min<int64_t>(64, std::max<int64_t>(1, (nQ + 1023) / 1024))
-                           : (quad ? kQuadPoints : 64);
+                           : (quad ? quad_points(e, nQ) : 64);
     std::vector<int64_t> boff(M + 1, 0);
     for (int k = 0; k < M; ++k) boff[k + 1] = boff[k] + (qoff[order[k] + 1] - qoff[order[k]] + bpts - 1) / bpts;
     int64_t nb = boff[M];
@@ -820,6 +820,7 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
         quad = cells >= kSpreadLeast;
         if (quad) nb = (nQ + kQuadPoints - 1) / kQuadPoints; // of one mesh: its b_off is not read
     }
+    const int quad_bpts = choice == Quads::Spread ? kQuadPoints : bpts;
 
     const int waves = e.opt.waves_per_block > 0 ? e.opt.waves_per_block : 1;
     const bool persist = (e.opt.launch_mode == FWN_LAUNCH_PERSISTENT) && !stats;
@@ -836,7 +837,7 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
     const float beta2 = e.opt.accuracy_scale * e.opt.accuracy_scale;
     FWN_HIP(hipEventRecord(e.ev[1], s));
     if (quad) {
-        launch_quads(e, dQ, vp, d_qoff, d_boff, d_order, M, nb, dOm, dIn, dflag, s);
+        launch_quads(e, dQ, vp, d_qoff, d_boff, d_order, M, nb, quad_bpts, dOm, dIn, dflag, s);
     } else {
         launch_traverse(stats != nullptr, waves, persist, banks, e.width, (unsigned)nblk, s, e.slots.as<uint32_t>(),
                         e.width, e.tris.as<uint32_t>(), e.roots.as<int32_t>(), e.mesh_info.as<float>(), dQ, vp, d_qoff,
