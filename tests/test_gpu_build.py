@@ -1,6 +1,6 @@
 """The tree build at the edges of its stages: segments of 16 / 17 triangles (row or wave), of 1,024 /
 1,025 (one workgroup or level by level), uneven splits that need more levels than a balanced tree,
-and many meshes.  Checker: the CPU restatement's tree, slot by slot."""
+and many meshes.  Oracle: the CPU restatement's tree, slot by slot."""
 import numpy as np
 import pytest
 
