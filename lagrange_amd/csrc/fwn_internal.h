@@ -209,8 +209,9 @@ SahMids build_topology_sah(Engine& e, Arena& ar, const float* cen, const float* 
 
 // queries (fwn_query.hip).  order: device positions -> points of one mesh that are already in an order
 // of waves (nullptr: the call sorts its points); not read by calls that need no order (few_points).
+// layer: the points lie in layers along a surface (a choice of kernel only, the results are the same).
 void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t nQ, float* omega, uint8_t* inside,
-                 int32_t* stats, bool device_ptrs, const uint32_t* order = nullptr);
+                 int32_t* stats, bool device_ptrs, const uint32_t* order = nullptr, bool layer = false);
 // whether a device call of nQ points of one mesh runs one wave per point
 bool few_points(const Engine& e, int64_t nQ);
 void run_bruteforce(Engine& e, const float* Q, int64_t nQ, double* out, bool device_ptrs);
@@ -229,10 +230,10 @@ void run_points(Engine& e, const float* Q, int64_t nQ, float* omega, uint8_t* in
 // near leaves are evaluated in the kernel, flag is set on a stack overflow.
 constexpr int kQuadPoints = 16;
 enum class Quads { No, Yes, Spread };
-Quads use_quads(const Engine& e, int64_t nQ, int banks);
+Quads use_quads(const Engine& e, int64_t nQ, int banks, bool layer);
 void launch_quads(Engine& e, const float* dQ, const uint32_t* perm, const int64_t* q_off, const int64_t* b_off,
-                  const int32_t* order, int M, int64_t nb, int bpts, float* omega, uint8_t* inside, int32_t* flag,
-                  hipStream_t s);
+                  const int32_t* order, int M, int64_t nb, int bpts, bool layer, float* omega, uint8_t* inside,
+                  int32_t* flag, hipStream_t s);
 int quad_points(const Engine& e, int64_t nQ); // points per wave, kQuadPoints at most
 // Pieces of a query that uses no engine scratch (single-mesh engine, device points): the 32-bit
 // point keys, and the traversal in sorted order `perm`; meta holds q_off {0, nQ}, b_off {0, batches} and the mesh order {0} (5 int64

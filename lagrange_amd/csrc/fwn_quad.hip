@@ -89,8 +89,8 @@ __global__ __launch_bounds__(64) void k_traverse_quad(
     const uint32_t* __restrict__ slots, const uint32_t* __restrict__ tris, const int32_t* __restrict__ roots,
     const float* __restrict__ minfo, const float* __restrict__ Q, const uint32_t* __restrict__ perm,
     const int64_t* __restrict__ q_off, const int64_t* __restrict__ b_off, const int32_t* __restrict__ mesh_order,
-    int M, int64_t n_batches, int bpts, int lds_nodes, float* __restrict__ omega, uint8_t* __restrict__ inside,
-    int32_t* __restrict__ flag)
+    int M, int64_t n_batches, int bpts, int run, int lds_nodes, float* __restrict__ omega,
+    uint8_t* __restrict__ inside, int32_t* __restrict__ flag)
 {
     extern __shared__ uint4 quad_lds[];
     uint2* queue = reinterpret_cast<uint2*>(reinterpret_cast<char*>(quad_lds) + (size_t)lds_nodes * kQuadNodeBytes);
@@ -99,7 +99,8 @@ __global__ __launch_bounds__(64) void k_traverse_quad(
     constexpr int kNode4 = kQuadNodeBytes / 16; // uint4 per node
     const int lane = threadIdx.x;
     const int p = lane >> 2, s = lane & 3;
-    const int64_t batch = xcd_batch(blockIdx.x, gridDim.x, M);
+    const int64_t batch =
+        run > 0 ? xcd_remap_runs(blockIdx.x, gridDim.x, (uint32_t)run) : xcd_remap(blockIdx.x, gridDim.x);
     if (batch >= n_batches) return;
     const int pos = mesh_of64(b_off, M, batch);
     const int m = mesh_order[pos];
@@ -300,11 +301,17 @@ __global__ __launch_bounds__(64) void k_traverse_quad(
 // 300 / 333 us at 588k points and 660 / 990 at 2.3M, one 1 % off 858 / 744 and 1521 / 1955; F =
 // 199,692 333 / 384 at 701k and 781 / 743.  Above kQuadAny points of one mesh the slots-in-lanes
 // traversal is therefore taken only for points that spread over the mesh's box (Quads::Spread).
-constexpr double kQuadCross = 24000.0, kQuadSparse = 2.0, kQuadAny = 500000.0;
-Quads use_quads(const Engine& e, int64_t nQ, int banks)
+// A caller that knows its points to lie along a surface (the orientation probes) has a line of its own,
+// kQuadLayer * cbrt(F), and no look at the points: whole calls of two probes a facet, 0.01 / 1 / 5 / 30 % of
+// the size off the surface, k_traverse 1060 / 818 / 394 / 231 us and this kernel 641 / 604 / 346 / 229 at 479k
+// probes, 1250 / 887 / 398 / 239 and 752 / 711 / 386 / 258 at 569k, 1707 / 1108 / 449 / 271 and 1135 / 981 /
+// 507 / - at 912k: the line lies where no distance loses.
+constexpr double kQuadCross = 24000.0, kQuadSparse = 2.0, kQuadAny = 500000.0, kQuadLayer = 8000.0;
+Quads use_quads(const Engine& e, int64_t nQ, int banks, bool layer)
 {
     if (e.width != 4 || banks != 1 || !default_shape(e)) return Quads::No;
     const double F = (double)e.h_f_off[e.n_meshes];
+    if (layer && e.n_meshes == 1) return (double)nQ <= kQuadLayer * std::cbrt(F) ? Quads::Yes : Quads::No;
     if ((double)nQ > kQuadCross * std::cbrt(F / e.n_meshes) + (e.n_meshes > 1 ? kQuadSparse * F : 0.0)) return Quads::No;
     return e.n_meshes == 1 && (double)nQ > kQuadAny ? Quads::Spread : Quads::Yes;
 }
@@ -320,8 +327,13 @@ int quad_points(const Engine& e, int64_t nQ)
 }
 
 void launch_quads(Engine& e, const float* dQ, const uint32_t* perm, const int64_t* q_off, const int64_t* b_off,
-                  const int32_t* order, int M, int64_t nb, int bpts, float* omega, uint8_t* inside, int32_t* flag, hipStream_t s)
+                  const int32_t* order, int M, int64_t nb, int bpts, bool layer, float* omega, uint8_t* inside,
+                  int32_t* flag, hipStream_t s)
 {
+    // Blocks to the XCDs in runs for several meshes (xcd_batch) and for layers of 8,192 waves or more, whose
+    // expensive waves lie together: probes 1 % off, one run per XCD / runs of 64, 400k points 488 / 454 us (F =
+    // 199,692) and 530 / 473 (F = 940,800), 500k 565 / 527 and 625 / 543; uniform points lose 8 to 18 % to runs
+    const int run = M > 1 ? 16 : (layer && nb >= 8192 ? 64 : 0);
     // node buffers per wave: 20 (9 KB, room for 4 waves per SIMD) while the call has no more waves
     // than that, else 12 (6 KB: 6 and a half); entries above them are rare.  F = 199,692, uniform and
     // near the surface, 9 / 12 / 20 buffers: 20k points 135 / 132 / 118 and 215 / 200 / 178 us, 400k
@@ -331,7 +343,7 @@ void launch_quads(Engine& e, const float* dQ, const uint32_t* perm, const int64_
 #define FWN_QUAD(BUCKET)                                                                                            \
     hipLaunchKernelGGL(k_traverse_quad<BUCKET>, dim3((unsigned)nb), dim3(64), lds, s, e.slots.as<uint32_t>(),      \
                        e.tris.as<uint32_t>(), e.roots.as<int32_t>(), e.mesh_info.as<float>(), dQ, perm, q_off,     \
-                       b_off, order, M, nb, bpts, lds_nodes, omega, inside, flag)
+                       b_off, order, M, nb, bpts, run, lds_nodes, omega, inside, flag)
     if (e.opt.leaf_max > 1) FWN_QUAD(true);
     else FWN_QUAD(false);
 #undef FWN_QUAD

@@ -667,7 +667,7 @@ bool few_points(const Engine& e, int64_t nQ)
 }
 
 void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t nQ, float* omega, uint8_t* inside,
-                 int32_t* stats, bool dev, const uint32_t* point_order)
+                 int32_t* stats, bool dev, const uint32_t* point_order, bool layer)
 {
     hipStream_t s = e.stream;
     const int M = e.n_meshes;
@@ -708,7 +708,7 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
     // points per wave: 64, or fewer for small calls so that their waves spread over the device
     // (a point's result does not depend on which points share its wave)
     const bool small = nQ <= kSmallBatch && !stats;
-    const Quads choice = small || stats ? Quads::No : use_quads(e, nQ, banks);
+    const Quads choice = small || stats ? Quads::No : use_quads(e, nQ, banks, layer);
     bool quad = choice == Quads::Yes; // Quads::Spread: known once the points are looked at
     const int bpts = small ? (int)std::min<int64_t>(64, std::max<int64_t>(1, (nQ + 1023) / 1024))
                            : (quad ? quad_points(e, nQ) : 64);
@@ -837,7 +837,7 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
     const float beta2 = e.opt.accuracy_scale * e.opt.accuracy_scale;
     FWN_HIP(hipEventRecord(e.ev[1], s));
     if (quad) {
-        launch_quads(e, dQ, vp, d_qoff, d_boff, d_order, M, nb, quad_bpts, dOm, dIn, dflag, s);
+        launch_quads(e, dQ, vp, d_qoff, d_boff, d_order, M, nb, quad_bpts, layer, dOm, dIn, dflag, s);
     } else {
         launch_traverse(stats != nullptr, waves, persist, banks, e.width, (unsigned)nblk, s, e.slots.as<uint32_t>(),
                         e.width, e.tris.as<uint32_t>(), e.roots.as<int32_t>(), e.mesh_info.as<float>(), dQ, vp, d_qoff,
