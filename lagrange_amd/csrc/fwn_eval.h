@@ -19,9 +19,14 @@ __device__ __forceinline__ int mesh_of64(const int64_t* off, int M, int64_t t)
     return lo;
 }
 
-// exact triangle solid angle, FP32, normalised-vector van Oosterom-Strackee form
+// Exact triangle solid angles.  Every rounding stands in the source (explicit fma, no contraction by the
+// compiler, which fuses a product and a sum only where both lie in one basic block): a leaf's value has
+// the same bits in every kernel, whatever else is compiled around it.
+
+// FP32, normalised-vector van Oosterom-Strackee form
 __device__ __forceinline__ float tri_f32(const float* __restrict__ t, float qx, float qy, float qz)
 {
+#pragma clang fp contract(off)
     float ax = t[0] - qx, ay = t[1] - qy, az = t[2] - qz;
     float bx = t[3] - qx, by = t[4] - qy, bz = t[5] - qz;
     float cx = t[6] - qx, cy = t[7] - qy, cz = t[8] - qz;
@@ -33,10 +38,10 @@ __device__ __forceinline__ float tri_f32(const float* __restrict__ t, float qx, 
     const bool corner = la2 == 0.0f || lb2 == 0.0f || lc2 == 0.0f;
     float ia = __builtin_amdgcn_rsqf(la2), ib = __builtin_amdgcn_rsqf(lb2), ic = __builtin_amdgcn_rsqf(lc2);
     ax *= ia; ay *= ia; az *= ia;
+    float ux = fmaf(bx, ib, -ax), uy = fmaf(by, ib, -ay), uz = fmaf(bz, ib, -az);
+    float vx = fmaf(cx, ic, -ax), vy = fmaf(cy, ic, -ay), vz = fmaf(cz, ic, -az);
     bx *= ib; by *= ib; bz *= ib;
     cx *= ic; cy *= ic; cz *= ic;
-    float ux = bx - ax, uy = by - ay, uz = bz - az;
-    float vx = cx - ax, vy = cy - ay, vz = cz - az;
     float nx = fmaf(uy, vz, -uz * vy);
     float ny = fmaf(uz, vx, -ux * vz);
     float nz = fmaf(ux, vy, -uy * vx);
@@ -48,21 +53,29 @@ __device__ __forceinline__ float tri_f32(const float* __restrict__ t, float qx, 
     return corner || num == 0.0f ? 0.0f : 2.0f * atan2f(num, den);
 }
 
-// exact triangle solid angle, FP64, 2 atan2(a.(b x c), |a||b||c| + (a.b)|c| + (b.c)|a| + (c.a)|b|)
+// a.b in FP64: products of the three axes, two of them fused into the sum
+__device__ __forceinline__ double dot_f64(double ax, double ay, double az, double bx, double by, double bz)
+{
+    return fma(az, bz, fma(ax, bx, ay * by));
+}
+
+// FP64, 2 atan2(a.(b x c), |a||b||c| + (a.b)|c| + (b.c)|a| + (c.a)|b|)
 __device__ __forceinline__ double tri_f64(const float* __restrict__ t, float qx, float qy, float qz)
 {
+#pragma clang fp contract(off)
     double q0 = qx, q1 = qy, q2 = qz;
     double ax = (double)t[0] - q0, ay = (double)t[1] - q1, az = (double)t[2] - q2;
     double bx = (double)t[3] - q0, by = (double)t[4] - q1, bz = (double)t[5] - q2;
     double cx = (double)t[6] - q0, cy = (double)t[7] - q1, cz = (double)t[8] - q2;
-    double la = sqrt(ax * ax + ay * ay + az * az);
-    double lb = sqrt(bx * bx + by * by + bz * bz);
-    double lc = sqrt(cx * cx + cy * cy + cz * cz);
+    double la = sqrt(dot_f64(ax, ay, az, ax, ay, az));
+    double lb = sqrt(dot_f64(bx, by, bz, bx, by, bz));
+    double lc = sqrt(dot_f64(cx, cy, cz, cx, cy, cz));
     if (la == 0.0 || lb == 0.0 || lc == 0.0) return 0.0;
-    double num = ax * (by * cz - bz * cy) + ay * (bz * cx - bx * cz) + az * (bx * cy - by * cx);
+    double num = dot_f64(ax, ay, az, fma(by, cz, -(bz * cy)), fma(bz, cx, -(bx * cz)), fma(bx, cy, -(by * cx)));
     if (num == 0.0) return 0.0;
-    double den = la * lb * lc + (ax * bx + ay * by + az * bz) * lc + (bx * cx + by * cy + bz * cz) * la +
-                 (cx * ax + cy * ay + cz * az) * lb;
+    double den = fma(la * lb, lc, dot_f64(ax, ay, az, bx, by, bz) * lc);
+    den = fma(la, dot_f64(bx, by, bz, cx, cy, cz), den);
+    den = fma(lb, dot_f64(cx, cy, cz, ax, ay, az), den);
     return 2.0 * atan2(num, den);
 }
 
