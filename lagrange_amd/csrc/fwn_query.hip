@@ -822,7 +822,7 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
     }
     const int quad_bpts = choice == Quads::Spread ? kQuadPoints : bpts;
 
-    const int waves = e.opt.waves_per_block > 0 ? e.opt.waves_per_block : 1;
+    const int waves = e.opt.waves_per_block > 0 && !stats ? e.opt.waves_per_block : 1; // stats: one wave a block
     const bool persist = (e.opt.launch_mode == FWN_LAUNCH_PERSISTENT) && !stats;
     int64_t nblk = (nb + waves - 1) / waves;
     if (persist) {
