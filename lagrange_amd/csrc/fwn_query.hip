@@ -458,6 +458,16 @@ constexpr int64_t kSmallBatch = 2048;
 // near the surface 162 / 208 and 208 / 404; 32,768 points 189 / 207 and 193 / 303, near the surface
 // 288 / 216 and 379 / 386.
 constexpr int64_t kPointCalls = 16384;
+//
+// Where the walks outgrow the LDS records (they are then done twice, the second time depth first), only
+// calls of up to kSmallBatch points take this path: a walk grows with the square of the accuracy scale and
+// with the depth of the tree.  16,384 points' walks fit while scale^2 log2(F / 64) <= kPointWalk and scale
+// <= kPointScale (8-wide and Morton trees outgrow them sooner).  8,192 points, uniform and near the
+// surface: F = 20,172, scale 3 (75) 81 / 184 and 111 / 216, scale 4 (132) 323 / 244 and 722 / 294, scale 8
+// 2222 / 586 and 3144 / 675; F = 199,692, scale 2.5 (73) 76 / 173 and 122 / 258, scale 3 (104) 228 / 216 and
+// 308 / 316.  Trees of buckets, whose near leaves hold more to add, cross at half as many points: 16,384
+// near the surface, buckets of 8, scale 1, F = 4,800 147 / 83, 8,192 91 / 83.
+constexpr double kPointWalk = 90.0, kPointScale = 3.0;
 
 } // namespace
 
@@ -663,7 +673,9 @@ void launch_traverse_inplace(Engine& e, int banks, const float* dQ, const uint32
 
 bool few_points(const Engine& e, int64_t nQ)
 {
-    return nQ <= kPointCalls && default_shape(e);
+    const double b = e.opt.accuracy_scale, F = (double)e.h_f_off[1];
+    const bool fits = b <= kPointScale && b * b * std::log2(std::max(F, 1.0) / 64.0) <= kPointWalk;
+    return nQ <= (!fits ? kSmallBatch : (e.opt.leaf_max > 1 ? kPointCalls / 2 : kPointCalls)) && default_shape(e);
 }
 
 void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t nQ, float* omega, uint8_t* inside,
