@@ -473,9 +473,10 @@ __global__ __launch_bounds__(1024) void k_publish(const uint4* __restrict__ om, 
 
 __global__ void k_clear(int32_t* p) { *p = 0; }
 
-// results of up to this many points go straight to host memory, one 8-byte store each; more are
-// collected in device memory first
-constexpr int64_t kPointDirect = 128;
+// Results of up to this many points go straight to host memory, one 8-byte store each; more are
+// collected in device memory first.  Host calls in us, stored / collected: 129 points 30.0 / 35.3 (F =
+// 20,172) and 32.6 / 37.6 (F = 874,800), 512 33.0 / 38.0 and 35.6 / 39.9, 2,048 37.0 / 40.4 and 39.7 / 44.0
+constexpr int64_t kPointDirect = 2048;
 // LDS of a k_point_bfs wave: as much as lets all waves of the call be resident, within these bounds
 constexpr size_t kPointLdsMax = 65536, kPointLdsMin = 20480;
 

@@ -32,7 +32,7 @@ def _noalloc(e, q):
     return om
 
 
-# 250,000: above the slots-in-lanes range of the small meshes; 30,000: within it; 16,384 and 2,000 (from
+# 250,000: above the slots-in-lanes range of the small meshes; 30,000: within it; 16,384 and 2,048 (from
 # host arrays): the per-point kernel
 @pytest.mark.parametrize("rel", [1e-4, 0.05])
 @pytest.mark.parametrize("name", MESHES)
@@ -45,7 +45,7 @@ def test_any_call(name, rel):
     q = torch.from_numpy(h).cuda()
     want = e.solid_angle_batch(q).cpu().numpy()
     got = {k: torch.cat([e.solid_angle_batch(x) for x in q.split(k)]).cpu().numpy() for k in (30000, 16384)}
-    got["host"] = np.concatenate([e.solid_angle_batch(h[k:k + 2000]) for k in range(0, n, 2000)])
+    got["host"] = np.concatenate([e.solid_angle_batch(h[k:k + 2048]) for k in range(0, n, 2048)])
     got["noalloc"] = torch.cat([_noalloc(e, x) for x in q.split(16384)]).cpu().numpy()
     for k, om in got.items():
         np.testing.assert_array_equal(om.view(np.uint32), want.view(np.uint32), err_msg=str(k))
