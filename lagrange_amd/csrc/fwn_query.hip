@@ -34,6 +34,7 @@
 
 #include "fwn_eval.h"
 #include "fwn_internal.h"
+#include "fwn_order.h"
 
 namespace fwn {
 
@@ -49,12 +50,10 @@ __device__ __forceinline__ int64_t wave_uniform64(int64_t v)
     return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
-// 32-bit point keys: mesh id in the top mesh_bits bits, then the leading bits of the point's
-// 30-bit Morton code in its mesh's box.  Only the 24 top bits are sorted: a wave needs its 64
-// points close together, not in exact curve order, and every point's result is independent of
-// which points share its wave.
+// The key of point i.  Only leading bits of the keys are sorted: a wave needs its points close together,
+// not in exact curve order, and every point's result is independent of which points share its wave.
 __device__ __forceinline__ uint32_t point_key(const float* __restrict__ Q, int64_t nQ, int64_t i,
-                                              const int64_t* __restrict__ q_off, int M, int mesh_bits,
+                                              const int64_t* __restrict__ q_off, int M, int mesh_bits, int first,
                                               const float* __restrict__ minfo)
 {
     int m = 0;
@@ -66,11 +65,8 @@ __device__ __forceinline__ uint32_t point_key(const float* __restrict__ Q, int64
         m = (m0 == m1) ? m0 : mesh_of64(q_off, M, i);
     }
     const float* mi = minfo + 8 * m;
-    uint32_t mc = morton30(Q[3 * i], Q[3 * i + 1], Q[3 * i + 2], mi, mi + 3);
-    const int mbits = 32 - mesh_bits; // bits left for the Morton code
-    uint32_t key = (mbits >= 30) ? mc : (mc >> (30 - mbits));
-    if (mesh_bits > 0) key |= (uint32_t)m << mbits;
-    return key; // the sort's first pass takes the values to be the positions i
+    // the sort's first pass takes the values to be the positions i
+    return point_key_of(morton30(Q[3 * i], Q[3 * i + 1], Q[3 * i + 2], mi, mi + 3), (uint32_t)m, mesh_bits, first);
 }
 
 // flags (nullptr: none): the traversal's overflow flag and work counter, cleared on the way
@@ -81,7 +77,7 @@ __global__ __launch_bounds__(QT) void k_query_keys(const float* __restrict__ Q, 
 {
     const int64_t i = (int64_t)blockIdx.x * QT + threadIdx.x;
     if (i < 2 && flags) flags[i] = 0;
-    if (i < nQ) keys[i] = point_key(Q, nQ, i, q_off, M, mesh_bits, minfo);
+    if (i < nQ) keys[i] = point_key(Q, nQ, i, q_off, M, mesh_bits, sort24_first(mesh_bits), minfo);
 }
 
 // the same in tiles of kFewTile points, with the tile's counts of the sort's first digit
@@ -98,7 +94,7 @@ __global__ __launch_bounds__(1024) void k_query_keys_few(const float* __restrict
     for (int r = 0; r < kFewTile / 1024; ++r) {
         const int64_t i = (int64_t)blockIdx.x * kFewTile + r * 1024 + threadIdx.x;
         const bool valid = i < nQ;
-        const uint32_t key = valid ? point_key(Q, nQ, i, q_off, M, mesh_bits, minfo) : 0u;
+        const uint32_t key = valid ? point_key(Q, nQ, i, q_off, M, mesh_bits, 0, minfo) : 0u;
         if (valid) keys[i] = key;
         count_digit(cnt, key >> 12 & 1023u, valid);
     }
@@ -809,8 +805,8 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
         int mesh_bits = 0;
         while ((1 << mesh_bits) < M) ++mesh_bits;
         if (mesh_bits > 24) fail(FWN_LIMIT_EXCEEDED, "more than 2^24 meshes in one engine");
-        // few tiles: 20 bits (the mesh among them) separate 2^20 cells, or about 60,000 along a
-        // surface, where at most 524,288 points leave nothing for more bits to order
+        // few tiles: 20 bits (the mesh among them) separate 2^20 cells of a mesh's box, or about 60,000 along
+        // a surface, where at most 524,288 points leave little for more bits to order
         if (few_tiles(nQ) <= kFewTiles && mesh_bits <= 8) {
             e.q_hist.reserve(sizeof(int32_t) * 1024 * (size_t)few_tiles(nQ));
             hipLaunchKernelGGL(k_query_keys_few, dim3(few_tiles(nQ)), dim3(1024), 0, s, dQ, nQ, d_qoff, M, mesh_bits,
