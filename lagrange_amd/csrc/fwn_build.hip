@@ -1035,6 +1035,9 @@ void build_engine(Engine& e, int32_t M, const float* V_host, const int64_t* v_of
     e.n_meshes = M;
     e.n_tris = nF;
     e.h_f_off.assign(f_off, f_off + M + 1);
+    int64_t largest = 0;
+    for (int m = 0; m < M; ++m) largest = std::max(largest, f_off[m + 1] - f_off[m]);
+    e.uneven = M > 1 && 2 * largest * M >= 3 * nF;
     const int leaf_max = e.opt.leaf_max;
     const int width = e.opt.tree_width;
     e.width = width;
@@ -1100,6 +1103,7 @@ void build_engine(Engine& e, int32_t M, const float* V_host, const int64_t* v_of
         if (h_err & 2) fail(FWN_INVALID_ARGUMENT, "non-finite vertex position");
         const float* mi = reinterpret_cast<const float*>(from + 16);
         for (int m = 0; m < M; ++m) e.h_tau[m] = mi[8 * m + 6];
+        e.h_info.assign(mi, mi + 8 * (size_t)M);
     };
     const size_t setup_b = 16 + sizeof(float) * 8 * (size_t)M;
 

@@ -173,7 +173,7 @@ void orientation_criterion(Engine& e, const float* V, int64_t nV, const int32_t*
     FWN_HIP(hipMemcpyAsync(&err, e.c_err.p, sizeof(int32_t), hipMemcpyDeviceToHost, s));
     FWN_HIP(hipStreamSynchronize(s));
     if (err) fail(FWN_INVALID_ARGUMENT, "facet index out of range");
-    run_queries(e, e.v_pts.as<float>(), nullptr, 2 * nF, e.v_om.as<float>(), nullptr, nullptr, true, nullptr, true);
+    run_queries(e, e.v_pts.as<float>(), nullptr, 2 * nF, e.v_om.as<float>(), nullptr, nullptr, true, nullptr, Points::Layer);
     double* dC = crit;
     if (!dev) {
         e.c_out.reserve(sizeof(double) * (size_t)nF);

@@ -86,6 +86,7 @@ struct Engine {
     fwn_options opt{};
 
     int32_t n_meshes = 0;
+    bool uneven = false; // several meshes, the largest of at least 1.5 times their mean number of triangles
     int32_t width = 4;         // slots per node
     int64_t n_tris = 0;
     int64_t n_nodes = 0;
@@ -102,6 +103,7 @@ struct Engine {
     DBuf mesh_info;  // per mesh: 8 floats: qbox lo[3], qbox inv[3], tau, pad
     std::vector<int32_t> h_roots;
     std::vector<float> h_tau;
+    std::vector<float> h_info; // host copy of mesh_info
     std::vector<int64_t> h_f_off;
 
     // query scratch (grown on demand)
@@ -207,11 +209,13 @@ SahMids build_topology_sah(Engine& e, Arena& ar, const float* cen, const float* 
                            const int64_t* f_off, int M, int32_t* items, int32_t* left, int32_t* right, int32_t* parent,
                            int32_t* first, int32_t* last, uint8_t* is_root, int32_t* root_bin);
 
+// What a caller knows of its points (a choice of kernel only, the results are the same): nothing, that they
+// lie in layers along a surface, or that they are a dense grid, spread over the mesh's box or not.
+enum class Points { Any, Layer, Spread, Close };
 // queries (fwn_query.hip).  order: device positions -> points of one mesh that are already in an order
 // of waves (nullptr: the call sorts its points); not read by calls that need no order (few_points).
-// layer: the points lie in layers along a surface (a choice of kernel only, the results are the same).
 void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t nQ, float* omega, uint8_t* inside,
-                 int32_t* stats, bool device_ptrs, const uint32_t* order = nullptr, bool layer = false);
+                 int32_t* stats, bool device_ptrs, const uint32_t* order = nullptr, Points where = Points::Any);
 // whether a device call of nQ points of one mesh runs one wave per point
 bool few_points(const Engine& e, int64_t nQ);
 void run_bruteforce(Engine& e, const float* Q, int64_t nQ, double* out, bool device_ptrs);
@@ -225,14 +229,25 @@ inline bool default_shape(const Engine& e)
 }
 // Calls of few points of a single-mesh engine, one wave per point (fwn_point.hip).
 void run_points(Engine& e, const float* Q, int64_t nQ, float* omega, uint8_t* inside, int banks, bool device_ptrs);
-// The slots-in-lanes traversal (fwn_quad.hip): whether a call goes to it (Spread: if its points spread
-// over the mesh's box), and its launch over nb batches of bpts points (metadata as k_traverse's); FP64
-// near leaves are evaluated in the kernel, flag is set on a stack overflow.
+// The slots-in-lanes traversal (fwn_quad.hip): whether a call goes to it, and its launch over nb batches of
+// bpts points (metadata as k_traverse's); FP64 near leaves are evaluated in the kernel, flag is set on a
+// stack overflow.  Look: quads_after_look says, once points of the mesh with the most of them (`most`) have
+// been looked at: how many of 2^kLookBits cells of its box hold one of as many points, and (0 unless
+// quads_near_surface) how many of kLookWalks walks reached a leaf.
 constexpr int kQuadPoints = 16;
-enum class Quads { No, Yes, Spread };
-Quads use_quads(const Engine& e, int64_t nQ, int banks, bool layer);
+constexpr int kLookBits = 13, kLookWalks = 256;
+// Layers cross where 64 neighbours extend over about 1.8 times their distance from the surface, and the last
+// slot's threshold is about twice that distance^2.  k_traverse / slots in lanes in us at extent / distance: 64
+// meshes of 199,692 triangles, 1 % of the diagonal off, 8 (12k points each) 1647 / 836, 5.5 (25k) 2039 / 1337, 3.9
+// (50k) 2733 / 2135; 16 of them 2.8 (100k) 1087 / 974, 1.6 (300k) 2171 / 2364; 5 % off 1.6 (64 x 12k) 337 / 342,
+// 1.1 (64 x 25k) 460 / 534, 0.8 (16 x 50k) 278 / 310
+constexpr float kLookNear = 0.6f;
+enum class Quads { No, Yes, Look };
+Quads use_quads(const Engine& e, int64_t nQ, int64_t most, int banks, Points where);
+bool quads_near_surface(const Engine& e, int64_t nQ);
+bool quads_after_look(int cells, int reached);
 void launch_quads(Engine& e, const float* dQ, const uint32_t* perm, const int64_t* q_off, const int64_t* b_off,
-                  const int32_t* order, int M, int64_t nb, int bpts, bool layer, float* omega, uint8_t* inside,
+                  const int32_t* order, int M, int64_t nb, int bpts, Points where, float* omega, uint8_t* inside,
                   int32_t* flag, hipStream_t s);
 int quad_points(const Engine& e, int64_t nQ); // points per wave, kQuadPoints at most
 // Pieces of a query that uses no engine scratch (single-mesh engine, device points): the 32-bit
@@ -467,13 +482,14 @@ __device__ __forceinline__ uint32_t xcd_remap_runs(uint32_t b, uint32_t nb, uint
     const uint32_t x = b % 8u, i = b / 8u;
     return (i / run * 8u + x) * run + i % run;
 }
-// Batches of several meshes are numbered from the largest mesh to the smallest: in one run per XCD
-// the last XCDs end early.  32 meshes of 1.7k to 181k triangles, 3.7M points, k_traverse_quad 1581 us
-// in one run per XCD, 1411 in runs of 16, 1448 in runs of 64 or more; a single mesh loses up to 8 %
-// (100k points, F = 199,692) to runs, its neighbouring waves sharing less of an L2.
-__device__ __forceinline__ uint32_t xcd_batch(uint32_t b, uint32_t nb, int M)
+// Batches of several meshes are numbered from the largest mesh to the smallest: in one run per XCD the last
+// XCDs end early where the meshes are uneven (Engine::uneven), while even ones share less of an L2 in several.
+// k_traverse in one run per XCD / in runs of 16 / 64: 32 meshes of 1.7k to 200k triangles, 50,000 points each,
+// uniform 1636 / 1038 / 1073 us, near the surface 4141 / 1648 / 1648; 64 even ones of 20,172 triangles, a layer 12k
+// 358 / 377 / 369 and 50k 713 / 750 / 735
+__device__ __forceinline__ uint32_t xcd_batch(uint32_t b, uint32_t nb, int run)
 {
-    return M > 1 ? xcd_remap_runs(b, nb, 16u) : xcd_remap(b, nb);
+    return run > 0 ? xcd_remap_runs(b, nb, (uint32_t)run) : xcd_remap(b, nb);
 }
 
 } // namespace fwn

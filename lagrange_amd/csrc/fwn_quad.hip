@@ -11,6 +11,7 @@
 
 #include "fwn_eval.h"
 #include "fwn_internal.h"
+#include "fwn_order.h"
 
 namespace fwn {
 
@@ -281,9 +282,10 @@ __global__ __launch_bounds__(64) void k_traverse_quad(
 // of the default launch shape (the other shapes are k_traverse's, chosen by the tuner or the
 // caller), up to kQuadCross * cbrt(F) points for a mesh of F triangles (several: of the mean F)
 // and, for several meshes, kQuadSparse points a triangle more, as each mesh's share of the points
-// is sparse on it however many the call has.  The two kernels' costs cross where the 64 points of a k_traverse wave are close together compared with the nodes they
-// visit, for points near the surface (both kernels walk to the triangles) at fewer points than for
-// uniform ones; the line lies between the two crossings.  k_traverse / this kernel in us, with the
+// is sparse on it however many the call has.  The two kernels' costs cross where the 64 points of a
+// k_traverse wave are close together compared with the nodes they visit, for points near the surface
+// (both kernels walk to the triangles) at fewer points than for uniform ones; the line lies between the
+// two crossings.  k_traverse / this kernel in us, with the
 // sort,
 //   uniform: F = 972 138 / 120 (200k points) and 170 / 182 (400k); F = 20,172 349 / 336 (800k), 455 /
 //     516 (1.5M); F = 199,692 731 / 567 (1.5M), 858 / 814 (2.5M), 1038 / 1215 (4M); F = 940,800
@@ -296,24 +298,45 @@ __global__ __launch_bounds__(64) void k_traverse_quad(
 //     713; 32 x 100k points, F = 19,200 1322 / 1169 and 1920 / 2164; 8 meshes of 14k to 48k, 1M
 //     points, 703 / 409; 32 of 1.7k to 181k, 3.7M points, 1199 / 1214.
 //
-// Points in a thin layer (at a distance from the surface above all, where few walks go deep) are close
-// together at far fewer points than these lines say: a layer 5 % of the diagonal off F = 940,800 takes
-// 300 / 333 us at 588k points and 660 / 990 at 2.3M, one 1 % off 858 / 744 and 1521 / 1955; F =
-// 199,692 333 / 384 at 701k and 781 / 743.  Above kQuadAny points of one mesh the slots-in-lanes
-// traversal is therefore taken only for points that spread over the mesh's box (Quads::Spread).
+// Points in a layer at a distance from the surface, where few walks go deep, are close together at far fewer
+// points than these lines say.  k_traverse / this kernel for layers 5 % of the diagonal off: F = 199,692 170 /
+// 185 us (400k points), 208 / 244 (600k) and 249 / 327 (1M); 16 such meshes 379 / 485 (100k points each) and 762 /
+// 1178 (300k); 64 of 20,172 triangles 477 / 557 (25k each).  Above kQuadAny points the slots-in-lanes traversal
+// is therefore taken only for points that, looked at (k_point_look), spread over the box of the mesh with the
+// most of them, or are close to its surface for their density.  One mesh's points near the surface: up to
+// kQuadNear * log2(F / 170) of them, as the kernels cross early there (F = 20,172 454 / 435 at 499k points and 484
+// / 495 at 600k; 199,692 834 / 727 at 600k and 979 / 1026 at 1M; 874,800 1502 / 1483 at 1M).  Several meshes': up to
+// the line above (64 of 199,692 triangles, 12k points each near the surface 4780 / 2207, 1 % off 1647 / 836; 16
+// with 300k 5235 / 4904).  The look runs beside the sort: 0 to 12 us of a call that k_traverse then answers in
+// 130 to 250, nothing of longer ones.  (With a fixed stride, ahead of the sort and a copy back it took 25 to 35
+// us, did not look at several meshes and took grids of 128^3 points for layers: F = 750,000 1226 us, 785 now.)
+//
 // A caller that knows its points to lie along a surface (the orientation probes) has a line of its own,
 // kQuadLayer * cbrt(F), and no look at the points: whole calls of two probes a facet, 0.01 / 1 / 5 / 30 % of
 // the size off the surface, k_traverse 1060 / 818 / 394 / 231 us and this kernel 641 / 604 / 346 / 229 at 479k
 // probes, 1250 / 887 / 398 / 239 and 752 / 711 / 386 / 258 at 569k, 1707 / 1108 / 449 / 271 and 1135 / 981 /
 // 507 / - at 912k: the line lies where no distance loses.
-constexpr double kQuadCross = 24000.0, kQuadSparse = 2.0, kQuadAny = 500000.0, kQuadLayer = 8000.0;
-Quads use_quads(const Engine& e, int64_t nQ, int banks, bool layer)
+constexpr double kQuadCross = 24000.0, kQuadSparse = 2.0, kQuadAny = 400000.0, kQuadNear = 73000.0, kQuadLayer = 8000.0;
+constexpr int64_t kLookLeast = 1 << kLookBits;
+Quads use_quads(const Engine& e, int64_t nQ, int64_t most, int banks, Points where)
 {
     if (e.width != 4 || banks != 1 || !default_shape(e)) return Quads::No;
     const double F = (double)e.h_f_off[e.n_meshes];
-    if (layer && e.n_meshes == 1) return (double)nQ <= kQuadLayer * std::cbrt(F) ? Quads::Yes : Quads::No;
+    if (where == Points::Layer && e.n_meshes == 1)
+        return (double)nQ <= kQuadLayer * std::cbrt(F) ? Quads::Yes : Quads::No;
     if ((double)nQ > kQuadCross * std::cbrt(F / e.n_meshes) + (e.n_meshes > 1 ? kQuadSparse * F : 0.0)) return Quads::No;
-    return e.n_meshes == 1 && (double)nQ > kQuadAny ? Quads::Spread : Quads::Yes;
+    if ((double)nQ <= kQuadAny || most < kLookLeast || where == Points::Spread) return Quads::Yes;
+    return where == Points::Close ? Quads::No : Quads::Look;
+}
+
+bool quads_near_surface(const Engine& e, int64_t nQ)
+{
+    return e.n_meshes > 1 || (double)nQ <= kQuadNear * std::log2((double)e.h_f_off[1] / 170.0);
+}
+
+bool quads_after_look(int cells, int reached)
+{
+    return (double)cells >= kSpreadLeast * (double)(1 << kLookBits) || 2 * reached >= kLookWalks;
 }
 
 // Points per wave: 16, the wave's lanes, or 8 where so few waves run that the longest decides (up to 500
@@ -327,13 +350,13 @@ int quad_points(const Engine& e, int64_t nQ)
 }
 
 void launch_quads(Engine& e, const float* dQ, const uint32_t* perm, const int64_t* q_off, const int64_t* b_off,
-                  const int32_t* order, int M, int64_t nb, int bpts, bool layer, float* omega, uint8_t* inside,
+                  const int32_t* order, int M, int64_t nb, int bpts, Points where, float* omega, uint8_t* inside,
                   int32_t* flag, hipStream_t s)
 {
     // Blocks to the XCDs in runs for several meshes (xcd_batch) and for layers of 8,192 waves or more, whose
     // expensive waves lie together: probes 1 % off, one run per XCD / runs of 64, 400k points 488 / 454 us (F =
     // 199,692) and 530 / 473 (F = 940,800), 500k 565 / 527 and 625 / 543; uniform points lose 8 to 18 % to runs
-    const int run = M > 1 ? 16 : (layer && nb >= 8192 ? 64 : 0);
+    const int run = M > 1 ? 16 : (where == Points::Layer && nb >= 8192 ? 64 : 0);
     // node buffers per wave: 20 (9 KB, room for 4 waves per SIMD) while the call has no more waves
     // than that, else 12 (6 KB: 6 and a half); entries above them are rare.  F = 199,692, uniform and
     // near the surface, 9 / 12 / 20 buffers: 20k points 135 / 132 / 118 and 215 / 200 / 178 us, 400k

@@ -102,33 +102,85 @@ __global__ __launch_bounds__(1024) void k_query_keys_few(const float* __restrict
     hist[(int64_t)blockIdx.x * 1024 + threadIdx.x] = cnt[threadIdx.x];
 }
 
-// How many of the 32^3 cells of the mesh's box (points outside it count at its faces) hold one of 32,768
-// points taken evenly from the call: uniform points and grids in the box or 20 % beyond it fill 0.52 to
-// 0.63 of them, layers up to 10 % of the diagonal off the surface 0.12 to 0.22.  One block; about 6 us,
-// of which the host sees nothing: it reads the count while the sort runs.
-constexpr int kSpreadPoints = 32768, kSpreadCells = 32768, kSpreadLeast = (int)(0.3 * kSpreadCells);
-__global__ __launch_bounds__(1024) void k_point_spread(const float* __restrict__ Q, int64_t nQ,
-                                                       const float* __restrict__ minfo, int32_t* __restrict__ cells)
+// A look at the n points of one mesh, Q[0..n): how many of 2^kLookBits cells of the mesh's box hold one of as
+// many of them (kSpreadLeast), and how many of kLookWalks points are close to the surface for their density:
+// a walk from the root of a 4-wide tree, each time into the slot nearest in terms of its far threshold, ends
+// in a leaf or in a slot with a threshold below kLookNear times the extent^2 of 64 neighbouring points (64 times
+// the layer's area, about a mean face of a cell for each filled one, over n).  `depth` levels at most, a slot
+// per lane.  The result, with a mark above it, is one store to host memory.  One workgroup, 12 to 16 us on a
+// stream of its own while the points are sorted.
+typedef float point3 __attribute__((ext_vector_type(3), aligned(4)));
+__global__ __launch_bounds__(1024) void k_point_look(const float* __restrict__ Q, int64_t n,
+                                                     const float* __restrict__ minfo,
+                                                     const uint32_t* __restrict__ slots, int32_t root, int32_t root_ns,
+                                                     int depth, uint64_t* __restrict__ result)
 {
-    __shared__ uint32_t bits[kSpreadCells / 32];
-    __shared__ int32_t part[16];
-    bits[threadIdx.x] = 0u;
+    __shared__ uint32_t filled[(1 << kLookBits) / 32];
+    __shared__ float lasts[kLookWalks]; // per walk: the threshold of its last slot, 0: a leaf
+    __shared__ int32_t part[2][16];
+    const int tid = threadIdx.x, lane = tid & 63;
+    if (tid < (1 << kLookBits) / 32) filled[tid] = 0u;
     __syncthreads();
-#pragma unroll 8
-    for (int r = 0; r < kSpreadPoints / 1024; ++r) {
-        const int64_t i = (int64_t)(r * 1024 + threadIdx.x) * nQ / kSpreadPoints;
-        const uint32_t c = morton30(Q[3 * i], Q[3 * i + 1], Q[3 * i + 2], minfo, minfo + 3) >> 15;
-        atomicOr(&bits[c >> 5], 1u << (c & 31u));
+    point3 q[(1 << kLookBits) / 1024];
+#pragma unroll
+    for (int r = 0; r < (1 << kLookBits) / 1024; ++r)
+        q[r] = *reinterpret_cast<const point3*>(Q + 3 * look_index((uint32_t)(r * 1024 + tid), kLookBits, n));
+#pragma unroll
+    for (int r = 0; r < (1 << kLookBits) / 1024; ++r) {
+        const uint32_t c = morton30(q[r].x, q[r].y, q[r].z, minfo, minfo + 3) >> (30 - kLookBits);
+        atomicOr(&filled[c >> 5], 1u << (c & 31u));
+    }
+    if (root >= 0) {
+        constexpr uint32_t kStep = (1u << kLookBits) / kLookWalks;
+        const point3 w = *reinterpret_cast<const point3*>(Q + 3 * look_index((uint32_t)(tid >> 2) * kStep, kLookBits, n));
+        const int s = tid & 3;
+        uint32_t e = (uint32_t)root << 4 | (uint32_t)root_ns; // the same in the walk's four lanes
+        bool on = true;
+        float last = INFINITY; // threshold of the slot entered last
+        for (int level = 0; level < depth && __ballot(on) != 0ull; ++level) {
+            float near = INFINITY, thr = 0.0f; // distance over threshold
+            uint32_t link = FWN_LINK_EMPTY;
+            if (on && s < (int)(e & 15u)) {
+                const uint32_t* slot = slots + ((size_t)(e >> 4) * 4 + s) * kSlotWords;
+                const float4 p = *reinterpret_cast<const float4*>(slot); // centre, threshold
+                link = slot[FWN_W_LINK];
+                const float dx = p.x - w.x, dy = p.y - w.y, dz = p.z - w.z;
+                const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                if (d2 <= p.w && p.w > 0.0f) near = d2 / p.w;
+                thr = p.w;
+            }
+            const float least = fminf(fminf(near, __shfl_xor(near, 1)), fminf(__shfl_xor(near, 2), __shfl_xor(near, 3)));
+            const uint64_t pick = __ballot(near == least && least < INFINITY) >> (lane & 60) & 15u;
+            const int from = (lane & 60) + (pick ? (int)__builtin_ctzll(pick) : 0);
+            e = (uint32_t)__shfl((int)link, from);
+            thr = __shfl(thr, from);
+            on = on && pick != 0ull;
+            if (on) last = (int32_t)e < 0 ? 0.0f : thr;
+            on = on && (int32_t)e >= 0;
+        }
+        if (s == 0) lasts[tid >> 2] = last;
+    } else if ((tid & 3) == 0) {
+        lasts[tid >> 2] = INFINITY;
     }
     __syncthreads();
-    int32_t n = __popc(bits[threadIdx.x]);
-    for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = n;
+    int32_t cells = tid < (1 << kLookBits) / 32 ? __popc(filled[tid]) : 0;
+    for (int o = 32; o > 0; o >>= 1) cells += __shfl_xor(cells, o);
+    if (lane == 0) part[0][tid >> 6] = cells;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        n = 0;
-        for (int w = 0; w < 16; ++w) n += part[w];
-        *cells = n;
+    cells = 0;
+    for (int k = 0; k < 16; ++k) cells += part[0][k];
+    float side[3]; // of a cell: 32 x 16 x 16 of them
+    for (int d = 0; d < 3; ++d) side[d] = minfo[3 + d] > 0.0f ? (d == 0 ? 1.0f / 32 : 1.0f / 16) / minfo[3 + d] : 0.0f;
+    const float face = (side[0] * side[1] + side[1] * side[2] + side[2] * side[0]) * (1.0f / 3);
+    const float line = kLookNear * 64.0f * (float)cells * face / (float)n;
+    const uint64_t hits = __ballot(tid < kLookWalks && lasts[tid & (kLookWalks - 1)] <= line);
+    if (lane == 0) part[1][tid >> 6] = (int32_t)__popcll(hits);
+    __syncthreads();
+    if (tid == 0) {
+        int32_t walks = 0;
+        for (int k = 0; k < 16; ++k) walks += part[1][k];
+        __hip_atomic_store(result, (uint64_t)1 << 63 | (uint64_t)walks << 32 | (uint64_t)cells, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -346,15 +398,16 @@ __global__ __launch_bounds__(WAVES * 64) void k_traverse(
     const uint32_t* __restrict__ slots, int width, const uint32_t* __restrict__ tris,
     const int32_t* __restrict__ roots, const float* __restrict__ minfo, const float* __restrict__ Q,
     const uint32_t* __restrict__ perm, const int64_t* __restrict__ q_off, const int64_t* __restrict__ b_off,
-    const int32_t* __restrict__ mesh_order, int M, int64_t n_batches, int bpts, float beta2, float* __restrict__ omega,
-    uint8_t* __restrict__ inside, int32_t* __restrict__ stats, int32_t* __restrict__ flag, uint32_t* __restrict__ work)
+    const int32_t* __restrict__ mesh_order, int M, int64_t n_batches, int bpts, int run, float beta2,
+    float* __restrict__ omega, uint8_t* __restrict__ inside, int32_t* __restrict__ stats, int32_t* __restrict__ flag,
+    uint32_t* __restrict__ work)
 {
     extern __shared__ uint4 traverse_lds[];
     char* lds = reinterpret_cast<char*>(traverse_lds) + (size_t)(threadIdx.x >> 6) * traverse_lds_bytes(width);
     unsigned long long* acc = reinterpret_cast<unsigned long long*>(lds);
     uint2* queue = reinterpret_cast<uint2*>(acc + 64);
     if (!PERSIST) {
-        const int64_t batch = (int64_t)xcd_batch(blockIdx.x, gridDim.x, M) * WAVES + (threadIdx.x >> 6);
+        const int64_t batch = (int64_t)xcd_batch(blockIdx.x, gridDim.x, run) * WAVES + (threadIdx.x >> 6);
         if (batch >= n_batches) return; // whole wave
         traverse_batch<STATS, NB>(batch, slots, width, tris, roots, minfo, Q, perm, q_off, b_off, mesh_order, M, bpts,
                                   beta2, omega, inside, stats, flag, queue, acc);
@@ -601,8 +654,8 @@ void run_queries_pipelined(Engine& e, const float* Q, int64_t nQ, float* omega, 
             FWN_HIP(hipEventRecord(e.tev[2 * k], s));
             launch_traverse(false, waves, persist, banks, e.width, (unsigned)nblk, s, e.slots.as<uint32_t>(), e.width,
                             e.tris.as<uint32_t>(), e.roots.as<int32_t>(), e.mesh_info.as<float>(), dQ, vp, d_qoff,
-                            d_boff, d_order, 1, nb, 64, beta2, dOm + off, dIn ? dIn + off : nullptr, (int32_t*)nullptr,
-                            dflag, dwork);
+                            d_boff, d_order, 1, nb, 64, 0, beta2, dOm + off, dIn ? dIn + off : nullptr,
+                            (int32_t*)nullptr, dflag, dwork);
             FWN_LAUNCH_CHECK("k_traverse");
             FWN_HIP(hipEventRecord(e.tev[2 * k + 1], s));
             FWN_HIP(hipEventRecord(e.pev[2 + sl], s));
@@ -663,7 +716,7 @@ void launch_traverse_inplace(Engine& e, int banks, const float* dQ, const uint32
     const int32_t* order = reinterpret_cast<const int32_t*>(meta + 4);
     launch_traverse(false, 1, false, banks, e.width, (unsigned)nb, s, e.slots.as<uint32_t>(), e.width,
                     e.tris.as<uint32_t>(), e.roots.as<int32_t>(), e.mesh_info.as<float>(), dQ, perm, q_off, b_off,
-                    order, 1, nb, 64, beta2, omega, inside, (int32_t*)nullptr, flag, (uint32_t*)nullptr);
+                    order, 1, nb, 64, 0, beta2, omega, inside, (int32_t*)nullptr, flag, (uint32_t*)nullptr);
     FWN_LAUNCH_CHECK("k_traverse");
 }
 
@@ -675,7 +728,7 @@ bool few_points(const Engine& e, int64_t nQ)
 }
 
 void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t nQ, float* omega, uint8_t* inside,
-                 int32_t* stats, bool dev, const uint32_t* point_order, bool layer)
+                 int32_t* stats, bool dev, const uint32_t* point_order, Points where)
 {
     hipStream_t s = e.stream;
     const int M = e.n_meshes;
@@ -716,25 +769,37 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
     // points per wave: 64, or fewer for small calls so that their waves spread over the device
     // (a point's result does not depend on which points share its wave)
     const bool small = nQ <= kSmallBatch && !stats;
-    const Quads choice = small || stats ? Quads::No : use_quads(e, nQ, banks, layer);
-    bool quad = choice == Quads::Yes; // Quads::Spread: known once the points are looked at
+    int most = order[0]; // the mesh with the most points, of several the one with the most triangles
+    for (int m : order)
+        if (qoff[m + 1] - qoff[m] > qoff[most + 1] - qoff[most]) most = m;
+    const int64_t n_most = qoff[most + 1] - qoff[most];
+    const Quads choice = small || stats ? Quads::No : use_quads(e, nQ, n_most, banks, where);
+    bool quad = choice == Quads::Yes; // Quads::Look: known once the points are looked at
     const int bpts = small ? (int)std::min<int64_t>(64, std::max<int64_t>(1, (nQ + 1023) / 1024))
                            : (quad ? quad_points(e, nQ) : 64);
-    std::vector<int64_t> boff(M + 1, 0);
-    for (int k = 0; k < M; ++k) boff[k + 1] = boff[k] + (qoff[order[k] + 1] - qoff[order[k]] + bpts - 1) / bpts;
+    auto batches = [&](int pts) {
+        std::vector<int64_t> off(M + 1, 0);
+        for (int k = 0; k < M; ++k) off[k + 1] = off[k] + (qoff[order[k] + 1] - qoff[order[k]] + pts - 1) / pts;
+        return off;
+    };
+    const std::vector<int64_t> boff = batches(bpts);
+    // a call that is looked at has its batches for the slots-in-lanes traversal behind the others
+    const std::vector<int64_t> boff_quad = choice == Quads::Look ? batches(kQuadPoints) : std::vector<int64_t>();
     int64_t nb = boff[M];
 
     const bool stage_io = small && !dev; // points in and results out through the pinned stage
-    // metadata (and the points of a small host batch) in one staged copy:
-    // q_off[M+1] (int64), b_off[M+1] (int64), mesh order[M] (int32), then the points at 16 B
-    const size_t meta_b = (sizeof(int64_t) * 2 * (M + 1) + sizeof(int32_t) * M + 15) & ~(size_t)15;
+    // metadata (and the points of a small host batch) in one staged copy: q_off[M+1], b_off[M+1], the other
+    // b_off[M+1] of a call that is looked at (int64), mesh order[M] (int32), then the points at 16 B
+    const size_t off_b = sizeof(int64_t) * (M + 1), offs = choice == Quads::Look ? 3 : 2;
+    const size_t meta_b = (offs * off_b + sizeof(int32_t) * M + 15) & ~(size_t)15;
     const size_t in_b = meta_b + (stage_io ? sizeof(float) * 3 * (size_t)nQ : 0);
     const size_t out_b = stage_io ? 16 + (sizeof(float) + 1) * (size_t)nQ : 0; // flags, omega, inside
-    const size_t spread_at = (std::max(in_b, out_b) + 15) & ~(size_t)15; // the spread comes back behind it all
-    char* hs = host_stage(e, spread_at + 16);
-    std::memcpy(hs, qoff.data(), sizeof(int64_t) * (M + 1));
-    std::memcpy(hs + sizeof(int64_t) * (M + 1), boff.data(), sizeof(int64_t) * (M + 1));
-    std::memcpy(hs + sizeof(int64_t) * 2 * (M + 1), order.data(), sizeof(int32_t) * M);
+    const size_t look_at = (std::max(in_b, out_b) + 15) & ~(size_t)15; // the look's result behind it all
+    char* hs = host_stage(e, look_at + 16);
+    std::memcpy(hs, qoff.data(), off_b);
+    std::memcpy(hs + off_b, boff.data(), off_b);
+    if (choice == Quads::Look) std::memcpy(hs + 2 * off_b, boff_quad.data(), off_b);
+    std::memcpy(hs + offs * off_b, order.data(), sizeof(int32_t) * M);
     if (stage_io) std::memcpy(hs + meta_b, Q, sizeof(float) * 3 * (size_t)nQ);
     const void* meta_before = e.q_meta.p;
     e.q_meta.reserve(in_b);
@@ -748,7 +813,7 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
     }
     const int64_t* d_qoff = e.q_meta.as<int64_t>();
     const int64_t* d_boff = d_qoff + (M + 1);
-    const int32_t* d_order = reinterpret_cast<const int32_t*>(d_qoff + 2 * (M + 1));
+    const int32_t* d_order = reinterpret_cast<const int32_t*>(d_qoff + offs * (M + 1));
 
     const float* dQ = Q;
     float* dOm = omega;
@@ -787,12 +852,6 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
     FWN_HIP(hipEventRecord(e.ev[0], s));
     int32_t* dflag = e.q_flag.as<int32_t>();
     uint32_t* dwork = reinterpret_cast<uint32_t*>(dflag + 1);
-    if (choice == Quads::Spread) {
-        hipLaunchKernelGGL(k_point_spread, dim3(1), dim3(1024), 0, s, dQ, nQ, e.mesh_info.as<float>(), dflag + 2);
-        FWN_LAUNCH_CHECK("k_point_spread");
-        FWN_HIP(hipMemcpyAsync(hs + spread_at, dflag + 2, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-        FWN_HIP(hipEventRecord(e.ev[3], s));
-    }
     // sorted position -> input index (nullptr: small calls keep the input order)
     const uint32_t* vp = small ? nullptr : point_order;
     if (small || point_order) {
@@ -821,14 +880,32 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
         }
         vp = vals;
     }
-    if (choice == Quads::Spread) {
-        FWN_HIP(hipEventSynchronize(e.ev[3])); // the sort is under way
-        int32_t cells = 0;
-        std::memcpy(&cells, hs + spread_at, sizeof(cells));
-        quad = cells >= kSpreadLeast;
-        if (quad) nb = (nQ + kQuadPoints - 1) / kQuadPoints; // of one mesh: its b_off is not read
+    int quad_bpts = bpts;
+    if (choice == Quads::Look) {
+        volatile uint64_t* word = reinterpret_cast<volatile uint64_t*>(hs + look_at);
+        *word = 0;
+        if (!e.cs_in) FWN_HIP(hipStreamCreateWithFlags(&e.cs_in, hipStreamNonBlocking));
+        FWN_HIP(hipStreamWaitEvent(e.cs_in, e.ev[0], 0)); // the points and the metadata are there
+        hipLaunchKernelGGL(k_point_look, dim3(1), dim3(1024), 0, e.cs_in, dQ + 3 * qoff[most], n_most,
+                           e.mesh_info.as<float>() + 8 * most, e.slots.as<uint32_t>(), e.h_roots[2 * most],
+                           e.h_roots[2 * most + 1], quads_near_surface(e, nQ) ? e.max_depth : 0,
+                           const_cast<uint64_t*>(word));
+        FWN_LAUNCH_CHECK("k_point_look");
+        // the sort is under way; a failed launch ends the wait
+        for (uint32_t spin = 1; *word == 0; ++spin)
+            if ((spin & 255u) == 0u && hipStreamQuery(e.cs_in) != hipErrorNotReady) {
+                FWN_HIP(hipStreamSynchronize(e.cs_in));
+                break;
+            }
+        const uint64_t seen = *word;
+        if (seen == 0) fail(FWN_HIP_ERROR, "no result of the look at the points");
+        quad = quads_after_look((int)(seen & 0xFFFFFFFFu), (int)(seen >> 32 & 0x7FFFFFFFu));
+        if (quad) {
+            nb = boff_quad[M];
+            d_boff += M + 1;
+            quad_bpts = kQuadPoints;
+        }
     }
-    const int quad_bpts = choice == Quads::Spread ? kQuadPoints : bpts;
 
     const int waves = e.opt.waves_per_block > 0 && !stats ? e.opt.waves_per_block : 1; // stats: one wave a block
     const bool persist = (e.opt.launch_mode == FWN_LAUNCH_PERSISTENT) && !stats;
@@ -845,11 +922,11 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
     const float beta2 = e.opt.accuracy_scale * e.opt.accuracy_scale;
     FWN_HIP(hipEventRecord(e.ev[1], s));
     if (quad) {
-        launch_quads(e, dQ, vp, d_qoff, d_boff, d_order, M, nb, quad_bpts, layer, dOm, dIn, dflag, s);
+        launch_quads(e, dQ, vp, d_qoff, d_boff, d_order, M, nb, quad_bpts, where, dOm, dIn, dflag, s);
     } else {
         launch_traverse(stats != nullptr, waves, persist, banks, e.width, (unsigned)nblk, s, e.slots.as<uint32_t>(),
                         e.width, e.tris.as<uint32_t>(), e.roots.as<int32_t>(), e.mesh_info.as<float>(), dQ, vp, d_qoff,
-                        d_boff, d_order, M, nb, bpts, beta2, dOm, dIn, dSt, dflag, dwork);
+                        d_boff, d_order, M, nb, bpts, e.uneven ? 64 : 0, beta2, dOm, dIn, dSt, dflag, dwork);
         FWN_LAUNCH_CHECK("k_traverse");
     }
     FWN_HIP(hipEventRecord(e.ev[2], s));

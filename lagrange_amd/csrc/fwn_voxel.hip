@@ -12,6 +12,7 @@
 #include <cstring>
 
 #include "fwn_internal.h"
+#include "fwn_order.h"
 
 namespace fwn {
 namespace {
@@ -90,7 +91,7 @@ __global__ __launch_bounds__(256) void k_voxel_list(const int32_t* __restrict__ 
 // Generate the centres (and, for a box, their order) into the engine's scratch and answer them;
 // outputs host or device.
 static void sign_centres(Engine& e, int64_t n, uint8_t* inside, float* omega, bool dev,
-                         const uint32_t* (*gen)(Engine&, float*, const void*), const void* arg)
+                         const uint32_t* (*gen)(Engine&, float*, const void*), const void* arg, Points where)
 {
     hipStream_t s = e.stream;
     e.v_pts.reserve(sizeof(float) * 3 * n);
@@ -105,7 +106,7 @@ static void sign_centres(Engine& e, int64_t n, uint8_t* inside, float* omega, bo
         e.v_in.reserve(n);
         dIn = e.v_in.as<uint8_t>();
     }
-    run_queries(e, e.v_pts.as<float>(), nullptr, n, dOm, dIn, nullptr, true, order);
+    run_queries(e, e.v_pts.as<float>(), nullptr, n, dOm, dIn, nullptr, true, order, where);
     if (!dev) {
         FWN_HIP(hipMemcpyAsync(inside, dIn, n, hipMemcpyDeviceToHost, s));
         if (omega) FWN_HIP(hipMemcpyAsync(omega, dOm, sizeof(float) * n, hipMemcpyDeviceToHost, s));
@@ -176,7 +177,17 @@ void sign_voxel_box(Engine& e, const int32_t lo[3], const int32_t dims[3], doubl
     b.vs = vs;
     if (b.n == 0) return;
     if (!inside) fail(FWN_INVALID_ARGUMENT, "inside_out is NULL");
-    sign_centres(e, b.n, inside, omega, dev, gen_box, &b);
+    // no sort runs while the points could be looked at, and a box says where they lie
+    Points where = Points::Any;
+    if (e.n_meshes == 1) {
+        double from[3], to[3];
+        for (int d = 0; d < 3; ++d) {
+            from[d] = vs * lo[d];
+            to[d] = vs * ((double)lo[d] + dims[d]);
+        }
+        where = box_spreads(from, to, e.h_info.data()) ? Points::Spread : Points::Close;
+    }
+    sign_centres(e, b.n, inside, omega, dev, gen_box, &b, where);
 }
 
 void sign_voxel_list(Engine& e, const int32_t* ijk, int64_t n, double vs, uint8_t* inside, float* omega, bool dev)
@@ -187,7 +198,7 @@ void sign_voxel_list(Engine& e, const int32_t* ijk, int64_t n, double vs, uint8_
     if (!ijk || !inside) fail(FWN_INVALID_ARGUMENT, "NULL voxel list or inside_out");
     if (n > (int64_t)UINT32_MAX / 2) fail(FWN_LIMIT_EXCEEDED, "more than 2^31 voxels in one call");
     ListArg l{ijk, n, vs, dev};
-    sign_centres(e, n, inside, omega, dev, gen_list, &l);
+    sign_centres(e, n, inside, omega, dev, gen_list, &l, Points::Any);
 }
 
 } // namespace fwn
