@@ -24,8 +24,8 @@
 //   k_collapse_*    level by level, each wide node takes the binary node's children and
 //                   repeatedly opens the largest non-leaf slot until it has tree_width slots (Morton
 //                   trees), or whole binary levels (SAH trees)
-//   k_write_slots   FP64 records -> the 32-word FP32 slot format of fwn.h, plus each slot's box
-//                   (6 floats, rounded outward) and link for distance queries
+//   k_write_slots   FP64 records -> the 24-word FP32 slot format of fwn.h, plus each slot's 64-byte
+//                   record for distance queries: its box (6 floats, rounded outward) and link
 //   k_slot_disks    each slot's disk (a slab around its triangles) for distance queries
 //
 // Several meshes are built together: their keys carry the mesh id above the Morton bits, so

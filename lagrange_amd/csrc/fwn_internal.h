@@ -114,8 +114,10 @@ struct Engine {
     DBuf d_d2, d_tri, d_cp;                               // closest-point outputs for host callers
     int n_cu = 0;
 
-    // pinned host staging for small calls: metadata, points and results in one copy each way
-    // (reused only after the call that filled it has synchronised its stream)
+    // pinned host staging: metadata, points and results of small calls, and the words the host polls.  A call
+    // that has polled its words returns before its kernels have retired, and the next one writes the stage at
+    // once: no kernel touches the stage after the mark that the host waits for (k_point_bfs and k_publish
+    // fence the overflow flag before it), and every other use ends with the stream synchronised.
     void* h_stage = nullptr;
     size_t h_stage_bytes = 0;
     DBuf q_ptflag; // overflow flag of few-point calls

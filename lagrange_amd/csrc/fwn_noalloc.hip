@@ -4,8 +4,8 @@
 // single-mesh engine, bit for bit, for callers that cannot allocate device memory during a call.
 // Its scratch lives in one file-scope device array of fixed size; the host reaches each device's
 // copy through hipGetSymbolAddress, taken once per device with that device current.  The same
-// kernels as the allocating path run: point keys, the 24-bit radix sort (histograms in the
-// array) and the traversal.
+// kernels as the allocating path run: point keys, the radix sort of their bits 8 to 31 (histograms
+// in the array) and the traversal.
 #include <hip/hip_runtime.h>
 
 #include <mutex>

@@ -441,7 +441,7 @@ __global__ __launch_bounds__(64) void k_point_bfs(const uint32_t* __restrict__ s
     if (v != 0) om = (float)((double)om + (double)v * (1.0 / kFixScale));
     const uint32_t in = ((double)om / (4.0 * 3.14159265358979323846) > 0.5) ? 1u : 0u;
     if (lane == 0) {
-        if (packed) { // omega, the flag and the mark in one store: they arrive together
+        if (packed) { // omega, the flag and the mark in one store, the wave's last access to the pinned stage
             __hip_atomic_store(packed + i, (uint64_t)__float_as_uint(om) | ((uint64_t)(2u | in) << 32),
                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         } else {
@@ -468,7 +468,7 @@ __global__ __launch_bounds__(1024) void k_publish(const uint4* __restrict__ om, 
     }
     __threadfence_system();
     __syncthreads();
-    if (threadIdx.x == 0) *hdone = token;
+    if (threadIdx.x == 0) *hdone = token; // the last access to the pinned stage
 }
 
 __global__ void k_clear(int32_t* p) { *p = 0; }

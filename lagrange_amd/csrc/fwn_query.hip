@@ -7,7 +7,7 @@
 // Points are sorted by mesh and 30-bit Morton code, then each wave64 takes 64 consecutive
 // points (one per lane) and walks its mesh's wide tree once for all of them:
 //  * the wave pops a (node, lane mask) pair from a wave-private stack held in three VGPRs
-//    (entry i lives in lane i%64 of bank i/64; pushes are v_cndmask, pops v_readlane), so
+//    (entry i lives in lane i%64 of bank i/64; pushes are v_writelane, pops v_readlane), so
 //    node ids and masks stay scalar and slot/triangle loads are scalar (s_load) broadcasts;
 //  * for every slot each active lane tests |q - p|^2 > beta^2 r2: far lanes add the order-2
 //    expansion, near lanes either take the exact triangle solid angles (leaf slot) or stay
@@ -539,7 +539,9 @@ namespace {
 // copied (several host threads) into a pinned buffer and sent to the device on one copy stream
 // while chunk k-1 is answered on the engine's stream and chunk k-2's results come back on a
 // second copy stream and are copied out to the caller's arrays.  Each chunk is an independent
-// Morton-sorted query (a point's result does not depend on the other points of its call).
+// Morton-sorted query (a point's result does not depend on the other points of its call).  Chunks run
+// k_traverse and the 24-bit sort whatever their size: the slots-in-lanes traversal, which answers 2M spread
+// points of F = 874,800 in 0.65 of the time, is not chosen here.
 constexpr int64_t kPipeChunk = 1 << 21; // points per chunk
 
 void parallel_copy(void* dst, const void* src, size_t bytes)
