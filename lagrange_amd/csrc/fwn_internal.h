@@ -233,9 +233,9 @@ inline bool default_shape(const Engine& e)
 void run_points(Engine& e, const float* Q, int64_t nQ, float* omega, uint8_t* inside, int banks, bool device_ptrs);
 // The slots-in-lanes traversal (fwn_quad.hip): whether a call goes to it, and its launch over nb batches of
 // bpts points (metadata as k_traverse's); FP64 near leaves are evaluated in the kernel, flag is set on a
-// stack overflow.  Look: quads_after_look says, once points of the mesh with the most of them (`most`) have
-// been looked at: how many of 2^kLookBits cells of its box hold one of as many points, and (0 unless
-// quads_near_surface) how many of kLookWalks walks reached a leaf.
+// stack overflow.  Look: quads_after_look says, once the n points of the mesh with the most of them (`most`)
+// have been looked at: how many of 2^kLookBits cells of its box hold one of as many points, and (none unless
+// quads_near_surface) the threshold of the last slot of kLookWalks walks.
 constexpr int kQuadPoints = 16;
 constexpr int kLookBits = 13, kLookWalks = 256;
 // Layers cross where 64 neighbours extend over about 1.8 times their distance from the surface, and the last
@@ -247,7 +247,7 @@ constexpr float kLookNear = 0.6f;
 enum class Quads { No, Yes, Look };
 Quads use_quads(const Engine& e, int64_t nQ, int64_t most, int banks, Points where);
 bool quads_near_surface(const Engine& e, int64_t nQ);
-bool quads_after_look(int cells, int reached);
+bool quads_after_look(const Engine& e, int mesh, int64_t n, int cells, const float* last, int walks);
 void launch_quads(Engine& e, const float* dQ, const uint32_t* perm, const int64_t* q_off, const int64_t* b_off,
                   const int32_t* order, int M, int64_t nb, int bpts, Points where, float* omega, uint8_t* inside,
                   int32_t* flag, hipStream_t s);

@@ -302,21 +302,21 @@ __global__ __launch_bounds__(64) void k_traverse_quad(
 // points than these lines say.  k_traverse / this kernel for layers 5 % of the diagonal off: F = 199,692 170 /
 // 185 us (400k points), 208 / 244 (600k) and 249 / 327 (1M); 16 such meshes 379 / 485 (100k points each) and 762 /
 // 1178 (300k); 64 of 20,172 triangles 477 / 557 (25k each).  Above kQuadAny points the slots-in-lanes traversal
-// is therefore taken only for points that, looked at (k_point_look), spread over the box of the mesh with the
+// is therefore taken only for points that, looked at (look_at_points), spread over the box of the mesh with the
 // most of them, or are close to its surface for their density.  One mesh's points near the surface: up to
 // kQuadNear * log2(F / 170) of them, as the kernels cross early there (F = 20,172 454 / 435 at 499k points and 484
 // / 495 at 600k; 199,692 834 / 727 at 600k and 979 / 1026 at 1M; 874,800 1502 / 1483 at 1M).  Several meshes': up to
 // the line above (64 of 199,692 triangles, 12k points each near the surface 4780 / 2207, 1 % off 1647 / 836; 16
-// with 300k 5235 / 4904).  The look runs beside the sort: 0 to 12 us of a call that k_traverse then answers in
-// 130 to 250, nothing of longer ones.  (With a fixed stride, ahead of the sort and a copy back it took 25 to 35
-// us, did not look at several meshes and took grids of 128^3 points for layers: F = 750,000 1226 us, 785 now.)
+// with 300k 5235 / 4904).  The look costs 7 to 9 us.  (As a kernel of its own ahead of the sort, with a fixed
+// stride and a copy back, it cost 25 to 35, did not see several meshes, and took grids of 128^3 points for layers:
+// F = 750,000 1226 us, 785 now.)
 //
 // A caller that knows its points to lie along a surface (the orientation probes) has a line of its own,
 // kQuadLayer * cbrt(F), and no look at the points: whole calls of two probes a facet, 0.01 / 1 / 5 / 30 % of
 // the size off the surface, k_traverse 1060 / 818 / 394 / 231 us and this kernel 641 / 604 / 346 / 229 at 479k
 // probes, 1250 / 887 / 398 / 239 and 752 / 711 / 386 / 258 at 569k, 1707 / 1108 / 449 / 271 and 1135 / 981 /
 // 507 / - at 912k: the line lies where no distance loses.
-constexpr double kQuadCross = 24000.0, kQuadSparse = 2.0, kQuadAny = 400000.0, kQuadNear = 73000.0, kQuadLayer = 8000.0;
+constexpr double kQuadCross = 24000.0, kQuadSparse = 2.0, kQuadAny = 450000.0, kQuadNear = 73000.0, kQuadLayer = 8000.0;
 constexpr int64_t kLookLeast = 1 << kLookBits;
 Quads use_quads(const Engine& e, int64_t nQ, int64_t most, int banks, Points where)
 {
@@ -334,9 +334,18 @@ bool quads_near_surface(const Engine& e, int64_t nQ)
     return e.n_meshes > 1 || (double)nQ <= kQuadNear * std::log2((double)e.h_f_off[1] / 170.0);
 }
 
-bool quads_after_look(int cells, int reached)
+// Close to the surface for their density: the last slot's threshold of half of the walks is below kLookNear
+// times the extent^2 of 64 neighbours, 64 times the layer's area over n, with about a cell's mean face of area
+// for each filled cell.
+bool quads_after_look(const Engine& e, int mesh, int64_t n, int cells, const float* last, int walks)
 {
-    return (double)cells >= kSpreadLeast * (double)(1 << kLookBits) || 2 * reached >= kLookWalks;
+    if ((double)cells >= kSpreadLeast * (double)(1 << kLookBits)) return true;
+    const float* inv = &e.h_info[8 * (size_t)mesh + 3];
+    double side[3]; // of a cell: 32 x 16 x 16 of them
+    for (int d = 0; d < 3; ++d) side[d] = inv[d] > 0.0f ? (d == 0 ? 1.0 / 32 : 1.0 / 16) / inv[d] : 0.0;
+    const double face = (side[0] * side[1] + side[1] * side[2] + side[2] * side[0]) / 3.0;
+    const double line = kLookNear * 64.0 * cells * face / (double)n;
+    return walks > 0 && 2 * std::count_if(last, last + walks, [&](float t) { return t <= line; }) >= walks;
 }
 
 // Points per wave: 16, the wave's lanes, or 8 where so few waves run that the longest decides (up to 500

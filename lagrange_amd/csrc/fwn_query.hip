@@ -26,11 +26,13 @@
 // three kernels 3.44 + 0.30 + 0.27 -> 2.05 ms), the grid 3.54 -> 3.52 ms.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstring>
 #include <thread>
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "fwn_eval.h"
 #include "fwn_internal.h"
@@ -69,13 +71,119 @@ __device__ __forceinline__ uint32_t point_key(const float* __restrict__ Q, int64
     return point_key_of(morton30(Q[3 * i], Q[3 * i + 1], Q[3 * i + 2], mi, mi + 3), (uint32_t)m, mesh_bits, first);
 }
 
+// A look at the n points of one mesh, Q[0..n), by the first blocks of the kernel that makes the keys: how many of
+// 2^kLookBits cells of the mesh's box hold one of as many of them, and for kLookWalks points (depth > 0) the
+// threshold of the last slot of a walk from the root of a 4-wide tree, each time into the slot nearest in terms
+// of its threshold (0: the walk ended in a leaf; infinity: the root's slots are far).  Each result is one store
+// to host memory, which holds kLookUnset there before.  A block of 1,024 threads and one more for the walks, or
+// one and four of 256.  Bound: latency of its rounds of loads; the keys' kernel takes 13.7 us with it, 6.5
+// (499,000 points) and 4.8 (600,000) without.  (On a stream of its own beside the sort, 12 us, the calls for it
+// cost the host 10 us, and the stream 300 in an engine's first such call.)
+struct Look {
+    const float* Q = nullptr;
+    int64_t n = 0;
+    const float* minfo = nullptr;
+    const uint32_t* slots = nullptr;
+    int32_t root = -1, root_ns = 0, depth = 0;
+    uint32_t* result = nullptr; // cells, then kLookWalks thresholds
+    int blocks = 0;             // 0: no look
+};
+constexpr uint32_t kLookUnset = 0xFFFFFFFFu;
+__host__ __device__ constexpr int look_blocks(int threads, bool walks) { return 1 + (walks ? 4 * kLookWalks / threads : 0); }
+
+typedef float point3 __attribute__((ext_vector_type(3), aligned(4)));
+__device__ __forceinline__ point3 look_point(const Look& look, uint32_t part)
+{
+    return *reinterpret_cast<const point3*>(look.Q + 3 * look_index(part, kLookBits, look.n));
+}
+
+template <int THREADS>
+__device__ __forceinline__ void look_at_points(const Look& look)
+{
+    const int tid = threadIdx.x, lane = tid & 63;
+    if (blockIdx.x == 0) {
+        __shared__ uint32_t filled[(1 << kLookBits) / 32];
+        __shared__ int32_t part[THREADS / 64];
+        for (int k = tid; k < (1 << kLookBits) / 32; k += THREADS) filled[k] = 0u;
+        __syncthreads();
+        constexpr int kAhead = 4; // points in flight; 8 would take the keys' blocks to 80 registers
+        for (int r = 0; r < (1 << kLookBits) / THREADS; r += kAhead) {
+            point3 q[kAhead];
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k) q[k] = look_point(look, (uint32_t)((r + k) * THREADS + tid));
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k) {
+                const uint32_t c = morton30(q[k].x, q[k].y, q[k].z, look.minfo, look.minfo + 3) >> (30 - kLookBits);
+                atomicOr(&filled[c >> 5], 1u << (c & 31u));
+            }
+        }
+        __syncthreads();
+        int32_t cells = 0;
+        for (int k = tid; k < (1 << kLookBits) / 32; k += THREADS) cells += __popc(filled[k]);
+        for (int o = 32; o > 0; o >>= 1) cells += __shfl_xor(cells, o);
+        if (lane == 0) part[tid >> 6] = cells;
+        __syncthreads();
+        if (tid == 0) {
+            cells = 0;
+            for (int k = 0; k < THREADS / 64; ++k) cells += part[k];
+            __hip_atomic_store(look.result, (uint32_t)cells, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+        return;
+    }
+    // a walk in four lanes, a slot in each
+    const int walk = ((int)blockIdx.x - 1) * (THREADS / 4) + (tid >> 2), s = tid & 3;
+    const point3 w = look_point(look, (uint32_t)walk * ((1u << kLookBits) / kLookWalks));
+    uint32_t e = (uint32_t)look.root << 4 | (uint32_t)look.root_ns; // the same in the walk's four lanes
+    bool on = look.root >= 0;
+    float last = INFINITY;
+    for (int level = 0; level < look.depth && __ballot(on) != 0ull; ++level) {
+        float near = INFINITY, thr = 0.0f; // distance over threshold
+        uint32_t link = FWN_LINK_EMPTY;
+        if (on && s < (int)(e & 15u)) {
+            const uint32_t* slot = look.slots + ((size_t)(e >> 4) * 4 + s) * kSlotWords;
+            const float4 p = *reinterpret_cast<const float4*>(slot); // centre, threshold
+            link = slot[FWN_W_LINK];
+            const float dx = p.x - w.x, dy = p.y - w.y, dz = p.z - w.z;
+            const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+            if (d2 <= p.w && p.w > 0.0f) near = d2 / p.w;
+            thr = p.w;
+        }
+        // the nearest of the four lanes' slots, the lower one of equals
+        float least = INFINITY, best = 0.0f;
+        e = 0u;
+        auto take = [&](auto lane_of_quad) __attribute__((always_inline)) {
+            constexpr int kPerm = lane_of_quad.value * 0x55; // quad_perm: that lane in all four
+            const float d = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(near), kPerm, 0xF, 0xF, true));
+            const uint32_t l = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)link, kPerm, 0xF, 0xF, true);
+            const float t = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(thr), kPerm, 0xF, 0xF, true));
+            const bool nearer = d < least;
+            least = nearer ? d : least;
+            e = nearer ? l : e;
+            best = nearer ? t : best;
+        };
+        take(std::integral_constant<int, 0>{});
+        take(std::integral_constant<int, 1>{});
+        take(std::integral_constant<int, 2>{});
+        take(std::integral_constant<int, 3>{});
+        on = on && least < INFINITY;
+        if (on) last = (int32_t)e < 0 ? 0.0f : best;
+        on = on && (int32_t)e >= 0;
+    }
+    if (s == 0)
+        __hip_atomic_store(look.result + 1 + walk, __float_as_uint(last), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // flags (nullptr: none): the traversal's overflow flag and work counter, cleared on the way
 __global__ __launch_bounds__(QT) void k_query_keys(const float* __restrict__ Q, int64_t nQ,
                                                    const int64_t* __restrict__ q_off, int M, int mesh_bits,
                                                    const float* __restrict__ minfo, uint32_t* __restrict__ keys,
-                                                   int32_t* __restrict__ flags)
+                                                   int32_t* __restrict__ flags, Look look)
 {
-    const int64_t i = (int64_t)blockIdx.x * QT + threadIdx.x;
+    if ((int)blockIdx.x < look.blocks) {
+        look_at_points<QT>(look);
+        return;
+    }
+    const int64_t i = (int64_t)((int)blockIdx.x - look.blocks) * QT + threadIdx.x;
     if (i < 2 && flags) flags[i] = 0;
     if (i < nQ) keys[i] = point_key(Q, nQ, i, q_off, M, mesh_bits, sort24_first(mesh_bits), minfo);
 }
@@ -84,104 +192,28 @@ __global__ __launch_bounds__(QT) void k_query_keys(const float* __restrict__ Q, 
 __global__ __launch_bounds__(1024) void k_query_keys_few(const float* __restrict__ Q, int64_t nQ,
                                                          const int64_t* __restrict__ q_off, int M, int mesh_bits,
                                                          const float* __restrict__ minfo, uint32_t* __restrict__ keys,
-                                                         int32_t* __restrict__ hist, int32_t* __restrict__ flags)
+                                                         int32_t* __restrict__ hist, int32_t* __restrict__ flags,
+                                                         Look look)
 {
+    if ((int)blockIdx.x < look.blocks) {
+        look_at_points<1024>(look);
+        return;
+    }
     __shared__ int32_t cnt[1024];
-    if (blockIdx.x == 0 && threadIdx.x < 2) flags[threadIdx.x] = 0;
+    const int tile = (int)blockIdx.x - look.blocks;
+    if (tile == 0 && threadIdx.x < 2) flags[threadIdx.x] = 0;
     cnt[threadIdx.x] = 0;
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < kFewTile / 1024; ++r) {
-        const int64_t i = (int64_t)blockIdx.x * kFewTile + r * 1024 + threadIdx.x;
+        const int64_t i = (int64_t)tile * kFewTile + r * 1024 + threadIdx.x;
         const bool valid = i < nQ;
         const uint32_t key = valid ? point_key(Q, nQ, i, q_off, M, mesh_bits, 0, minfo) : 0u;
         if (valid) keys[i] = key;
         count_digit(cnt, key >> 12 & 1023u, valid);
     }
     __syncthreads();
-    hist[(int64_t)blockIdx.x * 1024 + threadIdx.x] = cnt[threadIdx.x];
-}
-
-// A look at the n points of one mesh, Q[0..n): how many of 2^kLookBits cells of the mesh's box hold one of as
-// many of them (kSpreadLeast), and how many of kLookWalks points are close to the surface for their density:
-// a walk from the root of a 4-wide tree, each time into the slot nearest in terms of its far threshold, ends
-// in a leaf or in a slot with a threshold below kLookNear times the extent^2 of 64 neighbouring points (64 times
-// the layer's area, about a mean face of a cell for each filled one, over n).  `depth` levels at most, a slot
-// per lane.  The result, with a mark above it, is one store to host memory.  One workgroup, 12 to 16 us on a
-// stream of its own while the points are sorted.
-typedef float point3 __attribute__((ext_vector_type(3), aligned(4)));
-__global__ __launch_bounds__(1024) void k_point_look(const float* __restrict__ Q, int64_t n,
-                                                     const float* __restrict__ minfo,
-                                                     const uint32_t* __restrict__ slots, int32_t root, int32_t root_ns,
-                                                     int depth, uint64_t* __restrict__ result)
-{
-    __shared__ uint32_t filled[(1 << kLookBits) / 32];
-    __shared__ float lasts[kLookWalks]; // per walk: the threshold of its last slot, 0: a leaf
-    __shared__ int32_t part[2][16];
-    const int tid = threadIdx.x, lane = tid & 63;
-    if (tid < (1 << kLookBits) / 32) filled[tid] = 0u;
-    __syncthreads();
-    point3 q[(1 << kLookBits) / 1024];
-#pragma unroll
-    for (int r = 0; r < (1 << kLookBits) / 1024; ++r)
-        q[r] = *reinterpret_cast<const point3*>(Q + 3 * look_index((uint32_t)(r * 1024 + tid), kLookBits, n));
-#pragma unroll
-    for (int r = 0; r < (1 << kLookBits) / 1024; ++r) {
-        const uint32_t c = morton30(q[r].x, q[r].y, q[r].z, minfo, minfo + 3) >> (30 - kLookBits);
-        atomicOr(&filled[c >> 5], 1u << (c & 31u));
-    }
-    if (root >= 0) {
-        constexpr uint32_t kStep = (1u << kLookBits) / kLookWalks;
-        const point3 w = *reinterpret_cast<const point3*>(Q + 3 * look_index((uint32_t)(tid >> 2) * kStep, kLookBits, n));
-        const int s = tid & 3;
-        uint32_t e = (uint32_t)root << 4 | (uint32_t)root_ns; // the same in the walk's four lanes
-        bool on = true;
-        float last = INFINITY; // threshold of the slot entered last
-        for (int level = 0; level < depth && __ballot(on) != 0ull; ++level) {
-            float near = INFINITY, thr = 0.0f; // distance over threshold
-            uint32_t link = FWN_LINK_EMPTY;
-            if (on && s < (int)(e & 15u)) {
-                const uint32_t* slot = slots + ((size_t)(e >> 4) * 4 + s) * kSlotWords;
-                const float4 p = *reinterpret_cast<const float4*>(slot); // centre, threshold
-                link = slot[FWN_W_LINK];
-                const float dx = p.x - w.x, dy = p.y - w.y, dz = p.z - w.z;
-                const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-                if (d2 <= p.w && p.w > 0.0f) near = d2 / p.w;
-                thr = p.w;
-            }
-            const float least = fminf(fminf(near, __shfl_xor(near, 1)), fminf(__shfl_xor(near, 2), __shfl_xor(near, 3)));
-            const uint64_t pick = __ballot(near == least && least < INFINITY) >> (lane & 60) & 15u;
-            const int from = (lane & 60) + (pick ? (int)__builtin_ctzll(pick) : 0);
-            e = (uint32_t)__shfl((int)link, from);
-            thr = __shfl(thr, from);
-            on = on && pick != 0ull;
-            if (on) last = (int32_t)e < 0 ? 0.0f : thr;
-            on = on && (int32_t)e >= 0;
-        }
-        if (s == 0) lasts[tid >> 2] = last;
-    } else if ((tid & 3) == 0) {
-        lasts[tid >> 2] = INFINITY;
-    }
-    __syncthreads();
-    int32_t cells = tid < (1 << kLookBits) / 32 ? __popc(filled[tid]) : 0;
-    for (int o = 32; o > 0; o >>= 1) cells += __shfl_xor(cells, o);
-    if (lane == 0) part[0][tid >> 6] = cells;
-    __syncthreads();
-    cells = 0;
-    for (int k = 0; k < 16; ++k) cells += part[0][k];
-    float side[3]; // of a cell: 32 x 16 x 16 of them
-    for (int d = 0; d < 3; ++d) side[d] = minfo[3 + d] > 0.0f ? (d == 0 ? 1.0f / 32 : 1.0f / 16) / minfo[3 + d] : 0.0f;
-    const float face = (side[0] * side[1] + side[1] * side[2] + side[2] * side[0]) * (1.0f / 3);
-    const float line = kLookNear * 64.0f * (float)cells * face / (float)n;
-    const uint64_t hits = __ballot(tid < kLookWalks && lasts[tid & (kLookWalks - 1)] <= line);
-    if (lane == 0) part[1][tid >> 6] = (int32_t)__popcll(hits);
-    __syncthreads();
-    if (tid == 0) {
-        int32_t walks = 0;
-        for (int k = 0; k < 16; ++k) walks += part[1][k];
-        __hip_atomic_store(result, (uint64_t)1 << 63 | (uint64_t)walks << 32 | (uint64_t)cells, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_SYSTEM);
-    }
+    hist[(int64_t)tile * 1024 + threadIdx.x] = cnt[threadIdx.x];
 }
 
 // One slot's 24 words held in SGPRs (a 16-dword and an 8-dword scalar load issued together at
@@ -644,7 +676,7 @@ void run_queries_pipelined(Engine& e, const float* Q, int64_t nQ, float* omega, 
             uint32_t* kp2 = e.q_keys[1].as<uint32_t>();
             uint32_t* vp2 = e.q_vals[1].as<uint32_t>();
             hipLaunchKernelGGL(k_query_keys, dim3(grid_blocks(ck, QT)), dim3(QT), 0, s, dQ, ck, d_qoff, 1, 0,
-                               e.mesh_info.as<float>(), kp, (int32_t*)nullptr);
+                               e.mesh_info.as<float>(), kp, (int32_t*)nullptr, Look());
             FWN_LAUNCH_CHECK("k_query_keys");
             radix_sort_pairs32(kp, vp, kp2, vp2, ck, 8, 32, true, e.q_hist, e.q_rowsum, s);
             const int64_t nb = (ck + 63) / 64;
@@ -703,7 +735,7 @@ void run_queries_pipelined(Engine& e, const float* Q, int64_t nQ, float* omega, 
 void launch_point_keys(Engine& e, const float* dQ, int64_t nQ, uint32_t* keys, hipStream_t s)
 {
     hipLaunchKernelGGL(k_query_keys, dim3(grid_blocks(nQ, QT)), dim3(QT), 0, s, dQ, nQ, (const int64_t*)nullptr, 1, 0,
-                       e.mesh_info.as<float>(), keys, (int32_t*)nullptr);
+                       e.mesh_info.as<float>(), keys, (int32_t*)nullptr, Look());
     FWN_LAUNCH_CHECK("k_query_keys");
 }
 
@@ -775,7 +807,7 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
     for (int m : order)
         if (qoff[m + 1] - qoff[m] > qoff[most + 1] - qoff[most]) most = m;
     const int64_t n_most = qoff[most + 1] - qoff[most];
-    const Quads choice = small || stats ? Quads::No : use_quads(e, nQ, n_most, banks, where);
+    const Quads choice = small || stats ? Quads::No : use_quads(e, nQ, n_most, banks, where); // Look: no point_order
     bool quad = choice == Quads::Yes; // Quads::Look: known once the points are looked at
     const int bpts = small ? (int)std::min<int64_t>(64, std::max<int64_t>(1, (nQ + 1023) / 1024))
                            : (quad ? quad_points(e, nQ) : 64);
@@ -796,8 +828,8 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
     const size_t meta_b = (offs * off_b + sizeof(int32_t) * M + 15) & ~(size_t)15;
     const size_t in_b = meta_b + (stage_io ? sizeof(float) * 3 * (size_t)nQ : 0);
     const size_t out_b = stage_io ? 16 + (sizeof(float) + 1) * (size_t)nQ : 0; // flags, omega, inside
-    const size_t look_at = (std::max(in_b, out_b) + 15) & ~(size_t)15; // the look's result behind it all
-    char* hs = host_stage(e, look_at + 16);
+    const size_t look_at = (std::max(in_b, out_b) + 15) & ~(size_t)15; // the look's results behind it all
+    char* hs = host_stage(e, look_at + sizeof(uint32_t) * (1 + kLookWalks));
     std::memcpy(hs, qoff.data(), off_b);
     std::memcpy(hs + off_b, boff.data(), off_b);
     if (choice == Quads::Look) std::memcpy(hs + 2 * off_b, boff_quad.data(), off_b);
@@ -854,6 +886,19 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
     FWN_HIP(hipEventRecord(e.ev[0], s));
     int32_t* dflag = e.q_flag.as<int32_t>();
     uint32_t* dwork = reinterpret_cast<uint32_t*>(dflag + 1);
+    Look look;
+    volatile uint32_t* seen = reinterpret_cast<volatile uint32_t*>(hs + look_at);
+    if (choice == Quads::Look) {
+        std::memset(hs + look_at, 0xFF, sizeof(uint32_t) * (1 + kLookWalks));
+        look.Q = dQ + 3 * qoff[most];
+        look.n = n_most;
+        look.minfo = e.mesh_info.as<float>() + 8 * most;
+        look.slots = e.slots.as<uint32_t>();
+        look.root = e.h_roots[2 * most];
+        look.root_ns = e.h_roots[2 * most + 1];
+        look.depth = quads_near_surface(e, nQ) ? std::max(e.max_depth, 1) : 0;
+        look.result = reinterpret_cast<uint32_t*>(hs + look_at);
+    }
     // sorted position -> input index (nullptr: small calls keep the input order)
     const uint32_t* vp = small ? nullptr : point_order;
     if (small || point_order) {
@@ -870,38 +915,41 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
         // a surface, where at most 524,288 points leave little for more bits to order
         if (few_tiles(nQ) <= kFewTiles && mesh_bits <= 8) {
             e.q_hist.reserve(sizeof(int32_t) * 1024 * (size_t)few_tiles(nQ));
-            hipLaunchKernelGGL(k_query_keys_few, dim3(few_tiles(nQ)), dim3(1024), 0, s, dQ, nQ, d_qoff, M, mesh_bits,
-                               e.mesh_info.as<float>(), kp, e.q_hist.as<int32_t>(), dflag);
+            if (choice == Quads::Look) look.blocks = look_blocks(1024, look.depth > 0);
+            hipLaunchKernelGGL(k_query_keys_few, dim3(few_tiles(nQ) + look.blocks), dim3(1024), 0, s, dQ, nQ, d_qoff, M,
+                               mesh_bits, e.mesh_info.as<float>(), kp, e.q_hist.as<int32_t>(), dflag, look);
             FWN_LAUNCH_CHECK("k_query_keys_few");
             sort_few_tiles(kp, kp2, vp2, vals, nQ, e.q_hist.as<int32_t>(), s);
         } else {
-            hipLaunchKernelGGL(k_query_keys, dim3(grid_blocks(nQ, QT)), dim3(QT), 0, s, dQ, nQ, d_qoff, M, mesh_bits,
-                               e.mesh_info.as<float>(), kp, dflag);
+            if (choice == Quads::Look) look.blocks = look_blocks(QT, look.depth > 0);
+            hipLaunchKernelGGL(k_query_keys, dim3(grid_blocks(nQ, QT) + look.blocks), dim3(QT), 0, s, dQ, nQ, d_qoff, M,
+                               mesh_bits, e.mesh_info.as<float>(), kp, dflag, look);
             FWN_LAUNCH_CHECK("k_query_keys");
             radix_sort_pairs32(kp, vals, kp2, vp2, nQ, 8, 32, true, e.q_hist, e.q_rowsum, s);
         }
         vp = vals;
     }
     int quad_bpts = bpts;
-    if (choice == Quads::Look) {
-        volatile uint64_t* word = reinterpret_cast<volatile uint64_t*>(hs + look_at);
-        *word = 0;
-        if (!e.cs_in) FWN_HIP(hipStreamCreateWithFlags(&e.cs_in, hipStreamNonBlocking));
-        FWN_HIP(hipStreamWaitEvent(e.cs_in, e.ev[0], 0)); // the points and the metadata are there
-        hipLaunchKernelGGL(k_point_look, dim3(1), dim3(1024), 0, e.cs_in, dQ + 3 * qoff[most], n_most,
-                           e.mesh_info.as<float>() + 8 * most, e.slots.as<uint32_t>(), e.h_roots[2 * most],
-                           e.h_roots[2 * most + 1], quads_near_surface(e, nQ) ? e.max_depth : 0,
-                           const_cast<uint64_t*>(word));
-        FWN_LAUNCH_CHECK("k_point_look");
-        // the sort is under way; a failed launch ends the wait
-        for (uint32_t spin = 1; *word == 0; ++spin)
-            if ((spin & 255u) == 0u && hipStreamQuery(e.cs_in) != hipErrorNotReady) {
-                FWN_HIP(hipStreamSynchronize(e.cs_in));
-                break;
+    if (choice == Quads::Look) { // its results come while the points are sorted; a failed launch ends the wait
+        const int words = 1 + (look.depth > 0 ? kLookWalks : 0);
+        int k = 0;
+        bool over = false;
+        for (uint32_t spin = 1;; ++spin) {
+            while (k < words && seen[k] != kLookUnset) ++k;
+            if (k == words) break;
+            if (over) fail(FWN_HIP_ERROR, "no result of the look at the points");
+            if ((spin & 255u) == 0u && hipStreamQuery(s) != hipErrorNotReady) {
+                FWN_HIP(hipStreamSynchronize(s));
+                over = true;
             }
-        const uint64_t seen = *word;
-        if (seen == 0) fail(FWN_HIP_ERROR, "no result of the look at the points");
-        quad = quads_after_look((int)(seen & 0xFFFFFFFFu), (int)(seen >> 32 & 0x7FFFFFFFu));
+        }
+        std::atomic_thread_fence(std::memory_order_acquire);
+        float last[kLookWalks];
+        for (int j = 0; j + 1 < words; ++j) {
+            const uint32_t u = seen[1 + j];
+            std::memcpy(last + j, &u, sizeof(u));
+        }
+        quad = quads_after_look(e, most, n_most, (int)seen[0], last, words - 1);
         if (quad) {
             nb = boff_quad[M];
             d_boff += M + 1;
@@ -928,7 +976,7 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
     } else {
         launch_traverse(stats != nullptr, waves, persist, banks, e.width, (unsigned)nblk, s, e.slots.as<uint32_t>(),
                         e.width, e.tris.as<uint32_t>(), e.roots.as<int32_t>(), e.mesh_info.as<float>(), dQ, vp, d_qoff,
-                        d_boff, d_order, M, nb, bpts, e.uneven ? 64 : 0, beta2, dOm, dIn, dSt, dflag, dwork);
+                        d_boff, d_order, M, nb, bpts, e.uneven ? 16 : 0, beta2, dOm, dIn, dSt, dflag, dwork);
         FWN_LAUNCH_CHECK("k_traverse");
     }
     FWN_HIP(hipEventRecord(e.ev[2], s));
@@ -973,7 +1021,7 @@ const uint32_t* sort_points_single(Engine& e, const float* dQ, int64_t nQ)
     uint32_t* kp2 = e.q_keys[1].as<uint32_t>();
     uint32_t* vp2 = e.q_vals[1].as<uint32_t>();
     hipLaunchKernelGGL(k_query_keys, dim3(grid_blocks(nQ, QT)), dim3(QT), 0, s, dQ, nQ, (const int64_t*)nullptr, 1, 0,
-                       e.mesh_info.as<float>(), kp, (int32_t*)nullptr);
+                       e.mesh_info.as<float>(), kp, (int32_t*)nullptr, Look());
     FWN_LAUNCH_CHECK("k_query_keys");
     radix_sort_pairs32(kp, vp, kp2, vp2, nQ, 8, 32, true, e.q_hist, e.q_rowsum, s);
     return vp;

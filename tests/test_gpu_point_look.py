@@ -1,4 +1,4 @@
-"""Which traversal calls above 400,000 points take: slots in lanes for points that spread over the mesh's box
+"""Which traversal calls above 450,000 points take: slots in lanes for points that spread over the mesh's box
 (random, regular grids of powers of two, dense voxel boxes) or, several meshes or few enough points, lie near
 the surface; the scalar-slot one for layers off the surface and boxes far smaller than the mesh.  By the
 kernels that run; the values are those of small calls."""
@@ -46,9 +46,9 @@ POINTS = {"random": (lambda V, F: np.random.default_rng(1).uniform(-1.2, 1.2, (5
           "on the surface": (lambda V, F: layer(V, F, 480000, 0.0, 2), "quad"),
           "on the surface, more": (lambda V, F: layer(V, F, 640000, 0.0, 2), "scalar"),
           "layer": (lambda V, F: layer(V, F, 480000, 0.3, 3), "scalar"),
-          "layer, few": (lambda V, F: layer(V, F, 399999, 0.3, 3), "quad"),
+          "layer, few": (lambda V, F: layer(V, F, 449999, 0.3, 3), "quad"),
           "one place": (lambda V, F: np.full((500000, 3), 0.3, np.float32), "scalar"),
-          "not a number": (lambda V, F: np.full((450000, 3), np.nan, np.float32), "scalar"),
+          "not a number": (lambda V, F: np.full((450001, 3), np.nan, np.float32), "scalar"),
           "past the line": (lambda V, F: np.random.default_rng(1).uniform(-1.2, 1.2, (700001, 3)).astype(np.float32), "scalar")}
 
 
@@ -77,7 +77,7 @@ def test_several_meshes(where, want, first):
     meshes.insert(2, (np.zeros((0, 3), np.float32), np.zeros((0, 3), np.int32)))
     n = [first, 100001, 0, 180003, 200001 - first // 2]
     off = np.concatenate([[0], np.cumsum(n)]).astype(np.int64)
-    assert 400000 < off[-1] < 24000 * np.cbrt(sum(F.shape[0] for _, F in meshes) / 5)
+    assert 450000 < off[-1] < 24000 * np.cbrt(sum(F.shape[0] for _, F in meshes) / 5)
     qs = []
     for k, (V, F) in enumerate(meshes):
         if where == "random" or n[k] == 0:
@@ -97,7 +97,7 @@ def test_several_meshes(where, want, first):
 
 @pytest.mark.parametrize("lo,dims,size,want", [((-40,) * 3, (80, 80, 80), 0.03, "quad"),
                                                ((-40,) * 3, (80, 80, 80), 0.002, "scalar"),
-                                               ((-100, -100, 0), (200, 200, 11), 0.012, "scalar"),
+                                               ((-100, -100, 0), (200, 200, 12), 0.012, "scalar"),
                                                ((-300,) * 3, (80, 80, 80), 0.03, "scalar")])
 def test_voxel_boxes(lo, dims, size, want):
     mesh = W.icosphere(32)
