@@ -455,19 +455,6 @@ __global__ __launch_bounds__(WAVES * 64) void k_traverse(
     }
 }
 
-__global__ __launch_bounds__(256) void k_bruteforce(const uint32_t* __restrict__ tris, int64_t first, int64_t cnt,
-                                                    const float* __restrict__ Q, int64_t nQ,
-                                                    double* __restrict__ out)
-{
-    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    bool valid = i < nQ;
-    float qx = valid ? Q[3 * i] : 0.0f, qy = valid ? Q[3 * i + 1] : 0.0f, qz = valid ? Q[3 * i + 2] : 0.0f;
-    double s = 0.0;
-    for (int64_t t = first; t < first + cnt; ++t)
-        s += tri_f64(reinterpret_cast<const float*>(tris + t * kTriWords), qx, qy, qz);
-    if (valid) out[i] = s;
-}
-
 __global__ void k_zero2(int32_t* a) // overflow flag, work counter
 {
     a[0] = 0;
@@ -1025,28 +1012,6 @@ const uint32_t* sort_points_single(Engine& e, const float* dQ, int64_t nQ)
     FWN_LAUNCH_CHECK("k_query_keys");
     radix_sort_pairs32(kp, vp, kp2, vp2, nQ, 8, 32, true, e.q_hist, e.q_rowsum, s);
     return vp;
-}
-
-void run_bruteforce(Engine& e, const float* Q, int64_t nQ, double* out, bool dev)
-{
-    hipStream_t s = e.stream;
-    if (nQ <= 0) return;
-    const float* dQ = Q;
-    double* dOut = out;
-    if (!dev) {
-        e.q_in.reserve(sizeof(float) * 3 * nQ);
-        e.q_bf.reserve(sizeof(double) * nQ);
-        FWN_HIP(hipMemcpyAsync(e.q_in.p, Q, sizeof(float) * 3 * nQ, hipMemcpyHostToDevice, s));
-        dQ = e.q_in.as<float>();
-        dOut = e.q_bf.as<double>();
-    }
-    // mesh 0's triangles are the first f_off[1] entries of the sorted triangle array
-    const int64_t cnt = e.h_f_off.size() > 1 ? e.h_f_off[1] : 0;
-    hipLaunchKernelGGL(k_bruteforce, dim3(grid_blocks(nQ, 256)), dim3(256), 0, s, e.tris.as<uint32_t>(), (int64_t)0,
-                       cnt, dQ, nQ, dOut);
-    FWN_LAUNCH_CHECK("k_bruteforce");
-    if (!dev) FWN_HIP(hipMemcpyAsync(out, dOut, sizeof(double) * nQ, hipMemcpyDeviceToHost, s));
-    FWN_HIP(hipStreamSynchronize(s));
 }
 
 } // namespace fwn
