@@ -179,8 +179,8 @@ int fwn_destroy(fwn_engine* e);
 /* Solid angle (steradians, as FastWindingNumber::solid_angle) of nQ points Q (nQ x 3 float).
  * inside_out (nullable) receives (omega / (4 pi) > 0.5) evaluated in double, byte per point
  * (FastWindingNumber.cpp:66).  flags: FWN_DEVICE_POINTERS.  Results do not depend on how the
- * points are batched: host calls above 2^21 points are answered in pipelined chunks, calls of at
- * most 2,048 points without the Morton sort. */
+ * points are batched: host calls above 2^21 points are answered in pipelined chunks, calls of few
+ * points (2,048, up to 16,384 of one mesh) without the Morton sort. */
 int fwn_solid_angle(fwn_engine* e, const float* Q, int64_t nQ, float* omega_out, uint8_t* inside_out,
                     int32_t flags);
 

@@ -794,7 +794,9 @@ void run_queries(Engine& e, const float* Q, const int64_t* q_off_host, int64_t n
     for (int m : order)
         if (qoff[m + 1] - qoff[m] > qoff[most + 1] - qoff[most]) most = m;
     const int64_t n_most = qoff[most + 1] - qoff[most];
-    const Quads choice = small || stats ? Quads::No : use_quads(e, nQ, n_most, banks, where); // Look: no point_order
+    // points that come in an order are not looked at (the kernel that makes the keys does)
+    if (point_order && where == Points::Any) where = Points::Close;
+    const Quads choice = small || stats ? Quads::No : use_quads(e, nQ, n_most, banks, where);
     bool quad = choice == Quads::Yes; // Quads::Look: known once the points are looked at
     const int bpts = small ? (int)std::min<int64_t>(64, std::max<int64_t>(1, (nQ + 1023) / 1024))
                            : (quad ? quad_points(e, nQ) : 64);
